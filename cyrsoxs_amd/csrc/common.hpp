@@ -217,7 +217,8 @@ struct ScratchArena {
   void *last_ptr = nullptr;
   hipStream_t stream = nullptr;
   std::vector<std::vector<unsigned char>> keep;
-  std::map<std::pair<uint32_t, int>, void *> tw;  // (length, precision) -> table
+  std::map<std::pair<uint32_t, int>, void *> tw;  // (length, precision) -> twiddle table
+  std::map<std::pair<uint32_t, int>, void *> lf;  // (length, precision) -> any-length transform tables
   // 256-byte-aligned slice of `bytes`, or nullptr when the region is exhausted
   void *carve(size_t bytes);
   bool owns(const void *p) const {

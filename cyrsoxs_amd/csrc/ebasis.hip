@@ -30,6 +30,8 @@
 //   ebasis_angles_kernel sums the chunks, applies the DC replacement, and for every
 //                        angle forms p~ = A(theta) F (A = frame x E coefficients,
 //                        3 x 5, FP64-built) and the Ewald intensity.
+// Grids whose Ny has no compile-time codelet take the band passes of mbasis.hip over
+// the five tensor fields instead of ebasis_yz_kernel.
 //
 // HBM traffic per (energy, k): morphology V (16 M) + Gx write 40 V + Gx read 40 V.
 #include <hip/hip_runtime.h>
@@ -40,8 +42,8 @@
 
 #include "fft.hpp"
 #include "geom.hpp"
-#include "kernels.hpp"
 #include "fftpolicy.hpp"
+#include "kernels.hpp"
 #include "stockham.hpp"
 #include "tensor.hpp"
 #include "xfields.hpp"
@@ -71,11 +73,11 @@ __global__ void __launch_bounds__(256) ebasis_bins_kernel(EwaldGeom g, int32_t *
 // Block = pp columns (kx) x tpp threads, one field, one z chunk.  Per z slice the
 // next slice's loads are issued before the current slice's FFT.
 template <typename T, class F, int NG, bool THREE, int WG>
-__global__ void __launch_bounds__(WG) ebasis_yz_kernel(StagePlan P, YzArgs<T> a) {
+__global__ void __launch_bounds__(WG) ebasis_yz_kernel(YzArgs<T> a) {
   constexpr int E = F::kE;
   extern __shared__ unsigned char smem_raw[];
   cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw);
-  const F fft(P, a.tpp, a.pp, false);
+  const F fft{typename F::Plan{}};
   const uint32_t pp = a.pp, tpp = a.tpp;
   // tile q = (z chunk, field, column group), column group fastest, in XCD order
   const uint32_t groups = (a.nx + pp - 1) / pp;
@@ -316,72 +318,39 @@ bool ct_yz_pp_ok(uint32_t n, uint32_t pp) {
   return (pp == 4 || pp == 8 || pp == 16) && pp * (n / ct_elements(n)) <= 1024;
 }
 
-template <int E> constexpr int rt_yz_wg() { return E <= 8 ? 1024 : 512; }
-
-template <typename T, int NG, bool THREE>
-hipError_t launch_yz_rt_e(uint32_t E, dim3 grid, dim3 block, size_t lds, hipStream_t st, const StagePlan &P,
-                          const YzArgs<T> &a, bool *found) {
-  *found = true;
-#define CYR_YZ(EV)                                                                                              \
-  case EV:                                                                                                      \
-    if constexpr (e_allowed<T>(EV)) {                                                                           \
-      hipLaunchKernelGGL((ebasis_yz_kernel<T, RtFft<T, EV>, NG, THREE, rt_yz_wg<EV>()>), grid, block, lds, st, P, \
-                         a);                                                                                    \
-      return hipGetLastError();                                                                                 \
-    }                                                                                                           \
-    break;
-  switch (E) {
-    CYR_YZ(2)
-    CYR_YZ(3)
-    CYR_YZ(4)
-    CYR_YZ(5)
-    CYR_YZ(6)
-    CYR_YZ(8)
-    CYR_YZ(12)
-    CYR_YZ(16)
-    CYR_YZ(24)
-    default:
-      break;
-  }
-#undef CYR_YZ
-  *found = false;
-  return hipSuccess;
-}
-
 template <typename T, int NG, bool THREE, int N, int PP>
-hipError_t launch_yz_ct_pp(dim3 grid, size_t lds, hipStream_t st, const StagePlan &P, const YzArgs<T> &a) {
+hipError_t launch_yz_ct_pp(dim3 grid, size_t lds, hipStream_t st, const YzArgs<T> &a) {
   using F = typename CtPlan<T, N, false, PP>::type;
   constexpr int WG = PP * F::TPP;
   if constexpr (WG <= 1024) {
-    hipLaunchKernelGGL((ebasis_yz_kernel<T, F, NG, THREE, WG>), grid, dim3(WG), lds, st, P, a);
+    hipLaunchKernelGGL((ebasis_yz_kernel<T, F, NG, THREE, WG>), grid, dim3(WG), lds, st, a);
     return hipGetLastError();
   }
   return hipErrorInvalidValue;
 }
 
 template <typename T, int NG, bool THREE, int N>
-hipError_t launch_yz_ct(dim3 grid, size_t lds, hipStream_t st, const StagePlan &P, const YzArgs<T> &a) {
+hipError_t launch_yz_ct(dim3 grid, size_t lds, hipStream_t st, const YzArgs<T> &a) {
   switch (a.pp) {
-    case 4: return launch_yz_ct_pp<T, NG, THREE, N, 4>(grid, lds, st, P, a);
-    case 8: return launch_yz_ct_pp<T, NG, THREE, N, 8>(grid, lds, st, P, a);
-    default: return launch_yz_ct_pp<T, NG, THREE, N, 16>(grid, lds, st, P, a);
+    case 4: return launch_yz_ct_pp<T, NG, THREE, N, 4>(grid, lds, st, a);
+    case 8: return launch_yz_ct_pp<T, NG, THREE, N, 8>(grid, lds, st, a);
+    default: return launch_yz_ct_pp<T, NG, THREE, N, 16>(grid, lds, st, a);
   }
 }
 
 template <typename T, int NG, bool THREE>
-hipError_t launch_yz_ct_n(uint32_t n, dim3 grid, size_t lds, hipStream_t st, const StagePlan &P, const YzArgs<T> &a,
-                          bool *found) {
+hipError_t launch_yz_ct_n(uint32_t n, dim3 grid, size_t lds, hipStream_t st, const YzArgs<T> &a, bool *found) {
   *found = true;
   switch (n) {
-    case 64: return launch_yz_ct<T, NG, THREE, 64>(grid, lds, st, P, a);
-    case 128: return launch_yz_ct<T, NG, THREE, 128>(grid, lds, st, P, a);
-    case 256: return launch_yz_ct<T, NG, THREE, 256>(grid, lds, st, P, a);
+    case 64: return launch_yz_ct<T, NG, THREE, 64>(grid, lds, st, a);
+    case 128: return launch_yz_ct<T, NG, THREE, 128>(grid, lds, st, a);
+    case 256: return launch_yz_ct<T, NG, THREE, 256>(grid, lds, st, a);
     case 384:
-      if constexpr (e_allowed<T>(12)) return launch_yz_ct<T, NG, THREE, 384>(grid, lds, st, P, a);
+      if constexpr (sizeof(T) == 4) return launch_yz_ct<T, NG, THREE, 384>(grid, lds, st, a);
       break;
-    case 512: return launch_yz_ct<T, NG, THREE, 512>(grid, lds, st, P, a);
-    case 1024: return launch_yz_ct<T, NG, THREE, 1024>(grid, lds, st, P, a);
-    case 2048: return launch_yz_ct<T, NG, THREE, 2048>(grid, lds, st, P, a);
+    case 512: return launch_yz_ct<T, NG, THREE, 512>(grid, lds, st, a);
+    case 1024: return launch_yz_ct<T, NG, THREE, 1024>(grid, lds, st, a);
+    case 2048: return launch_yz_ct<T, NG, THREE, 2048>(grid, lds, st, a);
     default: break;
   }
   *found = false;
@@ -396,8 +365,6 @@ uint32_t yz_chunks(uint32_t nx, uint32_t nz, uint32_t pp, uint32_t target_blocks
   if (nch < 1) nch = 1;
   return nch > nz ? nz : nch;
 }
-
-uint32_t yz_wg_of(uint32_t E) { return E <= 8 ? 1024u : 512u; }
 
 }  // namespace
 
@@ -418,27 +385,27 @@ void ebasis_set_yz_tuning(uint32_t nx, uint32_t ny, uint32_t nz, int precision, 
   else g_tune[std::make_tuple(nx, ny, nz, precision)] = t;
 }
 
-bool ebasis_supported(uint32_t nx, uint32_t ny, uint32_t nz, int precision) {
-  StagePlan P;
-  uint32_t lcm;
-  const size_t cs = precision == CYR_FP64 ? 16 : 8;
-  const uint32_t ecap = precision == CYR_FP64 ? 8 : 16;
-  const size_t lds = device_max_lds();
-  if (nx < 2 || ny < 2 || nz > 0xffffu) return false;
-  if (!ct_usable(nx, precision)) {  // run-time X plan: one row per <= 256 threads
-    if (!make_stage_plan(nx, P, lcm)) return false;
-    const uint32_t ex = choose_e(nx, lcm, 256, ecap);
-    if (!e_instantiated(ex, precision) || nx / ex > 256) return false;
-    const size_t pp = 256 / (nx / ex);
-    if (pp * nx * cs > lds) return false;  // row tile
+bool ebasis_yz_supported(uint32_t ny, uint32_t nz, int precision) {
+  // LDS: tile + (3D) Y and z twiddles
+  const size_t cs = precision == CYR_FP64 ? 16 : 8, tw = nz > 1 ? ((size_t)ny + nz) * cs : 0;
+  return ct_usable(ny, precision) && (size_t)ct_yz_pp_of(ny) * ny * cs + tw <= device_max_lds();
+}
+
+bool fused_supported(uint32_t nx, uint32_t ny, uint32_t nz, int precision) {
+  if (nx < 2 || ny < 2 || nz > 0xffffu || nx > 0xfffeu) return false;
+  // sides below 8 with a prime factor above 5: nothing to gain on grids this small
+  for (uint32_t n : {nx, ny, nz}) {
+    uint32_t r = n;
+    for (uint32_t p : {2u, 3u, 5u})
+      while (r % p == 0) r /= p;
+    if (n < 8 && r != 1) return false;
   }
-  // Y kernel LDS: tile + (3D) Y and z twiddles; the run-time plan can narrow to one column
-  const size_t tw = nz > 1 ? ((size_t)ny + nz) * cs : 0;
-  if (ct_usable(ny, precision) && (size_t)ct_yz_pp_of(ny) * ny * cs + tw <= lds) return true;
-  if (!make_stage_plan(ny, P, lcm)) return false;
-  const uint32_t ey = choose_e(ny, lcm, yz_wg_of(lcm), ecap);
-  if (!e_instantiated(ey, precision) || ny / ey > yz_wg_of(ey)) return false;
-  return (size_t)ny * cs + tw <= lds;
+  LfPlan P;
+  LfShape s;
+  uint32_t e;
+  if (!ct_usable(nx, precision) && !(lf_plan(nx, precision, P) && lf_x_shape(P, precision, s, e))) return false;
+  if (!ct_usable(ny, precision) && !(lf_plan(ny, precision, P) && lf_cols_shape(P, precision, 16, true, s))) return false;
+  return nz == 1 || mbasis_zband_supported(nz, precision);
 }
 
 uint32_t ebasis_max_chunks(uint32_t nx, uint32_t ny, uint32_t nz, int precision) {
@@ -455,62 +422,28 @@ cyr_status launch_ebasis_bins(const EwaldGeom &g, int32_t *kzt, hipStream_t st) 
   return CYR_OK;
 }
 
-template <typename T>
-cyr_status launch_ebasis_polx(PolxArgs<T> a, const void *vox, int storage, int morph, bool hann, hipStream_t st) {
-  return launch_xfields<T, kXTensor>(a, vox, storage, morph, hann, st);
-}
-
 template <typename T> cyr_status ebasis_yz_plan(YzArgs<T> &a, uint32_t target_blocks) {
-  StagePlan P;
-  uint32_t lcm;
-  if (!make_stage_plan(a.ny, P, lcm)) return fail(CYR_E_UNSUPPORTED, "E-basis: Ny must be 2^a 3^b 5^c");
   const int prec = sizeof(T) == 8 ? CYR_FP64 : CYR_FP32;
   const size_t tw = a.nz > 1 ? ((size_t)a.nz + a.ny) * sizeof(cx<T>) : 0;
-  auto lds_of = [&](uint32_t q) { return (size_t)q * a.ny * sizeof(cx<T>) + tw; };
   // explicit arguments win over the tuning table, which wins over the defaults
   const YzTuning tune = ebasis_yz_tuning(a.nx, a.ny, a.nz, prec);
   if (!target_blocks) target_blocks = tune.target_blocks ? tune.target_blocks : kYzTargetBlocks;
   const uint32_t want_pp = a.pp ? a.pp : tune.columns;
-  a.ct = 0;
-  if (!a.e && ct_usable(a.ny, prec)) {
-    const uint32_t pp = ct_yz_pp_ok(a.ny, want_pp) ? want_pp : ct_yz_pp_of(a.ny);
-    if (lds_of(pp) <= device_max_lds()) {
-      a.ct = 1;
-      a.e = ct_elements(a.ny);
-      a.pp = pp;
-      a.tpp = a.ny / a.e;
-    }
-  }
-  if (!a.ct) {
-    const uint32_t ecap = sizeof(T) == 8 ? 8 : 16;
-    uint32_t pp = want_pp ? want_pp : 16;
-    uint32_t E = a.e ? a.e : choose_e(a.ny, lcm, yz_wg_of(lcm) / pp, ecap);
-    if (E % lcm != 0 || a.ny % E != 0 || !e_instantiated(E, prec)) E = lcm;
-    const uint32_t tpp = a.ny / E;
-    const uint32_t wg = yz_wg_of(E);
-    while (pp > 1 && (lds_of(pp) > device_max_lds() || pp * tpp > wg)) pp /= 2;
-    if (lds_of(pp) > device_max_lds() || pp * tpp > wg) return fail(CYR_E_UNSUPPORTED, "E-basis: column does not fit");
-    a.e = E;
-    a.tpp = tpp;
-    a.pp = pp;
-  }
+  if (!ct_usable(a.ny, prec)) return fail(CYR_E_UNSUPPORTED, "E-basis: Ny has no compile-time plan");
+  a.pp = ct_yz_pp_ok(a.ny, want_pp) ? want_pp : ct_yz_pp_of(a.ny);
+  a.tpp = a.ny / ct_elements(a.ny);
+  if ((size_t)a.pp * a.ny * sizeof(cx<T>) + tw > device_max_lds())
+    return fail(CYR_E_UNSUPPORTED, "E-basis: column does not fit");
   if (!a.zchunk) a.zchunk = ceil_div(a.nz, yz_chunks(a.nx, a.nz, a.pp, target_blocks));
   a.nchunks = ceil_div(a.nz, a.zchunk);
   return CYR_OK;
 }
 
 template <typename T> cyr_status launch_ebasis_yz(YzArgs<T> a, int ng, hipStream_t st) {
-  StagePlan P;
-  uint32_t lcm;
-  // (the run-time plan's elements per thread are a multiple of its radix lcm; a
-  // compile-time plan has its own radix sequence)
-  if (!make_stage_plan(a.ny, P, lcm) || !a.e || !a.pp || !a.tpp || !a.zchunk || a.ny % a.e != 0 ||
-      (!a.ct && a.e % lcm != 0) || a.tpp != a.ny / a.e)
-    return fail(CYR_E_INVALID, "E-basis: Y plan missing (call ebasis_yz_plan)");
   const int prec = sizeof(T) == 8 ? CYR_FP64 : CYR_FP32;
-  if (a.ct && (!ct_usable(a.ny, prec) || a.e != ct_elements(a.ny) || !ct_yz_pp_ok(a.ny, a.pp)))
+  if (!a.pp || !a.tpp || !a.zchunk) return fail(CYR_E_INVALID, "E-basis: Y plan missing (call ebasis_yz_plan)");
+  if (!ct_usable(a.ny, prec) || a.tpp != a.ny / ct_elements(a.ny) || !ct_yz_pp_ok(a.ny, a.pp))
     return fail(CYR_E_INVALID, "E-basis: inconsistent compile-time Y plan");
-  if (!a.ct && a.pp * a.tpp > yz_wg_of(a.e)) return fail(CYR_E_INVALID, "E-basis: Y block larger than its launch bound");
   const bool three = a.nz > 1;
   if (three && (!a.twz || !a.kzt)) return fail(CYR_E_INVALID, "E-basis: z tables missing");
   if (three && a.nz > 0xffffu) return fail(CYR_E_UNSUPPORTED, "E-basis: Nz above 65535");
@@ -519,21 +452,15 @@ template <typename T> cyr_status launch_ebasis_yz(YzArgs<T> a, int ng, hipStream
   a.twy = twiddles<T>(a.ny, &s);
   if (!a.twy) return s;
   const uint32_t groups = ceil_div(a.nx, a.pp);
-  const dim3 grid(xcd_grid((uint64_t)groups * kEbFields * a.nchunks)), block(a.pp * a.tpp);
+  const dim3 grid(xcd_grid((uint64_t)groups * kEbFields * a.nchunks));
   const size_t lds =
       (size_t)a.pp * a.ny * sizeof(cx<T>) + (three ? ((size_t)a.nz + a.ny) * sizeof(cx<T>) : 0);
   if (lds > device_max_lds()) return fail(CYR_E_UNSUPPORTED, "E-basis: Y tile does not fit in LDS");
   bool found = false;
   hipError_t e;
-  if (a.ct) {
-    if (!three) e = launch_yz_ct_n<T, 1, false>(a.ny, grid, lds, st, P, a, &found);
-    else if (ng == 2) e = launch_yz_ct_n<T, 2, true>(a.ny, grid, lds, st, P, a, &found);
-    else e = launch_yz_ct_n<T, 1, true>(a.ny, grid, lds, st, P, a, &found);
-  } else {
-    if (!three) e = launch_yz_rt_e<T, 1, false>(a.e, grid, block, lds, st, P, a, &found);
-    else if (ng == 2) e = launch_yz_rt_e<T, 2, true>(a.e, grid, block, lds, st, P, a, &found);
-    else e = launch_yz_rt_e<T, 1, true>(a.e, grid, block, lds, st, P, a, &found);
-  }
+  if (!three) e = launch_yz_ct_n<T, 1, false>(a.ny, grid, lds, st, a, &found);
+  else if (ng == 2) e = launch_yz_ct_n<T, 2, true>(a.ny, grid, lds, st, a, &found);
+  else e = launch_yz_ct_n<T, 1, true>(a.ny, grid, lds, st, a, &found);
   if (e != hipSuccess) return hip_fail(e, "ebasis_yz_kernel", __FILE__, __LINE__);
   if (!found) return fail(CYR_E_UNSUPPORTED, "E-basis: no Y kernel for this length");
   return CYR_OK;
@@ -558,7 +485,6 @@ template <typename T> cyr_status launch_ebasis_angles(const AnglesArgs<T> &a, in
 }
 
 #define CYR_INST(T)                                                                                           \
-  template cyr_status launch_ebasis_polx<T>(PolxArgs<T>, const void *, int, int, bool, hipStream_t);        \
   template cyr_status ebasis_yz_plan<T>(YzArgs<T> &, uint32_t);                                              \
   template cyr_status launch_ebasis_yz<T>(YzArgs<T>, int, hipStream_t);                                      \
   template cyr_status launch_ebasis_dc<T>(const DcArgs<T> &, hipStream_t);                                   \

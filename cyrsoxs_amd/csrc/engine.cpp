@@ -532,6 +532,10 @@ cyr_status cyr_engine_submit(cyr_engine eng, const cyr_sim_desc *desc, const voi
   r->vox = voxels;
   r->out = out;
   r->footprint = cyr_footprint_bytes(&r->desc);
+  if (r->footprint > e.budget && plain_fallback(&r->desc, g)) {
+    r->desc.pipeline = CYR_PIPE_PLAIN;
+    r->footprint = cyr_footprint_bytes(&r->desc);
+  }
   r->t_submit = Clock::now();
   std::lock_guard<std::mutex> lk(e.mu);
   if (e.stop) return fail(CYR_E_INVALID, "engine is shutting down");

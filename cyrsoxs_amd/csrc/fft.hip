@@ -9,15 +9,17 @@
 //     pencil are consecutive lanes (row loads are unit-stride); for the strided
 //     Y/Z axes the lanes run across `pp` adjacent pencils (each element load is a
 //     pp*sizeof(complex) contiguous segment).
-//   * Each thread holds E elements in registers; every Stockham stage is
-//     radix R in {2,3,4,5,8} with E/R butterflies per thread.  Stage 0 reads
-//     straight from HBM and the last stage writes straight to HBM (both in the
-//     Stockham access order, which is coalesced); intermediate stages go through
-//     LDS.  Each element is read once and written once per pass.
+//   * The first stage's butterflies load from HBM, the stages exchange through LDS, and
+//     the last stage's butterflies store to HBM: each element is read once and written
+//     once per pass.  Lengths 64-2048 with a compile-time codelet run it (fftpolicy.hpp);
+//     every other length runs the any-length transform (lfft.hpp).
 //   * Twiddles come from a per-length table generated in FP64 on the host.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
+#include <complex>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -41,123 +43,12 @@ struct PassArgs {
   uint32_t outer_count;
   uint32_t groups;  // ceil(inner_count / pp)
   uint32_t pp;
-  uint32_t tpp;
   double2 *dcz;        // non-null: the Y pass adds the DC-neighbour partial sums (FftDc)
-  const void *dc_twz;  // Z twiddles of those sums (null in 2D)
+  const void *dc_twy;  // Y and Z twiddles of those sums (twz null in 2D)
+  const void *dc_twz;
   uint32_t dc_nz;
   const uint32_t *span;  // Y pass: per output row, the shifted x range it writes (null: all)
 };
-
-// ---- one Stockham stage ------------------------------------------------------
-//
-// Butterfly j (0 <= j < n/R) of a stage with sub-transform length Ls reads
-// x[j + r n/R], multiplies by W_{Ls R}^{r (j mod Ls)}, does an R-point DFT and
-// writes y[(j / Ls) Ls R + (j mod Ls) + r Ls].
-
-template <typename T, int E, int R, bool CONTIG>
-__device__ inline void run_stage(cx<T> (&v)[E], const StagePlan &P, uint32_t s, bool first, bool last,
-                                 uint32_t t, uint32_t p, const PassArgs &A, cx<T> *gbase, bool active,
-                                 cx<T> *lds, uint32_t lpitch, const cx<T> *__restrict__ tw) {
-  constexpr int NB = E / R;
-  const uint32_t n = P.n;
-  const uint32_t m = n / R;
-  const uint32_t Ls = P.ls[s];
-  const uint32_t tstep = P.tstep[s];
-  const uint32_t tpp = A.tpp;
-  // ---- gather inputs
-#pragma unroll
-  for (int b = 0; b < NB; b++) {
-    const uint32_t j = t + b * tpp;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const uint32_t idx = j + r * m;
-      if (first) {
-        v[b * R + r] = active ? gbase[(uint64_t)idx * A.elem_stride] : mk<T>(0, 0);
-      } else {
-        v[b * R + r] = CONTIG ? lds[p * lpitch + idx] : lds[idx * lpitch + p];
-      }
-    }
-  }
-  if (!first) __syncthreads();
-  // ---- twiddle and butterfly
-#pragma unroll
-  for (int b = 0; b < NB; b++) {
-    const uint32_t j = t + b * tpp;
-    const uint32_t k = j % Ls;
-    if (k != 0) {
-      if (last && tw_blocks<T>() == 2) {  // finest twiddles: compensated (hi + lo)
-#pragma unroll
-        for (int r = 1; r < R; r++) v[b * R + r] = cmul_tw<T>(v[b * R + r], tw, n, r * k * tstep);
-      } else {
-#pragma unroll
-        for (int r = 1; r < R; r++) v[b * R + r] = cmul<T>(v[b * R + r], tw[r * k * tstep]);
-      }
-    }
-    bfly<T, R>(&v[b * R]);
-  }
-  // ---- scatter outputs
-#pragma unroll
-  for (int b = 0; b < NB; b++) {
-    const uint32_t j = t + b * tpp;
-    const uint32_t k = j % Ls;
-    const uint32_t o0 = (j / Ls) * Ls * R + k;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const uint32_t o = o0 + r * Ls;
-      if (last) {
-        if (active) gbase[(uint64_t)o * A.elem_stride] = v[b * R + r];
-      } else {
-        if (CONTIG) lds[p * lpitch + o] = v[b * R + r];
-        else lds[o * lpitch + p] = v[b * R + r];
-      }
-    }
-  }
-  if (!last) __syncthreads();
-}
-
-template <typename T, int E, bool CONTIG>
-__global__ void __launch_bounds__(1024) fft_pencil_kernel(StagePlan P, PassArgs A,
-                                                          const cx<T> *__restrict__ tw) {
-  extern __shared__ unsigned char smem_raw[];
-  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw);
-  const uint32_t tid = threadIdx.x;
-  uint32_t t, p;
-  if (CONTIG) {
-    t = tid % A.tpp;
-    p = tid / A.tpp;
-  } else {
-    p = tid % A.pp;
-    t = tid / A.pp;
-  }
-  const uint32_t g = blockIdx.x % A.groups;
-  const uint32_t o = blockIdx.x / A.groups;
-  const uint32_t pencil = g * A.pp + p;
-  const bool active = pencil < A.inner_count;
-  cx<T> *gbase = reinterpret_cast<cx<T> *>(A.vol[blockIdx.y]) + (uint64_t)pencil * A.inner_stride +
-                 (uint64_t)o * A.outer_stride;
-  const uint32_t lpitch = CONTIG ? P.n : A.pp;
-  cx<T> v[E];
-  for (uint32_t s = 0; s < P.nstages; s++) {
-    const bool first = s == 0, last = s + 1 == P.nstages;
-    switch (P.radix[s]) {
-      case 2:
-        if constexpr (E % 2 == 0) run_stage<T, E, 2, CONTIG>(v, P, s, first, last, t, p, A, gbase, active, lds, lpitch, tw);
-        break;
-      case 3:
-        if constexpr (E % 3 == 0) run_stage<T, E, 3, CONTIG>(v, P, s, first, last, t, p, A, gbase, active, lds, lpitch, tw);
-        break;
-      case 4:
-        if constexpr (E % 4 == 0) run_stage<T, E, 4, CONTIG>(v, P, s, first, last, t, p, A, gbase, active, lds, lpitch, tw);
-        break;
-      case 5:
-        if constexpr (E % 5 == 0) run_stage<T, E, 5, CONTIG>(v, P, s, first, last, t, p, A, gbase, active, lds, lpitch, tw);
-        break;
-      default:
-        if constexpr (E % 8 == 0) run_stage<T, E, 8, CONTIG>(v, P, s, first, last, t, p, A, gbase, active, lds, lpitch, tw);
-        break;
-    }
-  }
-}
 
 // Compile-time codelet pass (lengths with a CtPlan): pencils held in registers,
 // stages exchanged through LDS with immediate offsets.  Contiguous pencils (X)
@@ -229,7 +120,7 @@ __global__ void __launch_bounds__(WG) fft_ct_kernel(PassArgs A, const cx<T> *__r
             A.dc_nz > 1 ? 2.0 * tw_cos<T>(reinterpret_cast<const cx<T> *>(A.dc_twz), A.dc_nz, o) : 0.0;
 #pragma unroll
         for (int i = 0; i < E; i++) {
-          const double w = which == 0 ? 2.0 * tw_cos<T>(tw, N, F::in_pos(t, i)) + cz : 1.0;
+          const double w = which == 0 ? 2.0 * tw_cos<T>(reinterpret_cast<const cx<T> *>(A.dc_twy), N, F::in_pos(t, i)) + cz : 1.0;
           sr += w * (double)v[i].x;
           si += w * (double)v[i].y;
         }
@@ -291,7 +182,6 @@ hipError_t launch_ct_n(bool contig, uint32_t nc, PassArgs &A, hipStream_t stream
     using F = typename CtPlan<T, N, true, 1>::type;
     constexpr int WG = TPP <= 64 ? 64 : TPP;
     A.pp = WG / TPP;
-    A.tpp = TPP;
     A.groups = (A.inner_count + A.pp - 1) / A.pp;
     const uint64_t blocks = (uint64_t)A.groups * A.outer_count;
     if (blocks > 0x7fffffffull) return hipErrorInvalidConfiguration;
@@ -302,7 +192,6 @@ hipError_t launch_ct_n(bool contig, uint32_t nc, PassArgs &A, hipStream_t stream
     using F = typename CtPlan<T, N, false, PP>::type;
     constexpr int WG = PP * TPP;
     A.pp = PP;
-    A.tpp = TPP;
     A.groups = (A.inner_count + PP - 1) / PP;
     A.nvol = nc;
     const uint64_t tiles = (uint64_t)A.groups * A.outer_count * nc;
@@ -334,8 +223,116 @@ hipError_t launch_ct(uint32_t n, bool contig, uint32_t nc, PassArgs &A, hipStrea
   return hipSuccess;
 }
 
-// Direct O(n^2) DFT of each pencil for lengths with prime factors > 5: the
-// pencil is staged in LDS, then every thread produces outputs.
+// Any-length pass (lfft.hpp): rows (CONTIG) or tiles of pp columns, tpp threads per
+// pencil.  In place: a block owns whole pencils, and its first stage has read every
+// element before its last stage writes (a barrier lies between them; a one-stage
+// transform's butterfly is the whole pencil).  DC sums and row spans as in
+// fft_ct_kernel.
+struct AnyShape {
+  uint32_t tpp, lpp, pitch, pad;
+};
+
+template <typename T, bool CONTIG> struct AnyIn {
+  const cx<T> *gp;
+  uint64_t es;
+  __device__ inline cx<T> load(uint32_t e, uint32_t r, uint32_t q) const {
+    if constexpr (CONTIG) return gp[e + r * q];
+    else return stream_load<T>(gp + e * es + r * (q * es));
+  }
+};
+
+// TAB: the tables are in LDS (false: the longest pencils, read from memory).
+template <typename T, bool CONTIG, bool TAB>
+__global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<T> tb, AnyShape sh, PassArgs A) {
+  extern __shared__ unsigned char smem_raw[];
+  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw);
+  uint32_t t, p, tile = blockIdx.x, vol = blockIdx.y;
+  if constexpr (CONTIG) {
+    t = threadIdx.x % sh.tpp;
+    p = threadIdx.x / sh.tpp;
+  } else {
+    const uint32_t q = xcd_tile(blockIdx.x, gridDim.x);
+    const uint32_t per_vol = A.groups * A.outer_count;
+    if (q >= per_vol * A.nvol) return;  // grid padding: the whole block leaves before any barrier
+    p = threadIdx.x & (A.pp - 1);
+    t = threadIdx.x >> sh.lpp;
+    vol = q / per_vol;
+    tile = q % per_vol;
+  }
+  const uint32_t g = tile % A.groups, o = tile / A.groups;
+  const uint32_t pencil = g * A.pp + p;
+  const bool active = pencil < A.inner_count;
+  // (idle pencils read pencil 0 and write nothing)
+  cx<T> *gp = reinterpret_cast<cx<T> *>(A.vol[vol]) + (uint64_t)o * A.outer_stride +
+              (uint64_t)(active ? pencil : 0) * A.inner_stride;
+  LfLds<T> tab{tb.tw, tb.pos};
+  cx<T> *after = lds + (CONTIG ? A.pp * sh.pitch : tb.m << sh.lpp);
+  const uint32_t *span = nullptr;
+  if constexpr (TAB) {
+    tab = lf_stage_tables<T>(tb, after);
+    if (!CONTIG && A.span) {
+      uint32_t *ls = reinterpret_cast<uint32_t *>(reinterpret_cast<unsigned char *>(after) +
+                                                  lf_lds_tables<T>(tb.m, tb.nlast));
+      for (uint32_t i = threadIdx.x; i < tb.n; i += blockDim.x) ls[i] = A.span[i];
+      span = ls;
+    }
+    lds_sync();
+  }
+  if constexpr (!CONTIG) {
+    // DC-neighbour sums (fft_ct_kernel has the formula) of columns 0, 1 and Nx - 1, in the
+    // blocks that hold them: one more read of those lines, ahead of the transform's own
+    if (A.dcz && (g == 0 || g == A.groups - 1)) {
+      const bool mine = active && (pencil <= 1 || pencil == A.inner_count - 1);
+      const uint32_t which = pencil <= 1 ? pencil : 2;
+      double sr = 0, si = 0;
+      if (mine) {
+        const double cz =
+            A.dc_nz > 1 ? 2.0 * tw_cos<T>(reinterpret_cast<const cx<T> *>(A.dc_twz), A.dc_nz, o) : 0.0;
+        for (uint32_t e = t; e < tb.n; e += sh.tpp) {
+          const cx<T> v = gp[e * A.elem_stride];
+          const double w =
+              which == 0 ? 2.0 * tw_cos<T>(reinterpret_cast<const cx<T> *>(A.dc_twy), tb.n, e) + cz : 1.0;
+          sr += w * (double)v.x;
+          si += w * (double)v.y;
+        }
+      }
+      for (uint32_t off = A.pp; off < 64; off <<= 1) {
+        sr += __shfl_xor(sr, (int)off);
+        si += __shfl_xor(si, (int)off);
+      }
+      if (mine && (threadIdx.x & 63) < A.pp)
+        A.dcz[(((uint64_t)vol * A.dc_nz + o) * 3 + which) * (blockDim.x / 64) + threadIdx.x / 64] =
+            make_double2(sr, si);
+    }
+  }
+  AnyIn<T, CONTIG> in{gp, A.elem_stride};
+  // the line's shifted x range (see fft_ct_kernel)
+  const uint32_t n = A.inner_count, m = n / 2;
+  const uint32_t x0 = g * A.pp, x1 = (x0 + A.pp < n ? x0 + A.pp : n) - 1;
+  const bool lo_part = x0 <= m, hi_part = x1 > m;
+  const uint32_t a0 = m - (x1 < m ? x1 : m), a1 = m - x0;
+  const uint32_t b0 = n + m - x1, b1 = n + m - (x0 > m + 1 ? x0 : m + 1);
+  auto out = [&](uint32_t k0, uint32_t r, uint32_t dk, cx<T> v) {
+    const uint32_t k = k0 + r * dk;
+    bool keep = active;
+    if constexpr (!CONTIG && TAB) {
+      if (A.span) {
+        const uint32_t sp = span[k], lo = sp & 0xffffu, hi = sp >> 16;
+        keep = keep && lo <= hi && ((lo_part && a0 <= hi && a1 >= lo) || (hi_part && b0 <= hi && b1 >= lo));
+      }
+    }
+    if (keep) {
+      if constexpr (CONTIG) gp[k] = v;
+      else gp[k0 * in.es + r * (dk * in.es)] = v;
+    }
+  };
+  if constexpr (CONTIG) lf_run<false, T>(tb, tab, lds, LfRow{p * sh.pitch, sh.pad}, t, sh.tpp, in, out);
+  else lf_run<false, T>(tb, tab, lds, LfCols{sh.lpp, p}, t, sh.tpp, in, out);
+}
+
+// Direct O(n^2) DFT of each pencil for lengths beyond the any-length tile (e.g. a
+// large prime whose convolution does not fit in LDS): the pencil is staged in LDS,
+// then every thread produces outputs.
 template <typename T>
 __global__ void __launch_bounds__(256) dft_pencil_kernel(uint32_t n, PassArgs A, const cx<T> *__restrict__ tw) {
   extern __shared__ unsigned char smem_raw[];
@@ -362,65 +359,11 @@ __global__ void __launch_bounds__(256) dft_pencil_kernel(uint32_t n, PassArgs A,
 
 // ---- host-side planning ------------------------------------------------------
 
-struct Factoring {
-  bool ok = false;
-  std::vector<uint32_t> radices;
-  uint32_t lcm = 1;
-};
-
-Factoring factor(uint32_t n) {
-  Factoring f;
-  uint32_t r = n, a = 0, b = 0, c = 0;
-  while (r % 2 == 0) { r /= 2; a++; }
-  while (r % 3 == 0) { r /= 3; b++; }
-  while (r % 5 == 0) { r /= 5; c++; }
-  if (r != 1) return f;
-  while (a >= 3) { f.radices.push_back(8); a -= 3; }
-  uint32_t p2 = 1;
-  for (uint32_t rr : f.radices) p2 = rr > p2 ? rr : p2;
-  if (a == 2) { f.radices.push_back(4); p2 = p2 > 4 ? p2 : 4; }
-  if (a == 1) { f.radices.push_back(2); p2 = p2 > 2 ? p2 : 2; }
-  for (uint32_t i = 0; i < b; i++) f.radices.push_back(3);
-  for (uint32_t i = 0; i < c; i++) f.radices.push_back(5);
-  f.lcm = p2 * (b ? 3 : 1) * (c ? 5 : 1);
-  f.ok = f.radices.size() <= (size_t)kMaxStages;
-  return f;
-}
-
 std::mutex g_mu;
 std::map<std::tuple<int, uint32_t, int>, DeviceBuffer> g_tw;  // (device, n, precision)
-std::map<std::tuple<uint32_t, int, int>, FftShape> g_shapes;   // (n, contig, precision)
+std::map<std::tuple<int, uint32_t, int>, DeviceBuffer> g_lf;  // (device, n, precision): lfft.hpp tables
 
 template <typename T> constexpr int prec_of() { return sizeof(T) == 8 ? CYR_FP64 : CYR_FP32; }
-
-template <typename T, bool CONTIG>
-hipError_t launch_e(uint32_t E, dim3 grid, dim3 block, size_t lds, hipStream_t st, const StagePlan &P,
-                    const PassArgs &A, const cx<T> *tw, bool *found) {
-  *found = true;
-#define CYR_FFT_CASE(EV)                                                                     \
-  case EV:                                                                                   \
-    hipLaunchKernelGGL((fft_pencil_kernel<T, EV, CONTIG>), grid, block, lds, st, P, A, tw); \
-    return hipGetLastError();
-  switch (E) {
-    CYR_FFT_CASE(2)
-    CYR_FFT_CASE(3)
-    CYR_FFT_CASE(4)
-    CYR_FFT_CASE(5)
-    CYR_FFT_CASE(6)
-    CYR_FFT_CASE(8)
-    CYR_FFT_CASE(10)
-    CYR_FFT_CASE(12)
-    CYR_FFT_CASE(16)
-    CYR_FFT_CASE(20)
-    CYR_FFT_CASE(24)
-    CYR_FFT_CASE(32)
-    CYR_FFT_CASE(40)
-    default:
-      *found = false;
-      return hipSuccess;
-  }
-#undef CYR_FFT_CASE
-}
 
 size_t max_lds_bytes() {
   static size_t v = 0;
@@ -436,23 +379,6 @@ size_t max_lds_bytes() {
 }
 
 }  // namespace
-
-bool make_stage_plan(uint32_t n, StagePlan &P, uint32_t &lcm) {
-  const Factoring f = factor(n);
-  if (!f.ok) return false;
-  P = StagePlan{};
-  P.n = n;
-  P.nstages = (uint32_t)f.radices.size();
-  uint32_t Ls = 1;
-  for (uint32_t s = 0; s < P.nstages; s++) {
-    P.radix[s] = f.radices[s];
-    P.ls[s] = Ls;
-    P.tstep[s] = n / (Ls * f.radices[s]);
-    Ls *= f.radices[s];
-  }
-  lcm = f.lcm;
-  return true;
-}
 
 size_t device_max_lds() { return max_lds_bytes(); }
 
@@ -529,48 +455,382 @@ template <typename T> const cx<T> *twiddles(uint32_t n, cyr_status *st) {
   return reinterpret_cast<const cx<T> *>(b.ptr);
 }
 
-void fft_set_shape(uint32_t n, int contig, int precision, FftShape s) {
-  std::lock_guard<std::mutex> lk(g_mu);
-  g_shapes[std::make_tuple(n, contig, precision)] = s;
-}
-
-void fft_clear_shapes() {
-  std::lock_guard<std::mutex> lk(g_mu);
-  g_shapes.clear();
-}
-
 void fft_release() {
   std::lock_guard<std::mutex> lk(g_mu);
   for (auto &kv : g_tw) free_buffer(kv.second);
   g_tw.clear();
+  for (auto &kv : g_lf) free_buffer(kv.second);
+  g_lf.clear();
 }
+
+// ---- any-length plans and tables (lfft.hpp) -------------------------------------
+namespace {
+
+// Radices in the order of their stages' preference (odd ones last: the late stages
+// step through LDS rows by the radix) and the relative cost of a stage: the LDS round
+// trip and barrier every radix pays, plus its arithmetic and registers.
+struct RadixCost {
+  uint32_t r;
+  double c;
+};
+constexpr RadixCost kRadices[] = {{10, 1.5}, {8, 1.25}, {6, 1.2}, {4, 1.05}, {2, 1.0}, {13, 2.4},
+                                  {11, 2.1}, {9, 1.45}, {7, 1.4}, {5, 1.15}, {3, 1.02}};
+
+// Cheapest sequence of radices (at most `cap`) with product n.
+void radix_search(uint32_t n, uint32_t cap, size_t from, double cost, std::vector<uint32_t> &cur, double &best,
+                  std::vector<uint32_t> &out) {
+  if (n == 1) {
+    if (cost < best && cur.size() <= (size_t)kLfStages) {
+      best = cost;
+      out = cur;
+    }
+    return;
+  }
+  for (size_t i = from; i < sizeof(kRadices) / sizeof(kRadices[0]); i++) {
+    const uint32_t r = kRadices[i].r;
+    if (r > cap || n % r != 0 || cost + kRadices[i].c >= best) continue;
+    cur.push_back(r);
+    radix_search(n / r, cap, i, cost + kRadices[i].c, cur, best, out);
+    cur.pop_back();
+  }
+}
+
+bool radix_sequence(uint32_t n, uint32_t cap, std::vector<uint32_t> &out, double &cost) {
+  uint32_t r = n;
+  for (uint32_t p : {2u, 3u, 5u, 7u, 11u, 13u})
+    while (p <= cap && r % p == 0) r /= p;
+  if (r != 1) return false;
+  std::vector<uint32_t> cur;
+  cost = 1e9;
+  out.clear();
+  radix_search(n, cap, 0, 0.0, cur, cost, out);
+  return !out.empty();
+}
+
+// Forward FFT of a host vector whose length is a product of small primes.
+void host_fft(std::vector<std::complex<double>> &x) {
+  const size_t n = x.size();
+  if (n == 1) return;
+  size_t p = 2;
+  while (n % p != 0) p++;
+  const size_t m = n / p;
+  std::vector<std::vector<std::complex<double>>> sub(p, std::vector<std::complex<double>>(m));
+  for (size_t i = 0; i < n; i++) sub[i % p][i / p] = x[i];
+  for (auto &v : sub) host_fft(v);
+  for (size_t k = 0; k < n; k++) {
+    std::complex<double> acc = 0;
+    for (size_t r = 0; r < p; r++) {
+      const double a = -2.0 * M_PI * (double)((r * k) % n) / (double)n;
+      acc += sub[r][k % m] * std::complex<double>(std::cos(a), std::sin(a));
+    }
+    x[k] = acc;
+  }
+}
+
+// exp(-i pi k^2 / n), the argument reduced exactly
+std::complex<double> chirp_of(uint64_t k, uint32_t n) {
+  const double a = -M_PI * (double)((k * k) % (2ull * n)) / (double)n;
+  return {std::cos(a), std::sin(a)};
+}
+
+size_t al64(size_t x) { return (x + 63) & ~(size_t)63; }
+
+template <typename T> struct LfOffsets {
+  size_t tw, chirp, spec, pos, total;  // (the stages come first)
+  explicit LfOffsets(const LfPlan &P) {
+    const size_t cs = sizeof(cx<T>);
+    tw = al64(sizeof(P.st));
+    chirp = tw + al64(cs * P.m);
+    spec = chirp + (P.blue ? al64(cs * P.n) : 0);
+    pos = spec + (P.blue ? al64(cs * P.m) : 0);
+    total = pos + al64(sizeof(uint16_t) * P.m);
+  }
+};
+
+// Host image of the tables of P.
+template <typename T> std::vector<unsigned char> lf_host(const LfPlan &P) {
+  const LfOffsets<T> o(P);
+  std::vector<unsigned char> h(o.total, 0);
+  std::memcpy(h.data(), P.st, sizeof(P.st));
+  cx<T> *tw = reinterpret_cast<cx<T> *>(h.data() + o.tw);
+  for (uint32_t k = 0; k < P.m; k++) {
+    const double a = 2.0 * M_PI * (double)k / (double)P.m;
+    tw[k] = mk<T>((T)std::cos(a), (T)-std::sin(a));
+  }
+  uint16_t *pos = reinterpret_cast<uint16_t *>(h.data() + o.pos);
+  for (uint32_t k = 0; k < P.m; k++) {
+    uint32_t x = k, at = 0;
+    for (uint32_t s = 0; s < P.nst; s++) {
+      at += (x % P.st[s].radix) * P.st[s].q;
+      x /= P.st[s].radix;
+    }
+    pos[k] = (uint16_t)at;
+  }
+  if (P.blue) {
+    cx<T> *ch = reinterpret_cast<cx<T> *>(h.data() + o.chirp), *sp = reinterpret_cast<cx<T> *>(h.data() + o.spec);
+    std::vector<std::complex<double>> b(P.m, 0.0);
+    for (uint32_t k = 0; k < P.n; k++) {
+      const std::complex<double> c = chirp_of(k, P.n);
+      ch[k] = mk<T>((T)c.real(), (T)c.imag());
+      b[k] = std::conj(c);
+      if (k) b[P.m - k] = std::conj(c);
+    }
+    host_fft(b);
+    for (uint32_t k = 0; k < P.m; k++)
+      sp[pos[k]] = mk<T>((T)(b[k].real() / P.m), (T)(b[k].imag() / P.m));
+  }
+  return h;
+}
+
+}  // namespace
+
+namespace {
+
+// (cached by lf_plan: the search for a convolution length tries hundreds)
+bool lf_search(uint32_t n, int precision, LfPlan &P) {
+  std::vector<uint32_t> seq;
+  double c;
+  P = LfPlan{};
+  P.n = P.m = n;
+  if (!radix_sequence(n, precision == CYR_FP64 ? 10 : 13, seq, c)) {
+    // Bluestein: the cheapest convolution length (radices <= 10: the stages also
+    // run backwards)
+    double best = 1e18;
+    std::vector<uint32_t> s2;
+    for (uint32_t m = 2 * n - 1; m <= std::min(kLfMaxLength, 3 * n); m++) {
+      if (!radix_sequence(m, 10, s2, c)) continue;
+      if (m * (2 * c + 2) < best) {
+        best = m * (2 * c + 2);
+        P.m = m;
+        seq = s2;
+      }
+    }
+    if (best > 1e17) return false;
+    P.blue = 1;
+  }
+  P.nst = (uint32_t)seq.size();
+  uint32_t L = P.m;
+  for (uint32_t s = 0; s < P.nst; s++) {
+    const uint32_t q = L / seq[s];
+    P.st[s] = LfStage{seq[s], L, q, q > 1 ? (uint32_t)(((1ull << 32) + q - 1) / q) : 0, P.m / seq[s], P.m / L};
+    L = q;
+  }
+  return true;
+}
+
+}  // namespace
+
+bool lf_plan(uint32_t n, int precision, LfPlan &P) {
+  if (n < 2 || n > kLfMaxLength) return false;
+  // by length and precision (at most 2 x kLfMaxLength small entries); n = 0: no plan
+  static std::mutex mu;
+  static std::map<std::pair<uint32_t, int>, LfPlan> plans;
+  std::lock_guard<std::mutex> lk(mu);
+  const auto key = std::make_pair(n, precision);
+  auto it = plans.find(key);
+  if (it == plans.end()) {
+    LfPlan p;
+    if (!lf_search(n, precision, p)) p.n = 0;
+    it = plans.emplace(key, p).first;
+  }
+  P = it->second;
+  return P.n != 0;
+}
+
+size_t lf_table_bytes(uint32_t n, int precision) {
+  LfPlan P;
+  if (!lf_plan(n, precision, P)) return 0;
+  return precision == CYR_FP64 ? LfOffsets<double>(P).total : LfOffsets<float>(P).total;
+}
+
+template <typename T> cyr_status lf_tables(const LfPlan &P, LfTab<T> &t) {
+  const LfOffsets<T> o(P);
+  const unsigned char *base = nullptr;
+  if (ScratchArena *a = scratch_arena()) {
+    // built into the arena for this call, never into the process-wide cache
+    const auto key = std::make_pair(P.n, prec_of<T>());
+    auto it = a->lf.find(key);
+    if (it == a->lf.end()) {
+      void *d = a->carve(o.total);
+      if (!d) return fail(CYR_E_NOMEM, "allocation-free call: transform tables exceed the scratch array");
+      a->keep.push_back(lf_host<T>(P));
+      CYR_HIP(hipMemcpyAsync(d, a->keep.back().data(), o.total, hipMemcpyHostToDevice, a->stream));
+      it = a->lf.emplace(key, d).first;
+    }
+    base = reinterpret_cast<const unsigned char *>(it->second);
+  } else {
+    int dev = 0;
+    CYR_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(g_mu);
+    const auto key = std::make_tuple(dev, P.n, prec_of<T>());
+    auto it = g_lf.find(key);
+    if (it == g_lf.end()) {
+      const std::vector<unsigned char> h = lf_host<T>(P);
+      DeviceBuffer b;
+      CYR_TRY(ensure_buffer(b, h.size()));
+      if (hipMemcpy(b.ptr, h.data(), h.size(), hipMemcpyHostToDevice) != hipSuccess) {
+        free_buffer(b);
+        return fail(CYR_E_DEVICE, "transform table upload failed");
+      }
+      it = g_lf.emplace(key, b).first;
+    }
+    base = reinterpret_cast<const unsigned char *>(it->second.ptr);
+  }
+  t.n = P.n;
+  t.m = P.m;
+  t.blue = P.blue;
+  t.nst = P.nst;
+  t.nlast = P.st[P.nst - 1].nb;
+  t.st = reinterpret_cast<const LfStage *>(base);
+  t.tw = reinterpret_cast<const cx<T> *>(base + o.tw);
+  t.chirp = reinterpret_cast<const cx<T> *>(base + o.chirp);
+  t.spec = reinterpret_cast<const cx<T> *>(base + o.spec);
+  t.pos = reinterpret_cast<const uint16_t *>(base + o.pos);
+  return CYR_OK;
+}
+
+// Threads per pencil, a multiple of `unit`: blocks of about 256 threads (more, smaller
+// blocks per CU overlap one block's loads with another's stages), the count whose
+// stages, in whole rounds of butterflies, keep the fewest threads idle.
+uint32_t lf_threads(const LfPlan &P, uint32_t unit, uint32_t pencils) {
+  uint32_t pick = 0;
+  double best = 1e30;
+  for (uint32_t t = unit; t * pencils <= 1024 && t < P.m / 2 + unit; t += unit) {
+    double c = 0;
+    for (uint32_t s = 0; s < P.nst; s++)
+      for (const RadixCost &k : kRadices)
+        if (k.r == P.st[s].radix) {
+          const uint32_t rounds = (P.st[s].nb + t - 1) / t;
+          c += (double)t * rounds * k.r * k.c + 0.1 * P.m * rounds;
+        }
+    const uint32_t wg = t * pencils;
+    if (wg < 256) c *= 1.0 + 0.1 * (256 - wg) / 64.0;
+    if (wg > 320) c *= 1.0 + 0.1 * (wg - 320) / 64.0;
+    if (c < best) {
+      best = c;
+      pick = t;
+    }
+  }
+  return pick;
+}
+
+size_t lf_tables_lds(const LfPlan &P, int precision) {
+  const uint32_t nlast = P.st[P.nst - 1].nb;
+  return precision == CYR_FP64 ? lf_lds_tables<double>(P.m, nlast) : lf_lds_tables<float>(P.m, nlast);
+}
+
+// Column tiles: max_cols adjacent pencils where three blocks of them (with room for a
+// row-span table) fit in a CU's LDS, else fewer; whole waves.
+bool lf_cols_shape(const LfPlan &P, int precision, uint32_t max_cols, bool need_tables, LfShape &s) {
+  const size_t cs = precision == CYR_FP64 ? 16 : 8, cap = max_lds_bytes();
+  s = LfShape{};
+  for (uint32_t lpp = 6; lpp-- > 0;) {
+    if (1u << lpp > max_cols) continue;
+    const uint32_t pp = 1u << lpp;
+    const size_t tile = cs * ((size_t)P.m << lpp), with = tile + lf_tables_lds(P, precision) + 4 * (size_t)P.n;
+    if (lpp > 2 && with > cap / 3) continue;
+    if (lpp > 0 && with > cap) continue;
+    const bool tables = with <= cap;
+    if (tile > cap || (need_tables && !tables)) continue;
+    const uint32_t tpp = lf_threads(P, 64 / pp, pp);
+    if (!tpp) continue;
+    s.pp = pp;
+    s.lpp = lpp;
+    s.tpp = tpp;
+    s.tables = tables;
+    s.lds = tables ? with : tile;
+    return true;
+  }
+  return false;
+}
+
+// Rows, as many as 256 threads hold.  e: elements per thread of kernels that keep a
+// row's elements in registers (0: the thread count is free).
+bool lf_rows_shape(const LfPlan &P, int precision, uint32_t e, uint32_t max_threads, bool need_tables, LfShape &s) {
+  const size_t cs = precision == CYR_FP64 ? 16 : 8, cap = max_lds_bytes(), tab = lf_tables_lds(P, precision);
+  s = LfShape{};
+  const uint32_t tpp = e ? (P.n + e - 1) / e : lf_threads(P, 1, 1);
+  if (!tpp || tpp > max_threads) return false;
+  uint32_t rows = tpp >= 256 ? 1 : 256 / tpp;
+  s.pad = kLfPad;
+  auto tile = [&] { return cs * (size_t)rows * lf_row_pitch(P.m, s.pad); };
+  while (rows > 1 && tile() + tab > cap / 3) rows /= 2;
+  s.tables = tile() + tab <= cap;
+  if (tile() > cap) s.pad = kLfNoPad;
+  if (tile() > cap || (need_tables && !s.tables)) return false;
+  s.pp = rows;
+  s.tpp = tpp;
+  s.pitch = lf_row_pitch(P.m, s.pad);
+  s.lds = tile() + (s.tables ? tab : 0);
+  return true;
+}
+
+namespace {
+
+// One pass by the any-length transform (*done = false: the length is beyond it).
+template <typename T>
+cyr_status launch_any(uint32_t n, bool contig, uint32_t nc, PassArgs &A, hipStream_t st, bool *done) {
+  LfPlan P;
+  LfShape s;
+  *done = false;
+  if (!lf_plan(n, prec_of<T>(), P)) return CYR_OK;
+  if (!(contig ? lf_rows_shape(P, prec_of<T>(), 0, 1024, false, s) : lf_cols_shape(P, prec_of<T>(), 16, false, s)))
+    return CYR_OK;
+  LfTab<T> tb;
+  CYR_TRY(lf_tables<T>(P, tb));
+  A.pp = s.pp;
+  A.groups = (A.inner_count + s.pp - 1) / s.pp;
+  A.nvol = nc;
+  const uint64_t tiles = (uint64_t)A.groups * A.outer_count;
+  if (tiles * (contig ? 1 : nc) > 0x7ffffff0ull)
+    return fail(CYR_E_UNSUPPORTED, "FFT grid too large");
+  const AnyShape sh{s.tpp, s.lpp, s.pitch, s.pad};
+  const dim3 block(s.pp * s.tpp), grid = contig ? dim3((unsigned)tiles, nc) : dim3(xcd_grid(tiles * nc));
+  if (!s.tables && (A.span || A.dcz)) return fail(CYR_E_INVALID, "FFT: DC sums and spans need the tables in LDS");
+#define CYR_ANY(C, TB) hipLaunchKernelGGL((fft_any_kernel<T, C, TB>), grid, block, s.lds, st, tb, sh, A)
+  if (contig && s.tables) CYR_ANY(true, true);
+  else if (contig) CYR_ANY(true, false);
+  else if (s.tables) CYR_ANY(false, true);
+  else CYR_ANY(false, false);
+#undef CYR_ANY
+  CYR_LAUNCHED();
+  *done = true;
+  return CYR_OK;
+}
+
+}  // namespace
 
 // Whether a strided pass of length n runs the compile-time codelets.
 template <typename T> bool strided_ct(uint32_t n) {
   if (!ct_length(n) || (sizeof(T) == 8 && ct_elements(n) > 8)) return false;
-  {
-    std::lock_guard<std::mutex> lk(g_mu);
-    if (g_shapes.count(std::make_tuple(n, 0, prec_of<T>()))) return false;
-  }
   const uint32_t pp = n <= 512 ? 16 : (n == 1024 ? 8 : 4);
   return ((size_t)pp * n + n) * sizeof(cx<T>) <= max_lds_bytes();
 }
 
-// Whether the strided codelet's block of length n also holds the row-span table
-// (4 bytes per row) without losing occupancy.
+// The compile-time block of length n also holds the row-span table (4 bytes per
+// row) when that costs no occupancy; the any-length pass reads it from memory.
 template <typename T> bool fft_span_fits(uint32_t n) {
-  if (!strided_ct<T>(n)) return false;
+  if (!strided_ct<T>(n)) {
+    LfPlan P;
+    LfShape s;
+    return lf_plan(n, prec_of<T>(), P) && lf_cols_shape(P, prec_of<T>(), 16, true, s);
+  }
   const uint32_t pp = n <= 512 ? 16 : (n == 1024 ? 8 : 4), wg = pp * (n / ct_elements(n));
   const bool lo = tw_lo_in_lds<T>((size_t)pp * n, n, wg);
   const size_t lds = ((size_t)pp * n + (lo ? 2 * n : n)) * sizeof(cx<T>), with = lds + 4 * (size_t)n;
   return with <= max_lds_bytes() && cu_blocks(with, wg) >= cu_blocks(lds, wg);
 }
 
-// (the strided codelet's block: pp pencils x n / E threads, in waves of 64)
+// (partials per wave of the pass's block: pp pencils x threads per pencil)
 template <typename T> uint32_t fft_dc_slots(uint32_t nx, uint32_t ny) {
-  if (nx < 3 || !strided_ct<T>(ny)) return 0;
-  const uint32_t pp = ny <= 512 ? 16 : (ny == 1024 ? 8 : 4);
-  return 3 * (pp * (ny / ct_elements(ny)) / 64);
+  if (nx < 3 || ny < 2) return 0;
+  if (strided_ct<T>(ny)) {
+    const uint32_t pp = ny <= 512 ? 16 : (ny == 1024 ? 8 : 4);
+    return 3 * (pp * (ny / ct_elements(ny)) / 64);
+  }
+  LfPlan P;
+  LfShape s;
+  return lf_plan(ny, prec_of<T>(), P) && lf_cols_shape(P, prec_of<T>(), 16, true, s) ? 3 * (s.pp * s.tpp / 64) : 0;
 }
 
 template <typename T>
@@ -602,16 +862,10 @@ cyr_status fft_axis(void *const *vols, uint32_t count, uint32_t nx, uint32_t ny,
     A.outer_stride = nx;
     A.outer_count = ny;
   }
-  const Factoring f = factor(n);
   const size_t lds_max = max_lds_bytes();
-  // compile-time codelets unless a shape override asks for the run-time plan
   bool use_ct;
   if (contig) {
     use_ct = ct_length(n) && (sizeof(T) == 4 || ct_elements(n) <= 8);
-    {
-      std::lock_guard<std::mutex> lk(g_mu);
-      if (g_shapes.count(std::make_tuple(n, 1, prec_of<T>()))) use_ct = false;
-    }
     if (use_ct) {
       const size_t need = (size_t)(64 / (n / ct_elements(n)) > 1 ? 64 / (n / ct_elements(n)) : 1) *
                           ct_row_pitch(n) * sizeof(cx<T>);
@@ -620,14 +874,13 @@ cyr_status fft_axis(void *const *vols, uint32_t count, uint32_t nx, uint32_t ny,
   } else {
     use_ct = strided_ct<T>(n);
   }
-  // DC-neighbour sums only ride along a Y pass on the compile-time codelets
   const uint64_t dc_per_vol = dc ? (uint64_t)nz * fft_dc_slots<T>(nx, ny) : 0;
-  if (dc && (axis != 1 || !use_ct || dc_per_vol == 0))
-    return fail(CYR_E_INVALID, "FFT: DC sums need a Y pass on a compile-time plan and Nx >= 3");
+  if (dc && (axis != 1 || dc_per_vol == 0)) return fail(CYR_E_INVALID, "FFT: DC sums need a Y pass and Nx >= 3");
   for (uint32_t c0 = 0; c0 < count; c0 += 8) {
     const uint32_t nc = count - c0 < 8 ? count - c0 : 8;
     for (uint32_t i = 0; i < nc; i++) A.vol[i] = vols[c0 + i];
     A.dcz = dc ? dc->dcz + c0 * dc_per_vol : nullptr;
+    A.dc_twy = tw;
     A.dc_twz = dc ? dc->twz : nullptr;
     A.dc_nz = nz;
     A.span = dc && dc->span && fft_span_fits<T>(ny) ? dc->span : nullptr;
@@ -638,57 +891,9 @@ cyr_status fft_axis(void *const *vols, uint32_t count, uint32_t nx, uint32_t ny,
       if (e != hipSuccess) return hip_fail(e, "fft_ct_kernel", __FILE__, __LINE__);
       done = found;
     }
-    if (!done && f.ok) {
-      // Elements per thread: the radix lcm, doubled while a pencil would need more
-      // than 256 threads; pencils per block: up to 256 threads (contiguous) or a
-      // 16-pencil coalescing group (strided), bounded by LDS.
-      FftShape shp;
-      {
-        std::lock_guard<std::mutex> lk(g_mu);
-        auto it = g_shapes.find(std::make_tuple(n, (int)contig, prec_of<T>()));
-        if (it != g_shapes.end()) shp = it->second;
-      }
-      uint32_t E = f.lcm;
-      const uint32_t tpp_cap = contig ? 256 : 32;  // strided: 16 pencils x 32 threads
-      const uint32_t e_cap = sizeof(T) == 8 ? 16 : 32;
-      if (shp.e && shp.e % f.lcm == 0 && n % shp.e == 0) E = shp.e;
-      else
-        while (n / E > tpp_cap && (E * 2) <= e_cap && n % (E * 2) == 0) E *= 2;
-      if (n % E == 0 && n >= E) {
-        const uint32_t tpp = n / E;
-        uint32_t pp;
-        if (shp.pp) pp = shp.pp;
-        else if (contig) pp = tpp >= 256 ? 1 : 256 / tpp;
-        else pp = 16;
-        while (pp > 1 && ((size_t)pp * n * sizeof(cx<T>) > lds_max || pp * tpp > 1024)) pp /= 2;
-        if (contig && pp > A.inner_count) pp = A.inner_count;
-        if ((size_t)pp * n * sizeof(cx<T>) <= lds_max && pp * tpp <= 1024) {
-          StagePlan P{};
-          P.n = n;
-          P.nstages = (uint32_t)f.radices.size();
-          uint32_t Ls = 1;
-          for (uint32_t s = 0; s < P.nstages; s++) {
-            P.radix[s] = f.radices[s];
-            P.ls[s] = Ls;
-            P.tstep[s] = n / (Ls * f.radices[s]);
-            Ls *= f.radices[s];
-          }
-          A.pp = pp;
-          A.tpp = tpp;
-          A.groups = (A.inner_count + pp - 1) / pp;
-          const uint64_t blocks = (uint64_t)A.groups * A.outer_count;
-          if (blocks > 0x7fffffffull) return fail(CYR_E_UNSUPPORTED, "FFT grid too large");
-          dim3 grid((unsigned)blocks, nc), block(pp * tpp);
-          const size_t lds = (size_t)pp * n * sizeof(cx<T>);
-          bool found = false;
-          hipError_t e = contig ? launch_e<T, true>(E, grid, block, lds, stream, P, A, tw, &found)
-                                : launch_e<T, false>(E, grid, block, lds, stream, P, A, tw, &found);
-          if (e != hipSuccess) return hip_fail(e, "fft_pencil_kernel", __FILE__, __LINE__);
-          done = found;
-        }
-      }
-    }
+    if (!done) CYR_TRY(launch_any<T>(n, contig, nc, A, stream, &done));
     if (!done) {
+      if (dc) return fail(CYR_E_INVALID, "FFT: DC sums need a tiled Y pass");
       if ((size_t)n * sizeof(cx<T>) > lds_max) return fail(CYR_E_UNSUPPORTED, "FFT length not supported");
       const uint64_t blocks = (uint64_t)A.inner_count * A.outer_count;
       if (blocks > 0x7fffffffull) return fail(CYR_E_UNSUPPORTED, "FFT grid too large");
@@ -708,6 +913,8 @@ cyr_status fft3d(void *const *vols, uint32_t count, uint32_t nx, uint32_t ny, ui
   return CYR_OK;
 }
 
+template cyr_status lf_tables<float>(const LfPlan &, LfTab<float> &);
+template cyr_status lf_tables<double>(const LfPlan &, LfTab<double> &);
 template const cx<float> *twiddles<float>(uint32_t, cyr_status *);
 template const cx<double> *twiddles<double>(uint32_t, cyr_status *);
 template cyr_status fft_axis<float>(void *const *, uint32_t, uint32_t, uint32_t, uint32_t, int, hipStream_t,

@@ -1,5 +1,5 @@
-// Hand-written forward C2C FFT for gfx950: Stockham autosort pencils staged in
-// LDS, one launch per axis for a batch of volumes.
+// Hand-written forward C2C FFT for gfx950: pencils staged in LDS, one launch per
+// axis for a batch of volumes.
 #pragma once
 
 #include <cstdint>
@@ -24,7 +24,7 @@ struct FftDc {
   const uint32_t *span = nullptr;
 };
 // Partials per (volume, z) of a Y pass that can take the DC sums; 0 when it
-// cannot (Nx < 3, or no compile-time plan for Ny).
+// cannot (Nx < 3, or Ny beyond the tiles).
 template <typename T> uint32_t fft_dc_slots(uint32_t nx, uint32_t ny);
 // Whether a Y pass of length ny honours FftDc::span.
 template <typename T> bool fft_span_fits(uint32_t ny);
@@ -46,17 +46,8 @@ cyr_status fft3d(void *const *vols, uint32_t count, uint32_t nx, uint32_t ny, ui
 // the block of rounding residuals, tw_len<T>(n) entries in all).
 template <typename T> const cx<T> *twiddles(uint32_t n, cyr_status *st);
 
-// Launch-shape override for the tuner: elements per thread and pencils per block
-// for an axis length (0 = automatic choice).
-struct FftShape { uint32_t e = 0, pp = 0; };
-void fft_set_shape(uint32_t n, int contig, int precision, FftShape s);
-void fft_clear_shapes();
-
 void fft_release();
 
-// Stockham stage plan of an axis length made of factors 2, 3, 5 (false otherwise);
-// lcm = least common multiple of the radices (the minimum elements per thread).
-bool make_stage_plan(uint32_t n, StagePlan &P, uint32_t &lcm);
 size_t device_max_lds();
 
 }  // namespace cyr

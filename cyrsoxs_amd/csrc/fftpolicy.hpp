@@ -1,56 +1,29 @@
-// Register/LDS FFT policies shared by the fused E-basis kernels.
+// Register/LDS FFT policies shared by the FFT passes and the fused kernels.
 //
 // A policy transforms one pencil held by tpp threads, E elements each:
-//   in_pos(t, i)   pencil index loaded into register slot i before run()
-//   out_pos(t, i)  pencil index held by register slot i after run()
-//   run(v, t, p, lds, tw)  Stockham stages, exchanging through LDS
-// Layouts: CONTIG pencils are rows of the LDS tile (element e of pencil p at
-// p*pitch + e); otherwise pencils are columns (e*pp + p), which keeps a wave's
-// accesses to consecutive pencils in consecutive LDS words.
+//   in_pos(t, i)   pencil index loaded into register slot i
+//   holds(t, i)    whether slot i is an element of the pencil at all
+//   stage(lds, pp, ...)  copies its tables behind the tile of pp pencils
+//   transform(v, t, p, pp, lds, out)  the transform, exchanging through LDS; out(k, v)
+//                  takes output k
+// Layouts: CONTIG pencils are rows of the LDS tile; otherwise pencils are
+// columns (element e of pencil p at e pp + p), which keeps a wave's accesses to
+// consecutive pencils in consecutive LDS words.
 //
-// RtFft runs a plan chosen at run time (any 2^a 3^b 5^c length); CtFft is the
-// same algorithm with the radix sequence, the pencil length and the LDS pitch
-// fixed at compile time, so every LDS offset and most index arithmetic fold
-// into immediates and the register footprint shrinks.
+// CtFft: Stockham autosort with the radix sequence, the pencil length and the LDS
+// pitch fixed at compile time, so every LDS offset and most index arithmetic fold
+// into immediates.  Butterfly j (0 <= j < n/R) of a stage with sub-transform length
+// Ls reads x[j + r n/R], multiplies by W_{Ls R}^{r (j mod Ls)}, does an R-point DFT
+// and writes y[(j / Ls) Ls R + (j mod Ls) + r Ls]; a thread holds E elements (E/R
+// butterflies, j = t + b tpp).  LfFft: any length (lfft.hpp).
 #pragma once
 
 #include <hip/hip_runtime.h>
 
+#include "lfft.hpp"
 #include "stockham.hpp"
 
 namespace cyr {
-
-template <typename T, int E> struct RtFft {
-  static constexpr int kE = E;
-  // the kernel argument itself (constant memory): a copy indexed by run-time
-  // stage numbers would be placed in scratch
-  const StagePlan &P;
-  uint32_t tpp;
-  LdsMap L;
-  __device__ RtFft(const StagePlan &plan, uint32_t tpp_, uint32_t pitch, bool contig)
-      : P(plan), tpp(tpp_), L{pitch, contig} {}
-  __device__ uint32_t in_pos(uint32_t t, int i) const {
-    const uint32_t R0 = P.radix[0];
-    return t + ((uint32_t)i / R0) * tpp + ((uint32_t)i % R0) * (P.n / R0);
-  }
-  __device__ uint32_t out_pos(uint32_t t, int i) const {
-    return final_index(t, tpp, P.n, P.radix[P.nstages - 1], i);
-  }
-  // in_pos(t, i) - in_pos(t, 0): the same for every thread
-  __device__ uint32_t in_delta(int i) const {
-    const uint32_t R0 = P.radix[0];
-    return ((uint32_t)i / R0) * tpp + ((uint32_t)i % R0) * (P.n / R0);
-  }
-  __device__ bool exchanges() const { return P.nstages > 1; }
-  // tw: the length-n twiddle block (global or an LDS copy); twlo: its FP32
-  // residual block (may sit elsewhere; unused for FP64).  COMP = false keeps
-  // plain products in every stage (twlo unused).
-  template <bool COMP = true>
-  __device__ void run(cx<T> (&v)[E], uint32_t t, uint32_t p, cx<T> *lds, const cx<T> *__restrict__ tw,
-                      const cx<T> *twlo) const {
-    stockham_from_regs<T, E>(v, P, t, tpp, p, lds, L, tw, COMP ? twlo : nullptr);
-  }
-};
 
 template <int A, int... B> struct FirstOf { static constexpr int value = A; };
 template <int A, int... B> struct LastOf { static constexpr int value = LastOf<B...>::value; };
@@ -183,16 +156,66 @@ template <typename T, int N, int E, bool CONTIG, int PP, int... R> struct CtFft 
   static constexpr int kE = E, TPP = N / E;
   static constexpr int R0 = FirstOf<R...>::value, RL = LastOf<R...>::value;
   static constexpr int PE = CONTIG ? 1 : PP;
-  __device__ CtFft(const StagePlan &, uint32_t, uint32_t, bool) {}
+  static constexpr bool kCt = true;
+  struct Plan {};
+  __device__ explicit CtFft(const Plan &) {}
+  __device__ static constexpr bool holds(uint32_t, int) { return true; }
+  // rows: twiddles staged behind them (a barrier must follow), plain twiddle products
+  __device__ static void stage(cx<T> *lds, uint32_t pp, const cx<T> *__restrict__ tw) {
+    for (uint32_t i = threadIdx.x; i < (uint32_t)N; i += blockDim.x) lds[pp * kPitch + i] = tw[i];
+  }
+  template <class OUT>
+  __device__ static void transform(cx<T> (&v)[E], uint32_t t, uint32_t p, uint32_t pp, cx<T> *lds, OUT out) {
+    run<false>(v, t, p, lds, lds + pp * kPitch, nullptr);
+#pragma unroll
+    for (int i = 0; i < E; i++) out(out_pos(t, i), v[i]);
+  }
   __device__ static uint32_t in_pos(uint32_t t, int i) { return t + (i / R0) * TPP + (i % R0) * (N / R0); }
   __device__ static uint32_t out_pos(uint32_t t, int i) { return t + (i / RL) * TPP + (i % RL) * (N / RL); }
   __device__ static constexpr uint32_t in_delta(int i) { return (i / R0) * TPP + (i % R0) * (N / R0); }
-  __device__ static constexpr bool exchanges() { return sizeof...(R) > 1; }
   template <bool COMP = true>
   __device__ static void run(cx<T> (&v)[E], uint32_t t, uint32_t p, cx<T> *lds, const cx<T> *__restrict__ tw,
                              const cx<T> *__restrict__ twlo) {
     cx<T> *lb = CONTIG ? lds + (size_t)p * kPitch : lds + p;
     ct_stages<T, N, E, PE, COMP, 1, R...>(v, t, lb, tw, twlo);
+  }
+};
+
+// Any length (lfft.hpp), rows: slot i of thread t is element t + i tpp (E tpp >= n;
+// the last slots may be empty).  Plain twiddle products.
+template <typename T, int E> struct LfRowFft {
+  static constexpr int kE = E;
+  static constexpr bool kCt = false;
+  struct Plan {
+    LfTab<T> tb;
+    uint32_t tpp;    // threads per row
+    uint32_t pitch;  // LDS elements per row
+    uint32_t pad;    // one slot of padding per 2^pad elements
+  };
+  const Plan P;
+  __device__ explicit LfRowFft(const Plan &plan) : P(plan) {}
+  __device__ uint32_t in_pos(uint32_t t, int i) const { return t + (uint32_t)i * P.tpp; }
+  __device__ bool holds(uint32_t t, int i) const { return t + (uint32_t)i * P.tpp < P.tb.n; }
+  // (the tables lie behind the rows: stage() copies them, a barrier must follow)
+  __device__ void stage(cx<T> *lds, uint32_t pp) const { lf_stage_tables<T>(P.tb, lds + pp * P.pitch); }
+  template <class OUT>
+  __device__ void transform(cx<T> (&v)[E], uint32_t t, uint32_t p, uint32_t pp, cx<T> *lds, OUT out) const {
+    const cx<T> *tw = lds + pp * P.pitch;
+    const LfLds<T> tab{tw, reinterpret_cast<const uint16_t *>(tw + P.tb.m)};
+    LfNoInput<T> in;
+    const LfRow ad{p * P.pitch, P.pad};
+#pragma unroll
+    for (int i = 0; i < E; i++)
+      if (holds(t, i)) {
+        const uint32_t e = in_pos(t, i);
+        lds[ad(e)] = P.tb.blue ? cmul<T>(v[i], P.tb.chirp[e]) : v[i];
+      }
+    if (P.tb.blue)
+      for (uint32_t e = P.tb.n + t; e < P.tb.m; e += P.tpp) lds[ad(e)] = mk<T>(0, 0);
+    lds_sync();
+    auto emit = [&](uint32_t k, uint32_t r, uint32_t dk, cx<T> x) { out(k + r * dk, x); };
+    lf_run<true, T>(P.tb, tab, lds, ad, t, P.tpp, in, emit);
+    lds_sync();  // the rows may be refilled
   }
 };
 

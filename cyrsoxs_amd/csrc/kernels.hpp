@@ -65,9 +65,11 @@ cyr_status launch_igor_shift(cx<T> *vol, uint32_t nx, uint32_t ny, uint32_t nz, 
 // p~ = A F.
 constexpr int kEbFields = 5;
 constexpr int kEbAmat = 3 * kEbFields;
-// True when the grid has Stockham plans and LDS tiles that fit the fused kernels
-// (other grids run the plain executor).
-bool ebasis_supported(uint32_t nx, uint32_t ny, uint32_t nz, int precision);
+// True when every side has a transform whose tile fits the fused kernels (other
+// grids run the plain executor).
+bool fused_supported(uint32_t nx, uint32_t ny, uint32_t nz, int precision);
+// True when the fused Y / z-bin kernel takes the grid (a compile-time plan for Ny).
+bool ebasis_yz_supported(uint32_t ny, uint32_t nz, int precision);
 // Grid size the Y/z kernel's z chunking aims for, and the most chunks any plan
 // for (nx, nz) uses (sizes the partial-sum buffer).
 constexpr uint32_t kYzTargetBlocks = 1024;
@@ -88,7 +90,7 @@ template <typename T> struct PolxArgs {
   Mat3<T> Q;                       // columns e1, e2, k^ (row-major)
   int32_t rot;                     // 0 when Q is the identity
   const cx<T> *twx;                // filled by the launcher
-  uint32_t tpp, pp, pitch;         // filled by the launcher
+  uint32_t tpp, pp;                // filled by the launcher
   cx<T> *out[kXMaxOut];            // X-transformed fields
 };
 template <typename T>
@@ -100,8 +102,7 @@ template <typename T> struct YzArgs {
   const int32_t *kzt;              // [Ny][Nx] (3D)
   const cx<T> *twy, *twz;          // twy filled by the launcher; twz null in 2D
   uint32_t nx, ny, nz;
-  uint32_t e, pp, tpp, zchunk, nchunks;  // 0 = automatic (ebasis_yz_plan fills)
-  uint32_t ct;                     // 1: compile-time FFT plan for Ny (set by ebasis_yz_plan)
+  uint32_t pp, tpp, zchunk, nchunks;  // 0 = automatic (ebasis_yz_plan fills)
 };
 // Launch choices of the Y/z kernel for one (Nx, Ny, Nz, precision) shape, set by
 // the autotuner: columns per block and the grid size the z chunking aims for
@@ -112,7 +113,7 @@ struct YzTuning {
 };
 YzTuning ebasis_yz_tuning(uint32_t nx, uint32_t ny, uint32_t nz, int precision);
 void ebasis_set_yz_tuning(uint32_t nx, uint32_t ny, uint32_t nz, int precision, YzTuning t);
-// Fills e, pp, tpp, zchunk, nchunks (fields left 0 are chosen automatically;
+// Fills pp, tpp, zchunk, nchunks (fields left 0 are chosen automatically;
 // target_blocks is the grid size the z chunking aims for, 0 = tuned/default).
 template <typename T> cyr_status ebasis_yz_plan(YzArgs<T> &a, uint32_t target_blocks);
 template <typename T> cyr_status launch_ebasis_yz(YzArgs<T> a, int ng, hipStream_t st);
@@ -166,14 +167,14 @@ template <typename T> struct BandArgs {
   uint32_t count, vbase;           // volumes, global index of vol[0]
   const int32_t *band;             // [Ny][Nx] band table
   const uint32_t *span;            // [Ny] row spans (null: every column)
-  cx<T> *own, *mir;                // [volumes][J][Ny][Nx]
+  cx<T> *own, *mir;                // [volumes][J][Ny][Nx] (mir null: complex fields, no mirrored bins)
   uint32_t J, nx, ny, nz;
 };
 template <typename T> cyr_status launch_mbasis_extract(const BandArgs<T> &a, hipStream_t st);
 // Z FFT of the Y-transformed volumes writing only the band values (vol[] is read,
-// not overwritten); *done = false when Nz has no compile-time plan (then run the
-// Z FFT pass and launch_mbasis_extract).
-template <typename T> cyr_status launch_mbasis_zband(const BandArgs<T> &a, hipStream_t st, bool *done);
+// not overwritten), 3D; launch_mbasis_extract copies them in 2D.
+bool mbasis_zband_supported(uint32_t nz, int precision);
+template <typename T> cyr_status launch_mbasis_zband(const BandArgs<T> &a, hipStream_t st);
 // DC-replacement values of the packed volumes from their per-slice neighbour sums.
 cyr_status launch_mbasis_dcsum(const double2 *dcz, uint32_t nvol, uint32_t nz, bool three, double2 *dcv,
                                hipStream_t st);
@@ -184,11 +185,11 @@ template <typename T> struct MbAnglesArgs {
   uint32_t J;
   const double2 *dcv;              // [volumes]
   const MatConst<T> *mats;         // this energy's M constants
-  uint32_t M;
+  uint32_t M;                      // 0: own holds one energy's five tensor fields (mir unused)
   const T *amat;                   // [nA][kEbAmat]
   uint32_t nA;
   T *proj;                         // [nA][Ny][Nx] (per-angle projections), or
-  T *quad;                         // [ne][P][4] in quad_index order: laboratory frame, the intensity's quadratic form
+  T *quad;                         // [ne][P][3] in quad_index order: laboratory frame, the intensity's quadratic form
   Mat3<T> Q;                       // frame e1, e2, k^ (quadratic form)
   const double *kmag;              // quadratic form: |k| of the ne energies (mats then holds ne x M)
   uint32_t ne;
@@ -242,7 +243,7 @@ void rotation_orbit_tile_order(uint32_t n, uint32_t *out);
 // `quarter` angle steps per 90 degrees (0: none); 0 when it does not apply.
 uint32_t rotation_quarter_turns(uint32_t nx, uint32_t ny, uint32_t nA, uint32_t quarter);
 // Laboratory frame: the same for ne energies from their per-pixel quadratic forms
-// quad[ne][P][4] (quad_index order; I(theta) = c^2 q0 + s^2 q1 + 2 c s q2) with
+// quad[ne][P][3] (quad_index order; I(theta) = c^2 q0 + s^2 q1 + 2 c s q2) with
 // coef[a] = (c^2, s^2, 2 c s) (FP64; coef_t: the same in the compute precision)
 // into avg[ne][Ny][Nx]; each angle's taps serve several energies.  quarter (angle
 // steps per 90 degrees, 0 = none) with otiles (orbit tile order) lets each tap

@@ -13,9 +13,9 @@
 // and at the mirrored bins of the opposite column.
 //
 // Launches per (k, energy group): mbasis_bands_kernel (+ band width reduction),
-// then per material pass xfields_kernel (pair/single mode) -> DC neighbour sums
-// -> Y FFT pass -> mbasis_zband_kernel (Z FFT writing only band values; for Nz
-// without a compile-time plan: Z FFT pass + mbasis_extract_kernel);
+// then per material pass xfields_kernel (pair/single mode) -> Y FFT pass with the
+// DC neighbour sums -> mbasis_zband_kernel (Z FFT writing only band values; in 2D
+// mbasis_extract_kernel);
 // mbasis_dcsum_kernel; then per energy mbasis_angles_kernel and the shared
 // rotation / detector kernels.
 #include <hip/hip_runtime.h>
@@ -24,6 +24,7 @@
 #include "fftpolicy.hpp"
 #include "geom.hpp"
 #include "kernels.hpp"
+#include "quadform.hpp"
 #include "xfields.hpp"
 
 namespace cyr {
@@ -179,24 +180,21 @@ __device__ inline bool bins_meet_span(uint32_t x0, uint32_t x1, uint32_t n, uint
   return false;
 }
 
-// ---- band values of the transformed packed volumes ----------------------------
-// own[v][j][col] = Z_v(col, kz(Zlo + j)),  mir[v][j][col] = Z_v(-col, -kz(Zlo + j))
-// for j < width(col).  Grid: (columns, j, volume).
+// ---- band values of the transformed packed planes (2D) ---------------------------
+// own[v][0][col] = Z_v(col),  mir[v][0][col] = Z_v(-col) for sampled columns.
+// Grid: (columns, volume).
 template <typename T>
 __global__ void __launch_bounds__(256) mbasis_extract_kernel(BandArgs<T> a) {
   const uint64_t P = (uint64_t)a.nx * a.ny;
   const uint64_t col = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t j = blockIdx.y, v = blockIdx.z;
-  if (col >= P) return;
-  const uint32_t b = (uint32_t)a.band[col];
-  if (j >= (b >> 16)) return;
-  const uint32_t kz = a.nz > 1 ? unshift((b & 0xffffu) + j, a.nz) : 0;
+  const uint32_t v = blockIdx.y;
+  if (col >= P || a.band[col] == 0) return;
   const uint32_t iy = (uint32_t)(col / a.nx), ix = (uint32_t)(col - (uint64_t)iy * a.nx);
-  const uint32_t mx = ix ? a.nx - ix : 0, my = iy ? a.ny - iy : 0, mz = kz ? a.nz - kz : 0;
+  const uint32_t mx = ix ? a.nx - ix : 0, my = iy ? a.ny - iy : 0;
   const cx<T> *Z = a.vol[v];
-  const uint64_t o = ((uint64_t)(a.vbase + v) * a.J + j) * P + col;
-  a.own[o] = Z[(uint64_t)kz * P + col];
-  a.mir[o] = Z[(uint64_t)mz * P + (uint64_t)my * a.nx + mx];
+  const uint64_t o = (uint64_t)(a.vbase + v) * a.J * P + col;
+  a.own[o] = Z[col];
+  if (a.mir) a.mir[o] = Z[(uint64_t)my * a.nx + mx];
 }
 
 // ---- Z FFT fused with the band extraction --------------------------------------
@@ -258,6 +256,7 @@ __global__ void __launch_bounds__(WG) mbasis_zband_kernel(BandArgs<T> a, const c
     const uint32_t kz = F::out_pos(t, i);
     const uint32_t j = unshift(kz, N) - lo;  // wraps above w when below the band
     if (j < w) own[(uint64_t)j * P + col] = r[i];
+    if (!a.mir) continue;  // (complex fields: no mirrored bins)
     const uint32_t jm = unshift(kz ? N - kz : 0, N) - lom;
     if (jm < wm) mir[(uint64_t)jm * P + cm] = r[i];
   }
@@ -283,6 +282,76 @@ hipError_t launch_zband_n(const BandArgs<T> &a, hipStream_t st, const cx<T> *tw)
   hipLaunchKernelGGL((mbasis_zband_kernel<T, F, WG>), dim3(xcd_chunk_grid(tiles, kZbandChunk)), dim3(WG), lds, st,
                      a, tw);
   return hipGetLastError();
+}
+
+// The same for any length (lfft.hpp): the first stage loads the column's elements, the
+// last hands its outputs to the band test, so nothing but the band values leaves.
+template <typename T>
+__global__ void __launch_bounds__(1024) mbasis_zband_any_kernel(LfTab<T> tb, uint32_t tpp, uint32_t lpp,
+                                                                BandArgs<T> a) {
+  extern __shared__ unsigned char smem_raw[];
+  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw);
+  const uint32_t PP = 1u << lpp, groups = (a.nx + PP - 1) >> lpp, per_vol = groups * a.ny;
+  const uint32_t q = xcd_chunk_tile(blockIdx.x, kZbandChunk);  // (as mbasis_zband_kernel)
+  if (q >= per_vol * a.count) return;  // grid padding: the whole block leaves before any barrier
+  const uint32_t p = threadIdx.x & (PP - 1), t = threadIdx.x >> lpp;
+  const uint32_t v = q / per_vol, tile = q % per_vol;
+  const uint32_t g = tile % groups, y = tile / groups;
+  const uint32_t sp = a.span ? a.span[y] : 0xffff0000u;
+  const uint32_t slo = sp & 0xffffu, shi = sp >> 16;
+  if (!bins_meet_span(g * PP, (g * PP + PP < a.nx ? g * PP + PP : a.nx) - 1, a.nx, slo, shi)) return;
+  const uint32_t x = g * PP + p;
+  const bool active = x < a.nx;
+  const uint32_t xx = active ? x : 0;
+  const uint64_t P = (uint64_t)a.nx * a.ny;
+  const uint64_t col = (uint64_t)y * a.nx + xx;
+  const uint32_t sx = unshift(xx, a.nx);
+  const bool need = active && sx >= slo && sx <= shi;
+  const cx<T> *base = a.vol[v] + col;
+  const uint32_t mx = xx ? a.nx - xx : 0, my = y ? a.ny - y : 0;
+  const uint64_t cm = (uint64_t)my * a.nx + mx;
+  const uint32_t b = active ? (uint32_t)a.band[col] : 0, bm = active ? (uint32_t)a.band[cm] : 0;
+  const uint32_t lo = b & 0xffffu, w = b >> 16;
+  const uint32_t lom = bm & 0xffffu, wm = a.mir ? bm >> 16 : 0;
+  cx<T> *own = a.own + (uint64_t)(a.vbase + v) * a.J * P + col;
+  cx<T> *mir = a.mir + (uint64_t)(a.vbase + v) * a.J * P + cm;
+  const LfLds<T> tab = lf_stage_tables<T>(tb, lds + ((size_t)tb.m << lpp));
+  lds_sync();
+  const uint32_t N = a.nz;
+  // (columns outside the span hold stale values: they transform to nothing that is kept)
+  struct {
+    const cx<T> *base;
+    uint64_t P;
+    bool need;
+    __device__ cx<T> load(uint32_t e, uint32_t r, uint32_t q) const {
+      return need ? base[(uint64_t)e * P + r * (q * P)] : mk<T>(0, 0);
+    }
+  } in{base, P, need};
+  auto out = [&](uint32_t k0, uint32_t ks, uint32_t dk, cx<T> r) {
+    const uint32_t kz = k0 + ks * dk;
+    const uint32_t j = unshift(kz, N) - lo;  // wraps above w when below the band
+    if (j < w) own[(uint64_t)j * P] = r;
+    const uint32_t jm = unshift(kz ? N - kz : 0, N) - lom;
+    if (jm < wm) mir[(uint64_t)jm * P] = r;
+  };
+  lf_run<false, T>(tb, tab, lds, LfCols{lpp, p}, t, tpp, in, out);
+}
+
+// Up to 32 columns.
+template <typename T> cyr_status launch_zband_any(const BandArgs<T> &a, hipStream_t st) {
+  const int prec = sizeof(T) == 8 ? CYR_FP64 : CYR_FP32;
+  LfPlan P;
+  LfShape s;
+  if (!lf_plan(a.nz, prec, P) || !lf_cols_shape(P, prec, 32, true, s))
+    return fail(CYR_E_UNSUPPORTED, "Z band pass: length beyond the tile");
+  LfTab<T> tb;
+  CYR_TRY(lf_tables<T>(P, tb));
+  const uint64_t tiles = (uint64_t)((a.nx + s.pp - 1) / s.pp) * a.ny * a.count;
+  if (tiles > 0x7ffffff0ull) return fail(CYR_E_UNSUPPORTED, "Z band pass: grid too large");
+  hipLaunchKernelGGL((mbasis_zband_any_kernel<T>), dim3(xcd_chunk_grid(tiles, kZbandChunk)), dim3(s.pp * s.tpp), s.lds,
+                     st, tb, s.tpp, s.lpp, a);
+  CYR_LAUNCHED();
+  return CYR_OK;
 }
 
 // dcv[v] = (sum_z dcz[v][z]) / cnt, fixed-order tree (deterministic); one block per volume
@@ -362,6 +431,19 @@ __device__ inline int mb_fields(const MbAnglesArgs<T> &a, uint32_t X, uint32_t Y
   for (int q = 0; q < NG; q++) dc[q] = ix == 0 && iy == 0 && (three ? unshift(z0 + q, g.nz) == 0 : true);
   const uint64_t slab = (uint64_t)a.J * P2;
   const cx<T> *own = a.own + (uint64_t)j0 * P2 + col, *mir = a.mir + (uint64_t)j0 * P2 + col;
+  w1 = (T)f;
+  if (a.M == 0) {  // five complex tensor fields, no packing
+#pragma unroll
+    for (int q = 0; q < NG; q++)
+#pragma unroll
+      for (int c = 0; c < kEbFields; c++) {
+        const double2 d = a.dcv[c];
+        F[q][c] = dc[q] ? mk<T>((T)d.x, (T)d.y) : own[(uint64_t)c * slab + (uint64_t)q * P2];
+      }
+#pragma unroll
+    for (int q = 0; q < NG; q++) scatter_matrix(g, X, Y, three ? z0 + q : 0, md[q]);
+    return kind;
+  }
   auto fetch = [&](uint32_t v, int q, cx<T> &z, cx<T> &zm) {
     if (dc[q]) {
       const double2 d = a.dcv[v];
@@ -416,7 +498,6 @@ __device__ inline int mb_fields(const MbAnglesArgs<T> &a, uint32_t X, uint32_t Y
     F[q][3].y += iso[q].y;
     scatter_matrix(g, X, Y, three ? z0 + q : 0, md[q]);
   }
-  w1 = (T)f;
   return kind;
 }
 
@@ -457,53 +538,6 @@ __global__ void __launch_bounds__(256) mbasis_angles_kernel(MbAnglesArgs<T> a) {
     if constexpr (NG == 2) out = (1 - w1) * I[0] + w1 * I[1];
     else out = I[0];
     a.proj[(uint64_t)an * P2 + t] = out;
-  }
-}
-
-// ---- per energy, laboratory frame: the intensity's quadratic form ---------------
-// With E(theta) = c e1 + s e2 the polarization is p = c u + s v, u = Q (F0, F1, F2),
-// v = Q (F1, F3, F4), so I(theta) = c^2 |M u|^2 + s^2 |M v|^2 + 2 c s Re<M u, M v>.
-// quad[pixel] = (|Mu|^2, |Mv|^2, Re<Mu, Mv>), interpolated between the bins.
-template <typename T, int NG>
-__device__ inline void quad_form_write(const Mat3<T> &Q, const cx<T> (&F)[NG][kEbFields], const double (&md)[NG][6],
-                                       T w1, T *o) {
-  T qa[NG], qb[NG], qm[NG];
-#pragma unroll
-  for (int q = 0; q < NG; q++) {
-    cx<T> u[3], v[3], mu[3], mv[3];
-    const cx<T> ue[3] = {F[q][0], F[q][1], F[q][2]}, ve[3] = {F[q][1], F[q][3], F[q][4]};
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-      u[i] = mk<T>(Q.m[3 * i] * ue[0].x + Q.m[3 * i + 1] * ue[1].x + Q.m[3 * i + 2] * ue[2].x,
-                   Q.m[3 * i] * ue[0].y + Q.m[3 * i + 1] * ue[1].y + Q.m[3 * i + 2] * ue[2].y);
-      v[i] = mk<T>(Q.m[3 * i] * ve[0].x + Q.m[3 * i + 1] * ve[1].x + Q.m[3 * i + 2] * ve[2].x,
-                   Q.m[3 * i] * ve[0].y + Q.m[3 * i + 1] * ve[1].y + Q.m[3 * i + 2] * ve[2].y);
-    }
-    const T m0 = (T)md[q][0], m1 = (T)md[q][1], m2 = (T)md[q][2], m3 = (T)md[q][3], m4 = (T)md[q][4],
-            m5 = (T)md[q][5];
-    const T mm[3][3] = {{m0, m1, m2}, {m1, m3, m4}, {m2, m4, m5}};
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-      mu[i] = mk<T>(mm[i][0] * u[0].x + mm[i][1] * u[1].x + mm[i][2] * u[2].x,
-                    mm[i][0] * u[0].y + mm[i][1] * u[1].y + mm[i][2] * u[2].y);
-      mv[i] = mk<T>(mm[i][0] * v[0].x + mm[i][1] * v[1].x + mm[i][2] * v[2].x,
-                    mm[i][0] * v[0].y + mm[i][1] * v[1].y + mm[i][2] * v[2].y);
-    }
-    qa[q] = mu[0].x * mu[0].x + mu[0].y * mu[0].y + mu[1].x * mu[1].x + mu[1].y * mu[1].y + mu[2].x * mu[2].x +
-            mu[2].y * mu[2].y;
-    qb[q] = mv[0].x * mv[0].x + mv[0].y * mv[0].y + mv[1].x * mv[1].x + mv[1].y * mv[1].y + mv[2].x * mv[2].x +
-            mv[2].y * mv[2].y;
-    qm[q] = mu[0].x * mv[0].x + mu[0].y * mv[0].y + mu[1].x * mv[1].x + mu[1].y * mv[1].y + mu[2].x * mv[2].x +
-            mu[2].y * mv[2].y;
-  }
-  if constexpr (NG == 2) {
-    o[0] = (1 - w1) * qa[0] + w1 * qa[1];
-    o[1] = (1 - w1) * qb[0] + w1 * qb[1];
-    o[2] = (1 - w1) * qm[0] + w1 * qm[1];
-  } else {
-    o[0] = qa[0];
-    o[1] = qb[0];
-    o[2] = qm[0];
   }
 }
 
@@ -679,9 +713,9 @@ uint32_t *mbasis_span_table(uint32_t *bmax, uint32_t nx, uint32_t ny) {
 
 template <typename T> cyr_status launch_mbasis_extract(const BandArgs<T> &a, hipStream_t st) {
   if (a.count == 0) return CYR_OK;
-  if (a.count > (uint32_t)kXMaxOut || a.J == 0 || a.J > 65535) return fail(CYR_E_INVALID, "band extraction: bad shape");
+  if (a.count > (uint32_t)kXMaxOut || a.J == 0 || a.nz != 1) return fail(CYR_E_INVALID, "band extraction: bad shape");
   const uint64_t P = (uint64_t)a.nx * a.ny;
-  hipLaunchKernelGGL((mbasis_extract_kernel<T>), dim3(ceil_div(P, 256), a.J, a.count), dim3(256), 0, st, a);
+  hipLaunchKernelGGL((mbasis_extract_kernel<T>), dim3(ceil_div(P, 256), a.count), dim3(256), 0, st, a);
   CYR_LAUNCHED();
   return CYR_OK;
 }
@@ -694,17 +728,28 @@ cyr_status launch_mbasis_dcsum(const double2 *dcz, uint32_t nvol, uint32_t nz, b
   return CYR_OK;
 }
 
-template <typename T> cyr_status launch_mbasis_zband(const BandArgs<T> &a, hipStream_t st, bool *done) {
-  *done = false;
-  const int prec = sizeof(T) == 8 ? CYR_FP64 : CYR_FP32;
-  if (a.count == 0 || a.nz < 2 || !ct_usable(a.nz, prec)) return CYR_OK;
-  if (a.count > (uint32_t)kXMaxOut || a.J == 0) return fail(CYR_E_INVALID, "Z band pass: bad shape");
-  const uint32_t pp = a.nz <= 128 ? 32 : (a.nz <= 512 ? 16 : (a.nz == 1024 ? 8 : 4));
-  if (((size_t)pp * a.nz + a.nz) * sizeof(cx<T>) > device_max_lds()) return CYR_OK;
+template <typename T> bool zband_ct(uint32_t nz) {
+  if (!ct_usable(nz, sizeof(T) == 8 ? CYR_FP64 : CYR_FP32)) return false;
+  const uint32_t pp = nz <= 128 ? 32 : (nz <= 512 ? 16 : (nz == 1024 ? 8 : 4));
+  return ((size_t)pp * nz + nz) * sizeof(cx<T>) <= device_max_lds();
+}
+
+bool mbasis_zband_supported(uint32_t nz, int precision) {
+  if (nz < 2) return false;
+  if (precision == CYR_FP64 ? zband_ct<double>(nz) : zband_ct<float>(nz)) return true;
+  LfPlan P;
+  LfShape s;
+  return lf_plan(nz, precision, P) && lf_cols_shape(P, precision, 32, true, s);
+}
+
+template <typename T> cyr_status launch_mbasis_zband(const BandArgs<T> &a, hipStream_t st) {
+  if (a.count == 0) return CYR_OK;
+  if (a.nz < 2 || a.count > (uint32_t)kXMaxOut || a.J == 0) return fail(CYR_E_INVALID, "Z band pass: bad shape");
+  if (!zband_ct<T>(a.nz)) return launch_zband_any<T>(a, st);
   cyr_status s;
   const cx<T> *tw = twiddles<T>(a.nz, &s);
   if (!tw) return s;
-  hipError_t e = hipSuccess;
+  hipError_t e = hipErrorInvalidValue;
   switch (a.nz) {
     case 64: e = launch_zband_n<T, 64>(a, st, tw); break;
     case 128: e = launch_zband_n<T, 128>(a, st, tw); break;
@@ -715,10 +760,9 @@ template <typename T> cyr_status launch_mbasis_zband(const BandArgs<T> &a, hipSt
     case 512: e = launch_zband_n<T, 512>(a, st, tw); break;
     case 1024: e = launch_zband_n<T, 1024>(a, st, tw); break;
     case 2048: e = launch_zband_n<T, 2048>(a, st, tw); break;
-    default: return CYR_OK;
+    default: break;
   }
   if (e != hipSuccess) return hip_fail(e, "mbasis_zband_kernel", __FILE__, __LINE__);
-  *done = true;
   return CYR_OK;
 }
 
@@ -755,18 +799,10 @@ template <typename T> cyr_status launch_mbasis_angles(const MbAnglesArgs<T> &a, 
   return CYR_OK;
 }
 
-template <typename T>
-cyr_status launch_mbasis_xfields(PolxArgs<T> a, bool pair, const void *vox, int storage, int morph, bool hann,
-                                 hipStream_t st) {
-  if (pair) return launch_xfields<T, kXPair>(a, vox, storage, morph, hann, st);
-  return launch_xfields<T, kXSingle>(a, vox, storage, morph, hann, st);
-}
-
 #define CYR_INST(T)                                                                                          \
   template cyr_status launch_mbasis_extract<T>(const BandArgs<T> &, hipStream_t);                          \
-  template cyr_status launch_mbasis_zband<T>(const BandArgs<T> &, hipStream_t, bool *);                    \
-  template cyr_status launch_mbasis_angles<T>(const MbAnglesArgs<T> &, int, hipStream_t);                  \
-  template cyr_status launch_mbasis_xfields<T>(PolxArgs<T>, bool, const void *, int, int, bool, hipStream_t);
+  template cyr_status launch_mbasis_zband<T>(const BandArgs<T> &, hipStream_t);                            \
+  template cyr_status launch_mbasis_angles<T>(const MbAnglesArgs<T> &, int, hipStream_t);
 CYR_INST(float)
 CYR_INST(double)
 #undef CYR_INST

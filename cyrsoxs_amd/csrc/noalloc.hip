@@ -20,7 +20,11 @@
 namespace cyr {
 namespace {
 
-constexpr size_t kScratchBytes = CYR_NOALLOC_SCRATCH_BYTES;
+// The array also holds the any-length transforms' tables (at most three lengths, of
+// 8 complex values and 2 bytes per point of a convolution up to 16384 points), so that
+// they take nothing from the documented size.
+constexpr size_t kTableBytes = 3u * 1024u * 1024u;
+constexpr size_t kScratchBytes = CYR_NOALLOC_SCRATCH_BYTES + kTableBytes;
 static_assert(kScratchBytes % 256 == 0, "scratch size must keep 256-byte alignment");
 
 // One copy per device, held from module load until the process ends.
@@ -84,13 +88,21 @@ extern "C" cyr_status cyr_simulate_device_noalloc(const cyr_sim_desc *desc, cons
   SimGeometry g;
   CYR_TRY(build_geometry(desc, g));
   if (!d_voxels || !mats || !d_out) return fail(CYR_E_INVALID, "null buffer");
-  const uint64_t need = scratch_need(desc, g);
-  if (need > kScratchBytes) {
+  cyr_sim_desc plain = *desc;
+  plain.pipeline = CYR_PIPE_PLAIN;
+  uint64_t need = scratch_need(desc, g);
+  bool fallback = plain_fallback(desc, g) && scratch_need(&plain, g) <= CYR_NOALLOC_SCRATCH_BYTES;
+  if (need > CYR_NOALLOC_SCRATCH_BYTES && fallback) {
+    desc = &plain;
+    fallback = false;
+    need = scratch_need(desc, g);
+  }
+  if (need > CYR_NOALLOC_SCRATCH_BYTES) {
     char buf[200];
     std::snprintf(buf, sizeof(buf),
                   "allocation-free call: this simulation needs %llu bytes of device scratch; the limit is %zu "
                   "(use cyr_simulate_device)",
-                  (unsigned long long)need, kScratchBytes);
+                  (unsigned long long)need, (size_t)CYR_NOALLOC_SCRATCH_BYTES);
     return fail(CYR_E_INVALID, buf);
   }
   ScratchSlot *slot;
@@ -99,20 +111,29 @@ extern "C" cyr_status cyr_simulate_device_noalloc(const cyr_sim_desc *desc, cons
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   // host images of the tables and twiddles live until the stream has drained
   std::vector<unsigned char> host_tables(table_bytes(desc, g));
-  ScratchArena arena;
-  arena.base = slot->ptr;
-  arena.cap = kScratchBytes;
-  arena.stream = st;
-  // constant tables first (the executors read them as resident tables)
   fill_tables(desc, g, mats, host_tables.data());
-  void *tables = arena.carve(host_tables.size());
-  if (!tables) return fail(CYR_E_NOMEM, "allocation-free call: tables exceed the scratch array");
-  CYR_HIP(hipMemcpyAsync(tables, host_tables.data(), host_tables.size(), hipMemcpyHostToDevice, st));
-  WorkBuffers wb;      // every buffer a slice of the arena
-  wb.max_lanes = 1;    // no second stream or events
-  set_scratch_arena(&arena);
-  const cyr_status s = run_simulation(desc, g, d_voxels, mats, d_out, wb, st, kRunResident, tables);
-  set_scratch_arena(nullptr);
+  ScratchArena arena;
+  auto attempt = [&](const cyr_sim_desc *d) -> cyr_status {
+    arena = ScratchArena{};
+    arena.base = slot->ptr;
+    arena.cap = kScratchBytes;
+    arena.stream = st;
+    // constant tables first (the executors read them as resident tables)
+    void *tables = arena.carve(host_tables.size());
+    if (!tables) return fail(CYR_E_NOMEM, "allocation-free call: tables exceed the scratch array");
+    CYR_HIP(hipMemcpyAsync(tables, host_tables.data(), host_tables.size(), hipMemcpyHostToDevice, st));
+    WorkBuffers wb;    // every buffer a slice of the arena
+    wb.max_lanes = 1;  // no second stream or events
+    set_scratch_arena(&arena);
+    const cyr_status s = run_simulation(d, g, d_voxels, mats, d_out, wb, st, kRunResident, tables);
+    set_scratch_arena(nullptr);
+    return s;
+  };
+  cyr_status s = attempt(desc);
+  if (s == CYR_E_NOMEM && fallback) {  // (Ewald bands wider than the model)
+    CYR_HIP(hipStreamSynchronize(st));
+    s = attempt(&plain);
+  }
   // drain the stream on errors too: no queued launch may outlive the host images
   const hipError_t se = hipStreamSynchronize(st);
   kt_collect();

@@ -27,11 +27,11 @@
 
 namespace cyr {
 
-// The fused E-basis kernels need 2^a 3^b 5^c in-plane lengths and tiles that fit
-// in LDS; FP64 runs them on native-precision morphologies only.  Other
-// simulations asking for E-basis run the plain executor.
+// The fused kernels need sides whose transforms fit their tiles (fused_supported:
+// any length up to 2048 and more); FP64 runs them on native-precision morphologies
+// only.  Other simulations run the plain executor.
 bool ebasis_usable(const cyr_sim_desc *d, const SimGeometry &g) {
-  return ebasis_supported(g.nx, g.ny, g.nz, d->precision) &&
+  return fused_supported(g.nx, g.ny, g.nz, d->precision) &&
          !(d->precision == CYR_FP64 && d->storage != CYR_STORE_NATIVE);
 }
 
@@ -50,6 +50,27 @@ int resolved_pipeline(const cyr_sim_desc *d, const SimGeometry &g) {
   const double eb = (double)g.nE * (double)g.V * (morph + 15.0 * cs);
   const double mb = (double)g.V * (morph + 4.0 * cs * nv) + (double)g.nE * (double)g.P * 4.0 * ng * nv * cs;
   return mb < eb ? CYR_PIPE_MBASIS : CYR_PIPE_EBASIS;
+}
+
+bool plain_fallback(const cyr_sim_desc *d, const SimGeometry &g) {
+  if (resolved_pipeline(d, g) == CYR_PIPE_PLAIN) return false;
+  for (uint32_t n : {g.nx, g.ny}) {
+    // radices 8 (or the remaining 4 or 2), 3 and 5: their least common multiple
+    uint32_t r = n, l = 1;
+    for (uint32_t p : {8u, 4u, 2u})
+      if (n % p == 0) {
+        l = p;
+        break;
+      }
+    if (n % 3 == 0) l *= 3;
+    if (n % 5 == 0) l *= 5;
+    for (uint32_t p : {2u, 3u, 5u})
+      while (r % p == 0) r /= p;
+    const bool ct = n == 64 || n == 128 || n == 256 || (n == 384 && d->precision != CYR_FP64) || n == 512 ||
+                    n == 1024 || n == 2048;
+    if (!ct && (r != 1 || l > (d->precision == CYR_FP64 ? 8u : 24u) || (l > 8 && l % 5 == 0))) return true;
+  }
+  return false;
 }
 
 namespace {
@@ -350,6 +371,22 @@ cyr_status run_plain(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
   return CYR_OK;
 }
 
+// Whether the quadratic-form coefficients (c^2, s^2, 2cs) of every angle a of the
+// first quarter turn equal, rounded to the compute precision, those of a + 2
+// quarter turns (and a + A4 those of a + 3 quarter turns): E turned by 180 degrees
+// gives the same intensity, so the orbit kernel forms one value for both pairs.
+template <typename T> bool quad_pairs_share(const SimGeometry &g, uint32_t k) {
+  const uint32_t A4 = g.quarter;
+  if (A4 == 0 || g.nA != 4 * A4) return false;
+  for (uint32_t a = 0; a < 2 * A4; a++) {
+    const double *x = &g.ebasis[2 * ((size_t)k * g.nA + a)], *y = &g.ebasis[2 * ((size_t)k * g.nA + a + 2 * A4)];
+    const double cx = x[0], sx = x[1], cy = y[0], sy = y[1];
+    if ((T)(cx * cx) != (T)(cy * cy) || (T)(sx * sx) != (T)(sy * sy) || (T)(2.0 * cx * sx) != (T)(2.0 * cy * sy))
+      return false;
+  }
+  return true;
+}
+
 // EBASIS: per (energy, k) unit the five tensor fields, their XY transforms, the
 // z DFT at the Ewald bins, then every angle as 2D work.  With two lanes, unit u
 // runs on stream u % 2 with its own work buffers and starts once unit u-1's
@@ -539,38 +576,25 @@ uint32_t mbasis_band_cap(const SimGeometry &g) {
   return cap > floor_cap ? cap : floor_cap;
 }
 
-// Whether the quadratic-form coefficients (c^2, s^2, 2cs) of every angle a of the
-// first quarter turn equal, rounded to the compute precision, those of a + 2
-// quarter turns (and a + A4 those of a + 3 quarter turns): E turned by 180 degrees
-// gives the same intensity, so the orbit kernel forms one value for both pairs.
-template <typename T> bool quad_pairs_share(const SimGeometry &g, uint32_t k) {
-  const uint32_t A4 = g.quarter;
-  if (A4 == 0 || g.nA != 4 * A4) return false;
-  for (uint32_t a = 0; a < 2 * A4; a++) {
-    const double *x = &g.ebasis[2 * ((size_t)k * g.nA + a)], *y = &g.ebasis[2 * ((size_t)k * g.nA + a + 2 * A4)];
-    const double cx = x[0], sx = x[1], cy = y[0], sy = y[1];
-    if ((T)(cx * cx) != (T)(cy * cy) || (T)(sx * sx) != (T)(sy * sy) || (T)(2.0 * cx * sx) != (T)(2.0 * cy * sy))
-      return false;
-  }
-  return true;
-}
-
 // MBASIS: per (k, energy group) the seven real basis fields of every material
 // (packed two per complex volume), their 3D FFTs, and their values in the band
 // of Ewald bins the group samples (plus the mirrored bins); then per energy the
 // transformed tensor fields at its bins as combinations with its constants, and
-// every angle as 2D work.
+// every angle as 2D work.  tensor: the same passes over the five complex tensor
+// fields of one energy at a time (E-basis on grids whose Ny has no compile-time
+// plan for the fused Y/z kernel).
 template <typename T>
-cyr_status run_mbasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d_vox, T *d_out, WorkBuffers &wb,
-                      hipStream_t s, const Setup<T> &su) {
+cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_vox, T *d_out, WorkBuffers &wb,
+                     hipStream_t s, const Setup<T> &su, bool tensor) {
   const uint64_t V = g.V, P = g.P;
   const bool hann = d->windowing == 1 && d->algorithm != 1;
   const bool three = g.nz > 1;
   const int ng = (three && d->interpolation == 1) ? 2 : 1;
-  const uint32_t nvol = mbasis_volumes(g.M), pass_max = nvol < 7 ? nvol : 7;
+  const uint32_t nvol = tensor ? kEbFields : mbasis_volumes(g.M), pass_max = nvol < 7 ? nvol : 7;
+  const uint64_t planes = tensor ? 1 : 2;  // band values: own, and those of the mirrored bins
   // laboratory frame: one quadratic form per pixel instead of every angle's projection
   const bool lab = d->reference_frame != 0;
-  const uint32_t nb = lab ? std::min(mbasis_energy_batch(g, sizeof(T)), g.nE) : 1;
+  const uint32_t nb = lab && !tensor ? std::min(mbasis_energy_batch(g, sizeof(T)), g.nE) : 1;
   LaneBuffers &lb = wb.lane[0];
   CYR_TRY(ensure_buffer(lb.pol, sizeof(cx<T>) * V * pass_max));
   CYR_TRY(ensure_buffer(lb.proj, sizeof(T) * P * (lab ? 4 * (uint64_t)nb : g.nA)));
@@ -596,7 +620,7 @@ cyr_status run_mbasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
   for (uint32_t k = 0; k < g.nK; k++) {
     const M3 Q = ebasis_frame(g, k);
     for (uint32_t e0 = 0; e0 < g.nE;) {
-      uint32_t ne = g.nE - e0, J = 0;
+      uint32_t ne = tensor ? 1 : g.nE - e0, J = 0;
       uint64_t wsum = 0;  // sum over columns of the band widths
       uint64_t ssum = 0;  // columns inside the row spans (those some band reads)
       uint64_t d4 = 0;    // (2 x the largest distance of a finite plane value from the centre)^2
@@ -608,14 +632,15 @@ cyr_status run_mbasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
         ne = (ne + 1) / 2;
       }
       if (J == 0) J = 1;  // no pixel sampled: the angles kernel writes NaN only
-      CYR_TRY(ensure_buffer(lb.part, sizeof(cx<T>) * 2 * (uint64_t)nvol * J * P));
+      CYR_TRY(ensure_buffer(lb.part, sizeof(cx<T>) * planes * nvol * J * P));
       cx<T> *own = reinterpret_cast<cx<T> *>(lb.part.ptr);
-      cx<T> *mir = own + (uint64_t)nvol * J * P;
+      cx<T> *mir = tensor ? nullptr : own + (uint64_t)nvol * J * P;
       // ---- basis spectra in the band: one pass per material pair (or single)
       for (uint32_t m0 = 0, vb = 0; m0 < g.M;) {
         const bool pair = m0 + 1 < g.M;
-        const uint32_t nv = pair ? 7 : 4;
+        const uint32_t nv = tensor ? kEbFields : pair ? 7 : 4;
         PolxArgs<T> xa{};
+        xa.mats = su.mats + (size_t)e0 * g.M;  // (tensor mode)
         xa.M = g.M;
         xa.m0 = m0;
         xa.V = V;
@@ -634,8 +659,9 @@ cyr_status run_mbasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
           vptr[c] = xa.out[c];
         }
         kt_begin(s);
-        CYR_TRY(launch_mbasis_xfields<T>(xa, pair, d_vox, d->storage, d->morphology_type, hann, s));
-        kt_end("xfields", s, (pair ? 2.0 : 1.0) * 4.0 * vel * V + nv * (double)V * cxb);
+        if (tensor) CYR_TRY(launch_ebasis_polx<T>(xa, d_vox, d->storage, d->morphology_type, hann, s));
+        else CYR_TRY(launch_mbasis_xfields<T>(xa, pair, d_vox, d->storage, d->morphology_type, hann, s));
+        kt_end("xfields", s, (tensor ? g.M : pair ? 2.0 : 1.0) * 4.0 * vel * V + nv * (double)V * cxb);
         FftDc fdc{dcz + (uint64_t)vb * dc_per, su.twz, span};
         if (!dc_slots) {
           DcArgs<T> da{};
@@ -669,26 +695,17 @@ cyr_status run_mbasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
         ba.nx = g.nx;
         ba.ny = g.ny;
         ba.nz = g.nz;
-        bool fused_z = false;
+        kt_begin(s);
         if (three) {
-          kt_begin(s);
-          CYR_TRY(launch_mbasis_zband<T>(ba, s, &fused_z));
           // reads the volumes' columns inside the row spans; writes each column's band
           // values and those of its mirror column (own + mir)
-          const double zcols = ba.span ? (double)ssum : (double)P;
-          if (fused_z) kt_end("mbasis_zband", s, nv * zcols * g.nz * cxb + 2.0 * nv * (double)wsum * cxb);
-          if (!fused_z) {
-            kt_begin(s);
-            CYR_TRY(fft_axis<T>(vptr, nv, g.nx, g.ny, g.nz, 2, s));
-            kt_end("fft_z", s, 2.0 * nv * (double)V * cxb);
-          }
-        }
-        if (!fused_z) {
-          kt_begin(s);
+          CYR_TRY(launch_mbasis_zband<T>(ba, s));
+          kt_end("mbasis_zband", s, nv * (double)ssum * g.nz * cxb + (double)planes * nv * (double)wsum * cxb);
+        } else {
           CYR_TRY(launch_mbasis_extract<T>(ba, s));
-          kt_end("mbasis_extract", s);
+          kt_end("mbasis_extract", s, 2.0 * planes * nv * (double)wsum * cxb);
         }
-        m0 += pair ? 2 : 1;
+        m0 += tensor ? g.M : pair ? 2 : 1;
         vb += nv;
       }
       CYR_TRY(launch_mbasis_dcsum(dcz, nvol, (uint32_t)dc_per, three, dcv, s));
@@ -701,7 +718,7 @@ cyr_status run_mbasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
       aa.mir = mir;
       aa.J = J;
       aa.dcv = dcv;
-      aa.M = g.M;
+      aa.M = tensor ? 0 : g.M;
       aa.amat = su.amat + (size_t)kEbAmat * k * g.nA;
       aa.nA = g.nA;
       aa.Q = m3<T>(Q);
@@ -719,7 +736,7 @@ cyr_status run_mbasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
           // unique inputs: the group's band values (own + mirror, each column's band
           // width, shared by its energies) and the band table; outputs: n
           // quadratic-form planes
-          kt_end("mbasis_quad", s, 2.0 * nvol * (double)wsum * cxb + 4.0 * P + n * (double)kQuadRecord * P * sizeof(T));
+          kt_end("mbasis_quad", s, (double)planes * nvol * (double)wsum * cxb + 4.0 * P + n * (double)kQuadRecord * P * sizeof(T));
           kt_begin(s);
           CYR_TRY(launch_rotate_quad<T>(proj, inv, su.quad + (size_t)3 * k * g.nA, su.quad_t + (size_t)3 * k * g.nA,
                                         g.nA, g.nx, g.ny, d->rot_mask, avg, n, su.tiles, g.quarter, su.otiles,
@@ -735,7 +752,7 @@ cyr_status run_mbasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
           aa.proj = proj;
           kt_begin(s);
           CYR_TRY(launch_mbasis_angles<T>(aa, ng, s));
-          kt_end("mbasis_angles", s, 2.0 * ng * nvol * (double)P * cxb + (double)g.nA * P * sizeof(T));
+          kt_end("mbasis_angles", s, (double)planes * ng * nvol * (double)P * cxb + (double)g.nA * P * sizeof(T));
           kt_begin(s);
           CYR_TRY(launch_rotate_all<T>(proj, inv, g.nA, g.nx, g.ny, d->rot_mask, avg, su.tiles,
                                        0.5 * std::sqrt((double)d4), s));
@@ -766,9 +783,19 @@ cyr_status run_impl(const cyr_sim_desc *d, const SimGeometry &g, const void *d_v
   Setup<T> su{};
   CYR_TRY(setup_views<T>(d, g, tb, tables, su));
   const int pipe = resolved_pipeline(d, g);
-  const cyr_status s = pipe == CYR_PIPE_PLAIN ? run_plain<T>(d, g, d_vox, d_out, wb, st, su)
-                       : pipe == CYR_PIPE_MBASIS ? run_mbasis<T>(d, g, d_vox, d_out, wb, st, su)
-                                                 : run_ebasis<T>(d, g, d_vox, d_out, wb, st, su);
+  cyr_status s = pipe == CYR_PIPE_PLAIN ? run_plain<T>(d, g, d_vox, d_out, wb, st, su)
+                 : pipe == CYR_PIPE_MBASIS ? run_bands<T>(d, g, d_vox, d_out, wb, st, su, false)
+                 : ebasis_yz_supported(g.ny, g.nz, d->precision) ? run_ebasis<T>(d, g, d_vox, d_out, wb, st, su)
+                                                                 : run_bands<T>(d, g, d_vox, d_out, wb, st, su, true);
+  if (s == CYR_E_NOMEM && !scratch_arena() && plain_fallback(d, g)) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    CYR_HIP(hipStreamIsCapturing(st, &cap));
+    if (cap == hipStreamCaptureStatusNone) {  // (capture follows an eager run, which sized the buffers)
+      CYR_HIP(hipStreamSynchronize(st));
+      for (auto &l : wb.lane) l.release();
+      s = run_plain<T>(d, g, d_vox, d_out, wb, st, su);
+    }
+  }
   if (mode != kRunSync) return s;
   // drain the stream on errors too, so no queued launch outlives the call's buffers
   const hipError_t se = hipStreamSynchronize(st);
@@ -905,7 +932,13 @@ uint64_t work_bytes(const cyr_sim_desc *d, const SimGeometry &g) {
   const uint64_t cs = d->precision == CYR_FP64 ? 16 : 8, rs = cs / 2;
   const int pipe = resolved_pipeline(d, g);
   uint64_t b = 0;
-  if (pipe == CYR_PIPE_MBASIS) {
+  if (pipe == CYR_PIPE_EBASIS && !ebasis_yz_supported(g.ny, g.nz, d->precision)) {
+    // run_bands over the tensor fields of one energy: volumes, its one or two band
+    // rows (a column's own bin and its interpolation partner), tables, DC sums, planes
+    const uint64_t planes = d->reference_frame != 0 ? 4 : g.nA;
+    b += cs * g.V * kEbFields + cs * 2 * kEbFields * g.P + 4 * g.P + 4 * mbasis_bmax_words(g.nx, g.ny) +
+         16 * kEbFields * (mbasis_dc_per(d, g) + 1) + rs * g.P * planes + 8 * g.P;
+  } else if (pipe == CYR_PIPE_MBASIS) {
     // one pass of packed volumes, band values (own + mirror, at most the band cap),
     // band table, DC sums, per-angle projections, average
     const uint64_t nv = mbasis_volumes(g.M), pass = nv < 7 ? nv : 7;
@@ -980,8 +1013,8 @@ template <typename T>
 cyr_status autotune_impl(const cyr_sim_desc *d, const SimGeometry &g, WorkBuffers &wb, hipStream_t st,
                          YzTuning *chosen) {
   *chosen = YzTuning{};
-  const bool ebasis = ebasis_usable(d, g);
-  if (!ebasis || g.nz < 2) return CYR_OK;  // 2D: one slice, nothing to split
+  // nothing to choose without the fused Y/z kernel or in 2D (one slice, nothing to split)
+  if (!ebasis_usable(d, g) || !ebasis_yz_supported(g.ny, g.nz, d->precision) || g.nz < 2) return CYR_OK;
   const uint64_t V = g.V, P = g.P;
   const int ng = d->interpolation == 1 ? 2 : 1;
   LaneBuffers &lb = wb.lane[0];

@@ -1,13 +1,5 @@
-// Stockham autosort stages shared by the FFT pencil kernels and the fused
-// E-basis kernels.
-//
-// Butterfly j (0 <= j < n/R) of a stage with sub-transform length Ls reads
-// x[j + r n/R], multiplies by W_{Ls R}^{r (j mod Ls)}, does an R-point DFT and
-// writes y[(j / Ls) Ls R + (j mod Ls) + r Ls].  A thread holds E elements
-// (E/R butterflies, j = t + b tpp).  Stage 0 reads from HBM (or from a caller
-// functor), intermediate stages exchange through LDS, and the last stage either
-// writes HBM or leaves its outputs in registers: after the last stage element
-// v[b R + r] is output index j_b + r n/R.
+// Radix butterflies and the LDS barrier shared by the transform codelets
+// (fftpolicy.hpp) and the any-length transforms (lfft.hpp).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -15,16 +7,6 @@
 #include "common.hpp"
 
 namespace cyr {
-
-constexpr int kMaxStages = 16;
-
-struct StagePlan {
-  uint32_t n;
-  uint32_t nstages;
-  uint32_t radix[kMaxStages];
-  uint32_t ls[kMaxStages];
-  uint32_t tstep[kMaxStages];
-};
 
 // Work-group barrier that orders LDS accesses only: outstanding global loads and
 // stores stay in flight across it (a prefetched slice, or the previous field's
@@ -109,121 +91,6 @@ template <typename T, int R> __device__ inline void bfly(cx<T> *a) {
   else if constexpr (R == 4) bfly4<T>(a);
   else if constexpr (R == 5) bfly5<T>(a);
   else bfly8<T>(a);
-}
-
-// Twiddles and butterflies of one stage on registers.  twlo (the residual
-// block of an FP32 table, or null) turns the twiddles into compensated products;
-// the caller passes it for the last stage only.
-template <typename T, int E, int R>
-__device__ inline void stage_compute(cx<T> (&v)[E], uint32_t t, uint32_t tpp, uint32_t Ls, uint32_t tstep,
-                                     const cx<T> *__restrict__ tw, const cx<T> *twlo = nullptr) {
-  constexpr int NB = E / R;
-#pragma unroll
-  for (int b = 0; b < NB; b++) {
-    const uint32_t j = t + b * tpp;
-    const uint32_t k = j % Ls;
-    if (k != 0) {
-      if (tw_blocks<T>() == 2 && twlo) {
-#pragma unroll
-        for (int r = 1; r < R; r++) v[b * R + r] = cmul_comp<T>(v[b * R + r], tw[r * k * tstep], twlo[r * k * tstep]);
-      } else {
-#pragma unroll
-        for (int r = 1; r < R; r++) v[b * R + r] = cmul<T>(v[b * R + r], tw[r * k * tstep]);
-      }
-    }
-    bfly<T, R>(&v[b * R]);
-  }
-}
-
-// LDS addressing of element e of the block's pencil p.
-struct LdsMap {
-  uint32_t pitch;
-  bool contig;
-  __device__ inline uint32_t operator()(uint32_t p, uint32_t e) const {
-    return contig ? p * pitch + e : e * pitch + p;
-  }
-};
-
-// Stage input from LDS in Stockham order.
-template <typename T, int E, int R>
-__device__ inline void stage_load_lds(cx<T> (&v)[E], uint32_t t, uint32_t tpp, uint32_t m, uint32_t p,
-                                      const cx<T> *lds, LdsMap L) {
-  constexpr int NB = E / R;
-#pragma unroll
-  for (int b = 0; b < NB; b++) {
-    const uint32_t j = t + b * tpp;
-#pragma unroll
-    for (int r = 0; r < R; r++) v[b * R + r] = lds[L(p, j + r * m)];
-  }
-}
-
-// Stage output to LDS in Stockham order.
-template <typename T, int E, int R>
-__device__ inline void stage_store_lds(const cx<T> (&v)[E], uint32_t t, uint32_t tpp, uint32_t Ls, uint32_t p,
-                                       cx<T> *lds, LdsMap L) {
-  constexpr int NB = E / R;
-#pragma unroll
-  for (int b = 0; b < NB; b++) {
-    const uint32_t j = t + b * tpp;
-    const uint32_t o0 = (j / Ls) * Ls * R + (j % Ls);
-#pragma unroll
-    for (int r = 0; r < R; r++) lds[L(p, o0 + r * Ls)] = v[b * R + r];
-  }
-}
-
-// Input position of register slot (b, r) in stage 0 (and of any stage with m = n/R).
-__device__ inline uint32_t stage_in_index(uint32_t t, uint32_t tpp, uint32_t m, int b, int r) {
-  return t + b * tpp + r * m;
-}
-
-// Runs stages [1, nstages) on registers that already hold the stage-0 inputs:
-// stage 0 compute, then LDS exchange for every later stage.  After return the
-// registers hold the final outputs in last-stage order (v[b R + r] = output
-// j_b + r n/R_last).  Uniform control flow: every thread of the block calls it.
-// The last stage's twiddles are compensated products with the residual block
-// twlo of an FP32 table.
-template <typename T, int E>
-__device__ inline void stockham_from_regs(cx<T> (&v)[E], const StagePlan &P, uint32_t t, uint32_t tpp, uint32_t p,
-                                          cx<T> *lds, LdsMap L, const cx<T> *__restrict__ tw,
-                                          const cx<T> *__restrict__ twlo) {
-  for (uint32_t s = 0; s < P.nstages; s++) {
-    const uint32_t R = P.radix[s], Ls = P.ls[s], ts = P.tstep[s], m = P.n / R;
-    if (s > 0) {
-      switch (R) {
-        case 2: if constexpr (E % 2 == 0) stage_load_lds<T, E, 2>(v, t, tpp, m, p, lds, L); break;
-        case 3: if constexpr (E % 3 == 0) stage_load_lds<T, E, 3>(v, t, tpp, m, p, lds, L); break;
-        case 4: if constexpr (E % 4 == 0) stage_load_lds<T, E, 4>(v, t, tpp, m, p, lds, L); break;
-        case 5: if constexpr (E % 5 == 0) stage_load_lds<T, E, 5>(v, t, tpp, m, p, lds, L); break;
-        default: if constexpr (E % 8 == 0) stage_load_lds<T, E, 8>(v, t, tpp, m, p, lds, L); break;
-      }
-      lds_sync();
-    }
-    const cx<T> *lo = s + 1 == P.nstages && tw_blocks<T>() == 2 ? twlo : nullptr;
-    switch (R) {
-      case 2: if constexpr (E % 2 == 0) stage_compute<T, E, 2>(v, t, tpp, Ls, ts, tw, lo); break;
-      case 3: if constexpr (E % 3 == 0) stage_compute<T, E, 3>(v, t, tpp, Ls, ts, tw, lo); break;
-      case 4: if constexpr (E % 4 == 0) stage_compute<T, E, 4>(v, t, tpp, Ls, ts, tw, lo); break;
-      case 5: if constexpr (E % 5 == 0) stage_compute<T, E, 5>(v, t, tpp, Ls, ts, tw, lo); break;
-      default: if constexpr (E % 8 == 0) stage_compute<T, E, 8>(v, t, tpp, Ls, ts, tw, lo); break;
-    }
-    if (s + 1 < P.nstages) {
-      switch (R) {
-        case 2: if constexpr (E % 2 == 0) stage_store_lds<T, E, 2>(v, t, tpp, Ls, p, lds, L); break;
-        case 3: if constexpr (E % 3 == 0) stage_store_lds<T, E, 3>(v, t, tpp, Ls, p, lds, L); break;
-        case 4: if constexpr (E % 4 == 0) stage_store_lds<T, E, 4>(v, t, tpp, Ls, p, lds, L); break;
-        case 5: if constexpr (E % 5 == 0) stage_store_lds<T, E, 5>(v, t, tpp, Ls, p, lds, L); break;
-        default: if constexpr (E % 8 == 0) stage_store_lds<T, E, 8>(v, t, tpp, Ls, p, lds, L); break;
-      }
-      lds_sync();
-    }
-  }
-}
-
-// Output index held by register slot i after stockham_from_regs: slot i = b R + r
-// of the last stage with radix R holds output (t + b tpp) + r n/R.
-__device__ inline uint32_t final_index(uint32_t t, uint32_t tpp, uint32_t n, uint32_t R_last, int i) {
-  const uint32_t b = (uint32_t)i / R_last, r = (uint32_t)i % R_last;
-  return t + b * tpp + r * (n / R_last);
 }
 
 }  // namespace cyr

@@ -1,7 +1,8 @@
 // Per-voxel fields + X FFT: the first kernel of both fused executors.
 //
-// A block holds pp rows of tpp threads (F::kE elements each); WG = 64 makes
-// every row exchange wave-local (the barriers compile to LDS waits).  LDS: the
+// A block holds pp rows of tpp threads (F::kE elements each); the compile-time
+// plans' WG = 64 makes every row exchange wave-local (the barriers compile to LDS
+// waits).  LDS: the
 // pp x row tile, plus the X twiddle table: the 4-7 FFTs per row read their
 // twiddles from LDS (the pair kernel's vector-memory instructions drop from 124 to
 // 34 per wave: 731 -> 621 us at 512^2 x 128; the tensor kernel 780 -> 742 us).
@@ -37,9 +38,6 @@
 namespace cyr {
 
 enum XMode { kXTensor = 0, kXPair = 1, kXSingle = 2 };
-// Every mode runs 4-7 FFTs per row: the X twiddles are staged in LDS once per block.
-template <int MODE> constexpr bool x_lds_twiddles() { return true; }
-
 template <int MODE> constexpr int x_outputs() { return MODE == kXTensor ? kEbFields : (MODE == kXPair ? 7 : 4); }
 
 // ---- the five tensor fields of one voxel -------------------------------------
@@ -169,12 +167,12 @@ __device__ inline void voxel_fields(const S *__restrict__ vox, const PolxArgs<T>
 
 // ---- fields + X FFT --------------------------------------------------------------
 template <typename T, typename S, class F, int WG, int MODE>
-__global__ void __launch_bounds__(WG, (MODE == kXTensor && F::kE <= 8) ? 4 : 2)
-    xfields_kernel(StagePlan P, PolxArgs<T> a, const S *__restrict__ vox, int morph, int hann) {
+__global__ void __launch_bounds__(WG, F::kCt && MODE == kXTensor && F::kE <= 8 ? 4 : 2)
+    xfields_kernel(typename F::Plan plan, PolxArgs<T> a, const S *__restrict__ vox, int morph, int hann) {
   constexpr int E = F::kE, NO = x_outputs<MODE>();
   extern __shared__ unsigned char smem_raw[];
   cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw);
-  const F fft(P, a.tpp, a.nx, true);
+  const F fft(plan);
   const uint32_t tpp = a.tpp;
   const uint32_t t = threadIdx.x % tpp, p = threadIdx.x / tpp;
   const uint32_t row = blockIdx.x * a.pp + p;  // row = y + ny z
@@ -188,14 +186,41 @@ __global__ void __launch_bounds__(WG, (MODE == kXTensor && F::kE <= 8) ? 4 : 2)
   // products here cost 12% of its time (512^2 x 128, material pair) and left the
   // FP32 pattern error unchanged to three digits; the later Y and Z passes
   // apply them.
-  const cx<T> *twp = a.twx;
-  if constexpr (x_lds_twiddles<MODE>()) {
-    cx<T> *ltw = lds + (size_t)a.pp * a.pitch;
-    // (run-time plans launch pp x tpp <= WG threads: stride by the actual block)
-    for (uint32_t i = threadIdx.x; i < a.nx; i += blockDim.x) ltw[i] = a.twx[i];
-    lds_sync();  // (single-wave blocks: an LDS wait only)
-    twp = ltw;
-  }
+  if constexpr (F::kCt) fft.stage(lds, a.pp, a.twx);
+  else fft.stage(lds, a.pp);
+  lds_sync();  // (single-wave blocks: an LDS wait only)
+  // fill(c, v) forms output c, which is transformed and written.  Compile-time plans
+  // unroll the outputs; the any-length transform is too large to copy per output.
+  auto each_output = [&](auto fill) {
+    auto emit = [&](cx<T>(&v)[E], cx<T> *vol) {
+      cx<T> *o = vol + (uint64_t)(active ? row : 0) * a.nx;
+      // (transform() ends with a barrier after its last LDS reads, so the next
+      // output's first LDS store cannot overtake them)
+      fft.transform(v, t, p, a.pp, lds, [&](uint32_t k, cx<T> x) {
+        if (active) o[k] = x;
+      });
+    };
+    if constexpr (F::kCt) {
+      static_for<0, NO>([&](auto cc) {
+        cx<T> v[E];
+        fill(cc, v);
+        emit(v, a.out[decltype(cc)::value]);
+      });
+    } else {
+#pragma unroll 1
+      for (uint32_t c = blockIdx.y; c < (uint32_t)NO; c += gridDim.y) {
+        cx<T> v[E];
+        cx<T> *vol = nullptr;
+        static_for<0, NO>([&](auto cc) {  // (uniform)
+          if (c == (uint32_t)decltype(cc)::value) {
+            fill(cc, v);
+            vol = a.out[decltype(cc)::value];
+          }
+        });
+        emit(v, vol);
+      }
+    }
+  };
   if constexpr (MODE == kXPair) {
     // Material pair: a compact per-material state per element (window-weighted
     // phi_a, the second scalar field, the director s'; 5-6 values instead of the
@@ -209,11 +234,12 @@ __global__ void __launch_bounds__(WG, (MODE == kXTensor && F::kE <= 8) ? 4 : 2)
 #pragma unroll
       for (int i = 0; i < E; i++) {
         const uint32_t x = fft.in_pos(t, i);
-        const T w = active ? (hann ? a.hx[x] * wyz : wyz) : (T)0;
+        const bool in = active && fft.holds(t, i);
+        const T w = in ? (hann ? a.hx[x] * wyz : wyz) : (T)0;
 #pragma unroll
         for (int m = 0; m < 2; m++) {
           T vv[4] = {0, 0, 0, 0};
-          if (active) VoxLoad<T, S>::get(vox, (uint64_t)(a.m0 + m) * a.V + (uint64_t)row * a.nx + x, vv);
+          if (in) VoxLoad<T, S>::get(vox, (uint64_t)(a.m0 + m) * a.V + (uint64_t)row * a.nx + x, vv);
           T sx, sy, sz;
           if constexpr (MORPH == 1) {  // alpha = |s|^2, beta = phi_u, phi_a = 1
             sx = vv[0];
@@ -248,9 +274,8 @@ __global__ void __launch_bounds__(WG, (MODE == kXTensor && F::kE <= 8) ? 4 : 2)
       }
       // outputs c = 0..6: (alpha, beta, q00, q11, q01, q02, q12) of material m0
       // (real part) and m0 + 1 (imaginary part), q_ij = phi_a s'_i s'_j
-      static_for<0, NO>([&](auto cc) {
+      each_output([&](auto cc, cx<T>(&v)[E]) {
         constexpr int c = decltype(cc)::value;
-        cx<T> v[E];
 #pragma unroll
         for (int i = 0; i < E; i++) {
           T f[2];
@@ -266,12 +291,6 @@ __global__ void __launch_bounds__(WG, (MODE == kXTensor && F::kE <= 8) ? 4 : 2)
           }
           v[i] = mk<T>(f[0], f[1]);
         }
-        fft.template run<false>(v, t, p, lds, twp, nullptr);
-        if (active) {
-          cx<T> *o = a.out[c] + (uint64_t)row * a.nx;
-#pragma unroll
-          for (int i = 0; i < E; i++) o[fft.out_pos(t, i)] = v[i];
-        }
       });
     };
     if (morph == 1) pair_rows(std::integral_constant<int, 1>{});
@@ -283,7 +302,7 @@ __global__ void __launch_bounds__(WG, (MODE == kXTensor && F::kE <= 8) ? 4 : 2)
   for (int i = 0; i < E; i++) {
     const uint32_t x = fft.in_pos(t, i);
     T fr[NO], fi[NO];
-    if (active) {
+    if (active && fft.holds(t, i)) {
       const uint64_t idx = (uint64_t)row * a.nx + x;
       if (morph == 1) voxel_fields<T, S, 1, MODE>(vox, a, idx, rot, fr, fi);
       else voxel_fields<T, S, 0, MODE>(vox, a, idx, rot, fr, fi);
@@ -303,44 +322,26 @@ __global__ void __launch_bounds__(WG, (MODE == kXTensor && F::kE <= 8) ? 4 : 2)
       fim[c][i] = fi[c];
     }
   }
-  static_for<0, NO>([&](auto cc) {
+  each_output([&](auto cc, cx<T>(&v)[E]) {
     constexpr int c = decltype(cc)::value;
-    cx<T> v[E];
 #pragma unroll
     for (int i = 0; i < E; i++) v[i] = mk<T>(fre[c][i], fim[c][i]);
-    fft.template run<false>(v, t, p, lds, twp, nullptr);
-    if (active) {
-      cx<T> *o = a.out[c] + (uint64_t)row * a.nx;
-#pragma unroll
-      for (int i = 0; i < E; i++) o[fft.out_pos(t, i)] = v[i];
-    }
-    // (run() ends with a barrier after its last LDS reads, so the next field's
-    // first LDS store cannot overtake them)
   });
 }
 
 // ---- plan helpers shared by the fused executors ------------------------------
-// Elements-per-thread instantiations: FP32 up to 24 (radix lcm x 2^k), FP64 up to 8.
-template <typename T> constexpr bool e_allowed(int E) { return sizeof(T) == 4 || E <= 8; }
-
 // Launch shape of the compile-time X plans: rows of <= 64 threads share a wave.
 constexpr int ct_polx_wg(int N, int E) { return N / E <= 64 ? 64 : N / E; }
 
-// Elements per thread for a pencil of length n: the radix lcm, doubled while the
-// pencil would need more than `tpp_cap` threads.
-inline uint32_t choose_e(uint32_t n, uint32_t lcm, uint32_t tpp_cap, uint32_t e_cap) {
-  uint32_t E = lcm;
-  while (n / E > tpp_cap && E * 2 <= e_cap && n % (E * 2) == 0) E *= 2;
-  return E;
-}
-
-// Elements-per-thread values with a compiled run-time-plan kernel.
-inline bool e_instantiated(uint32_t E, int precision) {
-  switch (E) {
-    case 2: case 3: case 4: case 5: case 6: case 8: return true;
-    case 12: case 16: case 24: return precision != CYR_FP64;
-    default: return false;
-  }
+// Elements per thread of the any-length X plans (their per-element state fills the
+// registers): 4, and 8 for FP32 rows that would need more than kLfXThreads threads.
+constexpr uint32_t kLfXThreads = 512;
+constexpr uint64_t kXSplitThreads = 256 * 512;  // two waves per SIMD
+inline bool lf_x_shape(const LfPlan &P, int precision, LfShape &s, uint32_t &e) {
+  e = 4;
+  if (lf_rows_shape(P, precision, 4, kLfXThreads, true, s)) return true;
+  e = 8;
+  return precision != CYR_FP64 && lf_rows_shape(P, precision, 8, kLfXThreads, true, s);
 }
 
 // The compile-time plan applies (its elements per thread are compiled for T).
@@ -348,65 +349,51 @@ inline bool ct_usable(uint32_t n, int precision) {
   return ct_length(n) && (precision != CYR_FP64 || ct_elements(n) <= 8);
 }
 
-template <typename T, typename S, int E, int MODE>
-hipError_t launch_xfields_rt(dim3 grid, dim3 block, size_t lds, hipStream_t st, const StagePlan &P,
-                             const PolxArgs<T> &a, const void *vox, int morph, int hann) {
-  hipLaunchKernelGGL((xfields_kernel<T, S, RtFft<T, E>, 256, MODE>), grid, block, lds, st, P, a, (const S *)vox,
-                     morph, hann);
-  return hipGetLastError();
+// Blocks over which the any-length outputs are split (each evaluates the voxels again,
+// from L2): all of them when the rows alone leave the chip short of waves, so that the
+// chain of transforms that a block runs one after another is one transform long
+// (101 x 94 x 21, a pair: 120 -> 58 us).  Not for the compile-time plans, whose
+// transforms are short (64^3: 13.7 against 15.2 us), nor for FP64, whose sines cost
+// more than the chain (64^3: 40 against 79 us).
+template <typename T, int MODE> uint32_t x_split(uint64_t blocks, uint32_t threads) {
+  return sizeof(T) == 4 && blocks * threads < kXSplitThreads ? (uint32_t)x_outputs<MODE>() : 1;
 }
 
-template <typename T, typename S, int MODE>
-hipError_t launch_xfields_rt_e(uint32_t E, dim3 grid, dim3 block, size_t lds, hipStream_t st, const StagePlan &P,
-                               const PolxArgs<T> &a, const void *vox, int morph, int hann, bool *found) {
-  *found = true;
-#define CYR_PX(EV)                                                                                             \
-  case EV:                                                                                                     \
-    if constexpr (e_allowed<T>(EV))                                                                            \
-      return launch_xfields_rt<T, S, EV, MODE>(grid, block, lds, st, P, a, vox, morph, hann);                 \
-    break;
-  switch (E) {
-    CYR_PX(2)
-    CYR_PX(3)
-    CYR_PX(4)
-    CYR_PX(5)
-    CYR_PX(6)
-    CYR_PX(8)
-    CYR_PX(12)
-    CYR_PX(16)
-    CYR_PX(24)
-    default:
-      break;
-  }
-#undef CYR_PX
-  *found = false;
-  return hipSuccess;
+template <typename T, typename S, int E, int MODE>
+hipError_t launch_xfields_lf(const LfTab<T> &tb, const LfShape &sh, hipStream_t st, const PolxArgs<T> &a,
+                             const void *vox, int morph, int hann) {
+  using F = LfRowFft<T, E>;
+  const typename F::Plan plan{tb, sh.tpp, sh.pitch, sh.pad};
+  hipLaunchKernelGGL((xfields_kernel<T, S, F, kLfXThreads, MODE>),
+                     dim3(ceil_div(a.rows, sh.pp), x_split<T, MODE>(ceil_div(a.rows, sh.pp), sh.pp * sh.tpp)),
+                     dim3(sh.pp * sh.tpp), sh.lds, st, plan, a, (const S *)vox, morph, hann);
+  return hipGetLastError();
 }
 
 template <typename T, typename S, int N, int MODE>
-hipError_t launch_xfields_ct(dim3 grid, size_t lds, hipStream_t st, const StagePlan &P, const PolxArgs<T> &a,
-                             const void *vox, int morph, int hann) {
+hipError_t launch_xfields_ct(dim3 grid, size_t lds, hipStream_t st, const PolxArgs<T> &a, const void *vox, int morph,
+                             int hann) {
   using F = typename CtPlan<T, N, true, 1>::type;
   constexpr int WG = ct_polx_wg(N, F::kE);
-  hipLaunchKernelGGL((xfields_kernel<T, S, F, WG, MODE>), grid, dim3(WG), lds, st, P, a, (const S *)vox, morph,
-                     hann);
+  hipLaunchKernelGGL((xfields_kernel<T, S, F, WG, MODE>), grid, dim3(WG), lds, st, typename F::Plan{}, a,
+                     (const S *)vox, morph, hann);
   return hipGetLastError();
 }
 
 template <typename T, typename S, int MODE>
-hipError_t launch_xfields_ct_n(uint32_t n, dim3 grid, size_t lds, hipStream_t st, const StagePlan &P,
-                               const PolxArgs<T> &a, const void *vox, int morph, int hann, bool *found) {
+hipError_t launch_xfields_ct_n(uint32_t n, dim3 grid, size_t lds, hipStream_t st, const PolxArgs<T> &a,
+                               const void *vox, int morph, int hann, bool *found) {
   *found = true;
   switch (n) {
-    case 64: return launch_xfields_ct<T, S, 64, MODE>(grid, lds, st, P, a, vox, morph, hann);
-    case 128: return launch_xfields_ct<T, S, 128, MODE>(grid, lds, st, P, a, vox, morph, hann);
-    case 256: return launch_xfields_ct<T, S, 256, MODE>(grid, lds, st, P, a, vox, morph, hann);
+    case 64: return launch_xfields_ct<T, S, 64, MODE>(grid, lds, st, a, vox, morph, hann);
+    case 128: return launch_xfields_ct<T, S, 128, MODE>(grid, lds, st, a, vox, morph, hann);
+    case 256: return launch_xfields_ct<T, S, 256, MODE>(grid, lds, st, a, vox, morph, hann);
     case 384:
-      if constexpr (e_allowed<T>(12)) return launch_xfields_ct<T, S, 384, MODE>(grid, lds, st, P, a, vox, morph, hann);
+      if constexpr (sizeof(T) == 4) return launch_xfields_ct<T, S, 384, MODE>(grid, lds, st, a, vox, morph, hann);
       break;
-    case 512: return launch_xfields_ct<T, S, 512, MODE>(grid, lds, st, P, a, vox, morph, hann);
-    case 1024: return launch_xfields_ct<T, S, 1024, MODE>(grid, lds, st, P, a, vox, morph, hann);
-    case 2048: return launch_xfields_ct<T, S, 2048, MODE>(grid, lds, st, P, a, vox, morph, hann);
+    case 512: return launch_xfields_ct<T, S, 512, MODE>(grid, lds, st, a, vox, morph, hann);
+    case 1024: return launch_xfields_ct<T, S, 1024, MODE>(grid, lds, st, a, vox, morph, hann);
+    case 2048: return launch_xfields_ct<T, S, 2048, MODE>(grid, lds, st, a, vox, morph, hann);
     default: break;
   }
   *found = false;
@@ -416,32 +403,37 @@ hipError_t launch_xfields_ct_n(uint32_t n, dim3 grid, size_t lds, hipStream_t st
 // Plans and launches the fields + X FFT kernel of one MODE.
 template <typename T, int MODE>
 cyr_status launch_xfields(PolxArgs<T> a, const void *vox, int storage, int morph, bool hann, hipStream_t st) {
-  StagePlan P;
-  uint32_t lcm;
-  if (!make_stage_plan(a.nx, P, lcm)) return fail(CYR_E_UNSUPPORTED, "fused X kernel: Nx must be 2^a 3^b 5^c");
   const int prec = sizeof(T) == 8 ? CYR_FP64 : CYR_FP32;
   const bool ct = ct_usable(a.nx, prec);
-  const uint32_t E = ct ? ct_elements(a.nx) : choose_e(a.nx, lcm, 256, sizeof(T) == 8 ? 8 : 16);
-  a.tpp = a.nx / E;
-  if (a.tpp > 256) return fail(CYR_E_UNSUPPORTED, "fused X kernel: row needs more than 256 threads");
-  // compile-time plans: rows of <= 64 threads share one wave; the run-time plan
-  // packs rows into 256-thread blocks
-  const uint32_t wg = ct ? (a.tpp <= 64 ? 64u : a.tpp) : 256u;
-  a.pp = wg / a.tpp;
-  if (a.pp < 1) a.pp = 1;
-  a.pitch = ct ? ct_row_pitch(a.nx) : a.nx;
-  const size_t lds = ((size_t)a.pp * a.pitch + (x_lds_twiddles<MODE>() ? a.nx : 0)) * sizeof(cx<T>);
-  if (lds > device_max_lds()) return fail(CYR_E_UNSUPPORTED, "fused X kernel: row does not fit in LDS");
-  cyr_status s;
-  a.twx = twiddles<T>(a.nx, &s);
-  if (!a.twx) return s;
-  const dim3 grid(ceil_div(a.rows, a.pp)), block(a.pp * a.tpp);
-  bool found = false;
+  LfTab<T> tb{};
+  LfShape sh;
+  uint32_t e_lf = 0;
+  size_t lds = 0;
+  if (ct) {
+    // rows of <= 64 threads share one wave
+    a.tpp = a.nx / ct_elements(a.nx);
+    a.pp = a.tpp <= 64 ? 64 / a.tpp : 1;
+    lds = ((size_t)a.pp * ct_row_pitch(a.nx) + a.nx) * sizeof(cx<T>);
+    if (lds > device_max_lds()) return fail(CYR_E_UNSUPPORTED, "fused X kernel: row does not fit in LDS");
+    cyr_status s;
+    a.twx = twiddles<T>(a.nx, &s);
+    if (!a.twx) return s;
+  } else {
+    LfPlan P;
+    if (!lf_plan(a.nx, prec, P) || !lf_x_shape(P, prec, sh, e_lf))
+      return fail(CYR_E_UNSUPPORTED, "fused X kernel: row does not fit its block");
+    CYR_TRY(lf_tables<T>(P, tb));
+    a.tpp = sh.tpp;
+    a.pp = sh.pp;
+  }
+  const dim3 grid(ceil_div(a.rows, a.pp));
+  bool found = true;
   hipError_t e = hipSuccess;
   auto go = [&](auto tag) {
     using S = decltype(tag);
-    if (ct) e = launch_xfields_ct_n<T, S, MODE>(a.nx, grid, lds, st, P, a, vox, morph, hann ? 1 : 0, &found);
-    else e = launch_xfields_rt_e<T, S, MODE>(E, grid, block, lds, st, P, a, vox, morph, hann ? 1 : 0, &found);
+    if (ct) e = launch_xfields_ct_n<T, S, MODE>(a.nx, grid, lds, st, a, vox, morph, hann ? 1 : 0, &found);
+    else if (e_lf == 4) e = launch_xfields_lf<T, S, 4, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
+    else if constexpr (sizeof(T) == 4) e = launch_xfields_lf<T, S, 8, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
   };
   if constexpr (sizeof(T) == 4) {
     if (storage == CYR_STORE_FP16) go(half4{});
@@ -454,6 +446,19 @@ cyr_status launch_xfields(PolxArgs<T> a, const void *vox, int storage, int morph
   if (e != hipSuccess) return hip_fail(e, "xfields_kernel", __FILE__, __LINE__);
   if (!found) return fail(CYR_E_UNSUPPORTED, "fused X kernel: no kernel for this length");
   return CYR_OK;
+}
+
+// The launchers of kernels.hpp, instantiated per precision in a file of its own.
+template <typename T>
+cyr_status launch_ebasis_polx(PolxArgs<T> a, const void *vox, int storage, int morph, bool hann, hipStream_t st) {
+  return launch_xfields<T, kXTensor>(a, vox, storage, morph, hann, st);
+}
+
+template <typename T>
+cyr_status launch_mbasis_xfields(PolxArgs<T> a, bool pair, const void *vox, int storage, int morph, bool hann,
+                                 hipStream_t st) {
+  if (pair) return launch_xfields<T, kXPair>(a, vox, storage, morph, hann, st);
+  return launch_xfields<T, kXSingle>(a, vox, storage, morph, hann, st);
 }
 
 }  // namespace cyr
