@@ -15,7 +15,7 @@
 //     iso = (n_perp^2 - 1) |s|^2 + phi_u (n_iso^2 - 1)      (vector, phi_a = 1)
 // (the reference's "- Vfrac" on the diagonal is folded in analytically).
 //
-// Four launches per (energy, k):
+// Five launches per (energy, k), then the rotation:
 //   ebasis_bins_kernel   pixel -> FFT z bin of its (kx, ky) column (FP64 geometry);
 //                        with linear interpolation the second bin is bin - 1 (mod Nz)
 //   xfields_kernel       (xfields.hpp, tensor mode) the five fields evaluated at the
@@ -27,9 +27,12 @@
 //                        chunks with per-chunk partial sums (deterministic, no
 //                        atomics).  The DC replacement's neighbour bins are
 //                        accumulated on the side.  Gx is read exactly once.
-//   ebasis_angles_kernel sums the chunks, applies the DC replacement, and for every
-//                        angle forms p~ = A(theta) F (A = frame x E coefficients,
-//                        3 x 5, FP64-built) and the Ewald intensity.
+//   ebasis_dc_kernel     the DC replacement's neighbour sums
+//   ebasis_quad_kernel   laboratory frame: sums the chunks, applies the DC replacement
+//                        and writes the pixel's quadratic form (quadform.hpp), which
+//                        the rotation evaluates at every angle
+//   ebasis_angles_kernel material frame: for every angle p~ = A(theta) F (A = frame x
+//                        E coefficients, 3 x 5, FP64-built) and the Ewald intensity
 // Grids whose Ny has no compile-time codelet take the band passes of mbasis.hip over
 // the five tensor fields instead of ebasis_yz_kernel.
 //
@@ -44,6 +47,7 @@
 #include "geom.hpp"
 #include "fftpolicy.hpp"
 #include "kernels.hpp"
+#include "quadform.hpp"
 #include "stockham.hpp"
 #include "tensor.hpp"
 #include "xfields.hpp"
@@ -211,12 +215,14 @@ __global__ void __launch_bounds__(256) ebasis_dc_kernel(DcArgs<T> a) {
   }
 }
 
-// ---- chunk sums, DC, and every angle's intensity -----------------------------
+// ---- chunk sums and DC: the tensor fields at a pixel's Ewald bins ------------------
+// Pixel t of the block's range; false: a NaN pixel (or past the plane).  Every thread
+// of the block calls it (barriers inside).
 template <typename T, int NG>
-__global__ void __launch_bounds__(256) ebasis_angles_kernel(AnglesArgs<T> a) {
+__device__ inline bool eb_fields(const AnglesArgs<T> &a, uint64_t t, uint32_t &X, uint32_t &Y,
+                                 cx<T> (&F)[NG][kEbFields], double (&md)[NG][6], T &w1) {
   const EwaldGeom &g = a.g;
   const uint64_t P2 = (uint64_t)g.nx * g.ny;
-  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   // the block holding the pixel of FFT bin (0, 0) (X = Nx/2, Y = Ny/2) first sums
   // the per-slice DC-neighbour partials (fixed-order tree, deterministic)
   __shared__ double dcs[2 * kEbFields][256];
@@ -245,31 +251,30 @@ __global__ void __launch_bounds__(256) ebasis_angles_kernel(AnglesArgs<T> a) {
     }
     __syncthreads();
   }
-  if (t >= P2) return;
-  const uint32_t Y = (uint32_t)(t / g.nx), X = (uint32_t)(t - (uint64_t)Y * g.nx);
+  if (t >= P2) return false;
+  Y = (uint32_t)(t / g.nx);
+  X = (uint32_t)(t - (uint64_t)Y * g.nx);
   uint32_t z0 = 0;
   double f = 0;
-  const int kind = ewald_geometry(g, X, Y, &z0, &f);
-  if (kind == 0) {
-    for (uint32_t an = 0; an < a.nA; an++) a.proj[(uint64_t)an * P2 + t] = qnan<T>();
-    return;
-  }
+  if (ewald_geometry(g, X, Y, &z0, &f) == 0) return false;
   const uint32_t ix = unshift(X, g.nx), iy = unshift(Y, g.ny);
   const uint64_t col = (uint64_t)iy * g.nx + ix;
   const bool three = !g.enable2d;
-  cx<T> F[NG][kEbFields];
 #pragma unroll
   for (int q = 0; q < NG; q++)
 #pragma unroll
-    for (int c = 0; c < kEbFields; c++) {
-      cx<T> s = mk<T>(0, 0);
-      for (uint32_t ch = 0; ch < a.nchunks; ch++) {
+    for (int c = 0; c < kEbFields; c++) F[q][c] = mk<T>(0, 0);
+  // (a chunk's values are independent loads, all in flight together)
+  for (uint32_t ch = 0; ch < a.nchunks; ch++) {
+#pragma unroll
+    for (int q = 0; q < NG; q++)
+#pragma unroll
+      for (int c = 0; c < kEbFields; c++) {
         const cx<T> v = a.part[(((uint64_t)ch * NG + q) * kEbFields + c) * P2 + col];
-        s.x += v.x;
-        s.y += v.y;
+        F[q][c].x += v.x;
+        F[q][c].y += v.y;
       }
-      F[q][c] = s;
-    }
+  }
   if (ix == 0 && iy == 0) {
 #pragma unroll
     for (int q = 0; q < NG; q++) {
@@ -279,10 +284,49 @@ __global__ void __launch_bounds__(256) ebasis_angles_kernel(AnglesArgs<T> a) {
       for (int c = 0; c < kEbFields; c++) F[q][c] = dcv[c];
     }
   }
-  double md[NG][6];
 #pragma unroll
   for (int q = 0; q < NG; q++) scatter_matrix(g, X, Y, three ? z0 + q : 0, md[q]);
-  const T w1 = (T)f;
+  w1 = (T)f;
+  return true;
+}
+
+// ---- laboratory frame: the quadratic form ------------------------------------------
+// One record per pixel (12 B) in place of every angle's projection written here and
+// gathered again by the rotation (4 B per pixel and angle each way): one energy of
+// 256^2 x 64 with 36 angles, 47 + 33 us for the two kernels.
+template <typename T, int NG>
+__global__ void __launch_bounds__(256) ebasis_quad_kernel(AnglesArgs<T> a) {
+  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  uint32_t X, Y;
+  cx<T> F[NG][kEbFields];
+  double md[NG][6];
+  T w1;
+  const bool fine = eb_fields<T, NG>(a, t, X, Y, F, md, w1);
+  if (t >= (uint64_t)a.g.nx * a.g.ny) return;
+  if (!fine) {
+    Y = (uint32_t)(t / a.g.nx);
+    X = (uint32_t)(t - (uint64_t)Y * a.g.nx);
+  }
+  T *o = a.quad + (uint64_t)quad_index(X, Y, a.g.nx, a.g.ny) * kQuadRecord;
+  if (!fine) o[0] = o[1] = o[2] = qnan<T>();
+  else quad_form_write<T, NG>(a.Q, F, md, w1, o);
+}
+
+// ---- material frame: every angle's intensity ----------------------------------------
+template <typename T, int NG>
+__global__ void __launch_bounds__(256) ebasis_angles_kernel(AnglesArgs<T> a) {
+  const uint64_t P2 = (uint64_t)a.g.nx * a.g.ny;
+  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  uint32_t X, Y;
+  cx<T> F[NG][kEbFields];
+  double md[NG][6];
+  T w1;
+  const bool fine = eb_fields<T, NG>(a, t, X, Y, F, md, w1);
+  if (t >= P2) return;
+  if (!fine) {
+    for (uint32_t an = 0; an < a.nA; an++) a.proj[(uint64_t)an * P2 + t] = qnan<T>();
+    return;
+  }
 #pragma unroll 4
   for (uint32_t an = 0; an < a.nA; an++) {
     const T *A = a.amat + (uint64_t)kEbAmat * an;
@@ -478,8 +522,14 @@ template <typename T> cyr_status launch_ebasis_dc(const DcArgs<T> &a, hipStream_
 template <typename T> cyr_status launch_ebasis_angles(const AnglesArgs<T> &a, int ng, hipStream_t st) {
   const uint64_t P = (uint64_t)a.g.nx * a.g.ny;
   const dim3 grid(ceil_div(P, 256)), block(256);
-  if (ng == 2) hipLaunchKernelGGL((ebasis_angles_kernel<T, 2>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((ebasis_angles_kernel<T, 1>), grid, block, 0, st, a);
+  if (a.quad) {
+    if (ng == 2) hipLaunchKernelGGL((ebasis_quad_kernel<T, 2>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((ebasis_quad_kernel<T, 1>), grid, block, 0, st, a);
+  } else if (ng == 2) {
+    hipLaunchKernelGGL((ebasis_angles_kernel<T, 2>), grid, block, 0, st, a);
+  } else {
+    hipLaunchKernelGGL((ebasis_angles_kernel<T, 1>), grid, block, 0, st, a);
+  }
   CYR_LAUNCHED();
   return CYR_OK;
 }

@@ -135,7 +135,9 @@ template <typename T> struct AnglesArgs {
   const double2 *dcz;
   const T *amat;                   // [nA][kEbAmat]
   uint32_t nA;
-  T *proj;                         // [nA][Ny][Nx]
+  T *proj;                         // [nA][Ny][Nx] (material frame), or
+  T *quad;                         // [P][3] in quad_index order (laboratory frame)
+  Mat3<T> Q;                       // frame e1, e2, k^ (quadratic form)
 };
 template <typename T> cyr_status launch_ebasis_angles(const AnglesArgs<T> &a, int ng, hipStream_t st);
 

@@ -35,20 +35,32 @@ bool ebasis_usable(const cyr_sim_desc *d, const SimGeometry &g) {
          !(d->precision == CYR_FP64 && d->storage != CYR_STORE_NATIVE);
 }
 
-// HBM bytes per voxel (E-basis: per energy and k vector; material basis: per k
-// vector) and per pixel and energy.  The E-basis Y/z kernel is ALU-bound at about
-// twice its bytes, so its reads count double.  Measured at 512^2 x 128, 4
-// materials: E-basis 1.26 ms per energy, material basis 3.7 ms per k + 0.05 ms
-// per energy; the model's break-even (2.8 energies) matches.
+// The executor of CYR_PIPE_AUTO, by the HBM bytes each would move per k vector (a
+// launch counts as the 24 MB that move in its 4 us):
+//   E-basis, per energy: the morphology, five complex fields written and read by the
+//     fused Y/z kernel (ALU-bound at twice its bytes: 15 values; other Ny: written,
+//     transformed along Y and read, 20 values), 8 (11) launches;
+//   material basis: the morphology once and nv packed volumes written, transformed
+//     and read, 3 launches per material pass and 8 more; then, per energy, the band
+//     gathers of the pixels on the detector's Ewald disc, 2 ng nv values each.
+// Rotation and output are the same in both.  Measured at 512^2 x 128, 4 materials:
+// E-basis 1.26 ms per energy, material basis 3.7 ms per k + 0.05 ms per energy (model:
+// break-even at 2.8); 2048^2 x 1, 50 energies x 180 angles: 28 ms against 9.4 ms (a
+// model that charged every pixel the whole gathers chose E-basis).
 int resolved_pipeline(const cyr_sim_desc *d, const SimGeometry &g) {
   if (d->pipeline == CYR_PIPE_PLAIN || !ebasis_usable(d, g)) return CYR_PIPE_PLAIN;
   if (d->pipeline != CYR_PIPE_AUTO) return d->pipeline;
   const double cs = d->precision == CYR_FP64 ? 16.0 : 8.0;
   const double el = d->storage == CYR_STORE_NATIVE ? cs / 2 : 2.0;
   const double nv = mbasis_volumes(g.M), ng = (g.nz > 1 && d->interpolation == 1) ? 2.0 : 1.0;
-  const double morph = 4.0 * el * g.M;
-  const double eb = (double)g.nE * (double)g.V * (morph + 15.0 * cs);
-  const double mb = (double)g.V * (morph + 4.0 * cs * nv) + (double)g.nE * (double)g.P * 4.0 * ng * nv * cs;
+  const double morph = 4.0 * el * g.M, V = (double)g.V, nE = (double)g.nE, launch = 24e6;
+  const bool yz = ebasis_yz_supported(g.ny, g.nz, d->precision);
+  // share of the pixels with |q| < k: a disc of radius k in a square of side 2 pi / d
+  const double kd = g.kmag.empty() ? 0.0 : g.kmag.back() * d->phys_size;
+  const double disc = std::min(1.0, kd * kd / (4.0 * M_PI));
+  const double eb = nE * (V * (morph + (yz ? 15.0 : 20.0) * cs) + (yz ? 8.0 : 11.0) * launch);
+  const double mb = V * (morph + 4.0 * cs * nv) + (8.0 + 3.0 * ((g.M + 1) / 2)) * launch +
+                    nE * (double)g.P * disc * 2.0 * ng * nv * cs;
   return mb < eb ? CYR_PIPE_MBASIS : CYR_PIPE_EBASIS;
 }
 
@@ -387,6 +399,14 @@ template <typename T> bool quad_pairs_share(const SimGeometry &g, uint32_t k) {
   return true;
 }
 
+// Radius in pixels about the plane's centre (Nx/2, Ny/2) beyond which no pixel is on
+// the Ewald sphere: the disc |k k^ + q| <= k has its centre at the grid point of
+// q = -k k^ and the radius k in each grid step, plus two pixels against rounding.
+double ewald_radius(const EwaldGeom &g) {
+  const double cx = (-g.k * g.kx - g.start) / g.dx - g.nx / 2.0, cy = (-g.k * g.ky - g.start) / g.dy - g.ny / 2.0;
+  return std::hypot(cx, cy) + g.k / std::min(g.dx, g.dy) + 2.0;
+}
+
 // EBASIS: per (energy, k) unit the five tensor fields, their XY transforms, the
 // z DFT at the Ewald bins, then every angle as 2D work.  With two lanes, unit u
 // runs on stream u % 2 with its own work buffers and starts once unit u-1's
@@ -400,6 +420,8 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
   const int ng = (g.nz > 1 && d->interpolation == 1) ? 2 : 1;
   const uint32_t units = g.nE * g.nK;
   const uint32_t lanes = units > 1 ? std::min(energy_lanes(), wb.max_lanes) : 1;
+  // laboratory frame: one quadratic form per pixel instead of every angle's projection
+  const bool lab = d->reference_frame != 0;
   YzArgs<T> yz{};
   yz.nx = g.nx;
   yz.ny = g.ny;
@@ -408,7 +430,7 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
   for (uint32_t L = 0; L < lanes; L++) {
     LaneBuffers &lb = wb.lane[L];
     CYR_TRY(ensure_buffer(lb.pol, sizeof(cx<T>) * V * kEbFields));
-    CYR_TRY(ensure_buffer(lb.proj, sizeof(T) * P * g.nA));
+    CYR_TRY(ensure_buffer(lb.proj, sizeof(T) * P * (lab ? kQuadRecord : g.nA)));
     CYR_TRY(ensure_buffer(lb.avg, sizeof(double) * P));
     CYR_TRY(ensure_buffer(lb.bins, sizeof(int32_t) * P));
     CYR_TRY(ensure_buffer(lb.part, sizeof(cx<T>) * P * ng * kEbFields * yz.nchunks));
@@ -486,14 +508,28 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
     aa.dcz = dcz;
     aa.amat = su.amat + (size_t)kEbAmat * k * g.nA;
     aa.nA = g.nA;
-    aa.proj = proj;
-    kt_begin(s);
-    CYR_TRY(launch_ebasis_angles<T>(aa, ng, s));
-    kt_end("ebasis_angles", s, part_bytes + (double)g.nA * P * sizeof(T));
-    kt_begin(s);
-    CYR_TRY(launch_rotate_all<T>(proj, su.rotinv + (size_t)6 * k * g.nA, g.nA, g.nx, g.ny, d->rot_mask, avg,
-                                 su.tiles, -1.0, s));
-    kt_end("rotate_all", s, (double)(g.nA + 1) * P * sizeof(T));
+    const double *inv = su.rotinv + (size_t)6 * k * g.nA;
+    const double rfin = ewald_radius(geo);
+    if (lab) {
+      aa.quad = proj;
+      aa.Q = m3<T>(Q);
+      kt_begin(s);
+      CYR_TRY(launch_ebasis_angles<T>(aa, ng, s));
+      kt_end("ebasis_quad", s, part_bytes + (double)kQuadRecord * P * sizeof(T));
+      kt_begin(s);
+      CYR_TRY(launch_rotate_quad<T>(proj, inv, su.quad + (size_t)3 * k * g.nA, su.quad_t + (size_t)3 * k * g.nA, g.nA,
+                                    g.nx, g.ny, d->rot_mask, avg, 1, su.tiles, g.quarter, su.otiles,
+                                    quad_pairs_share<T>(g, k), rfin, s));
+      kt_end("rotate_quad", s, (double)kQuadRecord * P * sizeof(T) + 8.0 * P);
+    } else {
+      aa.proj = proj;
+      kt_begin(s);
+      CYR_TRY(launch_ebasis_angles<T>(aa, ng, s));
+      kt_end("ebasis_angles", s, part_bytes + (double)g.nA * P * sizeof(T));
+      kt_begin(s);
+      CYR_TRY(launch_rotate_all<T>(proj, inv, g.nA, g.nx, g.ny, d->rot_mask, avg, su.tiles, rfin, s));
+      kt_end("rotate_all", s, (double)(g.nA + 1) * P * sizeof(T));
+    }
     CYR_TRY(launch_detector_warp<T>(avg, out, g.nx, g.ny, &g.det_inv[(size_t)k * 6], d->rot_mask, s));
   }
   if (lanes > 1) {
@@ -952,7 +988,7 @@ uint64_t work_bytes(const cyr_sim_desc *d, const SimGeometry &g) {
     const uint64_t nch = ebasis_max_chunks(g.nx, g.ny, g.nz, d->precision);
     const uint64_t lanes = (uint64_t)g.nE * g.nK > 1 ? energy_lanes() : 1;
     b += lanes * (cs * g.V * kEbFields + 4 * g.P + cs * g.P * 2 * kEbFields * nch + 16 * kEbFields * g.nz +
-                  rs * g.P * g.nA + 8 * g.P);
+                  rs * g.P * (d->reference_frame != 0 ? kQuadRecord : g.nA) + 8 * g.P);
   } else {
     b += cs * g.V * 3 + rs * g.P + 8 * g.P * 2 + 4 * g.P;
     if (d->algorithm == 1) b += cs * g.V * 6;

@@ -260,6 +260,49 @@ __global__ void __launch_bounds__(256) rotate_quad_kernel(const T *__restrict__ 
   quad_store<NE>(avg, P, (uint64_t)Y * nx + X, e0, ne, nA, rot_mask, acc, cnt);
 }
 
+// The same for planes too small to fill the chip: S waves of a block take S runs of the
+// angles for one 8 x 8 quadrant of a tile and one energy, and their FP64 sums meet in
+// LDS in angle order.  The chain of dependent gathers per wave is S times shorter and
+// there are 4 S times as many waves as one tile per block and four energies give:
+// 256^2, one energy, 36 angles: 70 us (quarter-turn orbits, 64 blocks) -> 20 us; 64^2,
+// 3 energies, 6 angles: 32 -> 6.5 us.
+template <typename T, int S>
+__global__ void __launch_bounds__(64 * S) rotate_quad_split_kernel(const T *__restrict__ quad,
+                                                                   const double *__restrict__ inv_tab,
+                                                                   const double *__restrict__ coef, uint32_t nA,
+                                                                   uint32_t nx, uint32_t ny, int rot_mask,
+                                                                   double *__restrict__ avg,
+                                                                   const uint32_t *__restrict__ tiles,
+                                                                   uint32_t ntiles) {
+  __shared__ double sum[S][64];
+  __shared__ uint32_t num[S][64];
+  const uint64_t P = (uint64_t)nx * ny;
+  const uint32_t b = xcd_tile(blockIdx.x, gridDim.x);
+  if (b >= 4 * ntiles) return;  // (the whole block)
+  const uint32_t tt = tiles[b >> 2], w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const uint32_t X = (tt & 0xffffu) * 16 + (b & 1) * 8 + (l & 7);
+  const uint32_t Y = (tt >> 16) * 16 + ((b >> 1) & 1) * 8 + (l >> 3);
+  const uint32_t e = blockIdx.z;
+  const bool in = X < nx && Y < ny;
+  double acc[1] = {0};
+  uint32_t cnt[1] = {0};
+  if (in) {
+    const uint32_t a0 = (uint32_t)((uint64_t)nA * w / S), a1 = (uint32_t)((uint64_t)nA * (w + 1) / S);
+    const T *qp[1] = {quad + (uint64_t)e * P * kQuadRecord};
+    quad_pixel<T, 1>(qp, inv_tab + 6 * (uint64_t)a0, coef + 3 * (uint64_t)a0, a1 - a0, nx, ny, X, Y, rot_mask, acc,
+                     cnt);
+  }
+  sum[w][l] = acc[0];
+  num[w][l] = cnt[0];
+  __syncthreads();
+  if (w != 0 || !in) return;
+  for (int i = 1; i < S; i++) {
+    acc[0] += sum[i][l];
+    cnt[0] += num[i][l];
+  }
+  quad_store<1>(avg, P, (uint64_t)Y * nx + X, e, e + 1, nA, rot_mask, acc, cnt);
+}
+
 // Tiles of the general order beyond every finite plane value: the averages
 // rotate_quad_kernel would form there (NaN, or 0 with the rotation mask), as in
 // orbit_fill_kernel.  Same tile and pixel layout as tile_pixel.
@@ -284,7 +327,7 @@ __global__ void __launch_bounds__(256) quad_fill_kernel(double *__restrict__ avg
 // of A4 steps: angle a + q A4 is angle a plus 90q degrees).  The image rotation
 // turns about (N/2, N/2), so with s(X, Y) = (N - Y, X) (a 90-degree turn of the
 // pixel grid) the point pixel x samples at angle a + q A4 is the point pixel
-// s^q(x) samples at angle a.  One thread owns the orbit x, s x, s^2 x, s^3 x of a
+// s^q(x) samples at angle a.  One lane owns the orbit x, s x, s^2 x, s^3 x of a
 // pixel with X - N/2 in [1, N/2 - 1] and Y - N/2 in [0, N/2 - 1] (these orbits tile
 // [1, N-1]^2 minus the centre): it back-maps and gathers each (s^i x, a < A4) once
 // and serves the Q (pixel, angle) pairs that sample there.
@@ -331,6 +374,12 @@ template <typename T> __device__ inline typename Tap3<T>::v tap_load(__amdgpu_bu
 // Buffer resource word 3 of a raw (untyped) buffer on gfx9-family devices.
 constexpr int kRawBufferFlags = 0x00020000;
 
+// A block holds one 8 x 8 quadrant of a tile of orbits; its wave i samples the points of
+// orbit pixel i and serves pixel s^-q(i) from them (one pixel per wave, not four in
+// turn: four times the waves and a quarter of the chain of gathers for the same work;
+// 512^2 FP64 film, 10 energies x 72 angles: 128 us for one energy -> 111 us for all ten;
+// 2048^2 film, 10 energies x 180 angles: 1.19 ms, as before).  The waves' sums meet in LDS,
+// added in orbit order.
 template <typename T, int NE, int Q, bool RM>
 __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__ quad, const double *__restrict__ inv_tab,
                                                            const double *__restrict__ coef,
@@ -338,34 +387,54 @@ __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__
                                                            uint32_t n, double *__restrict__ avg, uint32_t ne,
                                                            const uint32_t *__restrict__ otiles, uint32_t n_otiles,
                                                            int share) {
+  __shared__ double sum[4][Q][NE][64];
+  __shared__ uint32_t num[RM ? 4 : 1][RM ? Q : 1][NE][64];
   const uint64_t P = (uint64_t)n * n;
   const uint32_t h = n / 2;
   const uint32_t qb = xcd_tile(blockIdx.x, gridDim.x);
   const uint32_t e0 = blockIdx.z * NE;
+  const uint32_t i = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
   const T *qp[NE];
 #pragma unroll
   for (int e = 0; e < NE; e++) qp[e] = quad + (uint64_t)(e0 + e < ne ? e0 + e : e0) * P * kQuadRecord;
-  if (qb >= n_otiles) {
-    // tail: row 0 (n pixels), column 0 below it (n - 1) and the centre
-    const uint32_t j = (qb - n_otiles) * 256 + threadIdx.x;
-    if (j >= 2 * n) return;
+  if (qb >= 4 * n_otiles) {
+    // tail: row 0 (n pixels), column 0 below it (n - 1) and the centre, 64 pixels a
+    // block, a quarter of the angles a wave
+    const uint32_t j = (qb - 4 * n_otiles) * 64 + l;
+    const bool in = j < 2 * n;
     const uint32_t X = j < n ? j : (j < 2 * n - 1 ? 0 : h);
     const uint32_t Y = j < n ? 0 : (j < 2 * n - 1 ? j - n + 1 : h);
     double acc[NE] = {};
     uint32_t cnt[NE] = {};
-    quad_pixel<T, NE>(qp, inv_tab, coef, nA, n, n, X, Y, RM, acc, cnt);
+    if (in) {
+      const uint32_t a0 = (uint32_t)((uint64_t)nA * i / 4), a1 = (uint32_t)((uint64_t)nA * (i + 1) / 4);
+      quad_pixel<T, NE>(qp, inv_tab + 6 * (uint64_t)a0, coef + 3 * (uint64_t)a0, a1 - a0, n, n, X, Y, RM, acc, cnt);
+    }
+#pragma unroll
+    for (int e = 0; e < NE; e++) {
+      sum[i][0][e][l] = acc[e];
+      if constexpr (RM) num[i][0][e][l] = cnt[e];
+    }
+    __syncthreads();
+    if (i != 0 || !in) return;
+#pragma unroll
+    for (int e = 0; e < NE; e++)
+      for (int w = 1; w < 4; w++) {
+        acc[e] += sum[w][0][e][l];
+        if constexpr (RM) cnt[e] += num[w][0][e][l];
+      }
     quad_store<NE>(avg, P, (uint64_t)Y * n + X, e0, ne, nA, RM, acc, cnt);
     return;
   }
-  const uint32_t tt = otiles[qb];
-  const uint32_t w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const uint32_t u = (tt & 0xffffu) * 16 + (w & 1) * 8 + (l & 7) + 1;
-  const uint32_t v = (tt >> 16) * 16 + (w >> 1) * 8 + (l >> 3);
-  if (u >= h || v >= h) return;
-  // orbit pixels s^i(x), i = 0..3
-  const uint32_t X0 = h + u, Y0 = h + v;
-  const uint32_t PX[4] = {X0, n - Y0, n - X0, Y0};
-  const uint32_t PY[4] = {Y0, X0, n - Y0, n - X0};
+  const uint32_t tt = otiles[qb >> 2];
+  const uint32_t u = (tt & 0xffffu) * 16 + (qb & 1) * 8 + (l & 7) + 1;
+  const uint32_t v = (tt >> 16) * 16 + ((qb >> 1) & 1) * 8 + (l >> 3);
+  const bool in = u < h && v < h;
+  // orbit pixels s^j(x), j = 0..3 (idle lanes: the orbit of (h, h), nothing stored)
+  const uint32_t X0 = in ? h + u : h, Y0 = in ? h + v : h;
+  auto px = [&](uint32_t j) { return j == 0 ? X0 : j == 1 ? n - Y0 : j == 2 ? n - X0 : Y0; };
+  auto py = [&](uint32_t j) { return j == 0 ? Y0 : j == 1 ? X0 : j == 2 ? n - Y0 : n - X0; };
+  const uint32_t PXi = px(i), PYi = py(i);
   const double hi = (double)(n - 1);
   const double m = 1e-9 + 1e-12 * (double)n;
   constexpr uint32_t rb = kQuadRecord * (uint32_t)sizeof(T);
@@ -373,128 +442,136 @@ __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__
 #pragma unroll
   for (int e = 0; e < NE; e++)
     rs[e] = __builtin_amdgcn_make_buffer_rsrc((void *)qp[e], (short)0, (int)(P * rb), kRawBufferFlags);
-  double acc[4][NE] = {};
-  uint32_t cnt[4][NE] = {};
-  bool dead[4] = {false, false, false, false};
-  static_for<0, 4>([&](auto ic) {
-    constexpr int i = decltype(ic)::value;
-    // angles in chunks of 64: bit (a - a0) of `defer` marks angle a of the chunk
-    // whose point takes the exact path
-    for (uint32_t a0 = 0; a0 < A4; a0 += 64) {
-      const uint32_t a1 = A4 - a0 > 64 ? a0 + 64 : A4;
-      uint64_t defer = 0;
-      for (uint32_t a = a0; a < a1; a++) {
-        const double *inv = inv_tab + 6 * (uint64_t)a;
-        const double sx = __builtin_fma(inv[0], (double)PX[i], __builtin_fma(inv[1], (double)PY[i], inv[2]));
-        const double sy = __builtin_fma(inv[3], (double)PX[i], __builtin_fma(inv[4], (double)PY[i], inv[5]));
-        const bool inside = sx >= 0 && sx <= hi && sy >= 0 && sy <= hi;
-        const double fx0 = floor(sx), fy0 = floor(sy);
-        const double fx = sx - fx0, fy = sy - fy0;
-        const bool safe = inside ? (fx >= m && fx <= 1 - m && fy >= m && fy <= 1 - m)
-                                 : (sx < -m || sx > hi + m || sy < -m || sy > hi + m);
-        const uint32_t x0 = inside ? (uint32_t)fx0 : 0u, y0 = inside ? (uint32_t)fy0 : 0u;
-        const uint32_t o00 = quad_index(x0, y0, n, n) * rb, o10 = quad_index(x0 + 1, y0, n, n) * rb;
-        const uint32_t o01 = quad_index(x0, y0 + 1, n, n) * rb, o11 = quad_index(x0 + 1, y0 + 1, n, n) * rb;
-        typename Tap3<T>::v t[NE][4];
+  // what the points of pixel i give to pixel s^-q(i), q < Q
+  double acc[Q][NE] = {};
+  uint32_t cnt[Q][NE] = {};
+  bool dead = false;
+  // angles in chunks of 64: bit (a - a0) of `defer` marks angle a of the chunk
+  // whose point takes the exact path
+  for (uint32_t a0 = 0; a0 < A4; a0 += 64) {
+    const uint32_t a1 = A4 - a0 > 64 ? a0 + 64 : A4;
+    uint64_t defer = 0;
+    for (uint32_t a = a0; a < a1; a++) {
+      const double *inv = inv_tab + 6 * (uint64_t)a;
+      const double sx = __builtin_fma(inv[0], (double)PXi, __builtin_fma(inv[1], (double)PYi, inv[2]));
+      const double sy = __builtin_fma(inv[3], (double)PXi, __builtin_fma(inv[4], (double)PYi, inv[5]));
+      const bool inside = sx >= 0 && sx <= hi && sy >= 0 && sy <= hi;
+      const double fx0 = floor(sx), fy0 = floor(sy);
+      const double fx = sx - fx0, fy = sy - fy0;
+      const bool safe = inside ? (fx >= m && fx <= 1 - m && fy >= m && fy <= 1 - m)
+                               : (sx < -m || sx > hi + m || sy < -m || sy > hi + m);
+      const uint32_t x0 = inside ? (uint32_t)fx0 : 0u, y0 = inside ? (uint32_t)fy0 : 0u;
+      const uint32_t o00 = quad_index(x0, y0, n, n) * rb, o10 = quad_index(x0 + 1, y0, n, n) * rb;
+      const uint32_t o01 = quad_index(x0, y0 + 1, n, n) * rb, o11 = quad_index(x0 + 1, y0 + 1, n, n) * rb;
+      typename Tap3<T>::v t[NE][4];
+#pragma unroll
+      for (int e = 0; e < NE; e++) {
+        t[e][0] = tap_load<T>(rs[e], o00);
+        t[e][1] = tap_load<T>(rs[e], o10);
+        t[e][2] = tap_load<T>(rs[e], o01);
+        t[e][3] = tap_load<T>(rs[e], o11);
+      }
+      if (!safe) {
+        defer |= 1ull << (a - a0);
+        continue;
+      }
+      // every pair shares this point's cell, validity and nonzero weights
+      const T fxT = (T)fx, fyT = (T)fy, gx = (T)1 - fxT, gy = (T)1 - fyT;
+      const T w00 = gx * gy, w10 = fxT * gy, w01 = gx * fyT, w11 = fxT * fyT;
+      T sm[NE][3];
+#pragma unroll
+      for (int e = 0; e < NE; e++) {
+        sm[e][0] = w00 * t[e][0].x + w10 * t[e][1].x + w01 * t[e][2].x + w11 * t[e][3].x;
+        sm[e][1] = w00 * t[e][0].y + w10 * t[e][1].y + w01 * t[e][2].y + w11 * t[e][3].y;
+        sm[e][2] = w00 * t[e][0].z + w10 * t[e][1].z + w01 * t[e][2].z + w11 * t[e][3].z;
+      }
+      auto add = [&](auto qc, const T(&vq)[NE]) {
+        constexpr int q = decltype(qc)::value;
 #pragma unroll
         for (int e = 0; e < NE; e++) {
-          t[e][0] = tap_load<T>(rs[e], o00);
-          t[e][1] = tap_load<T>(rs[e], o10);
-          t[e][2] = tap_load<T>(rs[e], o01);
-          t[e][3] = tap_load<T>(rs[e], o11);
-        }
-        if (!safe) {
-          defer |= 1ull << (a - a0);
-          continue;
-        }
-        // every pair shares this point's cell, validity and nonzero weights
-        const T fxT = (T)fx, fyT = (T)fy, gx = (T)1 - fxT, gy = (T)1 - fyT;
-        const T w00 = gx * gy, w10 = fxT * gy, w01 = gx * fyT, w11 = fxT * fyT;
-        T sm[NE][3];
-#pragma unroll
-        for (int e = 0; e < NE; e++) {
-          sm[e][0] = w00 * t[e][0].x + w10 * t[e][1].x + w01 * t[e][2].x + w11 * t[e][3].x;
-          sm[e][1] = w00 * t[e][0].y + w10 * t[e][1].y + w01 * t[e][2].y + w11 * t[e][3].y;
-          sm[e][2] = w00 * t[e][0].z + w10 * t[e][1].z + w01 * t[e][2].z + w11 * t[e][3].z;
-        }
-        auto add = [&](auto qc, const T(&vq)[NE]) {
-          constexpr int q = decltype(qc)::value;
-          constexpr int j = (i - q + 4) & 3;  // s^q(pixel j) = pixel i
-#pragma unroll
-          for (int e = 0; e < NE; e++) {
-            if constexpr (RM) {
-              const double vv = (double)vq[e];
-              const bool ok = inside && !isnan(vv);
-              acc[j][e] += ok ? vv : 0.0;
-              cnt[j][e] += ok ? 1u : 0u;
-            } else {
-              acc[j][e] += (double)vq[e];
-            }
-          }
-          if constexpr (!RM) dead[j] = dead[j] || !inside;
-        };
-        auto value = [&](int q, T(&vq)[NE]) {
-          const T *c = coef_t + 3 * (uint64_t)(a + q * A4);
-#pragma unroll
-          for (int e = 0; e < NE; e++) vq[e] = c[0] * sm[e][0] + c[1] * sm[e][1] + c[2] * sm[e][2];
-        };
-        bool shared = false;
-        if constexpr (Q == 4) {
-          if (share) {  // pairs q and q + 2 have equal coefficients
-            T v0[NE], v1[NE];
-            value(0, v0);
-            value(1, v1);
-            add(std::integral_constant<int, 0>{}, v0);
-            add(std::integral_constant<int, 1>{}, v1);
-            add(std::integral_constant<int, 2>{}, v0);
-            add(std::integral_constant<int, 3>{}, v1);
-            shared = true;
+          if constexpr (RM) {
+            const double vv = (double)vq[e];
+            const bool ok = inside && !isnan(vv);
+            acc[q][e] += ok ? vv : 0.0;
+            cnt[q][e] += ok ? 1u : 0u;
+          } else {
+            acc[q][e] += (double)vq[e];
           }
         }
-        if (!shared) {
-          static_for<0, Q>([&](auto qc) {
-            T vq[NE];
-            value(decltype(qc)::value, vq);
-            add(qc, vq);
-          });
+      };
+      if constexpr (!RM) dead = dead || !inside;
+      auto value = [&](int q, T(&vq)[NE]) {
+        const T *c = coef_t + 3 * (uint64_t)(a + q * A4);
+#pragma unroll
+        for (int e = 0; e < NE; e++) vq[e] = c[0] * sm[e][0] + c[1] * sm[e][1] + c[2] * sm[e][2];
+      };
+      bool shared = false;
+      if constexpr (Q == 4) {
+        if (share) {  // pairs q and q + 2 have equal coefficients
+          T v0[NE], v1[NE];
+          value(0, v0);
+          value(1, v1);
+          add(std::integral_constant<int, 0>{}, v0);
+          add(std::integral_constant<int, 1>{}, v1);
+          add(std::integral_constant<int, 2>{}, v0);
+          add(std::integral_constant<int, 3>{}, v1);
+          shared = true;
         }
       }
-      // points near a cell edge or the image border: every pair back-maps its own
-      // point exactly and gathers its own taps (one pair at a time, so the rare path
-      // holds few registers)
-      while (defer) {
-        const uint32_t a = a0 + (uint32_t)__builtin_ctzll(defer);
-        defer &= defer - 1;
+      if (!shared) {
+        static_for<0, Q>([&](auto qc) {
+          T vq[NE];
+          value(decltype(qc)::value, vq);
+          add(qc, vq);
+        });
+      }
+    }
+    // points near a cell edge or the image border: every pair back-maps its own
+    // point exactly and gathers its own taps (one pair at a time, so the rare path
+    // holds few registers)
+    while (defer) {
+      const uint32_t a = a0 + (uint32_t)__builtin_ctzll(defer);
+      defer &= defer - 1;
 #pragma unroll 1
-        for (uint32_t q = 0; q < (uint32_t)Q; q++) {
-          const uint32_t j = (i - q + 4) & 3;
-          const uint32_t aa = a + q * A4;
-          const QPoint d = quad_point(inv_tab + 6 * (uint64_t)aa, PX[j], PY[j], n, n);
-          Rec<T> td[NE][4];
-          quad_gather<T, NE>(qp, d, n, n, td);
-          T sm[NE][3];
-          quad_sums<T, NE>(d, td, sm);
-          const double *c = coef + 3 * (uint64_t)aa;
-          switch (j) {  // constant indices keep the accumulators in registers
-            case 0: quad_combine<T, NE>(d.inside, sm, c, RM, acc[0], cnt[0]); break;
-            case 1: quad_combine<T, NE>(d.inside, sm, c, RM, acc[1], cnt[1]); break;
-            case 2: quad_combine<T, NE>(d.inside, sm, c, RM, acc[2], cnt[2]); break;
-            default: quad_combine<T, NE>(d.inside, sm, c, RM, acc[3], cnt[3]); break;
-          }
-        }
+      for (uint32_t q = 0; q < (uint32_t)Q; q++) {
+        const uint32_t j = (i - q + 4) & 3;
+        const uint32_t aa = a + q * A4;
+        const QPoint d = quad_point(inv_tab + 6 * (uint64_t)aa, px(j), py(j), n, n);
+        Rec<T> td[NE][4];
+        quad_gather<T, NE>(qp, d, n, n, td);
+        T sm[NE][3];
+        quad_sums<T, NE>(d, td, sm);
+        const double *c = coef + 3 * (uint64_t)aa;
+        static_for<0, Q>([&](auto qc) {  // constant indices keep the accumulators in registers
+          constexpr int qq = decltype(qc)::value;
+          if (q == (uint32_t)qq) quad_combine<T, NE>(d.inside, sm, c, RM, acc[qq], cnt[qq]);
+        });
       }
     }
-  });
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    if constexpr (!RM) {
-      if (dead[i]) {
-#pragma unroll
-        for (int e = 0; e < NE; e++) acc[i][e] = __longlong_as_double(0x7ff8000000000000ll);
-      }
-    }
-    quad_store<NE>(avg, P, (uint64_t)PY[i] * n + PX[i], e0, ne, nA, RM, acc[i], cnt[i]);
   }
+#pragma unroll
+  for (int q = 0; q < Q; q++)
+#pragma unroll
+    for (int e = 0; e < NE; e++) {
+      sum[i][q][e][l] = dead ? __longlong_as_double(0x7ff8000000000000ll) : acc[q][e];
+      if constexpr (RM) num[i][q][e][l] = cnt[q][e];
+    }
+  __syncthreads();
+  if (!in) return;
+  // wave i now stores pixel i: the sums of the pixels j whose points serve it, q = j - i
+  double a[NE] = {};
+  uint32_t c[NE] = {};
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const uint32_t q = (j - i + 4) & 3;
+    if (q >= (uint32_t)Q) continue;  // (uniform)
+#pragma unroll
+    for (int e = 0; e < NE; e++) {
+      a[e] += sum[j][q][e][l];
+      if constexpr (RM) c[e] += num[j][q][e][l];
+    }
+  }
+  quad_store<NE>(avg, P, (uint64_t)PYi * n + PXi, e0, ne, nA, RM, a, c);
 }
 
 // Orbit tiles beyond every finite plane value (their pixels' taps, within 1.5
@@ -563,6 +640,9 @@ __global__ void __launch_bounds__(256) warp_kernel(const T *__restrict__ src, T 
   double v;
   if (bilinear_sample<T>(src, nx, ny, inv.c, X, Y, &v)) dst[t] = (T)v;
 }
+
+// Waves (8 per CU) below which the rotation splits the angles of a pixel.
+constexpr uint64_t kSplitWaves = 2048;
 
 Inv6 mk_inv(const double inv[6]) {
   Inv6 r;
@@ -700,6 +780,29 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
   if (ne == 0) return CYR_OK;
   if ((uint64_t)nx * ny > 0xffffffffull) return fail(CYR_E_UNSUPPORTED, "rotation: more than 2^32 pixels");
   if (!tiles) return fail(CYR_E_INVALID, "rotation: tile order missing");
+  const uint32_t ntiles = rotation_tile_count(nx, ny);
+  // tiles (in order of distance from the centre (Nx/2, Ny/2), about which the
+  // image turns) whose pixels all lie more than rfin + 2 pixels out are filled:
+  // a 16 x 16 tile's pixels are within 8 sqrt(2) of its centre
+  const uint32_t n_act = rfin >= 0 ? std::min(ntiles, rotation_tiles_within(nx, ny, rfin + 14.0)) : ntiles;
+  // planes whose sampled tiles, four waves each, give fewer waves than kSplitWaves over
+  // all energies: angles split over the waves of a block
+  if ((uint64_t)n_act * 4 * ne < kSplitWaves) {
+    const dim3 grid(xcd_grid(4ull * n_act), 1, ne);
+    if ((uint64_t)n_act * 16 * ne < kSplitWaves && nA >= 8)
+      hipLaunchKernelGGL((rotate_quad_split_kernel<T, 16>), grid, dim3(1024), 0, st, quad, inv_tab, coef, nA, nx, ny,
+                         rot_mask, avg, tiles, n_act);
+    else
+      hipLaunchKernelGGL((rotate_quad_split_kernel<T, 4>), grid, dim3(256), 0, st, quad, inv_tab, coef, nA, nx, ny,
+                         rot_mask, avg, tiles, n_act);
+    CYR_LAUNCHED();
+    if (n_act < ntiles) {
+      hipLaunchKernelGGL((quad_fill_kernel<1>), dim3(ntiles - n_act, 1, ne), dim3(256), 0, st, avg, nx, ny, ne,
+                         rot_mask, tiles, n_act);
+      CYR_LAUNCHED();
+    }
+    return CYR_OK;
+  }
   // the orbit kernel addresses a plane through 32-bit buffer offsets
   const bool small_plane = (uint64_t)nx * ny * kQuadRecord * sizeof(T) < (1ull << 31);
   const uint32_t Q = otiles && small_plane ? rotation_quarter_turns(nx, ny, nA, quarter) : 0;
@@ -709,31 +812,26 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
     // tiles (in order of distance from the centre) whose pixels all lie more than
     // rfin + 2 pixels out are filled, not sampled: a tile's pixels are within
     // 8 sqrt(2) < 11.4 pixels of its centre, hence the cut at rfin + 14
-    const uint32_t n_act = rfin >= 0 ? std::min(n_otiles, rotation_orbit_tiles_within(nx, rfin + 14.0)) : n_otiles;
+    const uint32_t o_act = rfin >= 0 ? std::min(n_otiles, rotation_orbit_tiles_within(nx, rfin + 14.0)) : n_otiles;
     // 2 energies per pass (measured against 1 and 4: 512^2 x 20 energies 415 / 384 us
     // for 4 / 2; 2048^2 film 7.30 / 6.75 / 8.92 ms per 10 energies for 1 / 2 / 4)
-    const uint64_t blocks = (uint64_t)n_act + ceil_div(2ull * nx, 256);
+    const uint64_t blocks = 4ull * o_act + ceil_div(2ull * nx, 64);
     const dim3 grid(xcd_grid(blocks), 1, ceil_div(ne, 2));
     hipError_t e =
         rot_mask ? launch_orbit_rm<T, 2, true>(Q, grid, st, quad, inv_tab, coef, coef_t, nA, quarter, nx, avg, ne,
-                                                otiles, n_act, share ? 1 : 0)
+                                                otiles, o_act, share ? 1 : 0)
                  : launch_orbit_rm<T, 2, false>(Q, grid, st, quad, inv_tab, coef, coef_t, nA, quarter, nx, avg, ne,
-                                                 otiles, n_act, share ? 1 : 0);
+                                                 otiles, o_act, share ? 1 : 0);
     if (e != hipSuccess) return hip_fail(e, "rotate_orbit_kernel", __FILE__, __LINE__);
-    if (n_act < n_otiles) {
-      const dim3 gf(n_otiles - n_act, 1, ceil_div(ne, 2));
-      if (rot_mask) hipLaunchKernelGGL((orbit_fill_kernel<2, true>), gf, dim3(256), 0, st, avg, nx, ne, otiles, n_act);
-      else hipLaunchKernelGGL((orbit_fill_kernel<2, false>), gf, dim3(256), 0, st, avg, nx, ne, otiles, n_act);
+    if (o_act < n_otiles) {
+      const dim3 gf(n_otiles - o_act, 1, ceil_div(ne, 2));
+      if (rot_mask) hipLaunchKernelGGL((orbit_fill_kernel<2, true>), gf, dim3(256), 0, st, avg, nx, ne, otiles, o_act);
+      else hipLaunchKernelGGL((orbit_fill_kernel<2, false>), gf, dim3(256), 0, st, avg, nx, ne, otiles, o_act);
       e = hipGetLastError();
       if (e != hipSuccess) return hip_fail(e, "orbit_fill_kernel", __FILE__, __LINE__);
     }
     return CYR_OK;
   }
-  const uint32_t ntiles = rotation_tile_count(nx, ny);
-  // tiles (in order of distance from the centre (Nx/2, Ny/2), about which the
-  // image turns) whose pixels all lie more than rfin + 2 pixels out are filled:
-  // a 16 x 16 tile's pixels are within 8 sqrt(2) of its centre
-  const uint32_t n_act = rfin >= 0 ? std::min(ntiles, rotation_tiles_within(nx, ny, rfin + 14.0)) : ntiles;
   // Energies per pass: 4 share each angle's taps; once a plane of quadratic forms
   // exceeds 16 MB (2048^2: 64 MB), one energy per pass keeps the gathers' working
   // set in cache (measured 19% faster there, equal at 512^2).
