@@ -22,7 +22,8 @@ OBJDIR = os.path.join(HERE, "_build")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("CYRSOXS_ARCH", "gfx950")
 
-LIB_SOURCES = ["xfields32.hip", "xfields64.hip", "fft.hip", "mbasis.hip", "ebasis.hip", "runtime.cpp",
+LIB_SOURCES = ["xfields_pair32.hip", "xfields_tensor32.hip", "xfields_single32.hip", "xfields_pair64.hip",
+               "xfields_tensor64.hip", "xfields_single64.hip", "fft.hip", "mbasis.hip", "ebasis.hip", "runtime.cpp",
                "host_math.cpp", "polarization.hip", "ewald.hip", "rotate.hip", "pipeline.hip", "noalloc.hip", "engine.cpp"]
 
 COMMON = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}",

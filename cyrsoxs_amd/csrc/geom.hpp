@@ -17,7 +17,9 @@ __device__ inline double sqrt_rn(double x) {
   double r = sqrt(x);
   if (!(x > 0) || !isfinite(x)) return r;
   double best = r, berr = fabs(fma(-r, r, x));
-  const double cand[2] = {nextafter(r, 0.0), nextafter(r, INFINITY)};
+  // the neighbours of a positive finite value: its bit pattern -1 and +1
+  const long long rb = __double_as_longlong(r);
+  const double cand[2] = {__longlong_as_double(rb - 1), __longlong_as_double(rb + 1)};
   for (int i = 0; i < 2; i++) {
     const double c = cand[i];
     const double e = fabs(fma(-c, c, x));

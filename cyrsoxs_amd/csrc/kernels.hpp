@@ -93,8 +93,11 @@ template <typename T> struct PolxArgs {
   uint32_t tpp, pp;                // filled by the launcher
   cx<T> *out[kXMaxOut];            // X-transformed fields
 };
-template <typename T>
-cyr_status launch_ebasis_polx(PolxArgs<T> a, const void *vox, int storage, int morph, bool hann, hipStream_t st);
+// Fields + X FFT of one mode: the five tensor fields of an energy (all materials), the
+// seven packed basis volumes of the material pair m0, m0 + 1, or the four of material m0.
+enum XMode { kXTensor = 0, kXPair = 1, kXSingle = 2 };
+template <typename T, int MODE>
+cyr_status launch_xfields(PolxArgs<T> a, const void *vox, int storage, int morph, bool hann, hipStream_t st);
 
 template <typename T> struct YzArgs {
   const cx<T> *vol[kEbFields];     // X-transformed fields
@@ -155,15 +158,12 @@ inline uint32_t mbasis_volumes(uint32_t M) { return 7 * (M / 2) + 4 * (M % 2); }
 // x coordinates that cover every column whose own or mirrored band is non-empty
 // (lo > hi: none); the Y pass writes and the Z band pass reads only those.
 constexpr uint32_t kBandHead = 7;
-cyr_status launch_mbasis_bands(const EwaldGeom &g, const double *kmag, uint32_t ne, int32_t *band, uint32_t *bmax,
+// kmax: the largest |k|; totals: also bmax[0..6] (else only the bands and spans).
+cyr_status launch_mbasis_bands(const EwaldGeom &g, const double *kmag, uint32_t ne, double kmax, int32_t *band,
+                               uint32_t *bmax, bool totals,
                                hipStream_t st);
 uint64_t mbasis_bmax_words(uint32_t nx, uint32_t ny);
 uint32_t *mbasis_span_table(uint32_t *bmax, uint32_t nx, uint32_t ny);
-// Fields + X FFT of one material pass: a pair (m0, m0 + 1, 7 outputs) or a single
-// material (m0, 4 outputs).
-template <typename T>
-cyr_status launch_mbasis_xfields(PolxArgs<T> a, bool pair, const void *vox, int storage, int morph, bool hann,
-                                 hipStream_t st);
 template <typename T> struct BandArgs {
   const cx<T> *vol[kXMaxOut];      // transformed packed volumes of this pass
   uint32_t count, vbase;           // volumes, global index of vol[0]
@@ -171,15 +171,16 @@ template <typename T> struct BandArgs {
   const uint32_t *span;            // [Ny] row spans (null: every column)
   cx<T> *own, *mir;                // [volumes][J][Ny][Nx] (mir null: complex fields, no mirrored bins)
   uint32_t J, nx, ny, nz;
+  const double2 *dcz;              // [volumes][dc_per] DC-neighbour partials; the pass also
+  double2 *dcv;                    // writes dcv[v] = their sum / dc_cnt for its volumes
+  uint64_t dc_per;
+  double dc_cnt;
 };
 template <typename T> cyr_status launch_mbasis_extract(const BandArgs<T> &a, hipStream_t st);
 // Z FFT of the Y-transformed volumes writing only the band values (vol[] is read,
 // not overwritten), 3D; launch_mbasis_extract copies them in 2D.
 bool mbasis_zband_supported(uint32_t nz, int precision);
 template <typename T> cyr_status launch_mbasis_zband(const BandArgs<T> &a, hipStream_t st);
-// DC-replacement values of the packed volumes from their per-slice neighbour sums.
-cyr_status launch_mbasis_dcsum(const double2 *dcz, uint32_t nvol, uint32_t nz, bool three, double2 *dcv,
-                               hipStream_t st);
 template <typename T> struct MbAnglesArgs {
   EwaldGeom g;                     // this energy's geometry
   const int32_t *band;

@@ -12,13 +12,15 @@
 // B^(k) = (Z - conj Zm) / 2i, so every column keeps Z at its own Ewald bins
 // and at the mirrored bins of the opposite column.
 //
-// Launches per (k, energy group): mbasis_bands_kernel (+ band width reduction),
+// Launches per (k, energy group): mbasis_bands_kernel (+ a reduction the first time),
 // then per material pass xfields_kernel (pair/single mode) -> Y FFT pass with the
 // DC neighbour sums -> mbasis_zband_kernel (Z FFT writing only band values; in 2D
-// mbasis_extract_kernel);
-// mbasis_dcsum_kernel; then per energy mbasis_angles_kernel and the shared
-// rotation / detector kernels.
+// mbasis_extract_kernel), which also forms the DC values; then per batch of energies
+// mbasis_quad_kernel (material frame: mbasis_angles_kernel) and the shared rotation /
+// detector kernels.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "fft.hpp"
 #include "fftpolicy.hpp"
@@ -35,83 +37,123 @@ template <typename T> __device__ inline T mb_qnan();
 template <> __device__ inline float mb_qnan<float>() { return __int_as_float(0x7fc00000); }
 template <> __device__ inline double mb_qnan<double>() { return __longlong_as_double(0x7ff8000000000000ll); }
 
-// ---- band of shifted z indices per column over the energy group ---------------
+// ---- bands and row spans ----------------------------------------------------------
 // band[col] = Zlo | (width << 16) over every energy's Ewald z index (and its
-// linear-interpolation partner z + 1); 0 = no energy samples the column.  Each
-// block also writes the widest band and the sum of the widths it saw (no atomics:
-// a second kernel reduces): bmax[kBandHead + 2b] = widest, bmax[kBandHead + 2b + 1]
-// = sum of block b.
-__global__ void __launch_bounds__(256) mbasis_bands_kernel(EwaldGeom g, const double *__restrict__ kmag, uint32_t ne,
-                                                           int32_t *__restrict__ band, uint32_t *__restrict__ bmax) {
-  __shared__ uint32_t red[2][256];
-  const uint64_t P = (uint64_t)g.nx * g.ny;
-  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  uint32_t w = 0;
-  if (t < P) {
-    const uint32_t Y = (uint32_t)(t / g.nx), X = (uint32_t)(t - (uint64_t)Y * g.nx);
-    uint32_t lo = 0xffffffffu, hi = 0;
-    for (uint32_t e = 0; e < ne; e++) {
-      EwaldGeom ge = g;
-      ge.k = kmag[e];
-      uint32_t z0 = 0;
-      double f = 0;
-      const int kind = ewald_geometry(ge, X, Y, &z0, &f);
-      if (kind == 0) continue;
-      lo = z0 < lo ? z0 : lo;
-      const uint32_t top = kind == 2 ? z0 + 1 : z0;
-      hi = top > hi ? top : hi;
-    }
-    w = lo == 0xffffffffu ? 0 : hi - lo + 1;
-    const uint64_t col = (uint64_t)unshift(Y, g.ny) * g.nx + unshift(X, g.nx);
-    band[col] = w ? (int32_t)(lo | (w << 16)) : 0;
+// linear-interpolation partner z + 1) at the column's pixel; 0 = no energy samples the
+// column.
+__device__ inline uint32_t column_band(EwaldGeom g, const double *__restrict__ kmag, uint32_t ne, double kmax,
+                                       uint32_t X, uint32_t Y) {
+  if (g.kx == 0 && g.ky == 0) {
+    // on-axis beam: k^2 - qx^2 - qy^2, as ewald_geometry rounds it, grows with k, so a
+    // pixel outside the largest energy's sphere is outside every one's
+    uint32_t z = 0;
+    double f = 0;
+    EwaldGeom gm = g;
+    gm.k = kmax;
+    gm.enable2d = 1;  // (validity alone)
+    if (ewald_geometry(gm, X, Y, &z, &f) == 0) return 0;
   }
-  red[0][threadIdx.x] = w;
-  red[1][threadIdx.x] = w;
-  __syncthreads();
-  for (uint32_t s = blockDim.x / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) {
-      red[0][threadIdx.x] = red[0][threadIdx.x + s] > red[0][threadIdx.x] ? red[0][threadIdx.x + s] : red[0][threadIdx.x];
-      red[1][threadIdx.x] += red[1][threadIdx.x + s];
-    }
-    __syncthreads();
+  uint32_t lo = 0xffffffffu, hi = 0;
+  for (uint32_t e = 0; e < ne; e++) {
+    g.k = kmag[e];
+    uint32_t z0 = 0;
+    double f = 0;
+    const int kind = ewald_geometry(g, X, Y, &z0, &f);
+    if (kind == 0) continue;
+    if (g.enable2d) return 1u << 16;  // (every energy samples plane 0)
+    lo = z0 < lo ? z0 : lo;
+    const uint32_t top = kind == 2 ? z0 + 1 : z0;
+    hi = top > hi ? top : hi;
   }
-  if (threadIdx.x == 0) {
-    bmax[kBandHead + 2 * blockIdx.x] = red[0][0];
-    bmax[kBandHead + 2 * blockIdx.x + 1] = red[1][0];
-  }
+  return lo == 0xffffffffu ? 0 : lo | ((hi - lo + 1) << 16);
 }
 
-// ---- columns whose transform some band reads, per row ----------------------------
 // Column c = (x, y) (FFT bins) is read by the band passes when its own band or
 // that of its mirror column (-x, -y) is non-empty.  span[y] = lo | (hi << 16)
 // covers every such column of FFT row y by its shifted x coordinate (unshift is
 // an involution: it also maps bins to shifted coordinates); lo > hi when the row
 // has none.  The Y pass writes, and the Z band pass reads, only columns inside
-// their row's span.  One block per row.
-__global__ void __launch_bounds__(256) mbasis_span_kernel(const int32_t *__restrict__ band, uint32_t nx, uint32_t ny,
-                                                          uint32_t *__restrict__ span) {
-  __shared__ uint32_t red[2][256];
-  const uint32_t y = blockIdx.x, my = y ? ny - y : 0;
-  uint32_t lo = 0xffffu, hi = 0;
-  for (uint32_t x = threadIdx.x; x < nx; x += blockDim.x) {
-    const uint32_t mx = x ? nx - x : 0;
-    if (band[(uint64_t)y * nx + x] != 0 || band[(uint64_t)my * nx + mx] != 0) {
-      const uint32_t X = unshift(x, nx);
-      lo = X < lo ? X : lo;
-      hi = X > hi ? X : hi;
+// their row's span.  One block per pair of mirrored rows (y, -y): which columns are
+// sampled stays in LDS, a bit each.  With bmax, block b also writes the widest band it
+// saw and the sum of the widths (no atomics: a second kernel reduces):
+// bmax[kBandHead + 2b], bmax[kBandHead + 2b + 1].
+// Bound by its FP64 geometry (a square root and a division per column and energy);
+// 2048^2 x 1, 50 energies: 277 us with a pass of its own over every energy and column
+// -> 58 us; 64^3, 3 energies: three launches of 14 us together -> one of 8.
+__global__ void __launch_bounds__(512) mbasis_bands_kernel(EwaldGeom g, const double *__restrict__ kmag, uint32_t ne,
+                                                           double kmax, int32_t *__restrict__ band,
+                                                           uint32_t *__restrict__ span, uint32_t *__restrict__ bmax) {
+  extern __shared__ unsigned long long sampled[];  // [2][ceil(nx / 64)]
+  __shared__ uint32_t red[4][8];
+  const uint32_t words = (g.nx + 63) / 64, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t y0 = blockIdx.x, y1 = y0 ? g.ny - y0 : 0;
+  const uint32_t rows = y1 == y0 ? 1 : 2;
+  uint32_t wmax = 0, wsum = 0;
+  for (uint32_t r = 0; r < rows; r++) {
+    const uint32_t y = r ? y1 : y0, Y = unshift(y, g.ny);
+    for (uint32_t i = wave; i < words; i += blockDim.x / 64) {
+      const uint32_t x = i * 64 + lane;
+      uint32_t b = 0;
+      if (x < g.nx) {
+        b = column_band(g, kmag, ne, kmax, unshift(x, g.nx), Y);
+        band[(uint64_t)y * g.nx + x] = (int32_t)b;
+      }
+      const unsigned long long m = __ballot(b != 0);
+      if (lane == 0) sampled[r * words + i] = m;
+      wmax = (b >> 16) > wmax ? b >> 16 : wmax;
+      wsum += b >> 16;
     }
   }
-  red[0][threadIdx.x] = lo;
-  red[1][threadIdx.x] = hi;
   __syncthreads();
-  for (uint32_t s = blockDim.x / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) {
-      red[0][threadIdx.x] = red[0][threadIdx.x + s] < red[0][threadIdx.x] ? red[0][threadIdx.x + s] : red[0][threadIdx.x];
-      red[1][threadIdx.x] = red[1][threadIdx.x + s] > red[1][threadIdx.x] ? red[1][threadIdx.x + s] : red[1][threadIdx.x];
+  for (uint32_t r = 0; r < rows; r++) {
+    const unsigned long long *own = sampled + r * words, *mirror = sampled + (rows - 1 - r) * words;
+    uint32_t lo = 0xffffu, hi = 0;
+    for (uint32_t x = threadIdx.x; x < g.nx; x += blockDim.x) {
+      const uint32_t mx = x ? g.nx - x : 0;
+      if (((own[x / 64] >> (x & 63)) | (mirror[mx / 64] >> (mx & 63))) & 1) {
+        const uint32_t X = unshift(x, g.nx);
+        lo = X < lo ? X : lo;
+        hi = X > hi ? X : hi;
+      }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      const uint32_t l2 = __shfl_xor(lo, off), h2 = __shfl_xor(hi, off);
+      lo = l2 < lo ? l2 : lo;
+      hi = h2 > hi ? h2 : hi;
+    }
+    if (lane == 0) {
+      red[0][wave] = lo;
+      red[1][wave] = hi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (uint32_t i = 1; i < blockDim.x / 64; i++) {
+        lo = red[0][i] < lo ? red[0][i] : lo;
+        hi = red[1][i] > hi ? red[1][i] : hi;
+      }
+      span[r ? y1 : y0] = lo | (hi << 16);
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) span[y] = red[0][0] | (red[1][0] << 16);
+  if (!bmax) return;
+  for (int off = 32; off > 0; off >>= 1) {
+    const uint32_t m2 = __shfl_xor(wmax, off);
+    wmax = m2 > wmax ? m2 : wmax;
+    wsum += __shfl_xor(wsum, off);
+  }
+  if (lane == 0) {
+    red[2][wave] = wmax;
+    red[3][wave] = wsum;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (uint32_t i = 1; i < blockDim.x / 64; i++) {
+      wmax = red[2][i] > wmax ? red[2][i] : wmax;
+      wsum += red[3][i];
+    }
+    bmax[kBandHead + 2 * blockIdx.x] = wmax;
+    bmax[kBandHead + 2 * blockIdx.x + 1] = wsum;
+  }
 }
 
 // bmax[0] = widest band, bmax[1..2] = sum of all widths (uint64, little endian)
@@ -180,14 +222,45 @@ __device__ inline bool bins_meet_span(uint32_t x0, uint32_t x1, uint32_t n, uint
   return false;
 }
 
+// ---- DC-replacement value of one volume ---------------------------------------------
+// dcv[v] = (sum of its dc_per neighbour partials) / dc_cnt, in a fixed order, by one
+// whole block of the band kernels below (the partials are complete before they start):
+// a launch of its own took 3-5 us of a 64^3 simulation's 94.
+template <typename T> __device__ inline void dc_value(const BandArgs<T> &a, uint32_t v) {
+  __shared__ double2 part[16];
+  double sr = 0, si = 0;
+  for (uint64_t i = threadIdx.x; i < a.dc_per; i += blockDim.x) {
+    const double2 x = a.dcz[(uint64_t)(a.vbase + v) * a.dc_per + i];
+    sr += x.x;
+    si += x.y;
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    sr += __shfl_down(sr, off);
+    si += __shfl_down(si, off);
+  }
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x / 64] = make_double2(sr, si);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (uint32_t w = 1; w < blockDim.x / 64; w++) {
+      sr += part[w].x;
+      si += part[w].y;
+    }
+    a.dcv[a.vbase + v] = make_double2(sr / a.dc_cnt, si / a.dc_cnt);
+  }
+}
+
 // ---- band values of the transformed packed planes (2D) ---------------------------
 // own[v][0][col] = Z_v(col),  mir[v][0][col] = Z_v(-col) for sampled columns.
-// Grid: (columns, volume).
+// Grid: (columns + 1 block, volume).
 template <typename T>
 __global__ void __launch_bounds__(256) mbasis_extract_kernel(BandArgs<T> a) {
   const uint64_t P = (uint64_t)a.nx * a.ny;
   const uint64_t col = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t v = blockIdx.y;
+  if (blockIdx.x == gridDim.x - 1) {  // one block past the columns
+    dc_value<T>(a, v);
+    return;
+  }
   if (col >= P || a.band[col] == 0) return;
   const uint32_t iy = (uint32_t)(col / a.nx), ix = (uint32_t)(col - (uint64_t)iy * a.nx);
   const uint32_t mx = ix ? a.nx - ix : 0, my = iy ? a.ny - iy : 0;
@@ -214,7 +287,10 @@ __global__ void __launch_bounds__(WG) mbasis_zband_kernel(BandArgs<T> a, const c
   // once, and they cluster at the rows far from ky = 0 (one contiguous tile range
   // per XCD left some XCDs with little work: 426 against 396 us at 512^2 x 128)
   const uint32_t q = xcd_chunk_tile(blockIdx.x, kZbandChunk);
-  if (q >= per_vol * a.count) return;  // grid padding: the whole block leaves before any barrier
+  if (q >= per_vol * a.count) {  // (the whole block: DC values, then grid padding)
+    if (q < (per_vol + 1) * a.count) dc_value<T>(a, q - per_vol * a.count);
+    return;
+  }
   const uint32_t p = threadIdx.x % PP, t = threadIdx.x / PP;
   const uint32_t v = q / per_vol, tile = q % per_vol;
   const uint32_t g = tile % groups, y = tile / groups;
@@ -279,7 +355,7 @@ hipError_t launch_zband_n(const BandArgs<T> &a, hipStream_t st, const cx<T> *tw)
   if (tiles > 0x7ffffff0ull) return hipErrorInvalidConfiguration;
   constexpr bool LO = tw_lo_in_lds<T>((size_t)PP * N, N, WG);
   const size_t lds = ((size_t)PP * N + (LO ? 2 * N : N)) * sizeof(cx<T>);
-  hipLaunchKernelGGL((mbasis_zband_kernel<T, F, WG>), dim3(xcd_chunk_grid(tiles, kZbandChunk)), dim3(WG), lds, st,
+  hipLaunchKernelGGL((mbasis_zband_kernel<T, F, WG>), dim3(xcd_chunk_grid(tiles + a.count, kZbandChunk)), dim3(WG), lds, st,
                      a, tw);
   return hipGetLastError();
 }
@@ -293,7 +369,10 @@ __global__ void __launch_bounds__(1024) mbasis_zband_any_kernel(LfTab<T> tb, uin
   cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw);
   const uint32_t PP = 1u << lpp, groups = (a.nx + PP - 1) >> lpp, per_vol = groups * a.ny;
   const uint32_t q = xcd_chunk_tile(blockIdx.x, kZbandChunk);  // (as mbasis_zband_kernel)
-  if (q >= per_vol * a.count) return;  // grid padding: the whole block leaves before any barrier
+  if (q >= per_vol * a.count) {  // (the whole block: DC values, then grid padding)
+    if (q < (per_vol + 1) * a.count) dc_value<T>(a, q - per_vol * a.count);
+    return;
+  }
   const uint32_t p = threadIdx.x & (PP - 1), t = threadIdx.x >> lpp;
   const uint32_t v = q / per_vol, tile = q % per_vol;
   const uint32_t g = tile % groups, y = tile / groups;
@@ -348,39 +427,10 @@ template <typename T> cyr_status launch_zband_any(const BandArgs<T> &a, hipStrea
   CYR_TRY(lf_tables<T>(P, tb));
   const uint64_t tiles = (uint64_t)((a.nx + s.pp - 1) / s.pp) * a.ny * a.count;
   if (tiles > 0x7ffffff0ull) return fail(CYR_E_UNSUPPORTED, "Z band pass: grid too large");
-  hipLaunchKernelGGL((mbasis_zband_any_kernel<T>), dim3(xcd_chunk_grid(tiles, kZbandChunk)), dim3(s.pp * s.tpp), s.lds,
+  hipLaunchKernelGGL((mbasis_zband_any_kernel<T>), dim3(xcd_chunk_grid(tiles + a.count, kZbandChunk)), dim3(s.pp * s.tpp), s.lds,
                      st, tb, s.tpp, s.lpp, a);
   CYR_LAUNCHED();
   return CYR_OK;
-}
-
-// dcv[v] = (sum_z dcz[v][z]) / cnt, fixed-order tree (deterministic); one block per volume
-__global__ void __launch_bounds__(1024) mbasis_dcsum_kernel(const double2 *__restrict__ dcz, uint32_t nz, double cnt,
-                                                            double2 *__restrict__ dcv) {
-  __shared__ double red[2][1024];
-  const uint32_t v = blockIdx.x;
-  double sr = 0, si = 0;
-  for (uint32_t z = threadIdx.x; z < nz; z += blockDim.x) {
-    const double2 x = dcz[(uint64_t)v * nz + z];
-    sr += x.x;
-    si += x.y;
-  }
-  red[0][threadIdx.x] = sr;
-  red[1][threadIdx.x] = si;
-  __syncthreads();
-  for (uint32_t s = blockDim.x / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) {
-      red[0][threadIdx.x] += red[0][threadIdx.x + s];
-      red[1][threadIdx.x] += red[1][threadIdx.x + s];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    double2 o;
-    o.x = red[0][0] / cnt;
-    o.y = red[1][0] / cnt;
-    dcv[v] = o;
-  }
 }
 
 template <typename T> __device__ inline void cmac(cx<T> &acc, T cr, T ci, const cx<T> &x) {
@@ -691,39 +741,30 @@ __global__ void __launch_bounds__(256) mbasis_quad2_kernel(MbAnglesArgs<T> a) {
 
 }  // namespace
 
-cyr_status launch_mbasis_bands(const EwaldGeom &g, const double *kmag, uint32_t ne, int32_t *band, uint32_t *bmax,
-                               hipStream_t st) {
-  const uint64_t P = (uint64_t)g.nx * g.ny;
-  const uint32_t blocks = ceil_div(P, 256);
+cyr_status launch_mbasis_bands(const EwaldGeom &g, const double *kmag, uint32_t ne, double kmax, int32_t *band,
+                               uint32_t *bmax, bool totals, hipStream_t st) {
   if (g.nx > 0xfffe) return fail(CYR_E_UNSUPPORTED, "material basis: Nx above 65534");
+  const uint32_t blocks = g.ny / 2 + 1;
   uint32_t *span = mbasis_span_table(bmax, g.nx, g.ny);
-  hipLaunchKernelGGL(mbasis_bands_kernel, dim3(blocks), dim3(256), 0, st, g, kmag, ne, band, bmax);
+  const uint32_t waves = std::min(8u, std::max(1u, ceil_div(g.nx, 64)));
+  hipLaunchKernelGGL(mbasis_bands_kernel, dim3(blocks), dim3(64 * waves), 16 * (size_t)ceil_div(g.nx, 64), st, g, kmag,
+                     ne, kmax, band, span, totals ? bmax : nullptr);
   CYR_LAUNCHED();
-  hipLaunchKernelGGL(mbasis_span_kernel, dim3(g.ny), dim3(256), 0, st, band, g.nx, g.ny, span);
-  CYR_LAUNCHED();
-  hipLaunchKernelGGL(mbasis_bmax_kernel, dim3(1), dim3(256), 0, st, bmax, blocks, span, g.nx, g.ny);
-  CYR_LAUNCHED();
+  if (totals) {
+    hipLaunchKernelGGL(mbasis_bmax_kernel, dim3(1), dim3(256), 0, st, bmax, blocks, span, g.nx, g.ny);
+    CYR_LAUNCHED();
+  }
   return CYR_OK;
 }
 
-uint64_t mbasis_bmax_words(uint32_t nx, uint32_t ny) { return kBandHead + 2 * ceil_div((uint64_t)nx * ny, 256) + ny; }
-uint32_t *mbasis_span_table(uint32_t *bmax, uint32_t nx, uint32_t ny) {
-  return bmax + kBandHead + 2 * ceil_div((uint64_t)nx * ny, 256);
-}
+uint64_t mbasis_bmax_words(uint32_t, uint32_t ny) { return kBandHead + 2 * ((uint64_t)ny / 2 + 1) + ny; }
+uint32_t *mbasis_span_table(uint32_t *bmax, uint32_t, uint32_t ny) { return bmax + kBandHead + 2 * (ny / 2 + 1); }
 
 template <typename T> cyr_status launch_mbasis_extract(const BandArgs<T> &a, hipStream_t st) {
   if (a.count == 0) return CYR_OK;
   if (a.count > (uint32_t)kXMaxOut || a.J == 0 || a.nz != 1) return fail(CYR_E_INVALID, "band extraction: bad shape");
   const uint64_t P = (uint64_t)a.nx * a.ny;
-  hipLaunchKernelGGL((mbasis_extract_kernel<T>), dim3(ceil_div(P, 256), a.count), dim3(256), 0, st, a);
-  CYR_LAUNCHED();
-  return CYR_OK;
-}
-
-cyr_status launch_mbasis_dcsum(const double2 *dcz, uint32_t nvol, uint32_t nz, bool three, double2 *dcv,
-                               hipStream_t st) {
-  if (nvol == 0) return CYR_OK;
-  hipLaunchKernelGGL(mbasis_dcsum_kernel, dim3(nvol), dim3(1024), 0, st, dcz, nz, three ? 6.0 : 4.0, dcv);
+  hipLaunchKernelGGL((mbasis_extract_kernel<T>), dim3(ceil_div(P, 256) + 1, a.count), dim3(256), 0, st, a);
   CYR_LAUNCHED();
   return CYR_OK;
 }

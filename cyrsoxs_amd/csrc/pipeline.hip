@@ -479,7 +479,7 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
     xa.rot = is_identity(Q) ? 0 : 1;
     for (int c = 0; c < kEbFields; c++) xa.out[c] = pol + (uint64_t)c * V;
     kt_begin(s);
-    CYR_TRY(launch_ebasis_polx<T>(xa, d_vox, d->storage, d->morphology_type, hann, s));
+    CYR_TRY((launch_xfields<T, kXTensor>(xa, d_vox, d->storage, d->morphology_type, hann, s)));
     kt_end("xfields", s, su.vox_bytes + kEbFields * (double)V * cxb);
     if (lanes > 1) CYR_HIP(hipEventRecord(wb.ev_polx[L], s));
     DcArgs<T> da{};
@@ -560,10 +560,11 @@ cyr_status mbasis_band(const cyr_sim_desc *d, const SimGeometry &g, uint32_t k, 
                        uint64_t *wsum, uint64_t *ssum, uint64_t *d4) {
   const double kv[3] = {g.kvec[k].x, g.kvec[k].y, g.kvec[k].z};
   const EwaldGeom geo = make_ewald_geom(g.nx, g.ny, g.nz, d->phys_size, g.kmag[e0], kv, d->interpolation);
-  CYR_TRY(launch_mbasis_bands(geo, d_kmag + e0, ne, band, bmax, s));
+  const double kmax = *std::max_element(g.kmag.begin() + e0, g.kmag.begin() + e0 + ne);
   std::vector<double> key = {(double)g.nx, (double)g.ny, (double)g.nz, d->phys_size, (double)d->interpolation,
                              kv[0], kv[1], kv[2]};
   key.insert(key.end(), g.kmag.begin() + e0, g.kmag.begin() + e0 + ne);
+  bool known = false;
   {
     std::lock_guard<std::mutex> lk(g_band_mu);
     auto it = g_band_widths.find(key);
@@ -572,13 +573,15 @@ cyr_status mbasis_band(const cyr_sim_desc *d, const SimGeometry &g, uint32_t k, 
       *wsum = it->second.wsum;
       *ssum = it->second.ssum;
       *d4 = it->second.d4;
-      return CYR_OK;
+      known = true;
     }
   }
+  if (known) return launch_mbasis_bands(geo, d_kmag + e0, ne, kmax, band, bmax, false, s);
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   CYR_HIP(hipStreamIsCapturing(s, &cap));
   if (cap != hipStreamCaptureStatusNone)
     return fail(CYR_E_INVALID, "material basis: Ewald band widths unknown under capture (run the simulation once first)");
+  CYR_TRY(launch_mbasis_bands(geo, d_kmag + e0, ne, kmax, band, bmax, true, s));
   uint32_t h[kBandHead] = {};
   CYR_HIP(hipMemcpyAsync(h, bmax, sizeof(h), hipMemcpyDeviceToHost, s));
   CYR_HIP(hipStreamSynchronize(s));
@@ -695,8 +698,8 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
           vptr[c] = xa.out[c];
         }
         kt_begin(s);
-        if (tensor) CYR_TRY(launch_ebasis_polx<T>(xa, d_vox, d->storage, d->morphology_type, hann, s));
-        else CYR_TRY(launch_mbasis_xfields<T>(xa, pair, d_vox, d->storage, d->morphology_type, hann, s));
+        const auto launch_x = tensor ? launch_xfields<T, kXTensor> : pair ? launch_xfields<T, kXPair> : launch_xfields<T, kXSingle>;
+        CYR_TRY(launch_x(xa, d_vox, d->storage, d->morphology_type, hann, s));
         kt_end("xfields", s, (tensor ? g.M : pair ? 2.0 : 1.0) * 4.0 * vel * V + nv * (double)V * cxb);
         FftDc fdc{dcz + (uint64_t)vb * dc_per, su.twz, span};
         if (!dc_slots) {
@@ -731,6 +734,10 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
         ba.nx = g.nx;
         ba.ny = g.ny;
         ba.nz = g.nz;
+        ba.dcz = dcz;
+        ba.dcv = dcv;
+        ba.dc_per = dc_per;
+        ba.dc_cnt = three ? 6.0 : 4.0;
         kt_begin(s);
         if (three) {
           // reads the volumes' columns inside the row spans; writes each column's band
@@ -744,7 +751,6 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
         m0 += tensor ? g.M : pair ? 2 : 1;
         vb += nv;
       }
-      CYR_TRY(launch_mbasis_dcsum(dcz, nvol, (uint32_t)dc_per, three, dcv, s));
       // ---- per energy: fields at the Ewald bins, angles, rotation
       const double kv[3] = {g.kvec[k].x, g.kvec[k].y, g.kvec[k].z};
       const double *inv = su.rotinv + (size_t)6 * k * g.nA;

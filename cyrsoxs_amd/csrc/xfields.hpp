@@ -37,7 +37,6 @@
 
 namespace cyr {
 
-enum XMode { kXTensor = 0, kXPair = 1, kXSingle = 2 };
 template <int MODE> constexpr int x_outputs() { return MODE == kXTensor ? kEbFields : (MODE == kXPair ? 7 : 4); }
 
 // ---- the five tensor fields of one voxel -------------------------------------
@@ -400,7 +399,8 @@ hipError_t launch_xfields_ct_n(uint32_t n, dim3 grid, size_t lds, hipStream_t st
   return hipSuccess;
 }
 
-// Plans and launches the fields + X FFT kernel of one MODE.
+// Plans and launches the fields + X FFT kernel of one MODE (instantiated per precision
+// and mode in a file of its own: xfields_*.hip).
 template <typename T, int MODE>
 cyr_status launch_xfields(PolxArgs<T> a, const void *vox, int storage, int morph, bool hann, hipStream_t st) {
   const int prec = sizeof(T) == 8 ? CYR_FP64 : CYR_FP32;
@@ -446,19 +446,6 @@ cyr_status launch_xfields(PolxArgs<T> a, const void *vox, int storage, int morph
   if (e != hipSuccess) return hip_fail(e, "xfields_kernel", __FILE__, __LINE__);
   if (!found) return fail(CYR_E_UNSUPPORTED, "fused X kernel: no kernel for this length");
   return CYR_OK;
-}
-
-// The launchers of kernels.hpp, instantiated per precision in a file of its own.
-template <typename T>
-cyr_status launch_ebasis_polx(PolxArgs<T> a, const void *vox, int storage, int morph, bool hann, hipStream_t st) {
-  return launch_xfields<T, kXTensor>(a, vox, storage, morph, hann, st);
-}
-
-template <typename T>
-cyr_status launch_mbasis_xfields(PolxArgs<T> a, bool pair, const void *vox, int storage, int morph, bool hann,
-                                 hipStream_t st) {
-  if (pair) return launch_xfields<T, kXPair>(a, vox, storage, morph, hann, st);
-  return launch_xfields<T, kXSingle>(a, vox, storage, morph, hann, st);
 }
 
 }  // namespace cyr
