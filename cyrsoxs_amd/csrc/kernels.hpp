@@ -191,14 +191,14 @@ template <typename T> struct MbAnglesArgs {
   uint32_t M;                      // 0: own holds one energy's five tensor fields (mir unused)
   const T *amat;                   // [nA][kEbAmat]
   uint32_t nA;
-  T *proj;                         // [nA][Ny][Nx] (per-angle projections), or
+  T *proj;                         // [ne][nA][Ny][Nx] (per-angle projections), or
   T *quad;                         // [ne][P][3] in quad_index order: laboratory frame, the intensity's quadratic form
   Mat3<T> Q;                       // frame e1, e2, k^ (quadratic form)
-  const double *kmag;              // quadratic form: |k| of the ne energies (mats then holds ne x M)
+  const double *kmag;              // |k| of the ne energies (mats holds ne x M)
   uint32_t ne;
 };
-// quad set: one quadratic form per pixel for each of ne energies in one launch
-// (laboratory frame), else every angle's projection of one energy.
+// ne energies in one launch: with quad one quadratic form per pixel (laboratory frame),
+// else every angle's projection.
 template <typename T> cyr_status launch_mbasis_angles(const MbAnglesArgs<T> &a, int ng, hipStream_t st);
 
 // Values per record of a plane of quadratic forms (q0, q1, q2 of one pixel, packed
@@ -230,11 +230,13 @@ uint32_t rotation_tile_count(uint32_t nx, uint32_t ny);
 // centre (a prefix of that order).
 uint32_t rotation_tiles_within(uint32_t nx, uint32_t ny, double r);
 void rotation_tile_order(uint32_t nx, uint32_t ny, uint32_t *out);
-// E-basis path: rotate every angle's projection, accumulate and average in one pass
-// (tiles: rotation_tile_order on the device).
+// Material frame: rotate every angle's projection proj[ne][nA][Ny][Nx], accumulate and
+// average into avg[ne][Ny][Nx] in one pass (tiles: rotation_tile_order on the device;
+// rfin as below).
 template <typename T>
 cyr_status launch_rotate_all(const T *proj, const double *inv_tab, uint32_t nA, uint32_t nx, uint32_t ny,
-                             int rot_mask, double *avg, const uint32_t *tiles, double rfin, hipStream_t st);
+                             int rot_mask, double *avg, uint32_t ne, const uint32_t *tiles, double rfin,
+                             hipStream_t st);
 // Quarter-turn orbits of a square N x N plane (N even): orbit representatives
 // in 16 x 16 tiles (ty << 16 | tx) ordered by distance from the rotation centre.
 uint32_t rotation_orbit_tile_count(uint32_t n);

@@ -286,11 +286,15 @@ __global__ void __launch_bounds__(WG) mbasis_zband_kernel(BandArgs<T> a, const c
   // chunks of 16 tiles over the XCDs: the tiles outside the row spans leave at
   // once, and they cluster at the rows far from ky = 0 (one contiguous tile range
   // per XCD left some XCDs with little work: 426 against 396 us at 512^2 x 128)
-  const uint32_t q = xcd_chunk_tile(blockIdx.x, kZbandChunk);
-  if (q >= per_vol * a.count) {  // (the whole block: DC values, then grid padding)
-    if (q < (per_vol + 1) * a.count) dc_value<T>(a, q - per_vol * a.count);
+  const uint32_t qb = xcd_chunk_tile(blockIdx.x, kZbandChunk);
+  // the first blocks form the DC values (last, they would be the launch's tail: 512^2 x
+  // 128, 395 -> 414 us); blocks past the tiles are grid padding
+  if (qb < a.count) {
+    dc_value<T>(a, qb);
     return;
   }
+  const uint32_t q = qb - a.count;
+  if (q >= per_vol * a.count) return;
   const uint32_t p = threadIdx.x % PP, t = threadIdx.x / PP;
   const uint32_t v = q / per_vol, tile = q % per_vol;
   const uint32_t g = tile % groups, y = tile / groups;
@@ -368,11 +372,13 @@ __global__ void __launch_bounds__(1024) mbasis_zband_any_kernel(LfTab<T> tb, uin
   extern __shared__ unsigned char smem_raw[];
   cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw);
   const uint32_t PP = 1u << lpp, groups = (a.nx + PP - 1) >> lpp, per_vol = groups * a.ny;
-  const uint32_t q = xcd_chunk_tile(blockIdx.x, kZbandChunk);  // (as mbasis_zband_kernel)
-  if (q >= per_vol * a.count) {  // (the whole block: DC values, then grid padding)
-    if (q < (per_vol + 1) * a.count) dc_value<T>(a, q - per_vol * a.count);
+  const uint32_t qb = xcd_chunk_tile(blockIdx.x, kZbandChunk);  // (as mbasis_zband_kernel)
+  if (qb < a.count) {
+    dc_value<T>(a, qb);
     return;
   }
+  const uint32_t q = qb - a.count;
+  if (q >= per_vol * a.count) return;
   const uint32_t p = threadIdx.x & (PP - 1), t = threadIdx.x >> lpp;
   const uint32_t v = q / per_vol, tile = q % per_vol;
   const uint32_t g = tile % groups, y = tile / groups;
@@ -551,12 +557,16 @@ __device__ inline int mb_fields(const MbAnglesArgs<T> &a, uint32_t X, uint32_t Y
   return kind;
 }
 
-// ---- per energy: every angle's projection ---------------------------------------
+// ---- every angle's projection (grid y: energies) ---------------------------------
 template <typename T, int NG>
 __global__ void __launch_bounds__(256) mbasis_angles_kernel(MbAnglesArgs<T> a) {
   const uint64_t P2 = (uint64_t)a.g.nx * a.g.ny;
   const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= P2) return;
+  const uint32_t e = blockIdx.y;
+  a.g.k = a.kmag[e];
+  a.mats += (uint64_t)e * a.M;
+  a.proj += (uint64_t)e * a.nA * P2;
   const uint32_t Y = (uint32_t)(t / a.g.nx), X = (uint32_t)(t - (uint64_t)Y * a.g.nx);
   cx<T> F[NG][kEbFields];
   double md[NG][6];
@@ -809,9 +819,9 @@ template <typename T> cyr_status launch_mbasis_zband(const BandArgs<T> &a, hipSt
 
 template <typename T> cyr_status launch_mbasis_angles(const MbAnglesArgs<T> &a, int ng, hipStream_t st) {
   const uint64_t P = (uint64_t)a.g.nx * a.g.ny;
-  const dim3 grid(ceil_div(P, 256)), block(256);
+  if (!a.kmag || a.ne == 0 || a.ne > 65535) return fail(CYR_E_INVALID, "material basis: energy table missing");
+  const dim3 grid(ceil_div(P, 256), a.ne), block(256);
   if (a.quad) {
-    if (!a.kmag || a.ne == 0 || a.ne > 65535) return fail(CYR_E_INVALID, "quadratic form: energy table missing");
     // FP32: energies in pairs (one thread per pixel and pair); FP64 (whose pair
     // kernel would hold 256 registers) and single energies: one at a time
     const bool paired = a.ne >= 2 && sizeof(T) == 4;

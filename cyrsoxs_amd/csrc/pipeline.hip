@@ -527,7 +527,7 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
       CYR_TRY(launch_ebasis_angles<T>(aa, ng, s));
       kt_end("ebasis_angles", s, part_bytes + (double)g.nA * P * sizeof(T));
       kt_begin(s);
-      CYR_TRY(launch_rotate_all<T>(proj, inv, g.nA, g.nx, g.ny, d->rot_mask, avg, su.tiles, rfin, s));
+      CYR_TRY(launch_rotate_all<T>(proj, inv, g.nA, g.nx, g.ny, d->rot_mask, avg, 1, su.tiles, rfin, s));
       kt_end("rotate_all", s, (double)(g.nA + 1) * P * sizeof(T));
     }
     CYR_TRY(launch_detector_warp<T>(avg, out, g.nx, g.ny, &g.det_inv[(size_t)k * 6], d->rot_mask, s));
@@ -788,19 +788,31 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
                                             g.ny, &g.det_inv[(size_t)k * 6], d->rot_mask, s));
         }
       } else {
-        for (uint32_t e = e0; e < e0 + ne; e++) {
-          aa.g = make_ewald_geom(g.nx, g.ny, g.nz, d->phys_size, g.kmag[e], kv, d->interpolation);
-          aa.mats = su.mats + (size_t)e * g.M;
-          aa.proj = proj;
+        // batches of energies whose projections and averages fit in the packed volumes,
+        // which the band passes have just finished with (one energy at a time in their
+        // own buffers when a single one does not)
+        const uint64_t per = sizeof(T) * P * g.nA + sizeof(double) * P;
+        const uint64_t fit = (sizeof(cx<T>) * V * pass_max) / per;
+        const uint32_t mbatch = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(fit, 32));
+        for (uint32_t b0 = e0; b0 < e0 + ne; b0 += mbatch) {
+          const uint32_t n = std::min(mbatch, e0 + ne - b0);
+          // (FP64 averages ahead of the projections: 8-byte aligned)
+          double *bavg = fit ? reinterpret_cast<double *>(pol) : avg;
+          T *pr = fit ? reinterpret_cast<T *>(bavg + (uint64_t)n * P) : proj;
+          aa.g = make_ewald_geom(g.nx, g.ny, g.nz, d->phys_size, g.kmag[b0], kv, d->interpolation);
+          aa.kmag = su.kmag + b0;
+          aa.ne = n;
+          aa.mats = su.mats + (size_t)b0 * g.M;
+          aa.proj = pr;
           kt_begin(s);
           CYR_TRY(launch_mbasis_angles<T>(aa, ng, s));
-          kt_end("mbasis_angles", s, (double)planes * ng * nvol * (double)P * cxb + (double)g.nA * P * sizeof(T));
+          kt_end("mbasis_angles", s, (double)planes * nvol * (double)wsum * cxb + n * (double)g.nA * P * sizeof(T));
           kt_begin(s);
-          CYR_TRY(launch_rotate_all<T>(proj, inv, g.nA, g.nx, g.ny, d->rot_mask, avg, su.tiles,
+          CYR_TRY(launch_rotate_all<T>(pr, inv, g.nA, g.nx, g.ny, d->rot_mask, bavg, n, su.tiles,
                                        0.5 * std::sqrt((double)d4), s));
-          kt_end("rotate_all", s, (double)(g.nA + 1) * P * sizeof(T));
-          T *out = d_out + ((uint64_t)e * g.nK + k) * P;
-          CYR_TRY(launch_detector_warp<T>(avg, out, g.nx, g.ny, &g.det_inv[(size_t)k * 6], d->rot_mask, s));
+          kt_end("rotate_all", s, n * (double)(g.nA + 1) * P * sizeof(T));
+          CYR_TRY(launch_detector_warp_n<T>(bavg, d_out + ((uint64_t)b0 * g.nK + k) * P, (uint64_t)g.nK * P, n, g.nx,
+                                            g.ny, &g.det_inv[(size_t)k * 6], d->rot_mask, s));
         }
       }
       e0 += ne;

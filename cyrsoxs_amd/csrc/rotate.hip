@@ -73,21 +73,36 @@ __global__ void __launch_bounds__(256) average_kernel(const double *__restrict__
   }
 }
 
+// Material frame: every angle's projection proj[ne][nA][P] rotated, masked and averaged
+// (grid z: energies).  A block holds one 8 x 8 quadrant of a tile, its four waves a
+// quarter of the angles each; their FP64 sums meet in LDS in angle order.  Each angle has
+// a plane of its own, so the split costs no sharing of taps, and small planes get four
+// times the waves (128^2, 18 angles: 16 us per energy in a launch of its own -> all of 6
+// energies 17 us).
 template <typename T>
 __global__ void __launch_bounds__(256) rotate_all_kernel(const T *__restrict__ proj, const double *__restrict__ inv_tab,
                                                          uint32_t nA, uint32_t nx, uint32_t ny, int rot_mask,
                                                          double *__restrict__ avg, const uint32_t *__restrict__ tiles,
                                                          uint32_t ntiles) {
+  __shared__ double sum[4][64];
+  __shared__ uint32_t num[4][64];
   const uint64_t P = (uint64_t)nx * ny;
-  uint32_t X, Y;
-  if (!tile_pixel(tiles, ntiles, nx, ny, X, Y)) return;
+  const uint32_t b = xcd_tile(blockIdx.x, gridDim.x);
+  if (b >= 4 * ntiles) return;  // (the whole block)
+  proj += (uint64_t)blockIdx.z * nA * P;
+  avg += (uint64_t)blockIdx.z * P;
+  const uint32_t tt = tiles[b >> 2], w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const uint32_t X = (tt & 0xffffu) * 16 + (b & 1) * 8 + (l & 7);
+  const uint32_t Y = (tt >> 16) * 16 + ((b >> 1) & 1) * 8 + (l >> 3);
+  const bool in = X < nx && Y < ny;
   const uint64_t t = (uint64_t)Y * nx + X;
   double acc = 0;
   uint32_t cnt = 0;
+  const uint32_t a0 = (uint32_t)((uint64_t)nA * w / 4), a1 = in ? (uint32_t)((uint64_t)nA * (w + 1) / 4) : a0;
   // independent gathers per angle; unrolling lets several be in flight (the sum
   // itself stays in angle order)
 #pragma unroll 4
-  for (uint32_t a = 0; a < nA; a++) {
+  for (uint32_t a = a0; a < a1; a++) {
     double inv[6];
 #pragma unroll
     for (int i = 0; i < 6; i++) inv[i] = inv_tab[6 * (uint64_t)a + i];
@@ -101,6 +116,14 @@ __global__ void __launch_bounds__(256) rotate_all_kernel(const T *__restrict__ p
     } else {
       acc += v;
     }
+  }
+  sum[w][l] = acc;
+  num[w][l] = cnt;
+  __syncthreads();
+  if (w != 0 || !in) return;
+  for (int i = 1; i < 4; i++) {
+    acc += sum[i][l];
+    cnt += num[i][l];
   }
   if (rot_mask) avg[t] = cnt == 0 ? 0.0 : acc * (1.0 / (cnt * 1.0));
   else avg[t] = acc * (1.0 / (double)nA);
@@ -735,18 +758,18 @@ cyr_status launch_average(const double *acc, const uint32_t *count, double *avg,
 
 template <typename T>
 cyr_status launch_rotate_all(const T *proj, const double *inv_tab, uint32_t nA, uint32_t nx, uint32_t ny, int rot_mask,
-                             double *avg, const uint32_t *tiles, double rfin, hipStream_t st) {
+                             double *avg, uint32_t ne, const uint32_t *tiles, double rfin, hipStream_t st) {
   const uint32_t ntiles = rotation_tile_count(nx, ny);
   if (!tiles) return fail(CYR_E_INVALID, "rotation: tile order missing");
   // the finite-radius cut of launch_rotate_quad (the projections are NaN where the
   // forms are)
   const uint32_t n_act = rfin >= 0 ? std::min(ntiles, rotation_tiles_within(nx, ny, rfin + 14.0)) : ntiles;
-  hipLaunchKernelGGL((rotate_all_kernel<T>), dim3(xcd_grid(n_act)), dim3(256), 0, st, proj, inv_tab, nA, nx, ny,
+  hipLaunchKernelGGL((rotate_all_kernel<T>), dim3(xcd_grid(4ull * n_act), 1, ne), dim3(256), 0, st, proj, inv_tab, nA, nx, ny,
                      rot_mask, avg, tiles, n_act);
   CYR_LAUNCHED();
   if (n_act < ntiles) {
-    hipLaunchKernelGGL((quad_fill_kernel<1>), dim3(ntiles - n_act), dim3(256), 0, st, avg, nx, ny, 1u, rot_mask, tiles,
-                       n_act);
+    hipLaunchKernelGGL((quad_fill_kernel<1>), dim3(ntiles - n_act, 1, ne), dim3(256), 0, st, avg, nx, ny, ne, rot_mask,
+                       tiles, n_act);
     CYR_LAUNCHED();
   }
   return CYR_OK;
@@ -895,7 +918,7 @@ cyr_status launch_warp(const T *src, T *dst, uint32_t nx, uint32_t ny, const dou
   template cyr_status launch_rotate_accumulate<T>(const T *, double *, uint32_t *, uint32_t, uint32_t,             \
                                                   const double *, int, hipStream_t);                               \
   template cyr_status launch_rotate_all<T>(const T *, const double *, uint32_t, uint32_t, uint32_t, int, double *, \
-                                           const uint32_t *, double, hipStream_t);                                 \
+                                           uint32_t, const uint32_t *, double, hipStream_t);                                 \
   template cyr_status launch_rotate_quad<T>(const T *, const double *, const double *, const T *, uint32_t,      \
                                             uint32_t, uint32_t, int, double *, uint32_t, const uint32_t *,        \
                                             uint32_t, const uint32_t *, bool, double, hipStream_t);                \
