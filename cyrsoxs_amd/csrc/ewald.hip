@@ -52,9 +52,14 @@ __device__ inline T intensity_at(const EwaldGeom &g, const cx<T> *px, const cx<T
 template <typename T>
 __global__ void __launch_bounds__(256) ewald_partial_kernel(EwaldGeom g, const cx<T> *__restrict__ px,
                                                             const cx<T> *__restrict__ py,
-                                                            const cx<T> *__restrict__ pz, T *__restrict__ proj) {
+                                                            const cx<T> *__restrict__ pz, T *__restrict__ proj,
+                                                            uint64_t vol_stride) {
   const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (uint64_t)g.nx * g.ny) return;
+  px += blockIdx.y * vol_stride;  // grid y: E angles
+  py += blockIdx.y * vol_stride;
+  pz += blockIdx.y * vol_stride;
+  proj += (uint64_t)blockIdx.y * g.nx * g.ny;
   const uint32_t Y = (uint32_t)(t / g.nx), X = (uint32_t)(t - (uint64_t)Y * g.nx);
   uint32_t z0 = 0;
   double f = 0;
@@ -108,7 +113,8 @@ __global__ void __launch_bounds__(256) ewald_full_kernel(EwaldGeom g, const T *_
 
 // F[0] <- mean of the periodic neighbours (4 in-plane, +2 along z when Nz > 1);
 // one thread per volume.
-template <typename T> struct DcVols { cx<T> *v[8]; };
+constexpr uint32_t kDcVols = 3 * kPolAngles;
+template <typename T> struct DcVols { cx<T> *v[kDcVols]; };
 
 template <typename T>
 __global__ void dc_replace_kernel(DcVols<T> vols, uint32_t count, uint32_t nx, uint32_t ny, uint32_t nz) {
@@ -148,9 +154,10 @@ __global__ void __launch_bounds__(256) igor_shift_kernel(cx<T> *vol, uint32_t nx
 
 template <typename T>
 cyr_status launch_ewald_partial(const EwaldGeom &g, const cx<T> *px, const cx<T> *py, const cx<T> *pz, T *proj,
-                                hipStream_t st) {
+                                hipStream_t st, uint32_t nb, uint64_t vol_stride) {
   const uint64_t P = (uint64_t)g.nx * g.ny;
-  hipLaunchKernelGGL((ewald_partial_kernel<T>), dim3(ceil_div(P, 256)), dim3(256), 0, st, g, px, py, pz, proj);
+  hipLaunchKernelGGL((ewald_partial_kernel<T>), dim3(ceil_div(P, 256), nb), dim3(256), 0, st, g, px, py, pz, proj,
+                     vol_stride);
   CYR_LAUNCHED();
   return CYR_OK;
 }
@@ -174,9 +181,9 @@ template <typename T> cyr_status launch_ewald_full(const EwaldGeom &g, const T *
 template <typename T>
 cyr_status launch_dc_replace(cx<T> *const *vols, uint32_t count, uint32_t nx, uint32_t ny, uint32_t nz,
                              hipStream_t st) {
-  for (uint32_t c0 = 0; c0 < count; c0 += 8) {
+  for (uint32_t c0 = 0; c0 < count; c0 += kDcVols) {
     DcVols<T> dv{};
-    const uint32_t nc = count - c0 < 8 ? count - c0 : 8;
+    const uint32_t nc = count - c0 < kDcVols ? count - c0 : kDcVols;
     for (uint32_t i = 0; i < nc; i++) dv.v[i] = vols[c0 + i];
     hipLaunchKernelGGL((dc_replace_kernel<T>), dim3(1), dim3(64), 0, st, dv, nc, nx, ny, nz);
     CYR_LAUNCHED();
@@ -193,7 +200,7 @@ template <typename T> cyr_status launch_igor_shift(cx<T> *vol, uint32_t nx, uint
 
 #define CYR_INST(T)                                                                                                  \
   template cyr_status launch_ewald_partial<T>(const EwaldGeom &, const cx<T> *, const cx<T> *, const cx<T> *, T *,   \
-                                              hipStream_t);                                                          \
+                                              hipStream_t, uint32_t, uint64_t);                                                          \
   template cyr_status launch_scatter3d<T>(const EwaldGeom &, const cx<T> *, const cx<T> *, const cx<T> *, T *,       \
                                           hipStream_t);                                                              \
   template cyr_status launch_ewald_full<T>(const EwaldGeom &, const T *, T *, hipStream_t);                          \

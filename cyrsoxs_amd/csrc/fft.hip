@@ -33,8 +33,9 @@ namespace cyr {
 
 namespace {
 
+constexpr uint32_t kPassVols = 24;  // volumes of one launch
 struct PassArgs {
-  void *vol[8];
+  void *vol[kPassVols];
   uint32_t nvol;  // volumes of this launch (1D XCD-ordered grids)
   uint64_t elem_stride;
   uint64_t inner_stride;
@@ -876,8 +877,8 @@ cyr_status fft_axis(void *const *vols, uint32_t count, uint32_t nx, uint32_t ny,
   }
   const uint64_t dc_per_vol = dc ? (uint64_t)nz * fft_dc_slots<T>(nx, ny) : 0;
   if (dc && (axis != 1 || dc_per_vol == 0)) return fail(CYR_E_INVALID, "FFT: DC sums need a Y pass and Nx >= 3");
-  for (uint32_t c0 = 0; c0 < count; c0 += 8) {
-    const uint32_t nc = count - c0 < 8 ? count - c0 : 8;
+  for (uint32_t c0 = 0; c0 < count; c0 += kPassVols) {
+    const uint32_t nc = count - c0 < kPassVols ? count - c0 : kPassVols;
     for (uint32_t i = 0; i < nc; i++) A.vol[i] = vols[c0 + i];
     A.dcz = dc ? dc->dcz + c0 * dc_per_vol : nullptr;
     A.dc_twy = tw;

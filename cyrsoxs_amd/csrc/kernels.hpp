@@ -8,6 +8,7 @@
 namespace cyr {
 
 // ---- polarization (polarization.hip) ----------------------------------------
+constexpr int kPolAngles = 8;  // E angles of one launch of the plain executor's kernels
 template <typename T> struct PolarArgs {
   const MatConst<T> *mats;  // this energy's M constants (device)
   uint32_t M;
@@ -15,11 +16,13 @@ template <typename T> struct PolarArgs {
   uint32_t nx, ny, nz;
   uint32_t rows, block, blocks_per_row;  // filled by the launcher
   const T *hx, *hy, *hz;                 // Hanning tables (device) or null
-  Vec3<T> e[2];                          // E basis vectors
-  Mat3<T> R;                             // E rotation (MATERIAL frame)
-  cx<T> *out[6];                         // [basis][component] volumes
+  Vec3<T> e[kPolAngles];                 // E vector of each angle
+  Mat3<T> R[kPolAngles];                 // E rotation of each angle (MATERIAL frame)
+  cx<T> *out[3];                         // component volumes of the first angle,
+  uint64_t angle_stride;                 // and the elements to the next angle's
 };
 
+// nb angles (1 .. kPolAngles) from one evaluation of the tensor.
 template <typename T>
 cyr_status launch_polarization(PolarArgs<T> a, const void *vox, int storage, int morph, int nb, bool hann,
                                bool matframe, hipStream_t st);
@@ -41,10 +44,11 @@ struct EwaldGeom {
 EwaldGeom make_ewald_geom(uint32_t nx, uint32_t ny, uint32_t nz, double phys_size, double k,
                           const double kvec[3], int interpolation);
 
-// Plain path: projection of one E angle from the three UNshifted FFT volumes.
+// Plain path: projections of nb E angles from their three UNshifted FFT volumes (angle
+// a's at px + a vol_stride, its projection at proj + a Nx Ny).
 template <typename T>
 cyr_status launch_ewald_partial(const EwaldGeom &g, const cx<T> *px, const cx<T> *py, const cx<T> *pz, T *proj,
-                                hipStream_t st);
+                                hipStream_t st, uint32_t nb = 1, uint64_t vol_stride = 0);
 // Full approach: I over the whole shifted volume, then the projection.
 template <typename T>
 cyr_status launch_scatter3d(const EwaldGeom &g, const cx<T> *px, const cx<T> *py, const cx<T> *pz, T *scatter,
@@ -216,10 +220,11 @@ __host__ __device__ inline uint32_t quad_index(uint32_t x, uint32_t y, uint32_t 
 }
 
 // ---- rotation / averaging (rotate.hip) --------------------------------------
-// Plain path: rotate one projection by the E angle and accumulate (FP64).
+// Plain path: rotate nb projections [nb][Ny][Nx] by their E angles (inv: nb x 6 inverse
+// coefficients on the device) and accumulate (FP64, in angle order).
 template <typename T>
 cyr_status launch_rotate_accumulate(const T *proj, double *acc, uint32_t *count, uint32_t nx, uint32_t ny,
-                                    const double inv[6], int rot_mask, hipStream_t st);
+                                    const double *inv, uint32_t nb, int rot_mask, hipStream_t st);
 // Average over angles into avg (FP64): mask division or 1/nA.
 cyr_status launch_average(const double *acc, const uint32_t *count, double *avg, uint64_t P, uint32_t nA,
                           int rot_mask, hipStream_t st);

@@ -305,17 +305,26 @@ cyr_status run_plain(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
   const bool full = d->scatter_approach == 1;
   const int ng = (g.nz > 1 && d->interpolation == 1) ? 2 : 1;
   LaneBuffers &lb = wb.lane[0];
-  CYR_TRY(ensure_buffer(lb.pol, sizeof(cx<T>) * V * 3));
+  // E angles per launch: small grids take several together (128^2 x 32: 8 launches of
+  // 3-12 us per angle, half of it gaps and unfilled kernels: 600 -> 296 us for 12
+  // angles), at most 64 MB of volumes beyond the first angle's; not beside other
+  // simulations or in the scratch array, whose memory is counted by the single angle
+  const uint64_t angle_bytes = sizeof(cx<T>) * V * 3;
+  uint32_t nb = 1;
+  if (!full && wb.max_lanes > 1 && !scratch_arena())
+    nb = (uint32_t)std::min<uint64_t>({(64ull << 20) / angle_bytes + 1, (uint64_t)kPolAngles, (uint64_t)g.nA});
+  if (nb > 1 && ensure_buffer(lb.pol, angle_bytes * nb) != CYR_OK) nb = 1;
+  CYR_TRY(ensure_buffer(lb.pol, angle_bytes * nb));
   cx<T> *pol = reinterpret_cast<cx<T> *>(lb.pol.ptr);
-  cx<T> *vols[3];
-  void *vptr[3];
-  for (uint32_t c = 0; c < 3; c++) {
+  cx<T> *vols[3 * kPolAngles];
+  void *vptr[3 * kPolAngles];
+  for (uint32_t c = 0; c < 3 * nb; c++) {
     vols[c] = pol + (uint64_t)c * V;
     vptr[c] = vols[c];
   }
   if (alg1) CYR_TRY(ensure_buffer(wb.nt, sizeof(cx<T>) * V * 6));
   if (full) CYR_TRY(ensure_buffer(wb.scatter, sizeof(T) * V));
-  CYR_TRY(ensure_buffer(lb.proj, sizeof(T) * P));
+  CYR_TRY(ensure_buffer(lb.proj, sizeof(T) * P * nb));
   CYR_TRY(ensure_buffer(wb.acc, sizeof(double) * P));
   CYR_TRY(ensure_buffer(wb.count, sizeof(uint32_t) * P));
   CYR_TRY(ensure_buffer(lb.avg, sizeof(double) * P));
@@ -335,6 +344,7 @@ cyr_status run_plain(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
   pa.hy = su.hy;
   pa.hz = su.hz;
   for (uint32_t c = 0; c < 3; c++) pa.out[c] = vols[c];
+  pa.angle_stride = 3 * V;
 
   for (uint32_t e = 0; e < g.nE; e++) {
     pa.mats = su.mats + (size_t)e * g.M;
@@ -346,21 +356,24 @@ cyr_status run_plain(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
       T *out = d_out + ((uint64_t)e * g.nK + k) * P;
       CYR_TRY(fill<double>(acc, 0.0, P, st));
       CYR_TRY(fill<uint32_t>(count, 0u, P, st));
-      for (uint32_t a = 0; a < g.nA; a++) {
-        const M3 &R = g.R[(size_t)k * g.nA + a];
-        pa.e[0] = Vec3<T>{(T)R.m[0], (T)R.m[3], (T)R.m[6]};  // E = R x^
-        pa.R = m3<T>(R);
+      for (uint32_t a0 = 0; a0 < g.nA; a0 += nb) {
+        const uint32_t n = std::min(nb, g.nA - a0);
+        for (uint32_t b = 0; b < n; b++) {
+          const M3 &R = g.R[(size_t)k * g.nA + a0 + b];
+          pa.e[b] = Vec3<T>{(T)R.m[0], (T)R.m[3], (T)R.m[6]};  // E = R x^
+          pa.R[b] = m3<T>(R);
+        }
         kt_begin(st);
         if (alg1)
-          CYR_TRY(launch_polarization_nt<T>(pa, reinterpret_cast<const cx<T> *>(wb.nt.ptr), 1, matframe, st));
+          CYR_TRY(launch_polarization_nt<T>(pa, reinterpret_cast<const cx<T> *>(wb.nt.ptr), (int)n, matframe, st));
         else
-          CYR_TRY(launch_polarization<T>(pa, d_vox, d->storage, d->morphology_type, 1, hann, matframe, st));
-        kt_end(alg1 ? "polarization_nt" : "polarization", st, (alg1 ? 6.0 * V * cxb : su.vox_bytes) + 3.0 * V * cxb);
+          CYR_TRY(launch_polarization<T>(pa, d_vox, d->storage, d->morphology_type, (int)n, hann, matframe, st));
+        kt_end(alg1 ? "polarization_nt" : "polarization", st, (alg1 ? 6.0 * V * cxb : su.vox_bytes) + 3.0 * n * V * cxb);
         kt_begin(st);
-        CYR_TRY(fft3d<T>(vptr, 3, g.nx, g.ny, g.nz, st));
-        kt_end("fft3d_3vol", st, (g.nz > 1 ? 3.0 : 2.0) * 3 * 2 * V * cxb);
+        CYR_TRY(fft3d<T>(vptr, 3 * n, g.nx, g.ny, g.nz, st));
+        kt_end("fft3d", st, (g.nz > 1 ? 3.0 : 2.0) * 3 * n * 2 * V * cxb);
         kt_begin(st);
-        CYR_TRY(launch_dc_replace<T>(vols, 3, g.nx, g.ny, g.nz, st));
+        CYR_TRY(launch_dc_replace<T>(vols, 3 * n, g.nx, g.ny, g.nz, st));
         kt_end("dc_replace", st);
         if (full) {
           T *sc = reinterpret_cast<T *>(wb.scatter.ptr);
@@ -368,13 +381,13 @@ cyr_status run_plain(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
           CYR_TRY(launch_ewald_full<T>(geo, sc, proj, st));
         } else {
           kt_begin(st);
-          CYR_TRY(launch_ewald_partial<T>(geo, vols[0], vols[1], vols[2], proj, st));
-          kt_end("ewald_partial", st, 3.0 * ng * P * cxb + (double)P * sizeof(T));
+          CYR_TRY(launch_ewald_partial<T>(geo, vols[0], vols[1], vols[2], proj, st, n, pa.angle_stride));
+          kt_end("ewald_partial", st, n * (3.0 * ng * P * cxb + (double)P * sizeof(T)));
         }
         kt_begin(st);
-        CYR_TRY(launch_rotate_accumulate<T>(proj, acc, count, g.nx, g.ny, &g.rot_inv[((size_t)k * g.nA + a) * 6],
+        CYR_TRY(launch_rotate_accumulate<T>(proj, acc, count, g.nx, g.ny, su.rotinv + ((size_t)k * g.nA + a0) * 6, n,
                                             d->rot_mask, st));
-        kt_end("rotate_accumulate", st, (double)P * (sizeof(T) + 2 * (8 + 4)));
+        kt_end("rotate_accumulate", st, (double)P * (n * sizeof(T) + 2 * (8 + 4)));
       }
       CYR_TRY(launch_average(acc, count, avg, P, g.nA, d->rot_mask, st));
       CYR_TRY(launch_detector_warp<T>(avg, out, g.nx, g.ny, &g.det_inv[(size_t)k * 6], d->rot_mask, st));
@@ -1271,7 +1284,7 @@ cyr_status cyr_polarization_device(const cyr_sim_desc *desc, const void *d_voxel
     pa.hy = h + g.nx;
     pa.hz = h + g.nx + g.ny;
     pa.e[0] = Vec3<T>{(T)R.m[0], (T)R.m[3], (T)R.m[6]};
-    pa.R = m3<T>(R);
+    pa.R[0] = m3<T>(R);
     pa.out[0] = reinterpret_cast<cx<T> *>(d_px);
     pa.out[1] = reinterpret_cast<cx<T> *>(d_py);
     pa.out[2] = reinterpret_cast<cx<T> *>(d_pz);

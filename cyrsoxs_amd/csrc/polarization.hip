@@ -14,7 +14,7 @@
 // d = n_par^2 - n_perp^2.  This is the reference's tensor with its "- Vfrac"
 // vacuum term cancelled analytically (phi_a |s|^2 + phi_u - Vfrac = 0 for Euler
 // angles; exact for vectors), which keeps FP32 free of 1 - n^2 cancellation.
-// Then p = N E / (4 pi) for each requested E basis vector; the MATERIAL frame
+// Then p = N E / (4 pi) for the E vector of each requested angle; the MATERIAL frame
 // rotates p by R^T; the Hanning window (Algorithm 0 only) multiplies p.
 #include <hip/hip_runtime.h>
 
@@ -26,9 +26,10 @@ namespace cyr {
 
 namespace {
 
-// Block = a run of `blockDim.x` voxels inside one X row (scalar row decode).
-template <typename T, typename S, int MORPH, int NB>
-__global__ void __launch_bounds__(256) polar_kernel(PolarArgs<T> a, const S *__restrict__ vox, int hann,
+// Block = a run of `blockDim.x` voxels inside one X row (scalar row decode).  The
+// tensor is evaluated once for the nb angles of the launch.
+template <typename T, typename S, int MORPH>
+__global__ void __launch_bounds__(256) polar_kernel(PolarArgs<T> a, const S *__restrict__ vox, int nb, int hann,
                                                     int matframe) {
   const uint32_t row = blockIdx.x / a.blocks_per_row;
   const uint32_t X = (blockIdx.x - row * a.blocks_per_row) * blockDim.x + threadIdx.x;
@@ -41,13 +42,12 @@ __global__ void __launch_bounds__(256) polar_kernel(PolarArgs<T> a, const S *__r
     const uint32_t Y = row % a.ny, Z = row / a.ny;
     w = a.hx[X] * a.hy[Y] * a.hz[Z];
   }
-#pragma unroll
-  for (int b = 0; b < NB; b++) {
+  for (int b = 0; b < nb; b++) {
     cx<T> p[3];
     apply_tensor<T>(nr, ni, a.e[b].x, a.e[b].y, a.e[b].z, p);
-    if (matframe) rotate_t<T>(a.R, p);
+    if (matframe) rotate_t<T>(a.R[b], p);
 #pragma unroll
-    for (int c = 0; c < 3; c++) a.out[b * 3 + c][idx] = cscale<T>(p[c], w);
+    for (int c = 0; c < 3; c++) a.out[c][b * a.angle_stride + idx] = cscale<T>(p[c], w);
   }
 }
 
@@ -63,8 +63,8 @@ __global__ void __launch_bounds__(256) nt_kernel(PolarArgs<T> a, const S *__rest
 }
 
 // p = Nt E / 4pi (+ R^T for MATERIAL); no Hanning (include/uniaxial.h:441-521).
-template <typename T, int NB, bool MATFRAME>
-__global__ void __launch_bounds__(256) polar_nt_kernel(PolarArgs<T> a, const cx<T> *__restrict__ nt) {
+template <typename T, bool MATFRAME>
+__global__ void __launch_bounds__(256) polar_nt_kernel(PolarArgs<T> a, const cx<T> *__restrict__ nt, int nb) {
   const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= a.V) return;
   T nr[6], ni[6];
@@ -74,13 +74,12 @@ __global__ void __launch_bounds__(256) polar_nt_kernel(PolarArgs<T> a, const cx<
     nr[j] = v.x;
     ni[j] = v.y;
   }
-#pragma unroll
-  for (int b = 0; b < NB; b++) {
+  for (int b = 0; b < nb; b++) {
     cx<T> p[3];
     apply_tensor<T>(nr, ni, a.e[b].x, a.e[b].y, a.e[b].z, p);
-    if (MATFRAME) rotate_t<T>(a.R, p);
+    if (MATFRAME) rotate_t<T>(a.R[b], p);
 #pragma unroll
-    for (int c = 0; c < 3; c++) a.out[b * 3 + c][idx] = p[c];
+    for (int c = 0; c < 3; c++) a.out[c][b * a.angle_stride + idx] = p[c];
   }
 }
 
@@ -90,11 +89,8 @@ hipError_t launch_polar_dispatch(const PolarArgs<T> &a, const void *vox, int mor
   const dim3 grid(a.blocks_per_row * a.rows), block(a.block);
   const int h = hann ? 1 : 0, mf = matframe ? 1 : 0;
   const S *v = (const S *)vox;
-  if (morph == 0 && nb == 1) hipLaunchKernelGGL((polar_kernel<T, S, 0, 1>), grid, block, 0, st, a, v, h, mf);
-  else if (morph == 0 && nb == 2) hipLaunchKernelGGL((polar_kernel<T, S, 0, 2>), grid, block, 0, st, a, v, h, mf);
-  else if (morph == 1 && nb == 1) hipLaunchKernelGGL((polar_kernel<T, S, 1, 1>), grid, block, 0, st, a, v, h, mf);
-  else if (morph == 1 && nb == 2) hipLaunchKernelGGL((polar_kernel<T, S, 1, 2>), grid, block, 0, st, a, v, h, mf);
-  else return hipErrorInvalidValue;
+  if (morph == 0) hipLaunchKernelGGL((polar_kernel<T, S, 0>), grid, block, 0, st, a, v, nb, h, mf);
+  else hipLaunchKernelGGL((polar_kernel<T, S, 1>), grid, block, 0, st, a, v, nb, h, mf);
   return hipGetLastError();
 }
 
@@ -103,8 +99,7 @@ hipError_t launch_polar_dispatch(const PolarArgs<T> &a, const void *vox, int mor
 template <typename T>
 cyr_status launch_polarization(PolarArgs<T> a, const void *vox, int storage, int morph, int nb, bool hann,
                                bool matframe, hipStream_t st) {
-  if (nb < 1 || nb > 2) return fail(CYR_E_INVALID, "polarization: 1 or 2 E bases");
-  if (matframe && nb != 1) return fail(CYR_E_INVALID, "polarization: MATERIAL frame needs one basis");
+  if (nb < 1 || nb > kPolAngles) return fail(CYR_E_INVALID, "polarization: too many angles");
   a.rows = (uint32_t)(a.V / a.nx);
   a.block = a.nx >= 256 ? 256 : ((a.nx + 63) / 64) * 64;
   a.blocks_per_row = ceil_div(a.nx, a.block);
@@ -135,10 +130,9 @@ cyr_status launch_nt(PolarArgs<T> a, const void *vox, int storage, int morph, cx
 template <typename T>
 cyr_status launch_polarization_nt(PolarArgs<T> a, const cx<T> *nt, int nb, bool matframe, hipStream_t st) {
   dim3 grid(ceil_div(a.V, 256)), block(256);
-  if (nb == 1 && matframe) hipLaunchKernelGGL((polar_nt_kernel<T, 1, true>), grid, block, 0, st, a, nt);
-  else if (nb == 1) hipLaunchKernelGGL((polar_nt_kernel<T, 1, false>), grid, block, 0, st, a, nt);
-  else if (nb == 2 && !matframe) hipLaunchKernelGGL((polar_nt_kernel<T, 2, false>), grid, block, 0, st, a, nt);
-  else return fail(CYR_E_INVALID, "polarization_nt: unsupported basis/frame combination");
+  if (nb < 1 || nb > kPolAngles) return fail(CYR_E_INVALID, "polarization_nt: too many angles");
+  if (matframe) hipLaunchKernelGGL((polar_nt_kernel<T, true>), grid, block, 0, st, a, nt, nb);
+  else hipLaunchKernelGGL((polar_nt_kernel<T, false>), grid, block, 0, st, a, nt, nb);
   CYR_LAUNCHED();
   return CYR_OK;
 }

@@ -42,23 +42,36 @@ __device__ inline bool tile_pixel(const uint32_t *__restrict__ tiles, uint32_t n
   return X < nx && Y < ny;
 }
 
+// (nb angles in turn: the sums stay in angle order)
 template <typename T>
 __global__ void __launch_bounds__(256) rotate_accumulate_kernel(const T *__restrict__ proj, double *__restrict__ acc,
                                                                 uint32_t *__restrict__ count, uint32_t nx, uint32_t ny,
-                                                                Inv6 inv, int rot_mask) {
+                                                                const double *__restrict__ inv_tab, uint32_t nb,
+                                                                int rot_mask) {
+  const uint64_t P = (uint64_t)nx * ny;
   const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (uint64_t)nx * ny) return;
+  if (t >= P) return;
   const uint32_t Y = (uint32_t)(t / nx), X = (uint32_t)(t - (uint64_t)Y * nx);
-  double v;
-  if (!bilinear_sample<T>(proj, nx, ny, inv.c, X, Y, &v)) v = __longlong_as_double(0x7ff8000000000000ll);
-  if (rot_mask) {
-    if (!isnan(v)) {
-      acc[t] += v;
-      count[t] += 1;
+  double s = acc[t];
+  uint32_t c = rot_mask ? count[t] : 0;
+#pragma unroll 2
+  for (uint32_t b = 0; b < nb; b++) {
+    double inv[6];
+#pragma unroll
+    for (int i = 0; i < 6; i++) inv[i] = inv_tab[6 * (uint64_t)b + i];
+    double v;
+    if (!bilinear_sample<T>(proj + (uint64_t)b * P, nx, ny, inv, X, Y, &v)) v = __longlong_as_double(0x7ff8000000000000ll);
+    if (rot_mask) {
+      if (!isnan(v)) {
+        s += v;
+        c += 1;
+      }
+    } else {
+      s += v;
     }
-  } else {
-    acc[t] += v;
   }
+  acc[t] = s;
+  if (rot_mask) count[t] = c;
 }
 
 __global__ void __launch_bounds__(256) average_kernel(const double *__restrict__ acc, const uint32_t *__restrict__ count,
@@ -741,10 +754,10 @@ uint32_t rotation_quarter_turns(uint32_t nx, uint32_t ny, uint32_t nA, uint32_t 
 
 template <typename T>
 cyr_status launch_rotate_accumulate(const T *proj, double *acc, uint32_t *count, uint32_t nx, uint32_t ny,
-                                    const double inv[6], int rot_mask, hipStream_t st) {
+                                    const double *inv, uint32_t nb, int rot_mask, hipStream_t st) {
   const uint64_t P = (uint64_t)nx * ny;
   hipLaunchKernelGGL((rotate_accumulate_kernel<T>), dim3(ceil_div(P, 256)), dim3(256), 0, st, proj, acc, count, nx,
-                     ny, mk_inv(inv), rot_mask);
+                     ny, inv, nb, rot_mask);
   CYR_LAUNCHED();
   return CYR_OK;
 }
@@ -916,7 +929,7 @@ cyr_status launch_warp(const T *src, T *dst, uint32_t nx, uint32_t ny, const dou
 
 #define CYR_INST(T)                                                                                                \
   template cyr_status launch_rotate_accumulate<T>(const T *, double *, uint32_t *, uint32_t, uint32_t,             \
-                                                  const double *, int, hipStream_t);                               \
+                                                  const double *, uint32_t, int, hipStream_t);                               \
   template cyr_status launch_rotate_all<T>(const T *, const double *, uint32_t, uint32_t, uint32_t, int, double *, \
                                            uint32_t, const uint32_t *, double, hipStream_t);                                 \
   template cyr_status launch_rotate_quad<T>(const T *, const double *, const double *, const T *, uint32_t,      \
