@@ -230,14 +230,16 @@ hipError_t launch_ct(uint32_t n, bool contig, uint32_t nc, PassArgs &A, hipStrea
 // transform's butterfly is the whole pencil).  DC sums and row spans as in
 // fft_ct_kernel.
 struct AnyShape {
-  uint32_t tpp, lpp, pitch, pad;
+  uint32_t tpp, lpp, pitch, pad;  // (tpp, lpp: columns; pitch, pad: rows)
 };
 
+// Inputs: of one column, or of the block's rows (rows past the last read the last).
 template <typename T, bool CONTIG> struct AnyIn {
   const cx<T> *gp;
-  uint64_t es;
-  __device__ inline cx<T> load(uint32_t e, uint32_t r, uint32_t q) const {
-    if constexpr (CONTIG) return gp[e + r * q];
+  uint64_t es;     // columns: element stride; rows: row stride
+  uint32_t rows;   // rows of this block
+  __device__ inline cx<T> load(uint32_t p, uint32_t e, uint32_t r, uint32_t q) const {
+    if constexpr (CONTIG) return gp[(uint64_t)(p < rows ? p : rows - 1) * es + e + r * q];
     else return stream_load<T>(gp + e * es + r * (q * es));
   }
 };
@@ -247,11 +249,8 @@ template <typename T, bool CONTIG, bool TAB>
 __global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<T> tb, AnyShape sh, PassArgs A) {
   extern __shared__ unsigned char smem_raw[];
   cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw);
-  uint32_t t, p, tile = blockIdx.x, vol = blockIdx.y;
-  if constexpr (CONTIG) {
-    t = threadIdx.x % sh.tpp;
-    p = threadIdx.x / sh.tpp;
-  } else {
+  uint32_t t = 0, p = 0, tile = blockIdx.x, vol = blockIdx.y;
+  if constexpr (!CONTIG) {
     const uint32_t q = xcd_tile(blockIdx.x, gridDim.x);
     const uint32_t per_vol = A.groups * A.outer_count;
     if (q >= per_vol * A.nvol) return;  // grid padding: the whole block leaves before any barrier
@@ -306,16 +305,17 @@ __global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<T> tb, AnyShape sh,
             make_double2(sr, si);
     }
   }
-  AnyIn<T, CONTIG> in{gp, A.elem_stride};
+  const uint32_t rows = CONTIG ? (A.inner_count - g * A.pp < A.pp ? A.inner_count - g * A.pp : A.pp) : 1;
+  AnyIn<T, CONTIG> in{gp, CONTIG ? A.inner_stride : A.elem_stride, rows};
   // the line's shifted x range (see fft_ct_kernel)
   const uint32_t n = A.inner_count, m = n / 2;
   const uint32_t x0 = g * A.pp, x1 = (x0 + A.pp < n ? x0 + A.pp : n) - 1;
   const bool lo_part = x0 <= m, hi_part = x1 > m;
   const uint32_t a0 = m - (x1 < m ? x1 : m), a1 = m - x0;
   const uint32_t b0 = n + m - x1, b1 = n + m - (x0 > m + 1 ? x0 : m + 1);
-  auto out = [&](uint32_t k0, uint32_t r, uint32_t dk, cx<T> v) {
+  auto out = [&](uint32_t row, uint32_t k0, uint32_t r, uint32_t dk, cx<T> v) {
     const uint32_t k = k0 + r * dk;
-    bool keep = active;
+    bool keep = CONTIG ? row < rows : active;
     if constexpr (!CONTIG && TAB) {
       if (A.span) {
         const uint32_t sp = span[k], lo = sp & 0xffffu, hi = sp >> 16;
@@ -323,12 +323,12 @@ __global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<T> tb, AnyShape sh,
       }
     }
     if (keep) {
-      if constexpr (CONTIG) gp[k] = v;
+      if constexpr (CONTIG) gp[row * in.es + k] = v;
       else gp[k0 * in.es + r * (dk * in.es)] = v;
     }
   };
-  if constexpr (CONTIG) lf_run<false, T>(tb, tab, lds, LfRow{p * sh.pitch, sh.pad}, t, sh.tpp, in, out);
-  else lf_run<false, T>(tb, tab, lds, LfCols{sh.lpp, p}, t, sh.tpp, in, out);
+  if constexpr (CONTIG) lf_run<false, false, T>(tb, tab, lds, LfRows{sh.pitch, sh.pad, A.pp}, in, out);
+  else lf_run<false, false, T>(tb, tab, lds, LfCols{sh.lpp, p, t, sh.tpp}, in, out);
 }
 
 // Direct O(n^2) DFT of each pencil for lengths beyond the any-length tile (e.g. a
@@ -362,7 +362,7 @@ __global__ void __launch_bounds__(256) dft_pencil_kernel(uint32_t n, PassArgs A,
 
 std::mutex g_mu;
 std::map<std::tuple<int, uint32_t, int>, DeviceBuffer> g_tw;  // (device, n, precision)
-std::map<std::tuple<int, uint32_t, int>, DeviceBuffer> g_lf;  // (device, n, precision): lfft.hpp tables
+std::map<std::tuple<int, uint32_t, int>, DeviceBuffer> g_lf;  // (device, n, precision + 2 narrow): lfft.hpp tables
 
 template <typename T> constexpr int prec_of() { return sizeof(T) == 8 ? CYR_FP64 : CYR_FP32; }
 
@@ -588,18 +588,19 @@ template <typename T> std::vector<unsigned char> lf_host(const LfPlan &P) {
 namespace {
 
 // (cached by lf_plan: the search for a convolution length tries hundreds)
-bool lf_search(uint32_t n, int precision, LfPlan &P) {
+bool lf_search(uint32_t n, int precision, bool narrow, LfPlan &P) {
   std::vector<uint32_t> seq;
   double c;
   P = LfPlan{};
   P.n = P.m = n;
-  if (!radix_sequence(n, precision == CYR_FP64 ? 10 : 13, seq, c)) {
+  P.narrow = narrow ? 1 : 0;
+  if (!radix_sequence(n, narrow ? 8 : precision == CYR_FP64 ? 10 : 13, seq, c)) {
     // Bluestein: the cheapest convolution length (radices <= 10: the stages also
     // run backwards)
     double best = 1e18;
     std::vector<uint32_t> s2;
     for (uint32_t m = 2 * n - 1; m <= std::min(kLfMaxLength, 3 * n); m++) {
-      if (!radix_sequence(m, 10, s2, c)) continue;
+      if (!radix_sequence(m, narrow ? 8 : 10, s2, c)) continue;
       if (m * (2 * c + 2) < best) {
         best = m * (2 * c + 2);
         P.m = m;
@@ -613,7 +614,8 @@ bool lf_search(uint32_t n, int precision, LfPlan &P) {
   uint32_t L = P.m;
   for (uint32_t s = 0; s < P.nst; s++) {
     const uint32_t q = L / seq[s];
-    P.st[s] = LfStage{seq[s], L, q, q > 1 ? (uint32_t)(((1ull << 32) + q - 1) / q) : 0, P.m / seq[s], P.m / L};
+    P.st[s] = LfStage{seq[s], L, q, q > 1 ? (uint32_t)(((1ull << 32) + q - 1) / q) : 0, P.m / seq[s], 0, P.m / L};
+    P.st[s].mb = P.st[s].nb > 1 ? (uint32_t)(((1ull << 32) + P.st[s].nb - 1) / P.st[s].nb) : 0;
     L = q;
   }
   return true;
@@ -621,27 +623,22 @@ bool lf_search(uint32_t n, int precision, LfPlan &P) {
 
 }  // namespace
 
-bool lf_plan(uint32_t n, int precision, LfPlan &P) {
+bool lf_plan(uint32_t n, int precision, bool narrow, LfPlan &P) {
   if (n < 2 || n > kLfMaxLength) return false;
-  // by length and precision (at most 2 x kLfMaxLength small entries); n = 0: no plan
+  // by length, precision and width (at most 4 x kLfMaxLength small entries); n = 0: no
+  // plan
   static std::mutex mu;
-  static std::map<std::pair<uint32_t, int>, LfPlan> plans;
+  static std::map<std::tuple<uint32_t, int, bool>, LfPlan> plans;
   std::lock_guard<std::mutex> lk(mu);
-  const auto key = std::make_pair(n, precision);
+  const auto key = std::make_tuple(n, precision, narrow);
   auto it = plans.find(key);
   if (it == plans.end()) {
     LfPlan p;
-    if (!lf_search(n, precision, p)) p.n = 0;
+    if (!lf_search(n, precision, narrow, p)) p.n = 0;
     it = plans.emplace(key, p).first;
   }
   P = it->second;
   return P.n != 0;
-}
-
-size_t lf_table_bytes(uint32_t n, int precision) {
-  LfPlan P;
-  if (!lf_plan(n, precision, P)) return 0;
-  return precision == CYR_FP64 ? LfOffsets<double>(P).total : LfOffsets<float>(P).total;
 }
 
 template <typename T> cyr_status lf_tables(const LfPlan &P, LfTab<T> &t) {
@@ -649,7 +646,7 @@ template <typename T> cyr_status lf_tables(const LfPlan &P, LfTab<T> &t) {
   const unsigned char *base = nullptr;
   if (ScratchArena *a = scratch_arena()) {
     // built into the arena for this call, never into the process-wide cache
-    const auto key = std::make_pair(P.n, prec_of<T>());
+    const auto key = std::make_pair(P.n, prec_of<T>() + 2 * (int)P.narrow);
     auto it = a->lf.find(key);
     if (it == a->lf.end()) {
       void *d = a->carve(o.total);
@@ -663,7 +660,7 @@ template <typename T> cyr_status lf_tables(const LfPlan &P, LfTab<T> &t) {
     int dev = 0;
     CYR_HIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lk(g_mu);
-    const auto key = std::make_tuple(dev, P.n, prec_of<T>());
+    const auto key = std::make_tuple(dev, P.n, prec_of<T>() + 2 * (int)P.narrow);
     auto it = g_lf.find(key);
     if (it == g_lf.end()) {
       const std::vector<unsigned char> h = lf_host<T>(P);
@@ -738,6 +735,7 @@ bool lf_cols_shape(const LfPlan &P, int precision, uint32_t max_cols, bool need_
     s.pp = pp;
     s.lpp = lpp;
     s.tpp = tpp;
+    s.threads = pp * tpp;
     s.tables = tables;
     s.lds = tables ? with : tile;
     return true;
@@ -745,14 +743,14 @@ bool lf_cols_shape(const LfPlan &P, int precision, uint32_t max_cols, bool need_
   return false;
 }
 
-// Rows, as many as 256 threads hold.  e: elements per thread of kernels that keep a
-// row's elements in registers (0: the thread count is free).
-bool lf_rows_shape(const LfPlan &P, int precision, uint32_t e, uint32_t max_threads, bool need_tables, LfShape &s) {
+// Rows: 2048 points of transforms for 256 threads, or, with e elements of a row per
+// thread, as many rows as 256 threads hold.
+bool lf_rows_shape(const LfPlan &P, int precision, uint32_t e, bool need_tables, LfShape &s) {
   const size_t cs = precision == CYR_FP64 ? 16 : 8, cap = max_lds_bytes(), tab = lf_tables_lds(P, precision);
   s = LfShape{};
-  const uint32_t tpp = e ? (P.n + e - 1) / e : lf_threads(P, 1, 1);
-  if (!tpp || tpp > max_threads) return false;
-  uint32_t rows = tpp >= 256 ? 1 : 256 / tpp;
+  s.tpp = e ? (P.n + e - 1) / e : 0;
+  if (s.tpp > kLfRowThreads) return false;
+  uint32_t rows = e ? std::max(1u, 256 / s.tpp) : std::max(1u, 2048 / P.m);
   s.pad = kLfPad;
   auto tile = [&] { return cs * (size_t)rows * lf_row_pitch(P.m, s.pad); };
   while (rows > 1 && tile() + tab > cap / 3) rows /= 2;
@@ -760,7 +758,7 @@ bool lf_rows_shape(const LfPlan &P, int precision, uint32_t e, uint32_t max_thre
   if (tile() > cap) s.pad = kLfNoPad;
   if (tile() > cap || (need_tables && !s.tables)) return false;
   s.pp = rows;
-  s.tpp = tpp;
+  s.threads = e ? rows * s.tpp : P.m > 4096 ? 512 : 256;
   s.pitch = lf_row_pitch(P.m, s.pad);
   s.lds = tile() + (s.tables ? tab : 0);
   return true;
@@ -774,8 +772,8 @@ cyr_status launch_any(uint32_t n, bool contig, uint32_t nc, PassArgs &A, hipStre
   LfPlan P;
   LfShape s;
   *done = false;
-  if (!lf_plan(n, prec_of<T>(), P)) return CYR_OK;
-  if (!(contig ? lf_rows_shape(P, prec_of<T>(), 0, 1024, false, s) : lf_cols_shape(P, prec_of<T>(), 16, false, s)))
+  if (!lf_plan(n, prec_of<T>(), false, P)) return CYR_OK;
+  if (!(contig ? lf_rows_shape(P, prec_of<T>(), 0, false, s) : lf_cols_shape(P, prec_of<T>(), 16, false, s)))
     return CYR_OK;
   LfTab<T> tb;
   CYR_TRY(lf_tables<T>(P, tb));
@@ -786,7 +784,7 @@ cyr_status launch_any(uint32_t n, bool contig, uint32_t nc, PassArgs &A, hipStre
   if (tiles * (contig ? 1 : nc) > 0x7ffffff0ull)
     return fail(CYR_E_UNSUPPORTED, "FFT grid too large");
   const AnyShape sh{s.tpp, s.lpp, s.pitch, s.pad};
-  const dim3 block(s.pp * s.tpp), grid = contig ? dim3((unsigned)tiles, nc) : dim3(xcd_grid(tiles * nc));
+  const dim3 block(s.threads), grid = contig ? dim3((unsigned)tiles, nc) : dim3(xcd_grid(tiles * nc));
   if (!s.tables && (A.span || A.dcz)) return fail(CYR_E_INVALID, "FFT: DC sums and spans need the tables in LDS");
 #define CYR_ANY(C, TB) hipLaunchKernelGGL((fft_any_kernel<T, C, TB>), grid, block, s.lds, st, tb, sh, A)
   if (contig && s.tables) CYR_ANY(true, true);
@@ -814,7 +812,7 @@ template <typename T> bool fft_span_fits(uint32_t n) {
   if (!strided_ct<T>(n)) {
     LfPlan P;
     LfShape s;
-    return lf_plan(n, prec_of<T>(), P) && lf_cols_shape(P, prec_of<T>(), 16, true, s);
+    return lf_plan(n, prec_of<T>(), false, P) && lf_cols_shape(P, prec_of<T>(), 16, true, s);
   }
   const uint32_t pp = n <= 512 ? 16 : (n == 1024 ? 8 : 4), wg = pp * (n / ct_elements(n));
   const bool lo = tw_lo_in_lds<T>((size_t)pp * n, n, wg);
@@ -831,7 +829,7 @@ template <typename T> uint32_t fft_dc_slots(uint32_t nx, uint32_t ny) {
   }
   LfPlan P;
   LfShape s;
-  return lf_plan(ny, prec_of<T>(), P) && lf_cols_shape(P, prec_of<T>(), 16, true, s) ? 3 * (s.pp * s.tpp / 64) : 0;
+  return lf_plan(ny, prec_of<T>(), false, P) && lf_cols_shape(P, prec_of<T>(), 16, true, s) ? 3 * (s.pp * s.tpp / 64) : 0;
 }
 
 template <typename T>

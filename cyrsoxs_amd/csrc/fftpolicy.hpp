@@ -4,8 +4,8 @@
 //   in_pos(t, i)   pencil index loaded into register slot i
 //   holds(t, i)    whether slot i is an element of the pencil at all
 //   stage(lds, pp, ...)  copies its tables behind the tile of pp pencils
-//   transform(v, t, p, pp, lds, out)  the transform, exchanging through LDS; out(k, v)
-//                  takes output k
+//   transform(v, t, p, pp, lds, out)  the transform, exchanging through LDS;
+//                  out(row, k, v) takes output k of a row
 // Layouts: CONTIG pencils are rows of the LDS tile; otherwise pencils are
 // columns (element e of pencil p at e pp + p), which keeps a wave's accesses to
 // consecutive pencils in consecutive LDS words.
@@ -168,7 +168,7 @@ template <typename T, int N, int E, bool CONTIG, int PP, int... R> struct CtFft 
   __device__ static void transform(cx<T> (&v)[E], uint32_t t, uint32_t p, uint32_t pp, cx<T> *lds, OUT out) {
     run<false>(v, t, p, lds, lds + pp * kPitch, nullptr);
 #pragma unroll
-    for (int i = 0; i < E; i++) out(out_pos(t, i), v[i]);
+    for (int i = 0; i < E; i++) out(p, out_pos(t, i), v[i]);
   }
   __device__ static uint32_t in_pos(uint32_t t, int i) { return t + (i / R0) * TPP + (i % R0) * (N / R0); }
   __device__ static uint32_t out_pos(uint32_t t, int i) { return t + (i / RL) * TPP + (i % RL) * (N / RL); }
@@ -183,9 +183,9 @@ template <typename T, int N, int E, bool CONTIG, int PP, int... R> struct CtFft 
 
 // Any length (lfft.hpp), rows: slot i of thread t is element t + i tpp (E tpp >= n;
 // the last slots may be empty).  Plain twiddle products.
-template <typename T, int E> struct LfRowFft {
+template <typename T, int E, bool NARROW> struct LfRowFft {
   static constexpr int kE = E;
-  static constexpr bool kCt = false;
+  static constexpr bool kCt = false, kNarrow = NARROW;
   struct Plan {
     LfTab<T> tb;
     uint32_t tpp;    // threads per row
@@ -202,19 +202,19 @@ template <typename T, int E> struct LfRowFft {
   __device__ void transform(cx<T> (&v)[E], uint32_t t, uint32_t p, uint32_t pp, cx<T> *lds, OUT out) const {
     const cx<T> *tw = lds + pp * P.pitch;
     const LfLds<T> tab{tw, reinterpret_cast<const uint16_t *>(tw + P.tb.m)};
-    LfNoInput<T> in;
-    const LfRow ad{p * P.pitch, P.pad};
+    const LfRows ad{P.pitch, P.pad, pp};
 #pragma unroll
     for (int i = 0; i < E; i++)
       if (holds(t, i)) {
         const uint32_t e = in_pos(t, i);
-        lds[ad(e)] = P.tb.blue ? cmul<T>(v[i], P.tb.chirp[e]) : v[i];
+        lds[ad.at(p, e)] = P.tb.blue ? cmul<T>(v[i], P.tb.chirp[e]) : v[i];
       }
     if (P.tb.blue)
-      for (uint32_t e = P.tb.n + t; e < P.tb.m; e += P.tpp) lds[ad(e)] = mk<T>(0, 0);
+      for (uint32_t e = P.tb.n + t; e < P.tb.m; e += P.tpp) lds[ad.at(p, e)] = mk<T>(0, 0);
     lds_sync();
-    auto emit = [&](uint32_t k, uint32_t r, uint32_t dk, cx<T> x) { out(k + r * dk, x); };
-    lf_run<true, T>(P.tb, tab, lds, ad, t, P.tpp, in, emit);
+    LfNoInput<T> in;
+    auto emit = [&](uint32_t row, uint32_t k, uint32_t r, uint32_t dk, cx<T> x) { out(row, k + r * dk, x); };
+    lf_run<true, NARROW, T>(P.tb, tab, lds, ad, in, emit);
     lds_sync();  // the rows may be refilled
   }
 };

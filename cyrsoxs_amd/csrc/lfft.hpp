@@ -42,6 +42,7 @@ struct LfStage {
   uint32_t q;   // L / radix
   uint32_t mg;  // ceil(2^32 / q): b / q = mulhi(b, mg) for b q < 2^32 (q > 1)
   uint32_t nb;  // butterflies, m / radix
+  uint32_t mb;  // ceil(2^32 / nb): i / nb = mulhi(i, mb) for i nb < 2^32 (nb > 1)
   uint32_t ts;  // twiddle step, m / L
 };
 
@@ -50,6 +51,7 @@ struct LfPlan {
   uint32_t m;     // transform length (n, or the convolution's)
   uint32_t blue;  // 1: Bluestein
   uint32_t nst;
+  uint32_t narrow;
   LfStage st[kLfStages];
 };
 
@@ -68,23 +70,24 @@ template <typename T> struct LfTab {
 
 // Plan of a length (false: longer than the tile limit).  lf_tables builds its
 // tables once per device (or in the caller's scratch arena).
-bool lf_plan(uint32_t n, int precision, LfPlan &P);
+// narrow: radices up to 8 only, for kernels that hold state of their own in registers.
+bool lf_plan(uint32_t n, int precision, bool narrow, LfPlan &P);
 template <typename T> cyr_status lf_tables(const LfPlan &P, LfTab<T> &t);
-// Bytes the tables of a length take in the compute precision.
-size_t lf_table_bytes(uint32_t n, int precision);
 
-// Launch shape of a tile: pencils, threads per pencil, row pitch and padding, the
+// Launch shape of a tile: pencils, threads per pencil and block, row pitch and padding, the
 // dynamic LDS and whether it includes the tables (returns false when the pencil does
-// not fit the tile).  Columns: at most max_cols (a power of two <= 32); rows: at most
-// max_threads threads each.
+// not fit the tile).  Columns: at most max_cols (a power of two <= 32).  Rows: e > 0 for
+// kernels that hold e elements of a row per thread (tpp threads of a row, at most
+// kLfRowThreads).
+constexpr uint32_t kLfRowThreads = 512;
 struct LfShape {
-  uint32_t pp = 0, lpp = 0, tpp = 0, pitch = 0, pad = 0;
+  uint32_t pp = 0, lpp = 0, tpp = 0, threads = 0, pitch = 0, pad = 0;
   bool tables = false;
   size_t lds = 0;
 };
 // Without `tables` in the request (need_tables false) the longest pencils go without.
 bool lf_cols_shape(const LfPlan &P, int precision, uint32_t max_cols, bool need_tables, LfShape &s);
-bool lf_rows_shape(const LfPlan &P, int precision, uint32_t e, uint32_t max_threads, bool need_tables, LfShape &s);
+bool lf_rows_shape(const LfPlan &P, int precision, uint32_t e, bool need_tables, LfShape &s);
 
 // ---- butterflies beyond stockham.hpp's 2, 3, 4, 5, 8 (forward) -------------------
 // cos and sin of 2 pi k / P, k = 1 .. (P - 1) / 2
@@ -210,21 +213,42 @@ template <typename T, int R> __device__ inline void bfly_any(cx<T> *a) {
   else bfly<T, R>(a);
 }
 
-// ---- LDS addressing ---------------------------------------------------------------
-// Column tiles: element e of column p at (e << lpp) + p (a wave's lanes run over
-// the columns).  Row tiles: the row's own base, one slot of padding per 8 elements
-// (the late stages' stride-R accesses then spread over the banks; rows that only fit
-// without it go unpadded).
-// slot(a0, e0, r, q): element e0 + r q, with a0 that of e0.
+// ---- who does which butterfly ------------------------------------------------------
+// Column tiles: the lanes run over the columns, thread t of column p takes butterflies
+// t, t + nt, ...; element e at (e << lpp) + p.
 struct LfCols {
-  uint32_t lpp, p;
-  __device__ inline uint32_t operator()(uint32_t e) const { return (e << lpp) + p; }
-  __device__ inline uint32_t slot(uint32_t a0, uint32_t, uint32_t r, uint32_t q) const { return a0 + r * (q << lpp); }
+  uint32_t lpp, p, t, nt;
+  __device__ inline uint32_t first() const { return t; }
+  __device__ inline uint32_t step() const { return nt; }
+  __device__ inline uint32_t count(const LfStage &S) const { return S.nb; }
+  __device__ inline void split(uint32_t i, const LfStage &, uint32_t &pencil, uint32_t &b) const {
+    pencil = p;
+    b = i;
+  }
+  // slot of element e0 + r q of the pencil, a0 that of e0
+  __device__ inline uint32_t at(uint32_t, uint32_t e) const { return (e << lpp) + p; }
+  __device__ inline uint32_t at(uint32_t, uint32_t a0, uint32_t, uint32_t r, uint32_t q) const {
+    return a0 + r * (q << lpp);
+  }
 };
-struct LfRow {
-  uint32_t base, pad;
-  __device__ inline uint32_t operator()(uint32_t e) const { return base + e + (e >> pad); }
-  __device__ inline uint32_t slot(uint32_t, uint32_t e0, uint32_t r, uint32_t q) const { return (*this)(e0 + r * q); }
+// Row tiles: the block's threads run over all butterflies of all its rows (a row's own
+// threads would leave half a wave idle in every stage with fewer butterflies); element e
+// of row p at p pitch + e + (e >> pad), one slot of padding per 8 elements (the late
+// stages' stride-R accesses then spread over the banks; rows that only fit without it go
+// unpadded).
+struct LfRows {
+  uint32_t pitch, pad, rows;
+  __device__ inline uint32_t first() const { return threadIdx.x; }
+  __device__ inline uint32_t step() const { return blockDim.x; }
+  __device__ inline uint32_t count(const LfStage &S) const { return rows * S.nb; }
+  __device__ inline void split(uint32_t i, const LfStage &S, uint32_t &pencil, uint32_t &b) const {
+    pencil = S.nb == 1 ? i : __umulhi(i, S.mb);
+    b = i - pencil * S.nb;
+  }
+  __device__ inline uint32_t at(uint32_t p, uint32_t e) const { return p * pitch + e + (e >> pad); }
+  __device__ inline uint32_t at(uint32_t p, uint32_t, uint32_t e0, uint32_t r, uint32_t q) const {
+    return at(p, e0 + r * q);
+  }
 };
 constexpr uint32_t kLfPad = 3, kLfNoPad = 31;
 inline uint32_t lf_row_pitch(uint32_t m, uint32_t pad) { return m + (m >> pad) + (pad == kLfNoPad ? 0 : 1); }
@@ -257,29 +281,31 @@ enum LfRole : uint32_t {
   kLfMid = 8   // Bluestein's turn: last forward butterfly, spectrum, first inverse one
 };
 
-// Stage S on the pencil behind ad: butterflies t, t + nt, ... (t >= nt: none).
+// Stage S of the block's pencils.
 template <typename T, int R, class AD, class IN, class OUT>
 __device__ inline void lf_stage(const LfTab<T> &P, const LfStage &S, uint32_t role, const LfLds<T> &tab, cx<T> *buf,
-                                AD ad, uint32_t t, uint32_t nt, IN &in, OUT &out) {
-  const uint32_t q = S.q;
+                                const AD &ad, IN &in, OUT &out) {
+  const uint32_t q = S.q, count = ad.count(S);
 #pragma unroll 1
-  for (uint32_t b = t; b < S.nb; b += nt) {
+  for (uint32_t i = ad.first(); i < count; i += ad.step()) {
+    uint32_t p, b;
+    ad.split(i, S, p, b);
     // (the last forward stage, q = 1, goes by output: block pos[b] / R)
     const bool last = q == 1;
     const uint32_t blk = last ? b : __umulhi(b, S.mg);
     const uint32_t j = last ? 0 : b - blk * q;
     const uint32_t e0 = (role & (kLfOut | kLfInv)) == kLfOut ? tab.pos[b] : blk * S.L + j;
-    const uint32_t a0 = ad(e0);
+    const uint32_t a0 = ad.at(p, e0);
     cx<T> v[R];
     if (role & kLfIn) {
       if (!P.blue) {
 #pragma unroll
-        for (int r = 0; r < R; r++) v[r] = in.load(e0, r, q);
+        for (int r = 0; r < R; r++) v[r] = in.load(p, e0, r, q);
       } else {
 #pragma unroll
         for (int r = 0; r < R; r++) {
           const uint32_t e = e0 + r * q, ec = e < P.n ? e : 0;
-          v[r] = in.load(ec, 0, 0);
+          v[r] = in.load(p, ec, 0, 0);
         }
 #pragma unroll
         for (int r = 0; r < R; r++) {
@@ -290,7 +316,7 @@ __device__ inline void lf_stage(const LfTab<T> &P, const LfStage &S, uint32_t ro
       }
     } else {
 #pragma unroll
-      for (int r = 0; r < R; r++) v[r] = buf[ad.slot(a0, e0, r, q)];
+      for (int r = 0; r < R; r++) v[r] = buf[ad.at(p, a0, e0, r, q)];
     }
     const uint32_t w = j * S.ts;
     if ((role & kLfInv) && !last) {
@@ -319,58 +345,58 @@ __device__ inline void lf_stage(const LfTab<T> &P, const LfStage &S, uint32_t ro
 #pragma unroll
         for (int r = 0; r < R; r++) {
           const uint32_t k = e0 + r * q;
-          if (k < P.n) out(k, 0, 0, cmul<T>(mk<T>(v[r].y, v[r].x), P.chirp[k]));
+          if (k < P.n) out(p, k, 0, 0, cmul<T>(mk<T>(v[r].y, v[r].x), P.chirp[k]));
         }
       } else {
 #pragma unroll
-        for (int r = 0; r < R; r++) out(b, r, S.nb, v[r]);
+        for (int r = 0; r < R; r++) out(p, b, r, S.nb, v[r]);
       }
     } else {
 #pragma unroll
-      for (int r = 0; r < R; r++) buf[ad.slot(a0, e0, r, q)] = v[r];
+      for (int r = 0; r < R; r++) buf[ad.at(p, a0, e0, r, q)] = v[r];
     }
   }
 }
 
-template <typename T, class AD, class IN, class OUT>
+template <bool NARROW, typename T, class AD, class IN, class OUT>
 __device__ inline void lf_stage_any(const LfTab<T> &P, uint32_t s, uint32_t role, const LfLds<T> &tab, cx<T> *buf,
-                                    AD ad, uint32_t t, uint32_t nt, IN &in, OUT &out) {
+                                    const AD &ad, IN &in, OUT &out) {
   const LfStage S = P.st[s];
-  switch (S.radix) {  // uniform over the grid
-    case 2: lf_stage<T, 2>(P, S, role, tab, buf, ad, t, nt, in, out); break;
-    case 3: lf_stage<T, 3>(P, S, role, tab, buf, ad, t, nt, in, out); break;
-    case 4: lf_stage<T, 4>(P, S, role, tab, buf, ad, t, nt, in, out); break;
-    case 5: lf_stage<T, 5>(P, S, role, tab, buf, ad, t, nt, in, out); break;
-    case 6: lf_stage<T, 6>(P, S, role, tab, buf, ad, t, nt, in, out); break;
-    case 7: lf_stage<T, 7>(P, S, role, tab, buf, ad, t, nt, in, out); break;
-    case 8: lf_stage<T, 8>(P, S, role, tab, buf, ad, t, nt, in, out); break;
-    case 9: lf_stage<T, 9>(P, S, role, tab, buf, ad, t, nt, in, out); break;
-    case 10: lf_stage<T, 10>(P, S, role, tab, buf, ad, t, nt, in, out); break;
-    // (FP64 butterflies of 11 and 13 would spill: those lengths run Bluestein)
-    case 11: if constexpr (sizeof(T) == 4) lf_stage<T, 11>(P, S, role, tab, buf, ad, t, nt, in, out); break;
-    default: if constexpr (sizeof(T) == 4) lf_stage<T, 13>(P, S, role, tab, buf, ad, t, nt, in, out); break;
+  // (uniform over the grid; FP64 butterflies of 11 and 13 would spill: those lengths run
+  // Bluestein)
+  switch (S.radix) {
+    case 2: lf_stage<T, 2>(P, S, role, tab, buf, ad, in, out); break;
+    case 3: lf_stage<T, 3>(P, S, role, tab, buf, ad, in, out); break;
+    case 4: lf_stage<T, 4>(P, S, role, tab, buf, ad, in, out); break;
+    case 5: lf_stage<T, 5>(P, S, role, tab, buf, ad, in, out); break;
+    case 6: lf_stage<T, 6>(P, S, role, tab, buf, ad, in, out); break;
+    case 7: lf_stage<T, 7>(P, S, role, tab, buf, ad, in, out); break;
+    case 8: lf_stage<T, 8>(P, S, role, tab, buf, ad, in, out); break;
+    case 9: if constexpr (!NARROW) lf_stage<T, 9>(P, S, role, tab, buf, ad, in, out); break;
+    case 10: if constexpr (!NARROW) lf_stage<T, 10>(P, S, role, tab, buf, ad, in, out); break;
+    case 11: if constexpr (!NARROW && sizeof(T) == 4) lf_stage<T, 11>(P, S, role, tab, buf, ad, in, out); break;
+    default: if constexpr (!NARROW && sizeof(T) == 4) lf_stage<T, 13>(P, S, role, tab, buf, ad, in, out); break;
   }
 }
 
 // Inputs already in LDS.
 template <typename T> struct LfNoInput {
-  __device__ inline cx<T> load(uint32_t, uint32_t, uint32_t) const { return mk<T>(0, 0); }
+  __device__ inline cx<T> load(uint32_t, uint32_t, uint32_t, uint32_t) const { return mk<T>(0, 0); }
 };
 
-// Transforms the block's pencils: in.load(e0, r, q) gives input e0 + r q < n, out(k0, r,
-// dk, v) takes output k0 + r dk (q and dk uniform: addresses step by scalars).  FROM_LDS: the inputs are already stored in LDS, behind a
-// barrier (Bluestein: times the chirp, zeros from n on).  Every thread of the block
-// calls it (t >= nt for the idle ones); barriers separate the stages, none follows the
-// last.
-template <bool FROM_LDS, typename T, class AD, class IN, class OUT>
-__device__ inline void lf_run(const LfTab<T> &P, const LfLds<T> &tab, cx<T> *buf, AD ad, uint32_t t, uint32_t nt,
-                              IN &in, OUT &out) {
+// Transforms the block's pencils: in.load(p, e0, r, q) gives input e0 + r q < n of pencil
+// p, out(p, k0, r, dk, v) takes its output k0 + r dk (q and dk uniform: addresses step by
+// scalars).  FROM_LDS: the inputs are already stored in LDS, behind a barrier (Bluestein:
+// times the chirp, zeros from n on).  NARROW: a narrow plan.  Every thread of the block
+// calls it; barriers separate the stages, none follows the last.
+template <bool FROM_LDS, bool NARROW, typename T, class AD, class IN, class OUT>
+__device__ inline void lf_run(const LfTab<T> &P, const LfLds<T> &tab, cx<T> *buf, const AD &ad, IN &in, OUT &out) {
   const uint32_t steps = P.blue ? 2 * P.nst - 1 : P.nst;
 #pragma unroll 1
   for (uint32_t i = 0; i < steps; i++) {
     uint32_t role = (!FROM_LDS && i == 0 ? kLfIn : 0) | (i + 1 == steps ? kLfOut : 0);
     if (P.blue) role |= i + 1 == P.nst ? kLfMid : i >= P.nst ? kLfInv : 0;
-    lf_stage_any<T>(P, i < P.nst ? i : steps - 1 - i, role, tab, buf, ad, t, nt, in, out);
+    lf_stage_any<NARROW, T>(P, i < P.nst ? i : steps - 1 - i, role, tab, buf, ad, in, out);
     if (i + 1 < steps) lds_sync();
   }
 }

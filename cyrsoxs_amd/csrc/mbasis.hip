@@ -408,18 +408,18 @@ __global__ void __launch_bounds__(1024) mbasis_zband_any_kernel(LfTab<T> tb, uin
     const cx<T> *base;
     uint64_t P;
     bool need;
-    __device__ cx<T> load(uint32_t e, uint32_t r, uint32_t q) const {
+    __device__ cx<T> load(uint32_t, uint32_t e, uint32_t r, uint32_t q) const {
       return need ? base[(uint64_t)e * P + r * (q * P)] : mk<T>(0, 0);
     }
   } in{base, P, need};
-  auto out = [&](uint32_t k0, uint32_t ks, uint32_t dk, cx<T> r) {
+  auto out = [&](uint32_t, uint32_t k0, uint32_t ks, uint32_t dk, cx<T> r) {
     const uint32_t kz = k0 + ks * dk;
     const uint32_t j = unshift(kz, N) - lo;  // wraps above w when below the band
     if (j < w) own[(uint64_t)j * P] = r;
     const uint32_t jm = unshift(kz ? N - kz : 0, N) - lom;
     if (jm < wm) mir[(uint64_t)jm * P] = r;
   };
-  lf_run<false, T>(tb, tab, lds, LfCols{lpp, p}, t, tpp, in, out);
+  lf_run<false, false, T>(tb, tab, lds, LfCols{lpp, p, t, tpp}, in, out);
 }
 
 // Up to 32 columns.
@@ -427,7 +427,7 @@ template <typename T> cyr_status launch_zband_any(const BandArgs<T> &a, hipStrea
   const int prec = sizeof(T) == 8 ? CYR_FP64 : CYR_FP32;
   LfPlan P;
   LfShape s;
-  if (!lf_plan(a.nz, prec, P) || !lf_cols_shape(P, prec, 32, true, s))
+  if (!lf_plan(a.nz, prec, false, P) || !lf_cols_shape(P, prec, 32, true, s))
     return fail(CYR_E_UNSUPPORTED, "Z band pass: length beyond the tile");
   LfTab<T> tb;
   CYR_TRY(lf_tables<T>(P, tb));
@@ -790,7 +790,7 @@ bool mbasis_zband_supported(uint32_t nz, int precision) {
   if (precision == CYR_FP64 ? zband_ct<double>(nz) : zband_ct<float>(nz)) return true;
   LfPlan P;
   LfShape s;
-  return lf_plan(nz, precision, P) && lf_cols_shape(P, precision, 32, true, s);
+  return lf_plan(nz, precision, false, P) && lf_cols_shape(P, precision, 32, true, s);
 }
 
 template <typename T> cyr_status launch_mbasis_zband(const BandArgs<T> &a, hipStream_t st) {

@@ -164,9 +164,16 @@ __device__ inline void voxel_fields(const S *__restrict__ vox, const PolxArgs<T>
   }
 }
 
+// Waves per SIMD the registers are held to: the any-length kernels wait on LDS and
+// barriers and want all that fit without spilling.
+template <typename T, class F, int MODE> constexpr int x_min_waves() {
+  if constexpr (F::kCt) return MODE == kXTensor && F::kE <= 8 ? 4 : 2;
+  else return sizeof(T) == 8 ? (F::kE <= 2 ? 3 : 2) : F::kNarrow && F::kE <= 4 ? 4 : 2;
+}
+
 // ---- fields + X FFT --------------------------------------------------------------
 template <typename T, typename S, class F, int WG, int MODE>
-__global__ void __launch_bounds__(WG, F::kCt && MODE == kXTensor && F::kE <= 8 ? 4 : 2)
+__global__ void __launch_bounds__(WG, (x_min_waves<T, F, MODE>()))
     xfields_kernel(typename F::Plan plan, PolxArgs<T> a, const S *__restrict__ vox, int morph, int hann) {
   constexpr int E = F::kE, NO = x_outputs<MODE>();
   extern __shared__ unsigned char smem_raw[];
@@ -190,14 +197,24 @@ __global__ void __launch_bounds__(WG, F::kCt && MODE == kXTensor && F::kE <= 8 ?
   lds_sync();  // (single-wave blocks: an LDS wait only)
   // fill(c, v) forms output c, which is transformed and written.  Compile-time plans
   // unroll the outputs; the any-length transform is too large to copy per output.
-  auto each_output = [&](auto fill) {
+  // (touch() marks what fill reads as changed: the products of every output would
+  // otherwise be hoisted out of the loop and held in registers)
+  auto each_output = [&](auto touch, auto fill) {
     auto emit = [&](cx<T>(&v)[E], cx<T> *vol) {
-      cx<T> *o = vol + (uint64_t)(active ? row : 0) * a.nx;
       // (transform() ends with a barrier after its last LDS reads, so the next
       // output's first LDS store cannot overtake them)
-      fft.transform(v, t, p, a.pp, lds, [&](uint32_t k, cx<T> x) {
-        if (active) o[k] = x;
-      });
+      if constexpr (F::kCt) {
+        cx<T> *o = vol + (uint64_t)(active ? row : 0) * a.nx;
+        fft.transform(v, t, p, a.pp, lds, [&](uint32_t, uint32_t k, cx<T> x) {
+          if (active) o[k] = x;
+        });
+      } else {
+        const uint32_t r0 = blockIdx.x * a.pp;
+        cx<T> *o = vol + (uint64_t)r0 * a.nx;
+        fft.transform(v, t, p, a.pp, lds, [&](uint32_t r, uint32_t k, cx<T> x) {
+          if (r0 + r < a.rows) o[(uint64_t)r * a.nx + k] = x;
+        });
+      }
     };
     if constexpr (F::kCt) {
       static_for<0, NO>([&](auto cc) {
@@ -210,6 +227,7 @@ __global__ void __launch_bounds__(WG, F::kCt && MODE == kXTensor && F::kE <= 8 ?
       for (uint32_t c = blockIdx.y; c < (uint32_t)NO; c += gridDim.y) {
         cx<T> v[E];
         cx<T> *vol = nullptr;
+        touch();
         static_for<0, NO>([&](auto cc) {  // (uniform)
           if (c == (uint32_t)decltype(cc)::value) {
             fill(cc, v);
@@ -273,7 +291,16 @@ __global__ void __launch_bounds__(WG, F::kCt && MODE == kXTensor && F::kE <= 8 ?
       }
       // outputs c = 0..6: (alpha, beta, q00, q11, q01, q02, q12) of material m0
       // (real part) and m0 + 1 (imaginary part), q_ij = phi_a s'_i s'_j
-      each_output([&](auto cc, cx<T>(&v)[E]) {
+      auto touch = [&] {
+#pragma unroll
+        for (int i = 0; i < E; i++)
+#pragma unroll
+          for (int m = 0; m < 2; m++) {
+            asm volatile("" : "+v"(wpa[m][i]), "+v"(wbe[m][i]), "+v"(sxa[m][i]), "+v"(sya[m][i]), "+v"(sza[m][i]));
+            if constexpr (MORPH == 1) asm volatile("" : "+v"(wal[m][i]));
+          }
+      };
+      each_output(touch, [&](auto cc, cx<T>(&v)[E]) {
         constexpr int c = decltype(cc)::value;
 #pragma unroll
         for (int i = 0; i < E; i++) {
@@ -321,7 +348,7 @@ __global__ void __launch_bounds__(WG, F::kCt && MODE == kXTensor && F::kE <= 8 ?
       fim[c][i] = fi[c];
     }
   }
-  each_output([&](auto cc, cx<T>(&v)[E]) {
+  each_output([] {}, [&](auto cc, cx<T>(&v)[E]) {
     constexpr int c = decltype(cc)::value;
 #pragma unroll
     for (int i = 0; i < E; i++) v[i] = mk<T>(fre[c][i], fim[c][i]);
@@ -332,15 +359,28 @@ __global__ void __launch_bounds__(WG, F::kCt && MODE == kXTensor && F::kE <= 8 ?
 // Launch shape of the compile-time X plans: rows of <= 64 threads share a wave.
 constexpr int ct_polx_wg(int N, int E) { return N / E <= 64 ? 64 : N / E; }
 
-// Elements per thread of the any-length X plans (their per-element state fills the
-// registers): 4, and 8 for FP32 rows that would need more than kLfXThreads threads.
-constexpr uint32_t kLfXThreads = 512;
+// Plan, shape and elements per thread of the any-length X transforms: FP32 4, FP64 2,
+// twice that for rows that would need more than kLfRowThreads threads.  Narrow plans: the
+// per-element state and butterflies of up to 8 then fit 128 registers in FP32, 4 waves per
+// SIMD, where radices up to 13 took 182 (200 x 240 x 50, 3 materials: 109 -> 84 us per
+// volume; 101 x 94 x 21: 58 -> 37 us).  Lengths with factors 11 and 13 would be
+// Bluestein's in a narrow plan, so those keep the wide one in FP32 (156 x 156 x 64, 4
+// materials: 183 us per volume by Bluestein, 98 so).
 constexpr uint64_t kXSplitThreads = 256 * 512;  // two waves per SIMD
-inline bool lf_x_shape(const LfPlan &P, int precision, LfShape &s, uint32_t &e) {
-  e = 4;
-  if (lf_rows_shape(P, precision, 4, kLfXThreads, true, s)) return true;
-  e = 8;
-  return precision != CYR_FP64 && lf_rows_shape(P, precision, 8, kLfXThreads, true, s);
+inline bool lf_x_shape(uint32_t n, int precision, LfPlan &P, LfShape &s, uint32_t &e) {
+  e = precision == CYR_FP64 ? 2 : 4;
+  const bool fits = lf_plan(n, precision, true, P);
+  if (precision == CYR_FP32 && fits && P.blue) {
+    LfPlan W;
+    if (lf_plan(n, precision, false, W) && !W.blue && lf_rows_shape(W, precision, e, true, s)) {
+      P = W;
+      return true;
+    }
+  }
+  if (!fits) return false;
+  if (lf_rows_shape(P, precision, e, true, s)) return true;
+  e *= 2;
+  return lf_rows_shape(P, precision, e, true, s);
 }
 
 // The compile-time plan applies (its elements per thread are compiled for T).
@@ -358,12 +398,12 @@ template <typename T, int MODE> uint32_t x_split(uint64_t blocks, uint32_t threa
   return sizeof(T) == 4 && blocks * threads < kXSplitThreads ? (uint32_t)x_outputs<MODE>() : 1;
 }
 
-template <typename T, typename S, int E, int MODE>
+template <typename T, typename S, int E, bool NARROW, int MODE>
 hipError_t launch_xfields_lf(const LfTab<T> &tb, const LfShape &sh, hipStream_t st, const PolxArgs<T> &a,
                              const void *vox, int morph, int hann) {
-  using F = LfRowFft<T, E>;
+  using F = LfRowFft<T, E, NARROW>;
   const typename F::Plan plan{tb, sh.tpp, sh.pitch, sh.pad};
-  hipLaunchKernelGGL((xfields_kernel<T, S, F, kLfXThreads, MODE>),
+  hipLaunchKernelGGL((xfields_kernel<T, S, F, kLfRowThreads, MODE>),
                      dim3(ceil_div(a.rows, sh.pp), x_split<T, MODE>(ceil_div(a.rows, sh.pp), sh.pp * sh.tpp)),
                      dim3(sh.pp * sh.tpp), sh.lds, st, plan, a, (const S *)vox, morph, hann);
   return hipGetLastError();
@@ -408,6 +448,7 @@ cyr_status launch_xfields(PolxArgs<T> a, const void *vox, int storage, int morph
   LfTab<T> tb{};
   LfShape sh;
   uint32_t e_lf = 0;
+  bool narrow = true;
   size_t lds = 0;
   if (ct) {
     // rows of <= 64 threads share one wave
@@ -420,8 +461,9 @@ cyr_status launch_xfields(PolxArgs<T> a, const void *vox, int storage, int morph
     if (!a.twx) return s;
   } else {
     LfPlan P;
-    if (!lf_plan(a.nx, prec, P) || !lf_x_shape(P, prec, sh, e_lf))
+    if (!lf_x_shape(a.nx, prec, P, sh, e_lf))
       return fail(CYR_E_UNSUPPORTED, "fused X kernel: row does not fit its block");
+    narrow = P.narrow;
     CYR_TRY(lf_tables<T>(P, tb));
     a.tpp = sh.tpp;
     a.pp = sh.pp;
@@ -429,11 +471,14 @@ cyr_status launch_xfields(PolxArgs<T> a, const void *vox, int storage, int morph
   const dim3 grid(ceil_div(a.rows, a.pp));
   bool found = true;
   hipError_t e = hipSuccess;
+  constexpr int E0 = sizeof(T) == 4 ? 4 : 2;
   auto go = [&](auto tag) {
     using S = decltype(tag);
     if (ct) e = launch_xfields_ct_n<T, S, MODE>(a.nx, grid, lds, st, a, vox, morph, hann ? 1 : 0, &found);
-    else if (e_lf == 4) e = launch_xfields_lf<T, S, 4, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
-    else if constexpr (sizeof(T) == 4) e = launch_xfields_lf<T, S, 8, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
+    else if (!narrow) {
+      if constexpr (sizeof(T) == 4) e = launch_xfields_lf<T, S, E0, false, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
+    } else if (e_lf == E0) e = launch_xfields_lf<T, S, E0, true, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
+    else e = launch_xfields_lf<T, S, 2 * E0, true, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
   };
   if constexpr (sizeof(T) == 4) {
     if (storage == CYR_STORE_FP16) go(half4{});

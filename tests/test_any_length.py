@@ -161,3 +161,23 @@ def test_engine_budget_falls_back_to_plain():
         rid = eng.submit(fused, vox, mats)
         assert eng.wait(rid) == 0
         assert np.array_equal(eng.result(rid), ref, equal_nan=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", [capi.FP64, capi.FP32])
+@pytest.mark.parametrize("dims", [(143, 10, 4), (9, 9, 1), (10, 50, 3), (1100, 4, 1), (1030, 6, 2), (2310, 4, 1),
+                                  (2048, 6, 1)])
+def test_x_rows_of_every_plan(dims, prec):
+    """Rows of the X kernel by each of its plans: radices up to 8, factors 11 and 13 (a
+    wide plan in FP32, Bluestein in FP64), the longer per-thread runs of long rows; several
+    rows a block with the last block short.  Bars as above."""
+    if prec == capi.FP64 and dims[0] > 2048:
+        pytest.skip("longer than the FP64 row limit")
+    print(f"X rows {dims} prec={prec}", flush=True)
+    M, energies, angles = 2, [283.0, 287.0], (0.0, 60.0, 120.0)
+    vox, mats = random_euler(dims, M, 12), random_constants(2, M, 13)
+    ref = O.simulate(O.Sim(dims, M, 3.0, energies, angles, interpolation=1, windowing=1), vox, mats)
+    for pipeline in (capi.PIPE_MBASIS, capi.PIPE_EBASIS):
+        sim = capi.Sim(dims, M, 3.0, energies, angles, precision=prec, pipeline=pipeline, interpolation=1, windowing=1)
+        err, same = pattern_rel_l2(capi.simulate(sim, vox, mats), ref)
+        assert same and err < (1e-10 if prec == capi.FP64 else 1e-4), (dims, pipeline, err)
