@@ -532,8 +532,8 @@ cyr_status cyr_engine_submit(cyr_engine eng, const cyr_sim_desc *desc, const voi
   r->vox = voxels;
   r->out = out;
   r->footprint = cyr_footprint_bytes(&r->desc);
-  if (r->footprint > e.budget && plain_fallback(&r->desc, g)) {
-    r->desc.pipeline = CYR_PIPE_PLAIN;
+  for (int p; r->footprint > e.budget && (p = smaller_pipeline(&r->desc, g)) >= 0;) {
+    r->desc.pipeline = p;
     r->footprint = cyr_footprint_bytes(&r->desc);
   }
   r->t_submit = Clock::now();

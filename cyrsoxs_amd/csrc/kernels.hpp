@@ -73,7 +73,7 @@ constexpr int kEbAmat = 3 * kEbFields;
 // grids run the plain executor).
 bool fused_supported(uint32_t nx, uint32_t ny, uint32_t nz, int precision);
 // True when the fused Y / z-bin kernel takes the grid (a compile-time plan for Ny).
-bool ebasis_yz_supported(uint32_t ny, uint32_t nz, int precision);
+bool ebasis_yz_supported(uint32_t nx, uint32_t ny, uint32_t nz, int precision);
 // Grid size the Y/z kernel's z chunking aims for, and the most chunks any plan
 // for (nx, nz) uses (sizes the partial-sum buffer).
 constexpr uint32_t kYzTargetBlocks = 1024;

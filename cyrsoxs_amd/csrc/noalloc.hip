@@ -88,14 +88,11 @@ extern "C" cyr_status cyr_simulate_device_noalloc(const cyr_sim_desc *desc, cons
   SimGeometry g;
   CYR_TRY(build_geometry(desc, g));
   if (!d_voxels || !mats || !d_out) return fail(CYR_E_INVALID, "null buffer");
-  cyr_sim_desc plain = *desc;
-  plain.pipeline = CYR_PIPE_PLAIN;
-  uint64_t need = scratch_need(desc, g);
-  bool fallback = plain_fallback(desc, g) && scratch_need(&plain, g) <= CYR_NOALLOC_SCRATCH_BYTES;
-  if (need > CYR_NOALLOC_SCRATCH_BYTES && fallback) {
-    desc = &plain;
-    fallback = false;
-    need = scratch_need(desc, g);
+  cyr_sim_desc fit = *desc;  // with the executor that fits
+  uint64_t need = scratch_need(&fit, g);
+  for (int p; need > CYR_NOALLOC_SCRATCH_BYTES && (p = smaller_pipeline(&fit, g)) >= 0;) {
+    fit.pipeline = p;
+    need = scratch_need(&fit, g);
   }
   if (need > CYR_NOALLOC_SCRATCH_BYTES) {
     char buf[200];
@@ -129,10 +126,13 @@ extern "C" cyr_status cyr_simulate_device_noalloc(const cyr_sim_desc *desc, cons
     set_scratch_arena(nullptr);
     return s;
   };
-  cyr_status s = attempt(desc);
-  if (s == CYR_E_NOMEM && fallback) {  // (Ewald bands wider than the model)
+  cyr_status s = attempt(&fit);
+  // (Ewald bands wider than the model)
+  for (int p; s == CYR_E_NOMEM && (p = smaller_pipeline(&fit, g)) >= 0;) {
+    fit.pipeline = p;
+    if (scratch_need(&fit, g) > CYR_NOALLOC_SCRATCH_BYTES) continue;
     CYR_HIP(hipStreamSynchronize(st));
-    s = attempt(&plain);
+    s = attempt(&fit);
   }
   // drain the stream on errors too: no queued launch may outlive the host images
   const hipError_t se = hipStreamSynchronize(st);

@@ -54,7 +54,7 @@ int resolved_pipeline(const cyr_sim_desc *d, const SimGeometry &g) {
   const double el = d->storage == CYR_STORE_NATIVE ? cs / 2 : 2.0;
   const double nv = mbasis_volumes(g.M), ng = (g.nz > 1 && d->interpolation == 1) ? 2.0 : 1.0;
   const double morph = 4.0 * el * g.M, V = (double)g.V, nE = (double)g.nE, launch = 24e6;
-  const bool yz = ebasis_yz_supported(g.ny, g.nz, d->precision);
+  const bool yz = ebasis_yz_supported(g.nx, g.ny, g.nz, d->precision);
   // share of the pixels with |q| < k: a disc of radius k in a square of side 2 pi / d
   const double kd = g.kmag.empty() ? 0.0 : g.kmag.back() * d->phys_size;
   const double disc = std::min(1.0, kd * kd / (4.0 * M_PI));
@@ -64,8 +64,18 @@ int resolved_pipeline(const cyr_sim_desc *d, const SimGeometry &g) {
   return mb < eb ? CYR_PIPE_MBASIS : CYR_PIPE_EBASIS;
 }
 
-bool plain_fallback(const cyr_sim_desc *d, const SimGeometry &g) {
-  if (resolved_pipeline(d, g) == CYR_PIPE_PLAIN) return false;
+int smaller_pipeline(const cyr_sim_desc *d, const SimGeometry &g) {
+  const int pipe = resolved_pipeline(d, g);
+  if (pipe == CYR_PIPE_PLAIN) return -1;
+  if (d->pipeline == CYR_PIPE_AUTO && pipe == CYR_PIPE_MBASIS) {
+    // (launches and the Ewald disc are matters of time: what fits a limit goes by the
+    // bytes of the volumes and planes alone, and does not move with the time model)
+    const double cs = d->precision == CYR_FP64 ? 16.0 : 8.0, el = d->storage == CYR_STORE_NATIVE ? cs / 2 : 2.0;
+    const double nv = mbasis_volumes(g.M), ng = (g.nz > 1 && d->interpolation == 1) ? 2.0 : 1.0;
+    const double eb = (double)g.nE * (double)g.V * (4.0 * el * g.M + 15.0 * cs);
+    const double mb = (double)g.V * (4.0 * el * g.M + 4.0 * cs * nv) + (double)g.nE * (double)g.P * 4.0 * ng * nv * cs;
+    if (mb >= eb) return CYR_PIPE_EBASIS;
+  }
   for (uint32_t n : {g.nx, g.ny}) {
     // radices 8 (or the remaining 4 or 2), 3 and 5: their least common multiple
     uint32_t r = n, l = 1;
@@ -80,9 +90,9 @@ bool plain_fallback(const cyr_sim_desc *d, const SimGeometry &g) {
       while (r % p == 0) r /= p;
     const bool ct = n == 64 || n == 128 || n == 256 || (n == 384 && d->precision != CYR_FP64) || n == 512 ||
                     n == 1024 || n == 2048;
-    if (!ct && (r != 1 || l > (d->precision == CYR_FP64 ? 8u : 24u) || (l > 8 && l % 5 == 0))) return true;
+    if (!ct && (r != 1 || l > (d->precision == CYR_FP64 ? 8u : 24u) || (l > 8 && l % 5 == 0))) return CYR_PIPE_PLAIN;
   }
-  return false;
+  return -1;
 }
 
 namespace {
@@ -633,8 +643,7 @@ uint32_t mbasis_band_cap(const SimGeometry &g) {
 // of Ewald bins the group samples (plus the mirrored bins); then per energy the
 // transformed tensor fields at its bins as combinations with its constants, and
 // every angle as 2D work.  tensor: the same passes over the five complex tensor
-// fields of one energy at a time (E-basis on grids whose Ny has no compile-time
-// plan for the fused Y/z kernel).
+// fields of one energy at a time (E-basis on grids that don't run the fused Y/z kernel).
 template <typename T>
 cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_vox, T *d_out, WorkBuffers &wb,
                      hipStream_t s, const Setup<T> &su, bool tensor) {
@@ -849,18 +858,27 @@ cyr_status run_impl(const cyr_sim_desc *d, const SimGeometry &g, const void *d_v
   }
   Setup<T> su{};
   CYR_TRY(setup_views<T>(d, g, tb, tables, su));
-  const int pipe = resolved_pipeline(d, g);
-  cyr_status s = pipe == CYR_PIPE_PLAIN ? run_plain<T>(d, g, d_vox, d_out, wb, st, su)
-                 : pipe == CYR_PIPE_MBASIS ? run_bands<T>(d, g, d_vox, d_out, wb, st, su, false)
-                 : ebasis_yz_supported(g.ny, g.nz, d->precision) ? run_ebasis<T>(d, g, d_vox, d_out, wb, st, su)
-                                                                 : run_bands<T>(d, g, d_vox, d_out, wb, st, su, true);
-  if (s == CYR_E_NOMEM && !scratch_arena() && plain_fallback(d, g)) {
+  auto execute = [&](const cyr_sim_desc *q) -> cyr_status {
+    switch (resolved_pipeline(q, g)) {
+      case CYR_PIPE_PLAIN: return run_plain<T>(q, g, d_vox, d_out, wb, st, su);
+      case CYR_PIPE_MBASIS: return run_bands<T>(q, g, d_vox, d_out, wb, st, su, false);
+      default:
+        return ebasis_yz_supported(g.nx, g.ny, g.nz, q->precision) ? run_ebasis<T>(q, g, d_vox, d_out, wb, st, su)
+                                                                   : run_bands<T>(q, g, d_vox, d_out, wb, st, su, true);
+    }
+  };
+  cyr_status s = execute(d);
+  if (s == CYR_E_NOMEM && !scratch_arena()) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     CYR_HIP(hipStreamIsCapturing(st, &cap));
     if (cap == hipStreamCaptureStatusNone) {  // (capture follows an eager run, which sized the buffers)
-      CYR_HIP(hipStreamSynchronize(st));
-      for (auto &l : wb.lane) l.release();
-      s = run_plain<T>(d, g, d_vox, d_out, wb, st, su);
+      cyr_sim_desc q = *d;
+      for (int p; s == CYR_E_NOMEM && (p = smaller_pipeline(&q, g)) >= 0;) {
+        CYR_HIP(hipStreamSynchronize(st));
+        for (auto &l : wb.lane) l.release();
+        q.pipeline = p;
+        s = execute(&q);
+      }
     }
   }
   if (mode != kRunSync) return s;
@@ -999,7 +1017,7 @@ uint64_t work_bytes(const cyr_sim_desc *d, const SimGeometry &g) {
   const uint64_t cs = d->precision == CYR_FP64 ? 16 : 8, rs = cs / 2;
   const int pipe = resolved_pipeline(d, g);
   uint64_t b = 0;
-  if (pipe == CYR_PIPE_EBASIS && !ebasis_yz_supported(g.ny, g.nz, d->precision)) {
+  if (pipe == CYR_PIPE_EBASIS && !ebasis_yz_supported(g.nx, g.ny, g.nz, d->precision)) {
     // run_bands over the tensor fields of one energy: volumes, its one or two band
     // rows (a column's own bin and its interpolation partner), tables, DC sums, planes
     const uint64_t planes = d->reference_frame != 0 ? 4 : g.nA;
@@ -1081,7 +1099,7 @@ cyr_status autotune_impl(const cyr_sim_desc *d, const SimGeometry &g, WorkBuffer
                          YzTuning *chosen) {
   *chosen = YzTuning{};
   // nothing to choose without the fused Y/z kernel or in 2D (one slice, nothing to split)
-  if (!ebasis_usable(d, g) || !ebasis_yz_supported(g.ny, g.nz, d->precision) || g.nz < 2) return CYR_OK;
+  if (!ebasis_usable(d, g) || !ebasis_yz_supported(g.nx, g.ny, g.nz, d->precision) || g.nz < 2) return CYR_OK;
   const uint64_t V = g.V, P = g.P;
   const int ng = d->interpolation == 1 ? 2 : 1;
   LaneBuffers &lb = wb.lane[0];

@@ -77,10 +77,11 @@ bool ebasis_usable(const cyr_sim_desc *d, const SimGeometry &g);
 // The executor a simulation runs: CYR_PIPE_PLAIN, CYR_PIPE_EBASIS or CYR_PIPE_MBASIS
 // (CYR_PIPE_AUTO resolved by HBM bytes; fused executors need ebasis_usable).
 int resolved_pipeline(const cyr_sim_desc *d, const SimGeometry &g);
-// Whether a fused simulation may run the plain executor where the fused one's
-// buffers do not fit (plain needs less): grids with a side other than 2^a 3^b or 5^c,
-// which had no fused executor before the any-length transforms.
-bool plain_fallback(const cyr_sim_desc *d, const SimGeometry &g);
+// The executor to try where the buffers of the simulation's own do not fit (-1: none; it
+// is refused).  AUTO's material basis, where the E-basis handles fewer bytes: the E-basis.
+// Grids with a side other than 2^a 3^b or 5^c, which had no fused executor before the
+// any-length transforms: plain.
+int smaller_pipeline(const cyr_sim_desc *d, const SimGeometry &g);
 
 // Autotunes the E-basis Y/z launch shape of the simulation's grid (see cyr_autotune).
 struct YzTuning;
