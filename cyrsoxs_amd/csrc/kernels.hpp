@@ -257,15 +257,25 @@ uint32_t rotation_quarter_turns(uint32_t nx, uint32_t ny, uint32_t nA, uint32_t 
 // coef[a] = (c^2, s^2, 2 c s) (FP64; coef_t: the same in the compute precision)
 // into avg[ne][Ny][Nx]; each angle's taps serve several energies.  quarter (angle
 // steps per 90 degrees, 0 = none) with otiles (orbit tile order) lets each tap
-// cell serve the angles a quarter turn apart; share: coef_t of angles a and
-// a + 2 quarter turns are equal (then one intensity serves both pairs).
+// cell serve the angles a quarter turn apart.  scratch: room for the sums over an angle's
+// quarter turns (not needed: none, or any size).
 // rfin >= 0: no plane value farther than rfin pixels from the centre is finite
 // (the tiles beyond it are then filled without sampling: every tap there is NaN,
 // so their averages are NaN, or 0 with the rotation mask).
+// Pixels farther than rfin + kQuadMargin are never read (a 16 x 16 tile whose centre is
+// within rfin + 14 samples points within 8 sqrt(2) of that, and taps 1.5 beyond).
+constexpr double kQuadMargin = 28.0;
+// What the coefficients of a list of whole turns share.
+struct QuadTurns {
+  bool share = false;  // coef_t of angles a and a + 2 quarter turns are equal
+  bool turn = false;   // and those of a + 1 quarter turn are (q1, q0, -q2) of a's
+  double rin = 0;      // pixels from the centre within which plane values are finite (a hint)
+};
 template <typename T>
 cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double *coef, const T *coef_t, uint32_t nA,
                               uint32_t nx, uint32_t ny, int rot_mask, double *avg, uint32_t ne, const uint32_t *tiles,
-                              uint32_t quarter, const uint32_t *otiles, bool share, double rfin, hipStream_t st);
+                              uint32_t quarter, const uint32_t *otiles, QuadTurns turns, double rfin, void *scratch,
+                              size_t scratch_bytes, hipStream_t st);
 // Detector warp of the averaged pattern into the output (prefill 0 or NaN).
 template <typename T>
 cyr_status launch_detector_warp(const double *avg, T *out, uint32_t nx, uint32_t ny, const double inv[6],

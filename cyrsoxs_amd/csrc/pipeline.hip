@@ -406,20 +406,31 @@ cyr_status run_plain(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
   return CYR_OK;
 }
 
-// Whether the quadratic-form coefficients (c^2, s^2, 2cs) of every angle a of the
-// first quarter turn equal, rounded to the compute precision, those of a + 2
-// quarter turns (and a + A4 those of a + 3 quarter turns): E turned by 180 degrees
-// gives the same intensity, so the orbit kernel forms one value for both pairs.
-template <typename T> bool quad_pairs_share(const SimGeometry &g, uint32_t k) {
+// What the quadratic-form coefficients (c^2, s^2, 2cs) of a list of whole turns share.
+// share: those of every angle a of the first two quarter turns equal, rounded to the
+// compute precision, those of a + 2 quarter turns: E turned by 180 degrees gives the same
+// intensity, so the orbit kernel forms one value for both pairs.  turn: a quarter turn
+// exchanges c^2 and s^2 and negates 2cs.  rin: the Ewald disc |k k^ + q| <= k of eg reaches
+// so far around the plane's centre (two pixels against rounding).
+template <typename T> QuadTurns quad_turns(const SimGeometry &g, uint32_t k, const EwaldGeom &eg) {
+  QuadTurns r;
   const uint32_t A4 = g.quarter;
-  if (A4 == 0 || g.nA != 4 * A4) return false;
-  for (uint32_t a = 0; a < 2 * A4; a++) {
-    const double *x = &g.ebasis[2 * ((size_t)k * g.nA + a)], *y = &g.ebasis[2 * ((size_t)k * g.nA + a + 2 * A4)];
-    const double cx = x[0], sx = x[1], cy = y[0], sy = y[1];
+  if (A4 == 0 || g.nA != 4 * A4) return r;
+  // a quarter turn takes (c, s) to (-s, c) up to the rounding of the angle table
+  r.share = r.turn = true;
+  const double cx = (-eg.k * eg.kx - eg.start) / eg.dx - eg.nx / 2.0;
+  const double cy = (-eg.k * eg.ky - eg.start) / eg.dy - eg.ny / 2.0;
+  r.rin = eg.k / std::max(eg.dx, eg.dy) - std::hypot(cx, cy) - 2.0;
+  for (uint32_t a = 0; a < 3 * A4; a++) {
+    const double *x = &g.ebasis[2 * ((size_t)k * g.nA + a)], *y = x + 2 * A4;
+    if (std::fabs(x[0] * x[0] - y[1] * y[1]) > 1e-13 || std::fabs(x[0] * x[1] + y[0] * y[1]) > 1e-13) r.turn = false;
+    if (a >= 2 * A4) continue;
+    const double *z = y + 2 * A4;
+    const double cx = x[0], sx = x[1], cy = z[0], sy = z[1];
     if ((T)(cx * cx) != (T)(cy * cy) || (T)(sx * sx) != (T)(sy * sy) || (T)(2.0 * cx * sx) != (T)(2.0 * cy * sy))
-      return false;
+      r.share = false;
   }
-  return true;
+  return r;
 }
 
 // Radius in pixels about the plane's centre (Nx/2, Ny/2) beyond which no pixel is on
@@ -542,7 +553,7 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
       kt_begin(s);
       CYR_TRY(launch_rotate_quad<T>(proj, inv, su.quad + (size_t)3 * k * g.nA, su.quad_t + (size_t)3 * k * g.nA, g.nA,
                                     g.nx, g.ny, d->rot_mask, avg, 1, su.tiles, g.quarter, su.otiles,
-                                    quad_pairs_share<T>(g, k), rfin, s));
+                                    quad_turns<T>(g, k, geo), rfin, pol, sizeof(cx<T>) * V * kEbFields, s));
       kt_end("rotate_quad", s, (double)kQuadRecord * P * sizeof(T) + 8.0 * P);
     } else {
       aa.proj = proj;
@@ -801,10 +812,13 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
           // width, shared by its energies) and the band table; outputs: n
           // quadratic-form planes
           kt_end("mbasis_quad", s, (double)planes * nvol * (double)wsum * cxb + 4.0 * P + n * (double)kQuadRecord * P * sizeof(T));
+          EwaldGeom gmin = aa.g;  // (the batch's smallest disc)
+          for (uint32_t i = 1; i < n; i++) gmin.k = std::min(gmin.k, g.kmag[b0 + i]);
           kt_begin(s);
           CYR_TRY(launch_rotate_quad<T>(proj, inv, su.quad + (size_t)3 * k * g.nA, su.quad_t + (size_t)3 * k * g.nA,
                                         g.nA, g.nx, g.ny, d->rot_mask, avg, n, su.tiles, g.quarter, su.otiles,
-                                        quad_pairs_share<T>(g, k), 0.5 * std::sqrt((double)d4), s));
+                                        quad_turns<T>(g, k, gmin), 0.5 * std::sqrt((double)d4), pol,
+                                        sizeof(cx<T>) * V * pass_max, s));
           kt_end("rotate_quad", s, n * ((double)kQuadRecord * P * sizeof(T) + 8.0 * P));
           CYR_TRY(launch_detector_warp_n<T>(avg, d_out + ((uint64_t)b0 * g.nK + k) * P, (uint64_t)g.nK * P, n, g.nx,
                                             g.ny, &g.det_inv[(size_t)k * 6], d->rot_mask, s));

@@ -410,6 +410,44 @@ template <typename T> __device__ inline typename Tap3<T>::v tap_load(__amdgpu_bu
 // Buffer resource word 3 of a raw (untyped) buffer on gfx9-family devices.
 constexpr int kRawBufferFlags = 0x00020000;
 
+// Row 0 (n pixels), column 0 below it (n - 1) and the centre, which are in no orbit: pixel
+// j of them by every angle, a quarter of the angles a wave.  Pixels farther than rcut from
+// the centre sample nothing finite.
+template <typename T, int NE, bool RM, int R>
+__device__ inline void orbit_tail(const T *const (&qp)[NE], const double *__restrict__ inv_tab,
+                                  const double *__restrict__ coef, uint32_t nA, uint32_t n, double rcut, uint32_t j,
+                                  uint32_t w, uint32_t l, uint32_t e0, uint32_t ne, double *__restrict__ avg,
+                                  double (&sum)[4][4][NE][64], uint32_t (&num)[R][R][NE][64]) {
+  const uint32_t h = n / 2;
+  const bool in = j < 2 * n;
+  const uint32_t X = j < n ? j : (j < 2 * n - 1 ? 0 : h);
+  const uint32_t Y = j < n ? 0 : (j < 2 * n - 1 ? j - n + 1 : h);
+  double acc[NE] = {};
+  uint32_t cnt[NE] = {};
+  const double dx = (double)X - h, dy = (double)Y - h;
+  if (in && dx * dx + dy * dy <= rcut * rcut) {
+    const uint32_t a0 = (uint32_t)((uint64_t)nA * w / 4), a1 = (uint32_t)((uint64_t)nA * (w + 1) / 4);
+    quad_pixel<T, NE>(qp, inv_tab + 6 * (uint64_t)a0, coef + 3 * (uint64_t)a0, a1 - a0, n, n, X, Y, RM, acc, cnt);
+  } else if constexpr (!RM) {
+#pragma unroll
+    for (int e = 0; e < NE; e++) acc[e] = __longlong_as_double(0x7ff8000000000000ll);
+  }
+#pragma unroll
+  for (int e = 0; e < NE; e++) {
+    sum[w][0][e][l] = acc[e];
+    if constexpr (RM) num[w][0][e][l] = cnt[e];
+  }
+  __syncthreads();
+  if (w != 0 || !in) return;
+#pragma unroll
+  for (int e = 0; e < NE; e++)
+    for (int i = 1; i < 4; i++) {
+      acc[e] += sum[i][0][e][l];
+      if constexpr (RM) cnt[e] += num[i][0][e][l];
+    }
+  quad_store<NE>(avg, (uint64_t)n * n, (uint64_t)Y * n + X, e0, ne, nA, RM, acc, cnt);
+}
+
 // A block holds one 8 x 8 quadrant of a tile of orbits; its wave i samples the points of
 // orbit pixel i and serves pixel s^-q(i) from them (one pixel per wave, not four in
 // turn: four times the waves and a quarter of the chain of gathers for the same work;
@@ -422,9 +460,9 @@ __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__
                                                            const T *__restrict__ coef_t, uint32_t nA, uint32_t A4,
                                                            uint32_t n, double *__restrict__ avg, uint32_t ne,
                                                            const uint32_t *__restrict__ otiles, uint32_t n_otiles,
-                                                           int share) {
-  __shared__ double sum[4][Q][NE][64];
-  __shared__ uint32_t num[RM ? 4 : 1][RM ? Q : 1][NE][64];
+                                                           double rcut, int share) {
+  __shared__ double sum[4][4][NE][64];
+  __shared__ uint32_t num[RM ? 4 : 1][RM ? 4 : 1][NE][64];
   const uint64_t P = (uint64_t)n * n;
   const uint32_t h = n / 2;
   const uint32_t qb = xcd_tile(blockIdx.x, gridDim.x);
@@ -434,32 +472,7 @@ __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__
 #pragma unroll
   for (int e = 0; e < NE; e++) qp[e] = quad + (uint64_t)(e0 + e < ne ? e0 + e : e0) * P * kQuadRecord;
   if (qb >= 4 * n_otiles) {
-    // tail: row 0 (n pixels), column 0 below it (n - 1) and the centre, 64 pixels a
-    // block, a quarter of the angles a wave
-    const uint32_t j = (qb - 4 * n_otiles) * 64 + l;
-    const bool in = j < 2 * n;
-    const uint32_t X = j < n ? j : (j < 2 * n - 1 ? 0 : h);
-    const uint32_t Y = j < n ? 0 : (j < 2 * n - 1 ? j - n + 1 : h);
-    double acc[NE] = {};
-    uint32_t cnt[NE] = {};
-    if (in) {
-      const uint32_t a0 = (uint32_t)((uint64_t)nA * i / 4), a1 = (uint32_t)((uint64_t)nA * (i + 1) / 4);
-      quad_pixel<T, NE>(qp, inv_tab + 6 * (uint64_t)a0, coef + 3 * (uint64_t)a0, a1 - a0, n, n, X, Y, RM, acc, cnt);
-    }
-#pragma unroll
-    for (int e = 0; e < NE; e++) {
-      sum[i][0][e][l] = acc[e];
-      if constexpr (RM) num[i][0][e][l] = cnt[e];
-    }
-    __syncthreads();
-    if (i != 0 || !in) return;
-#pragma unroll
-    for (int e = 0; e < NE; e++)
-      for (int w = 1; w < 4; w++) {
-        acc[e] += sum[w][0][e][l];
-        if constexpr (RM) cnt[e] += num[w][0][e][l];
-      }
-    quad_store<NE>(avg, P, (uint64_t)Y * n + X, e0, ne, nA, RM, acc, cnt);
+    orbit_tail<T, NE, RM>(qp, inv_tab, coef, nA, n, rcut, (qb - 4 * n_otiles) * 64 + l, i, l, e0, ne, avg, sum, num);
     return;
   }
   const uint32_t tt = otiles[qb >> 2];
@@ -608,6 +621,199 @@ __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__
     }
   }
   quad_store<NE>(avg, P, (uint64_t)PYi * n + PXi, e0, ne, nA, RM, a, c);
+}
+
+// Full turns (Q = 4): the sum over an angle's four quarter turns first, then the angles.
+// With y the point pixel x samples at angle a, x takes Q(s^q y) at angle a + q A4, whose
+// coefficients are those of a with c^2 and s^2 exchanged and 2cs negated for odd q.  So
+// the four add up to one sample at y of
+//   S = q(y) + P q(s y) + q(s^2 y) + P q(s^3 y),   P (q0, q1, q2) = (q1, q0, -q2),
+// and as S(s y) = P S(y), pixel s x takes the same sample with P, s^2 x and s^3 x the
+// values of x and s x: one gather per orbit and angle a < A4, a quarter of those
+// rotate_orbit_kernel makes, from the quadrant u, v in [0, n/2 - 1] about the centre alone
+// (every y turns into it; P where by an odd number of quarter turns).  Bound by its
+// gathers through L1, as rotate_orbit_kernel is: 2048^2 film, 10 energies x 180 angles
+// 1.19 ms by orbits -> 0.42 ms and 35 us for S (a wave replaying all four pixels of its
+// own deferred angles, not one pixel of all: 0.46 ms; 1 or 4 energies a pass, not 2: 0.51,
+// 0.46 ms).
+
+// The quadrant's S of ne planes.  Where a value is not finite the record says what the
+// samples that read it come to: q0 and q1 NaN, no pair there has a value (with the mask:
+// all four terms NaN; without: any); q0 alone NaN, the exact path decides.  Pixels beyond
+// rskip are not read by any sample: neither read nor written here.
+template <typename T, bool RM>
+__global__ void __launch_bounds__(256) quad_sym_kernel(const T *__restrict__ quad, T *__restrict__ sym, uint32_t n,
+                                                       uint32_t tx, double rskip) {
+  const uint32_t h = n / 2, w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const uint32_t u = (blockIdx.x % tx) * 16 + (w & 1) * 8 + (l & 7), v = (blockIdx.x / tx) * 16 + (w >> 1) * 8 + (l >> 3);
+  if (u >= h || v >= h || (double)u * u + (double)v * v > rskip * rskip) return;
+  const T *q = quad + (uint64_t)blockIdx.y * n * n * kQuadRecord;
+  T *o = sym + ((uint64_t)blockIdx.y * h * h + quad_index(u, v, h, h)) * kQuadRecord;
+  const uint32_t idx[4] = {quad_index(h + u, h + v, n, n), quad_index(h - v, h + u, n, n),
+                           quad_index(h - u, h - v, n, n), quad_index(h + v, h - u, n, n)};
+  T r[4][3];
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int c = 0; c < 3; c++) r[i][c] = q[(uint64_t)idx[i] * kQuadRecord + c];
+  const T nan = (T)__longlong_as_double(0x7ff8000000000000ll);
+  T s0 = (r[0][0] + r[2][0]) + (r[1][1] + r[3][1]), s1 = (r[0][1] + r[2][1]) + (r[1][0] + r[3][0]);
+  const T s2 = (r[0][2] + r[2][2]) - (r[1][2] + r[3][2]);
+  if (!(isfinite(s0) && isfinite(s1) && isfinite(s2))) {
+    uint32_t bad = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) bad += isnan(r[i][0]) || isnan(r[i][1]) || isnan(r[i][2]) ? 1 : 0;
+    s0 = nan;
+    s1 = bad >= (RM ? 4u : 1u) ? nan : (T)0;
+  }
+  o[0] = s0;
+  o[1] = s1;
+  o[2] = s2;
+}
+
+// A block holds one 8 x 8 quadrant of a tile of orbits; its waves take a quarter of the
+// angles each.  Points near a cell edge or the image border, and samples of records that
+// the exact path decides, are replayed pair by pair from the planes themselves, as in
+// rotate_orbit_kernel (the same margins), wave i taking those of orbit pixel i.
+template <typename T, int NE, bool RM>
+__global__ void __launch_bounds__(256) rotate_sym_kernel(const T *__restrict__ quad, const T *__restrict__ sym,
+                                                         const double *__restrict__ inv_tab,
+                                                         const double *__restrict__ coef, const T *__restrict__ coef_t,
+                                                         uint32_t nA, uint32_t A4, uint32_t n,
+                                                         double *__restrict__ avg, uint32_t ne,
+                                                         const uint32_t *__restrict__ otiles, uint32_t n_otiles,
+                                                         double rcut) {
+  __shared__ double sum[4][4][NE][64];
+  __shared__ unsigned long long later[4][64];
+  __shared__ uint32_t num[RM ? 4 : 1][RM ? 4 : 1][NE][64];
+  const uint64_t P = (uint64_t)n * n;
+  const uint32_t h = n / 2;
+  const uint32_t qb = xcd_tile(blockIdx.x, gridDim.x);
+  const uint32_t e0 = blockIdx.z * NE;
+  const uint32_t i = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+  const T *qp[NE];
+#pragma unroll
+  for (int e = 0; e < NE; e++) qp[e] = quad + (uint64_t)(e0 + e < ne ? e0 + e : e0) * P * kQuadRecord;
+  if (qb >= 4 * n_otiles) {
+    if constexpr (!RM)  // (with the mask rotate_orbit_kernel runs too, and takes them)
+      orbit_tail<T, NE, RM>(qp, inv_tab, coef, nA, n, rcut, (qb - 4 * n_otiles) * 64 + l, i, l, e0, ne, avg, sum, num);
+    return;
+  }
+  const uint32_t tt = otiles[qb >> 2];
+  const uint32_t u = (tt & 0xffffu) * 16 + (qb & 1) * 8 + (l & 7) + 1;
+  const uint32_t v = (tt >> 16) * 16 + ((qb >> 1) & 1) * 8 + (l >> 3);
+  const bool in = u < h && v < h;
+  const uint32_t X0 = h + u, Y0 = h + v;  // orbit pixels s^j(x), j = 0..3
+  auto px = [&](uint32_t j) { return j == 0 ? X0 : j == 1 ? n - Y0 : j == 2 ? n - X0 : Y0; };
+  auto py = [&](uint32_t j) { return j == 0 ? Y0 : j == 1 ? X0 : j == 2 ? n - Y0 : n - X0; };
+  const double hh = (double)h, hi = (double)(h - 1);
+  const double m = 1e-9 + 1e-12 * (double)n;
+  constexpr uint32_t rb = kQuadRecord * (uint32_t)sizeof(T);
+  __amdgpu_buffer_rsrc_t rs[NE];
+#pragma unroll
+  for (int e = 0; e < NE; e++)
+    rs[e] = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(sym + (uint64_t)(e0 + e < ne ? e0 + e : e0) * h * h * kQuadRecord), (short)0, (int)((uint64_t)h * h * rb),
+        kRawBufferFlags);
+  double acc[2][NE] = {};  // pixels x and s^2 x; s x and s^3 x
+  uint32_t cnt[NE] = {};
+  bool dead = false;
+  double ex[NE] = {};  // pixel i's pairs of the exact path
+  uint32_t exn[NE] = {};
+  const uint32_t chunks = ((A4 + 3) / 4 + 63) / 64, wa1 = in ? A4 * (i + 1) / 4 : 0;
+  for (uint32_t ch = 0; ch < chunks; ch++) {  // runs of 64 angles a wave, in step
+    const uint32_t a0 = A4 * i / 4 + 64 * ch, a1 = wa1 < a0 + 64 ? wa1 : a0 + 64;
+    uint64_t defer = 0;
+    for (uint32_t a = a0; a < a1; a++) {
+      const double *inv = inv_tab + 6 * (uint64_t)a;
+      const double du = __builtin_fma(inv[0], (double)X0, __builtin_fma(inv[1], (double)Y0, inv[2])) - hh;
+      const double dv = __builtin_fma(inv[3], (double)X0, __builtin_fma(inv[4], (double)Y0, inv[5])) - hh;
+      const bool odd = (du < 0) != (dv < 0);
+      const double p = fabs(odd ? dv : du), q = fabs(odd ? du : dv);
+      const bool inside = p <= hi && q <= hi;  // (all four turns of the point)
+      const double fx0 = floor(p), fy0 = floor(q);
+      const double fx = p - fx0, fy = q - fy0;
+      const bool safe = inside ? (fx >= m && fx <= 1 - m && fy >= m && fy <= 1 - m)
+                        : RM   ? p > hh + m || q > hh + m    // all four outside
+                               : p > hi + m || q > hi + m;   // one outside
+      const uint32_t x0 = inside ? (uint32_t)fx0 : 0u, y0 = inside ? (uint32_t)fy0 : 0u;
+      const uint32_t o00 = quad_index(x0, y0, h, h) * rb, o10 = quad_index(x0 + 1, y0, h, h) * rb;
+      const uint32_t o01 = quad_index(x0, y0 + 1, h, h) * rb, o11 = quad_index(x0 + 1, y0 + 1, h, h) * rb;
+      typename Tap3<T>::v t[NE][4];
+#pragma unroll
+      for (int e = 0; e < NE; e++) {
+        t[e][0] = tap_load<T>(rs[e], o00);
+        t[e][1] = tap_load<T>(rs[e], o10);
+        t[e][2] = tap_load<T>(rs[e], o01);
+        t[e][3] = tap_load<T>(rs[e], o11);
+      }
+      const T fxT = (T)fx, fyT = (T)fy, gx = (T)1 - fxT, gy = (T)1 - fyT;
+      const T w00 = gx * gy, w10 = fxT * gy, w01 = gx * fyT, w11 = fxT * fyT;
+      T sm[NE][3];
+      bool exact = !safe;
+#pragma unroll
+      for (int e = 0; e < NE; e++) {
+        sm[e][0] = w00 * t[e][0].x + w10 * t[e][1].x + w01 * t[e][2].x + w11 * t[e][3].x;
+        sm[e][1] = w00 * t[e][0].y + w10 * t[e][1].y + w01 * t[e][2].y + w11 * t[e][3].y;
+        sm[e][2] = w00 * t[e][0].z + w10 * t[e][1].z + w01 * t[e][2].z + w11 * t[e][3].z;
+        exact = exact || (inside && isnan(sm[e][0]) && !isnan(sm[e][1]));
+      }
+      if (exact) {
+        defer |= 1ull << (a - a0);
+        continue;
+      }
+      const T *c = coef_t + 3 * (uint64_t)a;
+      const T c0 = odd ? c[1] : c[0], c1 = odd ? c[0] : c[1], c2 = odd ? -c[2] : c[2];
+      if constexpr (!RM) dead = dead || !inside;
+#pragma unroll
+      for (int e = 0; e < NE; e++) {
+        const double v0 = (double)(c0 * sm[e][0] + c1 * sm[e][1] + c2 * sm[e][2]);
+        const double v1 = (double)(c1 * sm[e][0] + c0 * sm[e][1] - c2 * sm[e][2]);
+        if constexpr (RM) {
+          const bool ok = inside && !isnan(sm[e][1]);
+          acc[0][e] += ok ? v0 : 0.0;
+          acc[1][e] += ok ? v1 : 0.0;
+          cnt[e] += ok ? 4u : 0u;
+        } else {
+          acc[0][e] += v0;
+          acc[1][e] += v1;
+        }
+      }
+    }
+    if (ch) __syncthreads();  // (the masks have been read)
+    later[i][l] = defer;
+    __syncthreads();
+    for (uint32_t w = 0; w < 4; w++)
+      for (uint64_t mask = later[w][l]; mask; mask &= mask - 1) {
+        const uint32_t a = A4 * w / 4 + 64 * ch + (uint32_t)__builtin_ctzll(mask);
+#pragma unroll 2
+        for (uint32_t q = 0; q < 4; q++) {
+          const uint32_t aa = a + q * A4;
+          const QPoint d = quad_point(inv_tab + 6 * (uint64_t)aa, px(i), py(i), n, n);
+          Rec<T> td[NE][4];
+          quad_gather<T, NE>(qp, d, n, n, td);
+          quad_add<T, NE>(d, td, coef + 3 * (uint64_t)aa, RM, ex, exn);
+        }
+      }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+#pragma unroll
+    for (int e = 0; e < NE; e++) {
+      sum[i][j][e][l] = dead ? __longlong_as_double(0x7ff8000000000000ll) : acc[j & 1][e];
+      if constexpr (RM) num[i][j][e][l] = cnt[e];
+    }
+  __syncthreads();
+  if (!in) return;
+  // wave i stores pixel i
+#pragma unroll
+  for (int w = 0; w < 4; w++)
+#pragma unroll
+    for (int e = 0; e < NE; e++) {
+      ex[e] += sum[w][i][e][l];
+      if constexpr (RM) exn[e] += num[w][i][e][l];
+    }
+  quad_store<NE>(avg, P, (uint64_t)py(i) * n + px(i), e0, ne, nA, RM, ex, exn);
 }
 
 // Orbit tiles beyond every finite plane value (their pixels' taps, within 1.5
@@ -791,19 +997,19 @@ cyr_status launch_rotate_all(const T *proj, const double *inv_tab, uint32_t nA, 
 template <typename T, int NE, bool RM>
 hipError_t launch_orbit_rm(uint32_t Q, dim3 grid, hipStream_t st, const T *quad, const double *inv_tab,
                            const double *coef, const T *coef_t, uint32_t nA, uint32_t A4, uint32_t n, double *avg,
-                           uint32_t ne, const uint32_t *otiles, uint32_t n_otiles, int share) {
+                           uint32_t ne, const uint32_t *otiles, uint32_t n_otiles, double rcut, int share) {
   switch (Q) {
     case 2:
       hipLaunchKernelGGL((rotate_orbit_kernel<T, NE, 2, RM>), grid, dim3(256), 0, st, quad, inv_tab, coef, coef_t, nA,
-                         A4, n, avg, ne, otiles, n_otiles, share);
+                         A4, n, avg, ne, otiles, n_otiles, rcut, share);
       break;
     case 3:
       hipLaunchKernelGGL((rotate_orbit_kernel<T, NE, 3, RM>), grid, dim3(256), 0, st, quad, inv_tab, coef, coef_t, nA,
-                         A4, n, avg, ne, otiles, n_otiles, share);
+                         A4, n, avg, ne, otiles, n_otiles, rcut, share);
       break;
     default:
       hipLaunchKernelGGL((rotate_orbit_kernel<T, NE, 4, RM>), grid, dim3(256), 0, st, quad, inv_tab, coef, coef_t, nA,
-                         A4, n, avg, ne, otiles, n_otiles, share);
+                         A4, n, avg, ne, otiles, n_otiles, rcut, share);
       break;
   }
   return hipGetLastError();
@@ -812,7 +1018,8 @@ hipError_t launch_orbit_rm(uint32_t Q, dim3 grid, hipStream_t st, const T *quad,
 template <typename T>
 cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double *coef, const T *coef_t, uint32_t nA,
                               uint32_t nx, uint32_t ny, int rot_mask, double *avg, uint32_t ne, const uint32_t *tiles,
-                              uint32_t quarter, const uint32_t *otiles, bool share, double rfin, hipStream_t st) {
+                              uint32_t quarter, const uint32_t *otiles, QuadTurns turns, double rfin, void *scratch,
+                              size_t scratch_bytes, hipStream_t st) {
   if (ne == 0) return CYR_OK;
   if ((uint64_t)nx * ny > 0xffffffffull) return fail(CYR_E_UNSUPPORTED, "rotation: more than 2^32 pixels");
   if (!tiles) return fail(CYR_E_INVALID, "rotation: tile order missing");
@@ -852,13 +1059,50 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
     // 2 energies per pass (measured against 1 and 4: 512^2 x 20 energies 415 / 384 us
     // for 4 / 2; 2048^2 film 7.30 / 6.75 / 8.92 ms per 10 energies for 1 / 2 / 4)
     const uint64_t blocks = 4ull * o_act + ceil_div(2ull * nx, 64);
-    const dim3 grid(xcd_grid(blocks), 1, ceil_div(ne, 2));
-    hipError_t e =
-        rot_mask ? launch_orbit_rm<T, 2, true>(Q, grid, st, quad, inv_tab, coef, coef_t, nA, quarter, nx, avg, ne,
-                                                otiles, o_act, share ? 1 : 0)
-                 : launch_orbit_rm<T, 2, false>(Q, grid, st, quad, inv_tab, coef, coef_t, nA, quarter, nx, avg, ne,
-                                                 otiles, o_act, share ? 1 : 0);
-    if (e != hipSuccess) return hip_fail(e, "rotate_orbit_kernel", __FILE__, __LINE__);
+    const double rcut = rfin >= 0 ? rfin + 2.0 : 4.0 * nx;
+    hipError_t e;
+    // Full turns: summed over the quarter turns first, as many energies at a time as the
+    // scratch buffer has quadrants for.  With the mask only the tiles that sample finite
+    // values alone (turns.rin): near the disc's edge, which is not quite its own quarter
+    // turn, every angle of a pixel would take the exact path (512^2 FP64 film, 72 angles:
+    // 229 us for all tiles, 107 us so, 111 us by orbits alone).
+    const uint32_t h = nx / 2;
+    const uint64_t plane = (uint64_t)h * h * kQuadRecord, fit = scratch ? scratch_bytes / (plane * sizeof(T)) : 0;
+    uint32_t o_sym = 0;
+    if (Q == 4 && turns.turn && fit)
+      o_sym = rot_mask ? std::min(o_act, rotation_orbit_tiles_within(nx, std::max(0.0, turns.rin - 14.0))) : o_act;
+    if (o_sym) {
+      T *sym = reinterpret_cast<T *>(scratch);
+      const double rskip = rfin >= 0 ? rfin + kQuadMargin : 4.0 * nx;
+      const uint32_t tx = ceil_div(rfin >= 0 ? std::min(h, (uint32_t)rskip + 1) : h, 16);
+      for (uint32_t b0 = 0; b0 < ne;) {
+        const uint32_t nb = (uint32_t)std::min<uint64_t>(fit, ne - b0);
+        const T *qb = quad + (uint64_t)b0 * nx * nx * kQuadRecord;
+        double *ab = avg + (uint64_t)b0 * nx * nx;
+        const dim3 gs(tx * tx, nb);
+        const dim3 gr(xcd_grid(rot_mask ? 4ull * o_sym : blocks), 1, ceil_div(nb, 2));
+        auto run = [&](auto rm) {
+          constexpr bool RM = decltype(rm)::value;
+          hipLaunchKernelGGL((quad_sym_kernel<T, RM>), gs, dim3(256), 0, st, qb, sym, nx, tx, rskip);
+          hipLaunchKernelGGL((rotate_sym_kernel<T, 2, RM>), gr, dim3(256), 0, st, qb, sym, inv_tab, coef, coef_t, nA,
+                             quarter, nx, ab, nb, otiles, o_sym, rcut);
+        };
+        if (rot_mask) run(std::true_type{});
+        else run(std::false_type{});
+        e = hipGetLastError();
+        if (e != hipSuccess) return hip_fail(e, "rotate_sym_kernel", __FILE__, __LINE__);
+        b0 += nb;
+      }
+    }
+    if (!o_sym || rot_mask) {
+      const uint32_t o_n = o_act - o_sym;
+      const dim3 grid(xcd_grid(4ull * o_n + ceil_div(2ull * nx, 64)), 1, ceil_div(ne, 2));
+      e = rot_mask ? launch_orbit_rm<T, 2, true>(Q, grid, st, quad, inv_tab, coef, coef_t, nA, quarter, nx, avg, ne,
+                                                  otiles + o_sym, o_n, rcut, turns.share ? 1 : 0)
+                   : launch_orbit_rm<T, 2, false>(Q, grid, st, quad, inv_tab, coef, coef_t, nA, quarter, nx, avg, ne,
+                                                   otiles, o_n, rcut, turns.share ? 1 : 0);
+      if (e != hipSuccess) return hip_fail(e, "rotate_orbit_kernel", __FILE__, __LINE__);
+    }
     if (o_act < n_otiles) {
       const dim3 gf(n_otiles - o_act, 1, ceil_div(ne, 2));
       if (rot_mask) hipLaunchKernelGGL((orbit_fill_kernel<2, true>), gf, dim3(256), 0, st, avg, nx, ne, otiles, o_act);
@@ -934,7 +1178,8 @@ cyr_status launch_warp(const T *src, T *dst, uint32_t nx, uint32_t ny, const dou
                                            uint32_t, const uint32_t *, double, hipStream_t);                                 \
   template cyr_status launch_rotate_quad<T>(const T *, const double *, const double *, const T *, uint32_t,      \
                                             uint32_t, uint32_t, int, double *, uint32_t, const uint32_t *,        \
-                                            uint32_t, const uint32_t *, bool, double, hipStream_t);                \
+                                            uint32_t, const uint32_t *, QuadTurns, double, void *, size_t,         \
+                                            hipStream_t);                                                         \
   template cyr_status launch_detector_warp_n<T>(const double *, T *, uint64_t, uint32_t, uint32_t, uint32_t,       \
                                                 const double *, int, hipStream_t);                                 \
   template cyr_status launch_detector_warp<T>(const double *, T *, uint32_t, uint32_t, const double *, int,        \
