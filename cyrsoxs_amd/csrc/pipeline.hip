@@ -97,19 +97,6 @@ int smaller_pipeline(const cyr_sim_desc *d, const SimGeometry &g) {
 
 namespace {
 
-template <typename U>
-__global__ void __launch_bounds__(256) fill_kernel(U *__restrict__ p, U v, uint64_t n) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-
-template <typename U> cyr_status fill(U *p, U v, uint64_t n, hipStream_t st) {
-  if (n == 0) return CYR_OK;
-  hipLaunchKernelGGL((fill_kernel<U>), dim3(ceil_div(n, 256)), dim3(256), 0, st, p, v, n);
-  CYR_LAUNCHED();
-  return CYR_OK;
-}
-
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // n = (1 - delta) + i beta  ->  n^2 - 1 = delta^2 - 2 delta - beta^2 + 2i (1 - delta) beta
@@ -364,8 +351,8 @@ cyr_status run_plain(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
       const double kv[3] = {g.kvec[k].x, g.kvec[k].y, g.kvec[k].z};
       const EwaldGeom geo = make_ewald_geom(g.nx, g.ny, g.nz, d->phys_size, g.kmag[e], kv, d->interpolation);
       T *out = d_out + ((uint64_t)e * g.nK + k) * P;
-      CYR_TRY(fill<double>(acc, 0.0, P, st));
-      CYR_TRY(fill<uint32_t>(count, 0u, P, st));
+      const double *det = &g.det_inv[(size_t)k * 6];
+      const AvgSink<T> sink(avg, out, 0, P, det);
       for (uint32_t a0 = 0; a0 < g.nA; a0 += nb) {
         const uint32_t n = std::min(nb, g.nA - a0);
         for (uint32_t b = 0; b < n; b++) {
@@ -396,11 +383,10 @@ cyr_status run_plain(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
         }
         kt_begin(st);
         CYR_TRY(launch_rotate_accumulate<T>(proj, acc, count, g.nx, g.ny, su.rotinv + ((size_t)k * g.nA + a0) * 6, n,
-                                            d->rot_mask, st));
+                                            g.nA, a0 == 0, a0 + n == g.nA, d->rot_mask, sink, st));
         kt_end("rotate_accumulate", st, (double)P * (n * sizeof(T) + 2 * (8 + 4)));
       }
-      CYR_TRY(launch_average(acc, count, avg, P, g.nA, d->rot_mask, st));
-      CYR_TRY(launch_detector_warp<T>(avg, out, g.nx, g.ny, &g.det_inv[(size_t)k * 6], d->rot_mask, st));
+      CYR_TRY(launch_detector_warp<T>(avg, out, 0, 1, g.nx, g.ny, det, d->rot_mask, st));
     }
   }
   return CYR_OK;
@@ -544,6 +530,8 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
     aa.nA = g.nA;
     const double *inv = su.rotinv + (size_t)6 * k * g.nA;
     const double rfin = ewald_radius(geo);
+    const double *det = &g.det_inv[(size_t)k * 6];
+    const AvgSink<T> sink(avg, out, 0, P, det);
     if (lab) {
       aa.quad = proj;
       aa.Q = m3<T>(Q);
@@ -552,7 +540,7 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
       kt_end("ebasis_quad", s, part_bytes + (double)kQuadRecord * P * sizeof(T));
       kt_begin(s);
       CYR_TRY(launch_rotate_quad<T>(proj, inv, su.quad + (size_t)3 * k * g.nA, su.quad_t + (size_t)3 * k * g.nA, g.nA,
-                                    g.nx, g.ny, d->rot_mask, avg, 1, su.tiles, g.quarter, su.otiles,
+                                    g.nx, g.ny, d->rot_mask, sink, 1, su.tiles, g.quarter, su.otiles,
                                     quad_turns<T>(g, k, geo), rfin, pol, sizeof(cx<T>) * V * kEbFields, s));
       kt_end("rotate_quad", s, (double)kQuadRecord * P * sizeof(T) + 8.0 * P);
     } else {
@@ -561,10 +549,10 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
       CYR_TRY(launch_ebasis_angles<T>(aa, ng, s));
       kt_end("ebasis_angles", s, part_bytes + (double)g.nA * P * sizeof(T));
       kt_begin(s);
-      CYR_TRY(launch_rotate_all<T>(proj, inv, g.nA, g.nx, g.ny, d->rot_mask, avg, 1, su.tiles, rfin, s));
+      CYR_TRY(launch_rotate_all<T>(proj, inv, g.nA, g.nx, g.ny, d->rot_mask, sink, 1, su.tiles, rfin, s));
       kt_end("rotate_all", s, (double)(g.nA + 1) * P * sizeof(T));
     }
-    CYR_TRY(launch_detector_warp<T>(avg, out, g.nx, g.ny, &g.det_inv[(size_t)k * 6], d->rot_mask, s));
+    CYR_TRY(launch_detector_warp<T>(avg, out, 0, 1, g.nx, g.ny, det, d->rot_mask, s));
   }
   if (lanes > 1) {
     CYR_HIP(hipEventRecord(wb.ev_join, wb.aux));
@@ -787,6 +775,8 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
       // ---- per energy: fields at the Ewald bins, angles, rotation
       const double kv[3] = {g.kvec[k].x, g.kvec[k].y, g.kvec[k].z};
       const double *inv = su.rotinv + (size_t)6 * k * g.nA;
+      const double *det = &g.det_inv[(size_t)k * 6];
+      const uint64_t ostride = (uint64_t)g.nK * P;  // between an energy's pattern and the next
       MbAnglesArgs<T> aa{};
       aa.band = band;
       aa.own = own;
@@ -801,6 +791,7 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
         // batches of nb energies: quadratic forms, rotation + average, detector warp
         for (uint32_t b0 = e0; b0 < e0 + ne; b0 += nb) {
           const uint32_t n = std::min(nb, e0 + ne - b0);
+          T *out = d_out + ((uint64_t)b0 * g.nK + k) * P;
           aa.g = make_ewald_geom(g.nx, g.ny, g.nz, d->phys_size, g.kmag[b0], kv, d->interpolation);
           aa.kmag = su.kmag + b0;
           aa.ne = n;
@@ -816,12 +807,12 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
           for (uint32_t i = 1; i < n; i++) gmin.k = std::min(gmin.k, g.kmag[b0 + i]);
           kt_begin(s);
           CYR_TRY(launch_rotate_quad<T>(proj, inv, su.quad + (size_t)3 * k * g.nA, su.quad_t + (size_t)3 * k * g.nA,
-                                        g.nA, g.nx, g.ny, d->rot_mask, avg, n, su.tiles, g.quarter, su.otiles,
+                                        g.nA, g.nx, g.ny, d->rot_mask, AvgSink<T>(avg, out, ostride, P, det), n,
+                                        su.tiles, g.quarter, su.otiles,
                                         quad_turns<T>(g, k, gmin), 0.5 * std::sqrt((double)d4), pol,
                                         sizeof(cx<T>) * V * pass_max, s));
           kt_end("rotate_quad", s, n * ((double)kQuadRecord * P * sizeof(T) + 8.0 * P));
-          CYR_TRY(launch_detector_warp_n<T>(avg, d_out + ((uint64_t)b0 * g.nK + k) * P, (uint64_t)g.nK * P, n, g.nx,
-                                            g.ny, &g.det_inv[(size_t)k * 6], d->rot_mask, s));
+          CYR_TRY(launch_detector_warp<T>(avg, out, ostride, n, g.nx, g.ny, det, d->rot_mask, s));
         }
       } else {
         // batches of energies whose projections and averages fit in the packed volumes,
@@ -832,6 +823,7 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
         const uint32_t mbatch = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(fit, 32));
         for (uint32_t b0 = e0; b0 < e0 + ne; b0 += mbatch) {
           const uint32_t n = std::min(mbatch, e0 + ne - b0);
+          T *out = d_out + ((uint64_t)b0 * g.nK + k) * P;
           // (FP64 averages ahead of the projections: 8-byte aligned)
           double *bavg = fit ? reinterpret_cast<double *>(pol) : avg;
           T *pr = fit ? reinterpret_cast<T *>(bavg + (uint64_t)n * P) : proj;
@@ -844,11 +836,10 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
           CYR_TRY(launch_mbasis_angles<T>(aa, ng, s));
           kt_end("mbasis_angles", s, (double)planes * nvol * (double)wsum * cxb + n * (double)g.nA * P * sizeof(T));
           kt_begin(s);
-          CYR_TRY(launch_rotate_all<T>(pr, inv, g.nA, g.nx, g.ny, d->rot_mask, bavg, n, su.tiles,
+          CYR_TRY(launch_rotate_all<T>(pr, inv, g.nA, g.nx, g.ny, d->rot_mask, AvgSink<T>(bavg, out, ostride, P, det), n, su.tiles,
                                        0.5 * std::sqrt((double)d4), s));
           kt_end("rotate_all", s, n * (double)(g.nA + 1) * P * sizeof(T));
-          CYR_TRY(launch_detector_warp_n<T>(bavg, d_out + ((uint64_t)b0 * g.nK + k) * P, (uint64_t)g.nK * P, n, g.nx,
-                                            g.ny, &g.det_inv[(size_t)k * 6], d->rot_mask, s));
+          CYR_TRY(launch_detector_warp<T>(bavg, out, ostride, n, g.nx, g.ny, det, d->rot_mask, s));
         }
       }
       e0 += ne;

@@ -42,18 +42,21 @@ __device__ inline bool tile_pixel(const uint32_t *__restrict__ tiles, uint32_t n
   return X < nx && Y < ny;
 }
 
-// (nb angles in turn: the sums stay in angle order)
+// nb angles in turn (the sums stay in angle order): the first batch of a pattern starts
+// them, the last one divides and stores the average (128^2, 6 angles: two fills, the sum,
+// the average and the copy to the output, 5 launches of 4 to 6 us -> one).
 template <typename T>
 __global__ void __launch_bounds__(256) rotate_accumulate_kernel(const T *__restrict__ proj, double *__restrict__ acc,
                                                                 uint32_t *__restrict__ count, uint32_t nx, uint32_t ny,
                                                                 const double *__restrict__ inv_tab, uint32_t nb,
-                                                                int rot_mask) {
+                                                                uint32_t nA, int first, int last, int rot_mask,
+                                                                AvgSink<T> avg) {
   const uint64_t P = (uint64_t)nx * ny;
   const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= P) return;
   const uint32_t Y = (uint32_t)(t / nx), X = (uint32_t)(t - (uint64_t)Y * nx);
-  double s = acc[t];
-  uint32_t c = rot_mask ? count[t] : 0;
+  double s = first ? 0.0 : acc[t];
+  uint32_t c = rot_mask && !first ? count[t] : 0;
 #pragma unroll 2
   for (uint32_t b = 0; b < nb; b++) {
     double inv[6];
@@ -70,20 +73,12 @@ __global__ void __launch_bounds__(256) rotate_accumulate_kernel(const T *__restr
       s += v;
     }
   }
+  if (last) {
+    avg.store(0, t, rot_mask ? (c == 0 ? 0.0 : s * (1.0 / (c * 1.0))) : s * (1.0 / (double)nA));
+    return;
+  }
   acc[t] = s;
   if (rot_mask) count[t] = c;
-}
-
-__global__ void __launch_bounds__(256) average_kernel(const double *__restrict__ acc, const uint32_t *__restrict__ count,
-                                                      double *__restrict__ avg, uint64_t P, uint32_t nA, int rot_mask) {
-  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= P) return;
-  if (rot_mask) {
-    const uint32_t c = count[t];
-    avg[t] = c == 0 ? 0.0 : acc[t] * (1.0 / (c * 1.0));
-  } else {
-    avg[t] = acc[t] * (1.0 / (double)nA);
-  }
 }
 
 // Material frame: every angle's projection proj[ne][nA][P] rotated, masked and averaged
@@ -95,7 +90,7 @@ __global__ void __launch_bounds__(256) average_kernel(const double *__restrict__
 template <typename T>
 __global__ void __launch_bounds__(256) rotate_all_kernel(const T *__restrict__ proj, const double *__restrict__ inv_tab,
                                                          uint32_t nA, uint32_t nx, uint32_t ny, int rot_mask,
-                                                         double *__restrict__ avg, const uint32_t *__restrict__ tiles,
+                                                         AvgSink<T> avg, const uint32_t *__restrict__ tiles,
                                                          uint32_t ntiles) {
   __shared__ double sum[4][64];
   __shared__ uint32_t num[4][64];
@@ -103,7 +98,6 @@ __global__ void __launch_bounds__(256) rotate_all_kernel(const T *__restrict__ p
   const uint32_t b = xcd_tile(blockIdx.x, gridDim.x);
   if (b >= 4 * ntiles) return;  // (the whole block)
   proj += (uint64_t)blockIdx.z * nA * P;
-  avg += (uint64_t)blockIdx.z * P;
   const uint32_t tt = tiles[b >> 2], w = threadIdx.x >> 6, l = threadIdx.x & 63;
   const uint32_t X = (tt & 0xffffu) * 16 + (b & 1) * 8 + (l & 7);
   const uint32_t Y = (tt >> 16) * 16 + ((b >> 1) & 1) * 8 + (l >> 3);
@@ -138,8 +132,7 @@ __global__ void __launch_bounds__(256) rotate_all_kernel(const T *__restrict__ p
     acc += sum[i][l];
     cnt += num[i][l];
   }
-  if (rot_mask) avg[t] = cnt == 0 ? 0.0 : acc * (1.0 / (cnt * 1.0));
-  else avg[t] = acc * (1.0 / (double)nA);
+  avg.store(blockIdx.z, t, rot_mask ? (cnt == 0 ? 0.0 : acc * (1.0 / (cnt * 1.0))) : acc * (1.0 / (double)nA));
 }
 
 // Laboratory frame: every angle's intensity from the per-pixel quadratic form
@@ -250,15 +243,14 @@ __device__ inline void quad_add(const QPoint &p, const Rec<T> (&tp)[NE][4], cons
   quad_combine<T, NE>(p.inside, sm, c, rot_mask, acc, cnt);
 }
 
-template <int NE>
-__device__ inline void quad_store(double *avg, uint64_t P, uint64_t t, uint32_t e0, uint32_t ne, uint32_t nA,
+template <typename T, int NE>
+__device__ inline void quad_store(const AvgSink<T> &avg, uint64_t t, uint32_t e0, uint32_t ne, uint32_t nA,
                                   int rot_mask, const double (&acc)[NE], const uint32_t (&cnt)[NE]) {
 #pragma unroll
   for (int e = 0; e < NE; e++) {
     if (e0 + e >= ne) break;
-    double *o = avg + (uint64_t)(e0 + e) * P;
-    if (rot_mask) o[t] = cnt[e] == 0 ? 0.0 : acc[e] * (1.0 / (cnt[e] * 1.0));
-    else o[t] = acc[e] * (1.0 / (double)nA);
+    avg.store(e0 + e, t,
+              rot_mask ? (cnt[e] == 0 ? 0.0 : acc[e] * (1.0 / (cnt[e] * 1.0))) : acc[e] * (1.0 / (double)nA));
   }
 }
 
@@ -280,7 +272,7 @@ __device__ inline void quad_pixel(const T *const (&qp)[NE], const double *__rest
 template <typename T, int NE>
 __global__ void __launch_bounds__(256) rotate_quad_kernel(const T *__restrict__ quad, const double *__restrict__ inv_tab,
                                                           const double *__restrict__ coef, uint32_t nA, uint32_t nx,
-                                                          uint32_t ny, int rot_mask, double *__restrict__ avg,
+                                                          uint32_t ny, int rot_mask, AvgSink<T> avg,
                                                           uint32_t ne, const uint32_t *__restrict__ tiles,
                                                           uint32_t ntiles) {
   const uint64_t P = (uint64_t)nx * ny;
@@ -293,7 +285,7 @@ __global__ void __launch_bounds__(256) rotate_quad_kernel(const T *__restrict__ 
   double acc[NE] = {};
   uint32_t cnt[NE] = {};
   quad_pixel<T, NE>(qp, inv_tab, coef, nA, nx, ny, X, Y, rot_mask, acc, cnt);
-  quad_store<NE>(avg, P, (uint64_t)Y * nx + X, e0, ne, nA, rot_mask, acc, cnt);
+  quad_store<T, NE>(avg, (uint64_t)Y * nx + X, e0, ne, nA, rot_mask, acc, cnt);
 }
 
 // The same for planes too small to fill the chip: S waves of a block take S runs of the
@@ -307,7 +299,7 @@ __global__ void __launch_bounds__(64 * S) rotate_quad_split_kernel(const T *__re
                                                                    const double *__restrict__ inv_tab,
                                                                    const double *__restrict__ coef, uint32_t nA,
                                                                    uint32_t nx, uint32_t ny, int rot_mask,
-                                                                   double *__restrict__ avg,
+                                                                   AvgSink<T> avg,
                                                                    const uint32_t *__restrict__ tiles,
                                                                    uint32_t ntiles) {
   __shared__ double sum[S][64];
@@ -336,14 +328,14 @@ __global__ void __launch_bounds__(64 * S) rotate_quad_split_kernel(const T *__re
     acc[0] += sum[i][l];
     cnt[0] += num[i][l];
   }
-  quad_store<1>(avg, P, (uint64_t)Y * nx + X, e, e + 1, nA, rot_mask, acc, cnt);
+  quad_store<T, 1>(avg, (uint64_t)Y * nx + X, e, e + 1, nA, rot_mask, acc, cnt);
 }
 
 // Tiles of the general order beyond every finite plane value: the averages
 // rotate_quad_kernel would form there (NaN, or 0 with the rotation mask), as in
 // orbit_fill_kernel.  Same tile and pixel layout as tile_pixel.
-template <int NE>
-__global__ void __launch_bounds__(256) quad_fill_kernel(double *__restrict__ avg, uint32_t nx, uint32_t ny,
+template <typename T, int NE>
+__global__ void __launch_bounds__(256) quad_fill_kernel(AvgSink<T> avg, uint32_t nx, uint32_t ny,
                                                         uint32_t ne, int rot_mask, const uint32_t *__restrict__ tiles,
                                                         uint32_t first) {
   const uint64_t P = (uint64_t)nx * ny;
@@ -356,7 +348,7 @@ __global__ void __launch_bounds__(256) quad_fill_kernel(double *__restrict__ avg
   const double fill = rot_mask ? 0.0 : __longlong_as_double(0x7ff8000000000000ll);
 #pragma unroll
   for (int e = 0; e < NE; e++)
-    if (e0 + e < ne) avg[(uint64_t)(e0 + e) * P + (uint64_t)Y * nx + X] = fill;
+    if (e0 + e < ne) avg.store(e0 + e, (uint64_t)Y * nx + X, fill);
 }
 
 // Quarter-turn orbits (square N x N planes whose angle list holds Q quarter turns
@@ -416,7 +408,7 @@ constexpr int kRawBufferFlags = 0x00020000;
 template <typename T, int NE, bool RM, int R>
 __device__ inline void orbit_tail(const T *const (&qp)[NE], const double *__restrict__ inv_tab,
                                   const double *__restrict__ coef, uint32_t nA, uint32_t n, double rcut, uint32_t j,
-                                  uint32_t w, uint32_t l, uint32_t e0, uint32_t ne, double *__restrict__ avg,
+                                  uint32_t w, uint32_t l, uint32_t e0, uint32_t ne, AvgSink<T> avg,
                                   double (&sum)[4][4][NE][64], uint32_t (&num)[R][R][NE][64]) {
   const uint32_t h = n / 2;
   const bool in = j < 2 * n;
@@ -445,7 +437,7 @@ __device__ inline void orbit_tail(const T *const (&qp)[NE], const double *__rest
       acc[e] += sum[i][0][e][l];
       if constexpr (RM) cnt[e] += num[i][0][e][l];
     }
-  quad_store<NE>(avg, (uint64_t)n * n, (uint64_t)Y * n + X, e0, ne, nA, RM, acc, cnt);
+  quad_store<T, NE>(avg, (uint64_t)Y * n + X, e0, ne, nA, RM, acc, cnt);
 }
 
 // A block holds one 8 x 8 quadrant of a tile of orbits; its wave i samples the points of
@@ -458,7 +450,7 @@ template <typename T, int NE, int Q, bool RM>
 __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__ quad, const double *__restrict__ inv_tab,
                                                            const double *__restrict__ coef,
                                                            const T *__restrict__ coef_t, uint32_t nA, uint32_t A4,
-                                                           uint32_t n, double *__restrict__ avg, uint32_t ne,
+                                                           uint32_t n, AvgSink<T> avg, uint32_t ne,
                                                            const uint32_t *__restrict__ otiles, uint32_t n_otiles,
                                                            double rcut, int share) {
   __shared__ double sum[4][4][NE][64];
@@ -620,7 +612,7 @@ __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__
       if constexpr (RM) c[e] += num[j][q][e][l];
     }
   }
-  quad_store<NE>(avg, P, (uint64_t)PYi * n + PXi, e0, ne, nA, RM, a, c);
+  quad_store<T, NE>(avg, (uint64_t)PYi * n + PXi, e0, ne, nA, RM, a, c);
 }
 
 // Full turns (Q = 4): the sum over an angle's four quarter turns first, then the angles.
@@ -680,7 +672,7 @@ __global__ void __launch_bounds__(256) rotate_sym_kernel(const T *__restrict__ q
                                                          const double *__restrict__ inv_tab,
                                                          const double *__restrict__ coef, const T *__restrict__ coef_t,
                                                          uint32_t nA, uint32_t A4, uint32_t n,
-                                                         double *__restrict__ avg, uint32_t ne,
+                                                         AvgSink<T> avg, uint32_t ne,
                                                          const uint32_t *__restrict__ otiles, uint32_t n_otiles,
                                                          double rcut) {
   __shared__ double sum[4][4][NE][64];
@@ -813,15 +805,15 @@ __global__ void __launch_bounds__(256) rotate_sym_kernel(const T *__restrict__ q
       ex[e] += sum[w][i][e][l];
       if constexpr (RM) exn[e] += num[w][i][e][l];
     }
-  quad_store<NE>(avg, P, (uint64_t)py(i) * n + px(i), e0, ne, nA, RM, ex, exn);
+  quad_store<T, NE>(avg, (uint64_t)py(i) * n + px(i), e0, ne, nA, RM, ex, exn);
 }
 
 // Orbit tiles beyond every finite plane value (their pixels' taps, within 1.5
 // pixels of points as far from the centre as the pixel, are all NaN): the
 // averages rotate_orbit_kernel would form there, NaN, or 0 with the rotation
 // mask (no valid sample).  Same tile and pixel layout as rotate_orbit_kernel.
-template <int NE, bool RM>
-__global__ void __launch_bounds__(256) orbit_fill_kernel(double *__restrict__ avg, uint32_t n, uint32_t ne,
+template <typename T, int NE, bool RM>
+__global__ void __launch_bounds__(256) orbit_fill_kernel(AvgSink<T> avg, uint32_t n, uint32_t ne,
                                                          const uint32_t *__restrict__ otiles, uint32_t first) {
   const uint64_t P = (uint64_t)n * n;
   const uint32_t h = n / 2;
@@ -839,10 +831,11 @@ __global__ void __launch_bounds__(256) orbit_fill_kernel(double *__restrict__ av
   for (int i = 0; i < 4; i++)
 #pragma unroll
     for (int e = 0; e < NE; e++)
-      if (e0 + e < ne) avg[(uint64_t)(e0 + e) * P + (uint64_t)PY[i] * n + PX[i]] = fill;
+      if (e0 + e < ne) avg.store(e0 + e, (uint64_t)PY[i] * n + PX[i], fill);
 }
 
-// grid y = pattern: avg + y P -> out + y out_stride
+// The averaged pattern warped onto the detector (grid y = pattern: avg + y P -> out + y
+// out_stride).
 template <typename T>
 __global__ void __launch_bounds__(256) detector_warp_kernel(const double *__restrict__ avg, T *__restrict__ out,
                                                             uint32_t nx, uint32_t ny, Inv6 inv, int rot_mask,
@@ -856,21 +849,6 @@ __global__ void __launch_bounds__(256) detector_warp_kernel(const double *__rest
   if (!bilinear_sample<double>(avg, nx, ny, inv.c, X, Y, &v))
     v = rot_mask ? 0.0 : __longlong_as_double(0x7ff8000000000000ll);
   out[t] = (T)v;
-}
-
-// The same for an identity warp (the detector normal along the beam): every
-// destination pixel samples its own source pixel with weight 1, so the pattern
-// is the average converted (0 + a, as the weighted sum forms it).
-template <typename T>
-__global__ void __launch_bounds__(256) detector_copy_kernel(const double *__restrict__ avg, T *__restrict__ out,
-                                                            uint64_t P, uint64_t out_stride) {
-  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= P) return;
-  out[(uint64_t)blockIdx.y * out_stride + t] = (T)(0.0 + avg[(uint64_t)blockIdx.y * P + t]);
-}
-
-bool is_identity(const double inv[6]) {
-  return inv[0] == 1.0 && inv[1] == 0.0 && inv[2] == 0.0 && inv[3] == 0.0 && inv[4] == 1.0 && inv[5] == 0.0;
 }
 
 template <typename T>
@@ -960,24 +938,18 @@ uint32_t rotation_quarter_turns(uint32_t nx, uint32_t ny, uint32_t nA, uint32_t 
 
 template <typename T>
 cyr_status launch_rotate_accumulate(const T *proj, double *acc, uint32_t *count, uint32_t nx, uint32_t ny,
-                                    const double *inv, uint32_t nb, int rot_mask, hipStream_t st) {
+                                    const double *inv, uint32_t nb, uint32_t nA, bool first, bool last, int rot_mask,
+                                    const AvgSink<T> &avg, hipStream_t st) {
   const uint64_t P = (uint64_t)nx * ny;
   hipLaunchKernelGGL((rotate_accumulate_kernel<T>), dim3(ceil_div(P, 256)), dim3(256), 0, st, proj, acc, count, nx,
-                     ny, inv, nb, rot_mask);
-  CYR_LAUNCHED();
-  return CYR_OK;
-}
-
-cyr_status launch_average(const double *acc, const uint32_t *count, double *avg, uint64_t P, uint32_t nA, int rot_mask,
-                          hipStream_t st) {
-  hipLaunchKernelGGL(average_kernel, dim3(ceil_div(P, 256)), dim3(256), 0, st, acc, count, avg, P, nA, rot_mask);
+                     ny, inv, nb, nA, first ? 1 : 0, last ? 1 : 0, rot_mask, avg);
   CYR_LAUNCHED();
   return CYR_OK;
 }
 
 template <typename T>
 cyr_status launch_rotate_all(const T *proj, const double *inv_tab, uint32_t nA, uint32_t nx, uint32_t ny, int rot_mask,
-                             double *avg, uint32_t ne, const uint32_t *tiles, double rfin, hipStream_t st) {
+                             const AvgSink<T> &avg, uint32_t ne, const uint32_t *tiles, double rfin, hipStream_t st) {
   const uint32_t ntiles = rotation_tile_count(nx, ny);
   if (!tiles) return fail(CYR_E_INVALID, "rotation: tile order missing");
   // the finite-radius cut of launch_rotate_quad (the projections are NaN where the
@@ -987,7 +959,7 @@ cyr_status launch_rotate_all(const T *proj, const double *inv_tab, uint32_t nA, 
                      rot_mask, avg, tiles, n_act);
   CYR_LAUNCHED();
   if (n_act < ntiles) {
-    hipLaunchKernelGGL((quad_fill_kernel<1>), dim3(ntiles - n_act, 1, ne), dim3(256), 0, st, avg, nx, ny, ne, rot_mask,
+    hipLaunchKernelGGL((quad_fill_kernel<T, 1>), dim3(ntiles - n_act, 1, ne), dim3(256), 0, st, avg, nx, ny, ne, rot_mask,
                        tiles, n_act);
     CYR_LAUNCHED();
   }
@@ -996,7 +968,7 @@ cyr_status launch_rotate_all(const T *proj, const double *inv_tab, uint32_t nA, 
 
 template <typename T, int NE, bool RM>
 hipError_t launch_orbit_rm(uint32_t Q, dim3 grid, hipStream_t st, const T *quad, const double *inv_tab,
-                           const double *coef, const T *coef_t, uint32_t nA, uint32_t A4, uint32_t n, double *avg,
+                           const double *coef, const T *coef_t, uint32_t nA, uint32_t A4, uint32_t n, const AvgSink<T> &avg,
                            uint32_t ne, const uint32_t *otiles, uint32_t n_otiles, double rcut, int share) {
   switch (Q) {
     case 2:
@@ -1017,7 +989,8 @@ hipError_t launch_orbit_rm(uint32_t Q, dim3 grid, hipStream_t st, const T *quad,
 
 template <typename T>
 cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double *coef, const T *coef_t, uint32_t nA,
-                              uint32_t nx, uint32_t ny, int rot_mask, double *avg, uint32_t ne, const uint32_t *tiles,
+                              uint32_t nx, uint32_t ny, int rot_mask, const AvgSink<T> &avg, uint32_t ne,
+                              const uint32_t *tiles,
                               uint32_t quarter, const uint32_t *otiles, QuadTurns turns, double rfin, void *scratch,
                               size_t scratch_bytes, hipStream_t st) {
   if (ne == 0) return CYR_OK;
@@ -1040,7 +1013,7 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
                          rot_mask, avg, tiles, n_act);
     CYR_LAUNCHED();
     if (n_act < ntiles) {
-      hipLaunchKernelGGL((quad_fill_kernel<1>), dim3(ntiles - n_act, 1, ne), dim3(256), 0, st, avg, nx, ny, ne,
+      hipLaunchKernelGGL((quad_fill_kernel<T, 1>), dim3(ntiles - n_act, 1, ne), dim3(256), 0, st, avg, nx, ny, ne,
                          rot_mask, tiles, n_act);
       CYR_LAUNCHED();
     }
@@ -1078,7 +1051,7 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
       for (uint32_t b0 = 0; b0 < ne;) {
         const uint32_t nb = (uint32_t)std::min<uint64_t>(fit, ne - b0);
         const T *qb = quad + (uint64_t)b0 * nx * nx * kQuadRecord;
-        double *ab = avg + (uint64_t)b0 * nx * nx;
+        const AvgSink<T> ab = avg.from(b0);
         const dim3 gs(tx * tx, nb);
         const dim3 gr(xcd_grid(rot_mask ? 4ull * o_sym : blocks), 1, ceil_div(nb, 2));
         auto run = [&](auto rm) {
@@ -1105,8 +1078,8 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
     }
     if (o_act < n_otiles) {
       const dim3 gf(n_otiles - o_act, 1, ceil_div(ne, 2));
-      if (rot_mask) hipLaunchKernelGGL((orbit_fill_kernel<2, true>), gf, dim3(256), 0, st, avg, nx, ne, otiles, o_act);
-      else hipLaunchKernelGGL((orbit_fill_kernel<2, false>), gf, dim3(256), 0, st, avg, nx, ne, otiles, o_act);
+      if (rot_mask) hipLaunchKernelGGL((orbit_fill_kernel<T, 2, true>), gf, dim3(256), 0, st, avg, nx, ne, otiles, o_act);
+      else hipLaunchKernelGGL((orbit_fill_kernel<T, 2, false>), gf, dim3(256), 0, st, avg, nx, ne, otiles, o_act);
       e = hipGetLastError();
       if (e != hipSuccess) return hip_fail(e, "orbit_fill_kernel", __FILE__, __LINE__);
     }
@@ -1125,10 +1098,10 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
   CYR_LAUNCHED();
   if (n_act < ntiles) {
     if (one)
-      hipLaunchKernelGGL((quad_fill_kernel<1>), dim3(ntiles - n_act, 1, ne), dim3(256), 0, st, avg, nx, ny, ne, rot_mask,
+      hipLaunchKernelGGL((quad_fill_kernel<T, 1>), dim3(ntiles - n_act, 1, ne), dim3(256), 0, st, avg, nx, ny, ne, rot_mask,
                          tiles, n_act);
     else
-      hipLaunchKernelGGL((quad_fill_kernel<4>), dim3(ntiles - n_act, 1, ceil_div(ne, 4)), dim3(256), 0, st, avg, nx, ny,
+      hipLaunchKernelGGL((quad_fill_kernel<T, 4>), dim3(ntiles - n_act, 1, ceil_div(ne, 4)), dim3(256), 0, st, avg, nx, ny,
                          ne, rot_mask, tiles, n_act);
     CYR_LAUNCHED();
   }
@@ -1136,29 +1109,11 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
 }
 
 template <typename T>
-cyr_status launch_detector_warp(const double *avg, T *out, uint32_t nx, uint32_t ny, const double inv[6], int rot_mask,
-                                hipStream_t st) {
-  const uint64_t P = (uint64_t)nx * ny;
-  if (is_identity(inv))
-    hipLaunchKernelGGL((detector_copy_kernel<T>), dim3(ceil_div(P, 256)), dim3(256), 0, st, avg, out, P, (uint64_t)0);
-  else
-    hipLaunchKernelGGL((detector_warp_kernel<T>), dim3(ceil_div(P, 256)), dim3(256), 0, st, avg, out, nx, ny,
-                       mk_inv(inv), rot_mask, (uint64_t)0);
-  CYR_LAUNCHED();
-  return CYR_OK;
-}
-
-template <typename T>
-cyr_status launch_detector_warp_n(const double *avg, T *out, uint64_t out_stride, uint32_t ne, uint32_t nx,
-                                  uint32_t ny, const double inv[6], int rot_mask, hipStream_t st) {
-  const uint64_t P = (uint64_t)nx * ny;
-  if (ne == 0) return CYR_OK;
-  if (is_identity(inv))
-    hipLaunchKernelGGL((detector_copy_kernel<T>), dim3(ceil_div(P, 256), ne), dim3(256), 0, st, avg, out, P,
-                       out_stride);
-  else
-    hipLaunchKernelGGL((detector_warp_kernel<T>), dim3(ceil_div(P, 256), ne), dim3(256), 0, st, avg, out, nx, ny,
-                       mk_inv(inv), rot_mask, out_stride);
+cyr_status launch_detector_warp(const double *avg, T *out, uint64_t out_stride, uint32_t ne, uint32_t nx, uint32_t ny,
+                                const double inv[6], int rot_mask, hipStream_t st) {
+  if (ne == 0 || identity_warp(inv)) return CYR_OK;
+  hipLaunchKernelGGL((detector_warp_kernel<T>), dim3(ceil_div((uint64_t)nx * ny, 256), ne), dim3(256), 0, st, avg, out,
+                     nx, ny, mk_inv(inv), rot_mask, out_stride);
   CYR_LAUNCHED();
   return CYR_OK;
 }
@@ -1173,17 +1128,16 @@ cyr_status launch_warp(const T *src, T *dst, uint32_t nx, uint32_t ny, const dou
 
 #define CYR_INST(T)                                                                                                \
   template cyr_status launch_rotate_accumulate<T>(const T *, double *, uint32_t *, uint32_t, uint32_t,             \
-                                                  const double *, uint32_t, int, hipStream_t);                               \
-  template cyr_status launch_rotate_all<T>(const T *, const double *, uint32_t, uint32_t, uint32_t, int, double *, \
-                                           uint32_t, const uint32_t *, double, hipStream_t);                                 \
-  template cyr_status launch_rotate_quad<T>(const T *, const double *, const double *, const T *, uint32_t,      \
-                                            uint32_t, uint32_t, int, double *, uint32_t, const uint32_t *,        \
-                                            uint32_t, const uint32_t *, QuadTurns, double, void *, size_t,         \
-                                            hipStream_t);                                                         \
-  template cyr_status launch_detector_warp_n<T>(const double *, T *, uint64_t, uint32_t, uint32_t, uint32_t,       \
-                                                const double *, int, hipStream_t);                                 \
-  template cyr_status launch_detector_warp<T>(const double *, T *, uint32_t, uint32_t, const double *, int,        \
-                                              hipStream_t);                                                        \
+                                                  const double *, uint32_t, uint32_t, bool, bool, int,             \
+                                                  const AvgSink<T> &, hipStream_t);                                \
+  template cyr_status launch_rotate_all<T>(const T *, const double *, uint32_t, uint32_t, uint32_t, int,           \
+                                           const AvgSink<T> &, uint32_t, const uint32_t *, double, hipStream_t);   \
+  template cyr_status launch_rotate_quad<T>(const T *, const double *, const double *, const T *, uint32_t,        \
+                                            uint32_t, uint32_t, int, const AvgSink<T> &, uint32_t,                 \
+                                            const uint32_t *, uint32_t, const uint32_t *, QuadTurns, double,       \
+                                            void *, size_t, hipStream_t);                                          \
+  template cyr_status launch_detector_warp<T>(const double *, T *, uint64_t, uint32_t, uint32_t, uint32_t,         \
+                                              const double *, int, hipStream_t);                                   \
   template cyr_status launch_warp<T>(const T *, T *, uint32_t, uint32_t, const double *, hipStream_t);
 CYR_INST(float)
 CYR_INST(double)
