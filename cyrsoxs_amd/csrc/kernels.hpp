@@ -200,6 +200,7 @@ template <typename T> struct MbAnglesArgs {
   Mat3<T> Q;                       // frame e1, e2, k^ (quadratic form)
   const double *kmag;              // |k| of the ne energies (mats holds ne x M)
   uint32_t ne;
+  uint32_t bx, by, bw, bh;         // quadratic forms: of the pixels [bx, bx + bw) x [by, by + bh)
 };
 // ne energies in one launch: with quad one quadratic form per pixel (laboratory frame),
 // else every angle's projection.

@@ -788,6 +788,16 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
       aa.nA = g.nA;
       aa.Q = m3<T>(Q);
       if (lab) {
+        // the pixels the rotation may read: a box about the disc of finite values, its
+        // columns from a cache line's first record on
+        const double reach = 0.5 * std::sqrt((double)d4) + kQuadMargin + 1.0;
+        auto box = [&](uint32_t n, uint32_t &lo, uint32_t &len) {
+          const double a = std::max(0.0, n / 2.0 - reach), b = std::min((double)n, std::ceil(n / 2.0 + reach) + 1.0);
+          lo = (uint32_t)a / 16 * 16;
+          len = (uint32_t)b - lo;
+        };
+        box(g.nx, aa.bx, aa.bw);
+        box(g.ny, aa.by, aa.bh);
         // batches of nb energies: quadratic forms, rotation + average, detector warp
         for (uint32_t b0 = e0; b0 < e0 + ne; b0 += nb) {
           const uint32_t n = std::min(nb, e0 + ne - b0);
@@ -802,7 +812,8 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
           // unique inputs: the group's band values (own + mirror, each column's band
           // width, shared by its energies) and the band table; outputs: n
           // quadratic-form planes
-          kt_end("mbasis_quad", s, (double)planes * nvol * (double)wsum * cxb + 4.0 * P + n * (double)kQuadRecord * P * sizeof(T));
+          const double bp = (double)aa.bw * aa.bh;
+          kt_end("mbasis_quad", s, (double)planes * nvol * (double)wsum * cxb + 4.0 * bp + n * (double)kQuadRecord * bp * sizeof(T));
           EwaldGeom gmin = aa.g;  // (the batch's smallest disc)
           for (uint32_t i = 1; i < n; i++) gmin.k = std::min(gmin.k, g.kmag[b0 + i]);
           kt_begin(s);
