@@ -476,7 +476,7 @@ __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__
   auto px = [&](uint32_t j) { return j == 0 ? X0 : j == 1 ? n - Y0 : j == 2 ? n - X0 : Y0; };
   auto py = [&](uint32_t j) { return j == 0 ? Y0 : j == 1 ? X0 : j == 2 ? n - Y0 : n - X0; };
   const uint32_t PXi = px(i), PYi = py(i);
-  const double hi = (double)(n - 1);
+  const double hc = 0.5 * (double)(n - 1);
   const double m = 1e-9 + 1e-12 * (double)n;
   constexpr uint32_t rb = kQuadRecord * (uint32_t)sizeof(T);
   __amdgpu_buffer_rsrc_t rs[NE];
@@ -496,11 +496,13 @@ __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__
       const double *inv = inv_tab + 6 * (uint64_t)a;
       const double sx = __builtin_fma(inv[0], (double)PXi, __builtin_fma(inv[1], (double)PYi, inv[2]));
       const double sy = __builtin_fma(inv[3], (double)PXi, __builtin_fma(inv[4], (double)PYi, inv[5]));
-      const bool inside = sx >= 0 && sx <= hi && sy >= 0 && sy <= hi;
+      // (half the image's side from its middle: two tests, not four; a point that rounding
+      // puts on the wrong side of the border is within the margin of it)
+      const double dx = fabs(sx - hc), dy = fabs(sy - hc), far = dx > dy ? dx : dy;
+      const bool inside = far <= hc;
       const double fx0 = floor(sx), fy0 = floor(sy);
       const double fx = sx - fx0, fy = sy - fy0;
-      const bool safe = inside ? (fx >= m && fx <= 1 - m && fy >= m && fy <= 1 - m)
-                               : (sx < -m || sx > hi + m || sy < -m || sy > hi + m);
+      const bool safe = inside ? fabs(fx - 0.5) <= 0.5 - m && fabs(fy - 0.5) <= 0.5 - m : far > hc + m;
       const uint32_t x0 = inside ? (uint32_t)fx0 : 0u, y0 = inside ? (uint32_t)fy0 : 0u;
       const uint32_t o00 = quad_index(x0, y0, n, n) * rb, o10 = quad_index(x0 + 1, y0, n, n) * rb;
       const uint32_t o01 = quad_index(x0, y0 + 1, n, n) * rb, o11 = quad_index(x0 + 1, y0 + 1, n, n) * rb;
@@ -624,8 +626,8 @@ __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__
 // values of x and s x: one gather per orbit and angle a < A4, a quarter of those
 // rotate_orbit_kernel makes, from the quadrant u, v in [0, n/2 - 1] about the centre alone
 // (every y turns into it; P where by an odd number of quarter turns).  Bound by its
-// gathers through L1, as rotate_orbit_kernel is: 2048^2 film, 10 energies x 180 angles
-// 1.19 ms by orbits -> 0.42 ms and 35 us for S (a wave replaying all four pixels of its
+// gathers through L1 and its FP64 points: 2048^2 film, 10 energies x 180 angles 1.19 ms by
+// orbits -> 0.40 ms and 24 us for S (a wave replaying all four pixels of its
 // own deferred angles, not one pixel of all: 0.46 ms; 1 or 4 energies a pass, not 2: 0.51,
 // 0.46 ms).
 
@@ -668,7 +670,7 @@ __global__ void __launch_bounds__(256) quad_sym_kernel(const T *__restrict__ qua
 // the exact path decides, are replayed pair by pair from the planes themselves, as in
 // rotate_orbit_kernel (the same margins), wave i taking those of orbit pixel i.
 template <typename T, int NE, bool RM>
-__global__ void __launch_bounds__(256) rotate_sym_kernel(const T *__restrict__ quad, const T *__restrict__ sym,
+__global__ void __launch_bounds__(256, sizeof(T) == 4 ? 5 : 4) rotate_sym_kernel(const T *__restrict__ quad, const T *__restrict__ sym,
                                                          const double *__restrict__ inv_tab,
                                                          const double *__restrict__ coef, const T *__restrict__ coef_t,
                                                          uint32_t nA, uint32_t A4, uint32_t n,
@@ -722,12 +724,12 @@ __global__ void __launch_bounds__(256) rotate_sym_kernel(const T *__restrict__ q
       const double dv = __builtin_fma(inv[3], (double)X0, __builtin_fma(inv[4], (double)Y0, inv[5])) - hh;
       const bool odd = (du < 0) != (dv < 0);
       const double p = fabs(odd ? dv : du), q = fabs(odd ? du : dv);
-      const bool inside = p <= hi && q <= hi;  // (all four turns of the point)
+      const double far = p > q ? p : q;
+      const bool inside = far <= hi;  // (all four turns of the point)
       const double fx0 = floor(p), fy0 = floor(q);
       const double fx = p - fx0, fy = q - fy0;
-      const bool safe = inside ? (fx >= m && fx <= 1 - m && fy >= m && fy <= 1 - m)
-                        : RM   ? p > hh + m || q > hh + m    // all four outside
-                               : p > hi + m || q > hi + m;   // one outside
+      const bool safe = inside ? (fabs(fx - 0.5) <= 0.5 - m && fabs(fy - 0.5) <= 0.5 - m)
+                               : far > (RM ? hh : hi) + m;  // (with the mask all four outside, else one)
       const uint32_t x0 = inside ? (uint32_t)fx0 : 0u, y0 = inside ? (uint32_t)fy0 : 0u;
       const uint32_t o00 = quad_index(x0, y0, h, h) * rb, o10 = quad_index(x0 + 1, y0, h, h) * rb;
       const uint32_t o01 = quad_index(x0, y0 + 1, h, h) * rb, o11 = quad_index(x0 + 1, y0 + 1, h, h) * rb;
