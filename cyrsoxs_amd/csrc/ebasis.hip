@@ -33,8 +33,8 @@
 //                        the rotation evaluates at every angle
 //   ebasis_angles_kernel material frame: for every angle p~ = A(theta) F (A = frame x
 //                        E coefficients, 3 x 5, FP64-built) and the Ewald intensity
-// Grids whose Ny has no compile-time codelet take the band passes of mbasis.hip over
-// the five tensor fields instead of ebasis_yz_kernel.
+// Grids whose Ny has no compile-time codelet, and most in FP64 (ebasis_yz_supported), take
+// the band passes of mbasis.hip over the five tensor fields instead of ebasis_yz_kernel.
 //
 // HBM traffic per (energy, k): morphology V (16 M) + Gx write 40 V + Gx read 40 V.
 #include <hip/hip_runtime.h>

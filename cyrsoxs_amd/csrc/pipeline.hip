@@ -1023,7 +1023,7 @@ uint64_t output_bytes(const cyr_sim_desc *d, const SimGeometry &g) {
   return (uint64_t)g.nE * g.nK * g.P * (d->precision == CYR_FP64 ? 8 : 4);
 }
 
-// DC-neighbour partials per volume of the material basis (see run_mbasis)
+// DC-neighbour partials per volume of the material basis (see run_bands)
 static uint64_t mbasis_dc_per(const cyr_sim_desc *d, const SimGeometry &g) {
   const uint32_t slots = d->precision == CYR_FP64 ? fft_dc_slots<double>(g.nx, g.ny) : fft_dc_slots<float>(g.nx, g.ny);
   return (uint64_t)g.nz * (slots ? slots : 1);

@@ -249,7 +249,8 @@ cyr_status cyr_set_tuning(const uint32_t dims[3], int32_t precision, const cyr_y
 cyr_status cyr_get_tuning(const uint32_t dims[3], int32_t precision, cyr_yz_tuning *t);
 /* Times the candidate launch shapes for desc's grid on the current device (HIP
  * events, zero-filled fields) and records the fastest; *chosen (may be NULL)
- * receives it ({0, 0} when the grid has nothing to tune, e.g. 2D). */
+ * receives it ({0, 0} when the grid has nothing to tune: 2D, and grids whose
+ * E-basis runs separate Y and z passes). */
 cyr_status cyr_autotune(const cyr_sim_desc *desc, cyr_yz_tuning *chosen);
 
 /* (energy, k) units the E-basis executor keeps in flight on separate streams,
@@ -270,7 +271,8 @@ int cyr_device_count(void);
 uint32_t cyr_num_angles(double start, double increment, double end);
 /* The executor a descriptor runs: CYR_PIPE_PLAIN, CYR_PIPE_EBASIS or
  * CYR_PIPE_MBASIS (CYR_PIPE_AUTO resolved; grids without fused-kernel plans run
- * PLAIN); -1 for an invalid descriptor.  No counterpart in the reference. */
+ * PLAIN; where its buffers exceed a limit, a smaller one may run instead of an
+ * error); -1 for an invalid descriptor.  No counterpart in the reference. */
 int32_t cyr_resolved_pipeline(const cyr_sim_desc *desc);
 /* Device bytes a simulation holds while it runs (morphology + work volumes). */
 uint64_t cyr_footprint_bytes(const cyr_sim_desc *desc);
