@@ -42,14 +42,31 @@ struct PassArgs {
   uint64_t outer_stride;
   uint32_t inner_count;
   uint32_t outer_count;
-  uint32_t groups;  // ceil(inner_count / pp)
+  uint32_t groups;  // launched, of ceil(inner_count / pp)
   uint32_t pp;
+  uint32_t glo = 0xffffffffu, gskip = 0;  // groups from glo on lie gskip further (column_groups)
   double2 *dcz;        // non-null: the Y pass adds the DC-neighbour partial sums (FftDc)
   const void *dc_twy;  // Y and Z twiddles of those sums (twz null in 2D)
   const void *dc_twz;
   uint32_t dc_nz;
   const uint32_t *span;  // Y pass: per output row, the shifted x range it writes (null: all)
+  uint32_t reach = 0xffffffffu;  // Y pass: columns from bin 0, either way round, that are read later
 };
+
+// The column groups of a strided pass: all, or those within reach of bin 0 (the others are
+// neither read nor written; 2048^2 film at 1 nm, 7 and 4 volumes: 307 -> 175 us).
+inline void column_groups(PassArgs &A) {
+  const uint32_t n = A.inner_count, total = (n + A.pp - 1) / A.pp;
+  A.groups = total;
+  A.glo = 0xffffffffu;
+  A.gskip = 0;
+  if (A.reach >= n / 2) return;
+  const uint32_t lo = A.reach / A.pp + 1, hi = (n - A.reach) / A.pp;
+  if (hi <= lo) return;
+  A.glo = lo;
+  A.gskip = hi - lo;
+  A.groups = total - A.gskip;
+}
 
 // Compile-time codelet pass (lengths with a CtPlan): pencils held in registers,
 // stages exchanged through LDS with immediate offsets.  Contiguous pencils (X)
@@ -94,8 +111,9 @@ __global__ void __launch_bounds__(WG) fft_ct_kernel(PassArgs A, const cx<T> *__r
     vol = q / per_vol;
     tile = q % per_vol;
   }
-  const uint32_t g = tile % A.groups;
+  uint32_t g = tile % A.groups;
   const uint32_t o = tile / A.groups;
+  if (g >= A.glo) g += A.gskip;
   const uint32_t pencil = g * A.pp + p;
   const bool active = pencil < A.inner_count;
   cx<T> *gbase = reinterpret_cast<cx<T> *>(A.vol[vol]) + (uint64_t)(active ? pencil : 0) * A.inner_stride +
@@ -112,7 +130,7 @@ __global__ void __launch_bounds__(WG) fft_ct_kernel(PassArgs A, const cx<T> *__r
     // + 2 cos(2 pi z / Nz) (3D) at x = 0 and 1 otherwise; one FP64 partial per
     // (volume, z, column, wave), the lanes of a wave that hold one column (lane
     // stride pp) combined in a fixed order
-    if (A.dcz && (g == 0 || g == A.groups - 1)) {  // the same for the whole block
+    if (A.dcz && (g == 0 || g == A.groups + A.gskip - 1)) {  // the same for the whole block
       const bool mine = active && (pencil <= 1 || pencil == A.inner_count - 1);
       const uint32_t which = pencil <= 1 ? pencil : 2;
       double sr = 0, si = 0;
@@ -193,7 +211,7 @@ hipError_t launch_ct_n(bool contig, uint32_t nc, PassArgs &A, hipStream_t stream
     using F = typename CtPlan<T, N, false, PP>::type;
     constexpr int WG = PP * TPP;
     A.pp = PP;
-    A.groups = (A.inner_count + PP - 1) / PP;
+    column_groups(A);
     A.nvol = nc;
     const uint64_t tiles = (uint64_t)A.groups * A.outer_count * nc;
     if (tiles > 0x7ffffff0ull) return hipErrorInvalidConfiguration;
@@ -259,7 +277,9 @@ __global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<T> tb, AnyShape sh,
     vol = q / per_vol;
     tile = q % per_vol;
   }
-  const uint32_t g = tile % A.groups, o = tile / A.groups;
+  uint32_t g = tile % A.groups;
+  const uint32_t o = tile / A.groups;
+  if (g >= A.glo) g += A.gskip;
   const uint32_t pencil = g * A.pp + p;
   const bool active = pencil < A.inner_count;
   // (idle pencils read pencil 0 and write nothing)
@@ -281,7 +301,7 @@ __global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<T> tb, AnyShape sh,
   if constexpr (!CONTIG) {
     // DC-neighbour sums (fft_ct_kernel has the formula) of columns 0, 1 and Nx - 1, in the
     // blocks that hold them: one more read of those lines, ahead of the transform's own
-    if (A.dcz && (g == 0 || g == A.groups - 1)) {
+    if (A.dcz && (g == 0 || g == A.groups + A.gskip - 1)) {
       const bool mine = active && (pencil <= 1 || pencil == A.inner_count - 1);
       const uint32_t which = pencil <= 1 ? pencil : 2;
       double sr = 0, si = 0;
@@ -778,7 +798,7 @@ cyr_status launch_any(uint32_t n, bool contig, uint32_t nc, PassArgs &A, hipStre
   LfTab<T> tb;
   CYR_TRY(lf_tables<T>(P, tb));
   A.pp = s.pp;
-  A.groups = (A.inner_count + s.pp - 1) / s.pp;
+  column_groups(A);
   A.nvol = nc;
   const uint64_t tiles = (uint64_t)A.groups * A.outer_count;
   if (tiles * (contig ? 1 : nc) > 0x7ffffff0ull)
@@ -882,6 +902,7 @@ cyr_status fft_axis(void *const *vols, uint32_t count, uint32_t nx, uint32_t ny,
     A.dc_twy = tw;
     A.dc_twz = dc ? dc->twz : nullptr;
     A.dc_nz = nz;
+    A.reach = dc && dc->reach > 1 ? dc->reach : dc ? 1 : 0xffffffffu;
     A.span = dc && dc->span && fft_span_fits<T>(ny) ? dc->span : nullptr;
     bool done = false;
     if (use_ct) {

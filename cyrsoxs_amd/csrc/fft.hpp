@@ -17,11 +17,13 @@ namespace cyr {
 // entries, lo | (hi << 16)), when fft_span_fits(Ny), the pass writes output row y
 // only in the lines of adjacent columns (16 for Ny <= 512, 8 for 1024, 4 above)
 // holding a column whose shifted x coordinate (the bin -> shifted map m - x,
-// Nx + m - x, m = Nx/2) lies in lo..hi; the other columns keep their input.
+// Nx + m - x, m = Nx/2) lies in lo..hi; the other columns keep their input,
+// as do all columns farther than reach from column 0 (either way round).
 struct FftDc {
   double2 *dcz;
   const void *twz;
   const uint32_t *span = nullptr;
+  uint32_t reach = 0xffffffffu;
 };
 // Partials per (volume, z) of a Y pass that can take the DC sums; 0 when it
 // cannot (Nx < 3, or Ny beyond the tiles).

@@ -691,6 +691,8 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
         if (J <= cap || ne == 1) break;
         ne = (ne + 1) / 2;
       }
+      // columns that some band reads: bin x is the shifted column Nx/2 - x
+      const uint32_t reach = (uint32_t)std::min(0.5 * std::sqrt((double)d4) + 2.0, 4294967294.0);
       if (J == 0) J = 1;  // no pixel sampled: the angles kernel writes NaN only
       CYR_TRY(ensure_buffer(lb.part, sizeof(cx<T>) * planes * nvol * J * P));
       cx<T> *own = reinterpret_cast<cx<T> *>(lb.part.ptr);
@@ -722,7 +724,7 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
         const auto launch_x = tensor ? launch_xfields<T, kXTensor> : pair ? launch_xfields<T, kXPair> : launch_xfields<T, kXSingle>;
         CYR_TRY(launch_x(xa, d_vox, d->storage, d->morphology_type, hann, s));
         kt_end("xfields", s, (tensor ? g.M : pair ? 2.0 : 1.0) * 4.0 * vel * V + nv * (double)V * cxb);
-        FftDc fdc{dcz + (uint64_t)vb * dc_per, su.twz, span};
+        FftDc fdc{dcz + (uint64_t)vb * dc_per, su.twz, span, reach};
         if (!dc_slots) {
           DcArgs<T> da{};
           for (uint32_t c = 0; c < nv; c++) da.vol[c] = xa.out[c];
@@ -742,7 +744,8 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
         // reads every volume; writes the columns inside the row spans when it honours
         // them (algorithmic bytes: the lines at the span edges are written whole)
         const double ycols = dc_slots && fft_span_fits<T>(g.ny) ? (double)ssum : (double)P;
-        kt_end("fft_y", s, nv * (double)V * cxb + nv * ycols * g.nz * cxb);
+        const double near = std::min(1.0, (2.0 * reach + 1.0) / g.nx);
+        kt_end("fft_y", s, nv * near * (double)V * cxb + nv * ycols * near * g.nz * cxb);
         BandArgs<T> ba{};
         for (uint32_t c = 0; c < nv; c++) ba.vol[c] = xa.out[c];
         ba.count = nv;
