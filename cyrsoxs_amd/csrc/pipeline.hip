@@ -741,11 +741,11 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
         }
         kt_begin(s);
         CYR_TRY(fft_axis<T>(vptr, nv, g.nx, g.ny, g.nz, 1, s, dc_slots ? &fdc : nullptr));
-        // reads every volume; writes the columns inside the row spans when it honours
-        // them (algorithmic bytes: the lines at the span edges are written whole)
-        const double ycols = dc_slots && fft_span_fits<T>(g.ny) ? (double)ssum : (double)P;
-        const double near = std::min(1.0, (2.0 * reach + 1.0) / g.nx);
-        kt_end("fft_y", s, nv * near * (double)V * cxb + nv * ycols * near * g.nz * cxb);
+        // reads every volume's columns within reach; writes those inside the row spans when it
+        // honours them (algorithmic bytes: the lines at the span edges are written whole)
+        const double near = dc_slots ? std::min(1.0, (2.0 * reach + 1.0) / g.nx) : 1.0;
+        const double ycols = dc_slots && fft_span_fits<T>(g.ny) ? (double)ssum : (double)P * near;
+        kt_end("fft_y", s, nv * near * (double)V * cxb + nv * ycols * g.nz * cxb);
         BandArgs<T> ba{};
         for (uint32_t c = 0; c < nv; c++) ba.vol[c] = xa.out[c];
         ba.count = nv;
