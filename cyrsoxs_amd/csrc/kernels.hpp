@@ -282,7 +282,7 @@ uint32_t rotation_quarter_turns(uint32_t nx, uint32_t ny, uint32_t nA, uint32_t 
 // Laboratory frame: the same for ne energies from their per-pixel quadratic forms
 // quad[ne][P][3] (quad_index order; I(theta) = c^2 q0 + s^2 q1 + 2 c s q2) with
 // coef[a] = (c^2, s^2, 2 c s) (FP64; coef_t: the same in the compute precision)
-// into avg[ne][Ny][Nx]; each angle's taps serve several energies.  quarter (angle
+// into avg (ne patterns); each angle's taps serve several energies.  quarter (angle
 // steps per 90 degrees, 0 = none) with otiles (orbit tile order) lets each tap
 // cell serve the angles a quarter turn apart.  scratch: room for the sums over an angle's
 // quarter turns (not needed: none, or any size).
