@@ -300,8 +300,9 @@ __global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<T> tb, AnyShape sh,
   }
   if constexpr (!CONTIG) {
     // DC-neighbour sums (fft_ct_kernel has the formula) of columns 0, 1 and Nx - 1, in the
-    // blocks that hold them: one more read of those lines, ahead of the transform's own
-    if (A.dcz && (g == 0 || g == A.groups + A.gskip - 1)) {
+    // blocks that hold them (of one-column tiles, column 1 is group 1): one more read of
+    // those lines, ahead of the transform's own
+    if (A.dcz && (g * A.pp <= 1 || g == A.groups + A.gskip - 1)) {
       const bool mine = active && (pencil <= 1 || pencil == A.inner_count - 1);
       const uint32_t which = pencil <= 1 ? pencil : 2;
       double sr = 0, si = 0;
