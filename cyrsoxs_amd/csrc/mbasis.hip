@@ -225,9 +225,10 @@ __device__ inline bool bins_meet_span(uint32_t x0, uint32_t x1, uint32_t n, uint
 // ---- DC-replacement value of one volume ---------------------------------------------
 // dcv[v] = (sum of its dc_per neighbour partials) / dc_cnt, in a fixed order, by one
 // whole block of the band kernels below (the partials are complete before they start):
-// a launch of its own took 3-5 us of a 64^3 simulation's 94.
-template <typename T> __device__ inline void dc_value(const BandArgs<T> &a, uint32_t v) {
-  __shared__ double2 part[16];
+// a launch of its own took 3-5 us of a 64^3 simulation's 94.  part: a value per wave, in
+// the LDS that the other blocks keep their tile in (a variable of its own would add to
+// tiles that fill the LDS).
+template <typename T> __device__ inline void dc_value(const BandArgs<T> &a, uint32_t v, double2 *part) {
   double sr = 0, si = 0;
   for (uint64_t i = threadIdx.x; i < a.dc_per; i += blockDim.x) {
     const double2 x = a.dcz[(uint64_t)(a.vbase + v) * a.dc_per + i];
@@ -258,7 +259,8 @@ __global__ void __launch_bounds__(256) mbasis_extract_kernel(BandArgs<T> a) {
   const uint64_t col = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t v = blockIdx.y;
   if (blockIdx.x == gridDim.x - 1) {  // one block past the columns
-    dc_value<T>(a, v);
+    __shared__ double2 part[4];
+    dc_value<T>(a, v, part);
     return;
   }
   if (col >= P || a.band[col] == 0) return;
@@ -290,7 +292,7 @@ __global__ void __launch_bounds__(WG) mbasis_zband_kernel(BandArgs<T> a, const c
   // the first blocks form the DC values (last, they would be the launch's tail: 512^2 x
   // 128, 395 -> 414 us); blocks past the tiles are grid padding
   if (qb < a.count) {
-    dc_value<T>(a, qb);
+    dc_value<T>(a, qb, reinterpret_cast<double2 *>(smem_raw));
     return;
   }
   const uint32_t q = qb - a.count;
@@ -374,7 +376,7 @@ __global__ void __launch_bounds__(1024) mbasis_zband_any_kernel(LfTab<T> tb, uin
   const uint32_t PP = 1u << lpp, groups = (a.nx + PP - 1) >> lpp, per_vol = groups * a.ny;
   const uint32_t qb = xcd_chunk_tile(blockIdx.x, kZbandChunk);  // (as mbasis_zband_kernel)
   if (qb < a.count) {
-    dc_value<T>(a, qb);
+    dc_value<T>(a, qb, reinterpret_cast<double2 *>(smem_raw));
     return;
   }
   const uint32_t q = qb - a.count;

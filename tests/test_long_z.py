@@ -1,0 +1,29 @@
+"""Long Z pencils: tiles of the Z band pass that fill the 160 KB of LDS.  Bars as in every
+parity test (FP64 1e-10, FP32 1e-4 of the FP64 oracle, identical masks)."""
+import pytest
+
+from cyrsoxs_amd import capi
+from oracle import oracle as O
+from tests.helpers import pattern_rel_l2, random_constants, random_euler
+
+torch = pytest.importorskip("torch")
+
+# FP64 2048: the codelet's four columns take the LDS whole; 1944, 3125 and FP32 4460, 8100:
+# any-length tiles within 256 bytes of it
+CASES = [(capi.FP64, (12, 8, 2048)), (capi.FP64, (8, 10, 1944)), (capi.FP64, (6, 4, 3125)), (capi.FP32, (8, 6, 4460)),
+         (capi.FP32, (6, 4, 8100))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,dims", CASES)
+def test_z_tiles_that_fill_lds(prec, dims):
+    print(f"long z {dims} prec={prec}", flush=True)
+    M, energies, angles = 2, [283.0, 287.0], (0.0, 60.0, 120.0)
+    vox, mats = random_euler(dims, M, 31), random_constants(2, M, 32)
+    kw = dict(interpolation=1, windowing=1)
+    ref = O.simulate(O.Sim(dims, M, 3.0, energies, angles, **kw), vox, mats)
+    for pipeline in (capi.PIPE_MBASIS, capi.PIPE_EBASIS):
+        sim = capi.Sim(dims, M, 3.0, energies, angles, precision=prec, pipeline=pipeline, **kw)
+        assert sim.resolved_pipeline() == pipeline
+        err, same = pattern_rel_l2(capi.simulate(sim, vox, mats), ref)
+        assert same and err < (1e-10 if prec == capi.FP64 else 1e-4), (dims, pipeline, err)
