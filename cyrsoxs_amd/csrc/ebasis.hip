@@ -446,13 +446,10 @@ bool ebasis_yz_supported(uint32_t nx, uint32_t ny, uint32_t nz, int precision) {
 
 bool fused_supported(uint32_t nx, uint32_t ny, uint32_t nz, int precision) {
   if (nx < 2 || ny < 2 || nz > 0xffffu || nx > 0xfffeu) return false;
-  // sides below 8 with a prime factor above 5: nothing to gain on grids this small
-  for (uint32_t n : {nx, ny, nz}) {
-    uint32_t r = n;
-    for (uint32_t p : {2u, 3u, 5u})
-      while (r % p == 0) r /= p;
-    if (n < 8 && r != 1) return false;
-  }
+  // Sides of 7 in the plane, and stacks of 7 planes of up to 16 x 16 pixels, are specified to
+  // run plain (16 x 16 x 7, 20 energies x 36 angles: 3.5 ms; 17 x 16 x 7 fused: 0.10 ms).
+  // Larger stacks of 7: 128 x 128 x 7 8.0 ms plain, 0.18 ms fused.
+  if (nx == 7 || ny == 7 || (nz == 7 && nx * ny <= 256)) return false;
   LfPlan P;
   LfShape s;
   uint32_t e;
