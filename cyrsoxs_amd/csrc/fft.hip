@@ -287,7 +287,7 @@ __global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<T> tb, AnyShape sh,
               (uint64_t)(active ? pencil : 0) * A.inner_stride;
   LfLds<T> tab{tb.tw, tb.pos};
   cx<T> *after = lds + (CONTIG ? A.pp * sh.pitch : tb.m << sh.lpp);
-  const uint32_t *span = nullptr;
+  const uint32_t *span = A.span;
   if constexpr (TAB) {
     tab = lf_stage_tables<T>(tb, after);
     if (!CONTIG && A.span) {
@@ -337,7 +337,7 @@ __global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<T> tb, AnyShape sh,
   auto out = [&](uint32_t row, uint32_t k0, uint32_t r, uint32_t dk, cx<T> v) {
     const uint32_t k = k0 + r * dk;
     bool keep = CONTIG ? row < rows : active;
-    if constexpr (!CONTIG && TAB) {
+    if constexpr (!CONTIG) {
       if (A.span) {
         const uint32_t sp = span[k], lo = sp & 0xffffu, hi = sp >> 16;
         keep = keep && lo <= hi && ((lo_part && a0 <= hi && a1 >= lo) || (hi_part && b0 <= hi && b1 >= lo));
@@ -739,8 +739,9 @@ size_t lf_tables_lds(const LfPlan &P, int precision) {
 }
 
 // Column tiles: max_cols adjacent pencils where three blocks of them (with room for a
-// row-span table) fit in a CU's LDS, else fewer; whole waves.
-bool lf_cols_shape(const LfPlan &P, int precision, uint32_t max_cols, bool need_tables, LfShape &s) {
+// row-span table) fit in a CU's LDS, else fewer; whole waves.  One column that fits without
+// its tables reads them from memory.
+bool lf_cols_shape(const LfPlan &P, int precision, uint32_t max_cols, LfShape &s) {
   const size_t cs = precision == CYR_FP64 ? 16 : 8, cap = max_lds_bytes();
   s = LfShape{};
   for (uint32_t lpp = 6; lpp-- > 0;) {
@@ -750,7 +751,7 @@ bool lf_cols_shape(const LfPlan &P, int precision, uint32_t max_cols, bool need_
     if (lpp > 2 && with > cap / 3) continue;
     if (lpp > 0 && with > cap) continue;
     const bool tables = with <= cap;
-    if (tile > cap || (need_tables && !tables)) continue;
+    if (tile > cap) continue;
     const uint32_t tpp = lf_threads(P, 64 / pp, pp);
     if (!tpp) continue;
     s.pp = pp;
@@ -794,7 +795,7 @@ cyr_status launch_any(uint32_t n, bool contig, uint32_t nc, PassArgs &A, hipStre
   LfShape s;
   *done = false;
   if (!lf_plan(n, prec_of<T>(), false, P)) return CYR_OK;
-  if (!(contig ? lf_rows_shape(P, prec_of<T>(), 0, false, s) : lf_cols_shape(P, prec_of<T>(), 16, false, s)))
+  if (!(contig ? lf_rows_shape(P, prec_of<T>(), 0, false, s) : lf_cols_shape(P, prec_of<T>(), 16, s)))
     return CYR_OK;
   LfTab<T> tb;
   CYR_TRY(lf_tables<T>(P, tb));
@@ -806,7 +807,6 @@ cyr_status launch_any(uint32_t n, bool contig, uint32_t nc, PassArgs &A, hipStre
     return fail(CYR_E_UNSUPPORTED, "FFT grid too large");
   const AnyShape sh{s.tpp, s.lpp, s.pitch, s.pad};
   const dim3 block(s.threads), grid = contig ? dim3((unsigned)tiles, nc) : dim3(xcd_grid(tiles * nc));
-  if (!s.tables && (A.span || A.dcz)) return fail(CYR_E_INVALID, "FFT: DC sums and spans need the tables in LDS");
 #define CYR_ANY(C, TB) hipLaunchKernelGGL((fft_any_kernel<T, C, TB>), grid, block, s.lds, st, tb, sh, A)
   if (contig && s.tables) CYR_ANY(true, true);
   else if (contig) CYR_ANY(true, false);
@@ -828,12 +828,12 @@ template <typename T> bool strided_ct(uint32_t n) {
 }
 
 // The compile-time block of length n also holds the row-span table (4 bytes per
-// row) when that costs no occupancy; the any-length pass reads it from memory.
+// row) when that costs no occupancy; the any-length pass keeps it with its tables.
 template <typename T> bool fft_span_fits(uint32_t n) {
   if (!strided_ct<T>(n)) {
     LfPlan P;
     LfShape s;
-    return lf_plan(n, prec_of<T>(), false, P) && lf_cols_shape(P, prec_of<T>(), 16, true, s);
+    return lf_plan(n, prec_of<T>(), false, P) && lf_cols_shape(P, prec_of<T>(), 16, s);
   }
   const uint32_t pp = n <= 512 ? 16 : (n == 1024 ? 8 : 4), wg = pp * (n / ct_elements(n));
   const bool lo = tw_lo_in_lds<T>((size_t)pp * n, n, wg);
@@ -850,7 +850,7 @@ template <typename T> uint32_t fft_dc_slots(uint32_t nx, uint32_t ny) {
   }
   LfPlan P;
   LfShape s;
-  return lf_plan(ny, prec_of<T>(), false, P) && lf_cols_shape(P, prec_of<T>(), 16, true, s) ? 3 * (s.pp * s.tpp / 64) : 0;
+  return lf_plan(ny, prec_of<T>(), false, P) && lf_cols_shape(P, prec_of<T>(), 16, s) ? 3 * (s.pp * s.tpp / 64) : 0;
 }
 
 template <typename T>

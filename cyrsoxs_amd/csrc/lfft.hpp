@@ -85,8 +85,8 @@ struct LfShape {
   bool tables = false;
   size_t lds = 0;
 };
-// Without `tables` in the request (need_tables false) the longest pencils go without.
-bool lf_cols_shape(const LfPlan &P, int precision, uint32_t max_cols, bool need_tables, LfShape &s);
+// The longest columns go without tables, and rows do without `need_tables`.
+bool lf_cols_shape(const LfPlan &P, int precision, uint32_t max_cols, LfShape &s);
 bool lf_rows_shape(const LfPlan &P, int precision, uint32_t e, bool need_tables, LfShape &s);
 
 // ---- butterflies beyond stockham.hpp's 2, 3, 4, 5, 8 (forward) -------------------

@@ -368,7 +368,8 @@ hipError_t launch_zband_n(const BandArgs<T> &a, hipStream_t st, const cx<T> *tw)
 
 // The same for any length (lfft.hpp): the first stage loads the column's elements, the
 // last hands its outputs to the band test, so nothing but the band values leaves.
-template <typename T>
+// TAB: the tables are in LDS (false: the longest pencils, read from memory).
+template <typename T, bool TAB>
 __global__ void __launch_bounds__(1024) mbasis_zband_any_kernel(LfTab<T> tb, uint32_t tpp, uint32_t lpp,
                                                                 BandArgs<T> a) {
   extern __shared__ unsigned char smem_raw[];
@@ -402,8 +403,11 @@ __global__ void __launch_bounds__(1024) mbasis_zband_any_kernel(LfTab<T> tb, uin
   const uint32_t lom = bm & 0xffffu, wm = a.mir ? bm >> 16 : 0;
   cx<T> *own = a.own + (uint64_t)(a.vbase + v) * a.J * P + col;
   cx<T> *mir = a.mir + (uint64_t)(a.vbase + v) * a.J * P + cm;
-  const LfLds<T> tab = lf_stage_tables<T>(tb, lds + ((size_t)tb.m << lpp));
-  lds_sync();
+  LfLds<T> tab{tb.tw, tb.pos};
+  if constexpr (TAB) {
+    tab = lf_stage_tables<T>(tb, lds + ((size_t)tb.m << lpp));
+    lds_sync();
+  }
   const uint32_t N = a.nz;
   // (columns outside the span hold stale values: they transform to nothing that is kept)
   struct {
@@ -429,14 +433,15 @@ template <typename T> cyr_status launch_zband_any(const BandArgs<T> &a, hipStrea
   const int prec = sizeof(T) == 8 ? CYR_FP64 : CYR_FP32;
   LfPlan P;
   LfShape s;
-  if (!lf_plan(a.nz, prec, false, P) || !lf_cols_shape(P, prec, 32, true, s))
+  if (!lf_plan(a.nz, prec, false, P) || !lf_cols_shape(P, prec, 32, s))
     return fail(CYR_E_UNSUPPORTED, "Z band pass: length beyond the tile");
   LfTab<T> tb;
   CYR_TRY(lf_tables<T>(P, tb));
   const uint64_t tiles = (uint64_t)((a.nx + s.pp - 1) / s.pp) * a.ny * a.count;
   if (tiles > 0x7ffffff0ull) return fail(CYR_E_UNSUPPORTED, "Z band pass: grid too large");
-  hipLaunchKernelGGL((mbasis_zband_any_kernel<T>), dim3(xcd_chunk_grid(tiles + a.count, kZbandChunk)), dim3(s.pp * s.tpp), s.lds,
-                     st, tb, s.tpp, s.lpp, a);
+  const dim3 grid(xcd_chunk_grid(tiles + a.count, kZbandChunk)), block(s.pp * s.tpp);
+  if (s.tables) hipLaunchKernelGGL((mbasis_zband_any_kernel<T, true>), grid, block, s.lds, st, tb, s.tpp, s.lpp, a);
+  else hipLaunchKernelGGL((mbasis_zband_any_kernel<T, false>), grid, block, s.lds, st, tb, s.tpp, s.lpp, a);
   CYR_LAUNCHED();
   return CYR_OK;
 }
@@ -794,7 +799,7 @@ bool mbasis_zband_supported(uint32_t nz, int precision) {
   if (precision == CYR_FP64 ? zband_ct<double>(nz) : zband_ct<float>(nz)) return true;
   LfPlan P;
   LfShape s;
-  return lf_plan(nz, precision, false, P) && lf_cols_shape(P, precision, 32, true, s);
+  return lf_plan(nz, precision, false, P) && lf_cols_shape(P, precision, 32, s);
 }
 
 template <typename T> cyr_status launch_mbasis_zband(const BandArgs<T> &a, hipStream_t st) {

@@ -1,5 +1,6 @@
-"""Long Z pencils: tiles of the Z band pass that fill the 160 KB of LDS.  Bars as in every
-parity test (FP64 1e-10, FP32 1e-4 of the FP64 oracle, identical masks)."""
+"""Long columns: tiles of the Z band pass that fill the 160 KB of LDS, and Y and Z columns
+whose tables stay in memory.  Bars as in every parity test (FP64 1e-10, FP32 1e-4 of the
+FP64 oracle, identical masks)."""
 import pytest
 
 from cyrsoxs_amd import capi
@@ -11,13 +12,16 @@ torch = pytest.importorskip("torch")
 # FP64 2048: the codelet's four columns take the LDS whole; 1944, 3125 and FP32 4460, 8100:
 # any-length tiles within 256 bytes of it
 CASES = [(capi.FP64, (12, 8, 2048)), (capi.FP64, (8, 10, 1944)), (capi.FP64, (6, 4, 3125)), (capi.FP32, (8, 6, 4460)),
-         (capi.FP32, (6, 4, 8100))]
+         (capi.FP32, (6, 4, 8100)),
+         # tables in memory
+         (capi.FP64, (6, 4, 5000)), (capi.FP32, (4, 4, 9216)), (capi.FP32, (3, 9216, 1)), (capi.FP32, (4, 8192, 2)),
+         (capi.FP64, (3, 8192, 1))]
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("prec,dims", CASES)
-def test_z_tiles_that_fill_lds(prec, dims):
-    print(f"long z {dims} prec={prec}", flush=True)
+def test_long_columns(prec, dims):
+    print(f"long columns {dims} prec={prec}", flush=True)
     M, energies, angles = 2, [283.0, 287.0], (0.0, 60.0, 120.0)
     vox, mats = random_euler(dims, M, 31), random_constants(2, M, 32)
     kw = dict(interpolation=1, windowing=1)
@@ -27,3 +31,11 @@ def test_z_tiles_that_fill_lds(prec, dims):
         assert sim.resolved_pipeline() == pipeline
         err, same = pattern_rel_l2(capi.simulate(sim, vox, mats), ref)
         assert same and err < (1e-10 if prec == capi.FP64 else 1e-4), (dims, pipeline, err)
+
+
+@pytest.mark.parametrize("prec,dims", [(capi.FP32, (64, 64, 16000)), (capi.FP32, (64, 8192, 64)),
+                                       (capi.FP32, (64, 12288, 1)), (capi.FP64, (64, 64, 10000)),
+                                       (capi.FP64, (64, 8192, 1))])
+def test_long_columns_are_fused(prec, dims):
+    sim = capi.Sim(dims, 2, 2.0, [285.0, 286.0], (0, 30, 150), precision=prec, pipeline=capi.PIPE_MBASIS)
+    assert sim.resolved_pipeline() == capi.PIPE_MBASIS
