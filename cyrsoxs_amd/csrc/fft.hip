@@ -620,7 +620,7 @@ bool lf_search(uint32_t n, int precision, bool narrow, LfPlan &P) {
     // run backwards)
     double best = 1e18;
     std::vector<uint32_t> s2;
-    for (uint32_t m = 2 * n - 1; m <= std::min(kLfMaxLength, 3 * n); m++) {
+    for (uint32_t m = 2 * n - 1; m <= std::min(kLfMaxConvolution, 3 * n); m++) {
       if (!radix_sequence(m, narrow ? 8 : 10, s2, c)) continue;
       if (m * (2 * c + 2) < best) {
         best = m * (2 * c + 2);

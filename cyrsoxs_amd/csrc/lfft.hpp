@@ -34,7 +34,8 @@
 namespace cyr {
 
 constexpr int kLfStages = 12;
-constexpr uint32_t kLfMaxLength = 16384;
+constexpr uint32_t kLfMaxLength = 20480;       // one FP32 pencil in 160 KB of LDS
+constexpr uint32_t kLfMaxConvolution = 16384;  // Bluestein's
 
 struct LfStage {
   uint32_t radix;

@@ -1,11 +1,12 @@
 """Long columns: tiles of the Z band pass that fill the 160 KB of LDS, and Y and Z columns
 whose tables stay in memory.  Bars as in every parity test (FP64 1e-10, FP32 1e-4 of the
 FP64 oracle, identical masks)."""
+import numpy as np
 import pytest
 
 from cyrsoxs_amd import capi
 from oracle import oracle as O
-from tests.helpers import pattern_rel_l2, random_constants, random_euler
+from tests.helpers import pattern_rel_l2, random_constants, random_euler, rel_l2
 
 torch = pytest.importorskip("torch")
 
@@ -31,6 +32,20 @@ def test_long_columns(prec, dims):
         assert sim.resolved_pipeline() == pipeline
         err, same = pattern_rel_l2(capi.simulate(sim, vox, mats), ref)
         assert same and err < (1e-10 if prec == capi.FP64 else 1e-4), (dims, pipeline, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims", [(2, 18432, 1), (18432, 2, 1), (3, 20480, 1), (20480, 2, 1), (2, 2, 16875)])
+def test_transforms_longer_than_16384(dims):
+    """One FP32 pencil of up to 20480 points in LDS (tolerance as for the shorter lengths: 15
+    roundings of 6e-8 a butterfly, five stages, two axes, below 4e-6)."""
+    print(f"fft3d {dims}", flush=True)
+    rng = np.random.default_rng(dims[0] + dims[1])
+    v = rng.normal(size=dims[::-1]) + 1j * rng.normal(size=dims[::-1])
+    d = torch.from_numpy(v.astype(np.complex64)).cuda()
+    capi.fft3d_device([d], dims, capi.FP32)
+    torch.cuda.synchronize()
+    assert rel_l2(d.cpu().numpy(), np.fft.fftn(v)) < 4e-6
 
 
 @pytest.mark.parametrize("prec,dims", [(capi.FP32, (64, 64, 16000)), (capi.FP32, (64, 8192, 64)),
