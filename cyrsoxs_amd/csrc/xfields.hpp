@@ -359,8 +359,9 @@ __global__ void __launch_bounds__(WG, (x_min_waves<T, F, MODE>()))
 // Launch shape of the compile-time X plans: rows of <= 64 threads share a wave.
 constexpr int ct_polx_wg(int N, int E) { return N / E <= 64 ? 64 : N / E; }
 
-// Plan, shape and elements per thread of the any-length X transforms: FP32 4, FP64 2,
-// twice that for rows that would need more than kLfRowThreads threads.  Narrow plans: the
+// Plan, shape and elements per thread of the any-length X transforms: FP32 4, FP64 2, and
+// for rows that would need more than kLfRowThreads threads twice that, in FP32 up to four
+// times (rows of 4097 to 8192 points).  Narrow plans: the
 // per-element state and butterflies of up to 8 then fit 128 registers in FP32, 4 waves per
 // SIMD, where radices up to 13 took 182 (200 x 240 x 50, 3 materials: 109 -> 84 us per
 // volume; 101 x 94 x 21: 58 -> 37 us).  Lengths with factors 11 and 13 would be
@@ -378,9 +379,9 @@ inline bool lf_x_shape(uint32_t n, int precision, LfPlan &P, LfShape &s, uint32_
     }
   }
   if (!fits) return false;
-  if (lf_rows_shape(P, precision, e, true, s)) return true;
-  e *= 2;
-  return lf_rows_shape(P, precision, e, true, s);
+  for (const uint32_t last = precision == CYR_FP64 ? 4 : 16; e <= last; e *= 2)
+    if (lf_rows_shape(P, precision, e, true, s)) return true;
+  return false;
 }
 
 // The compile-time plan applies (its elements per thread are compiled for T).
@@ -478,7 +479,8 @@ cyr_status launch_xfields(PolxArgs<T> a, const void *vox, int storage, int morph
     else if (!narrow) {
       if constexpr (sizeof(T) == 4) e = launch_xfields_lf<T, S, E0, false, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
     } else if (e_lf == E0) e = launch_xfields_lf<T, S, E0, true, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
-    else e = launch_xfields_lf<T, S, 2 * E0, true, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
+    else if (e_lf == 2 * E0) e = launch_xfields_lf<T, S, 2 * E0, true, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
+    else if constexpr (sizeof(T) == 4) e = launch_xfields_lf<T, S, 4 * E0, true, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
   };
   if constexpr (sizeof(T) == 4) {
     if (storage == CYR_STORE_FP16) go(half4{});

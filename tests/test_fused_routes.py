@@ -1,10 +1,11 @@
-"""Grids that run the fused executors: stacks of seven planes."""
+"""Grids that run the fused executors: stacks of seven planes, FP32 rows of 4097 to 8192
+points."""
 import numpy as np
 import pytest
 
 from cyrsoxs_amd import capi
 from oracle import oracle as O
-from tests.helpers import pattern_rel_l2, random_constants, random_euler
+from tests.helpers import pattern_rel_l2, random_constants, random_euler, random_vector
 
 torch = pytest.importorskip("torch")
 
@@ -36,3 +37,26 @@ def test_seven_planes_match_the_oracle(dims, prec):
         sim = capi.Sim(dims, M, 2.0, energies, angles, precision=prec, pipeline=pipeline, **kw)
         err, same = pattern_rel_l2(capi.simulate(sim, vox, mats), ref)
         assert same and err < (1e-10 if prec == capi.FP64 else 1e-4), (dims, pipeline, err)
+
+
+@pytest.mark.parametrize("nx", [4608, 5184, 5832, 6144])
+def test_long_rows_are_fused(nx):
+    for dims in ((nx, 64, 1), (nx, 96, 12)):
+        for pipeline in (capi.PIPE_EBASIS, capi.PIPE_MBASIS):
+            assert _resolved(dims, capi.FP32, pipeline) == pipeline
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,M,morph", [(4100, 2, 0), (4608, 1, 0), (6144, 2, 0), (6144, 3, 1), (8192, 2, 0)])
+def test_long_rows_match_the_oracle(nx, M, morph):
+    """The X kernel's longest runs per thread (FP32, 1e-4 of the oracle, identical masks)."""
+    dims, energies, angles = (nx, 4, 2), [283.0, 287.0], (0.0, 60.0, 120.0)
+    print(f"long rows {dims} M={M} morph={morph}", flush=True)
+    vox, mats = (random_vector if morph else random_euler)(dims, M, 43), random_constants(2, M, 44)
+    kw = dict(interpolation=1, windowing=1, rot_mask=1, morphology_type=morph)
+    ref = O.simulate(O.Sim(dims, M, 3.0, energies, angles, **kw), vox, mats)
+    for pipeline in (capi.PIPE_MBASIS, capi.PIPE_EBASIS):
+        sim = capi.Sim(dims, M, 3.0, energies, angles, precision=capi.FP32, pipeline=pipeline, **kw)
+        assert sim.resolved_pipeline() == pipeline
+        err, same = pattern_rel_l2(capi.simulate(sim, vox, mats), ref)
+        assert same and err < 1e-4, (dims, pipeline, err)
