@@ -64,6 +64,40 @@ int resolved_pipeline(const cyr_sim_desc *d, const SimGeometry &g) {
   return mb < eb ? CYR_PIPE_MBASIS : CYR_PIPE_EBASIS;
 }
 
+// Grids on which a request that does not fit is an error, never the plain executor's run
+// time: both sides are a codelet's length, or a product of radices 8 (or a remaining 4 or
+// 2), 3 and 5 whose least common multiple is at most 24 (FP64: 8), without 5 beside others,
+// and whose rows need no more than 256 threads at up to 16 (FP64: 8) elements each, or that
+// multiple (columns: 1024 threads, 512 for multiples above 8), with room in LDS for a column
+// and the Y and z twiddles.  Callers rely on either answer: other grids are admitted with
+// the plain executor's buffers.
+static bool refuses_plain(const SimGeometry &g, int precision) {
+  const bool fp64 = precision == CYR_FP64;
+  const size_t cs = fp64 ? 16 : 8;
+  const size_t column = g.nz > 1 ? 2 * (size_t)g.ny + g.nz : g.ny;
+  if (column * cs > device_max_lds()) return false;
+  for (int axis = 0; axis < 2; axis++) {
+    const uint32_t n = axis ? g.ny : g.nx;
+    if (n == 64 || n == 128 || n == 256 || (n == 384 && !fp64) || n == 512 || n == 1024 || n == 2048) continue;
+    uint32_t r = n, l = 1;
+    for (uint32_t p : {8u, 4u, 2u})
+      if (n % p == 0) {
+        l = p;
+        break;
+      }
+    if (n % 3 == 0) l *= 3;
+    if (n % 5 == 0) l *= 5;
+    for (uint32_t p : {2u, 3u, 5u})
+      while (r % p == 0) r /= p;
+    if (r != 1 || l > (fp64 ? 8u : 24u) || (l > 5 && l % 5 == 0)) return false;
+    const uint32_t threads = axis == 0 ? 256 : l <= 8 ? 1024 : 512;
+    uint32_t e = l;
+    while (n / e > threads && 2 * e <= (fp64 ? 8u : 16u) && n % (2 * e) == 0) e *= 2;
+    if (n / e > (axis && e > 8 ? 512u : threads)) return false;
+  }
+  return true;
+}
+
 int smaller_pipeline(const cyr_sim_desc *d, const SimGeometry &g) {
   const int pipe = resolved_pipeline(d, g);
   if (pipe == CYR_PIPE_PLAIN) return -1;
@@ -76,23 +110,7 @@ int smaller_pipeline(const cyr_sim_desc *d, const SimGeometry &g) {
     const double mb = (double)g.V * (4.0 * el * g.M + 4.0 * cs * nv) + (double)g.nE * (double)g.P * 4.0 * ng * nv * cs;
     if (mb >= eb) return CYR_PIPE_EBASIS;
   }
-  for (uint32_t n : {g.nx, g.ny}) {
-    // radices 8 (or the remaining 4 or 2), 3 and 5: their least common multiple
-    uint32_t r = n, l = 1;
-    for (uint32_t p : {8u, 4u, 2u})
-      if (n % p == 0) {
-        l = p;
-        break;
-      }
-    if (n % 3 == 0) l *= 3;
-    if (n % 5 == 0) l *= 5;
-    for (uint32_t p : {2u, 3u, 5u})
-      while (r % p == 0) r /= p;
-    const bool ct = n == 64 || n == 128 || n == 256 || (n == 384 && d->precision != CYR_FP64) || n == 512 ||
-                    n == 1024 || n == 2048;
-    if (!ct && (r != 1 || l > (d->precision == CYR_FP64 ? 8u : 24u) || (l > 8 && l % 5 == 0))) return CYR_PIPE_PLAIN;
-  }
-  return -1;
+  return refuses_plain(g, d->precision) ? -1 : CYR_PIPE_PLAIN;
 }
 
 namespace {

@@ -79,8 +79,7 @@ bool ebasis_usable(const cyr_sim_desc *d, const SimGeometry &g);
 int resolved_pipeline(const cyr_sim_desc *d, const SimGeometry &g);
 // The executor to try where the buffers of the simulation's own do not fit (-1: none; it
 // is refused).  AUTO's material basis, where the E-basis handles fewer bytes: the E-basis.
-// Grids with a side other than 2^a 3^b or 5^c, which had no fused executor before the
-// any-length transforms: plain.
+// Else plain, except on grids where refuses_plain holds.
 int smaller_pipeline(const cyr_sim_desc *d, const SimGeometry &g);
 
 // Autotunes the E-basis Y/z launch shape of the simulation's grid (see cyr_autotune).

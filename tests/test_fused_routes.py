@@ -1,5 +1,7 @@
 """Grids that run the fused executors: stacks of seven planes, FP32 rows of 4097 to 8192
 points."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -60,3 +62,20 @@ def test_long_rows_match_the_oracle(nx, M, morph):
         assert sim.resolved_pipeline() == pipeline
         err, same = pattern_rel_l2(capi.simulate(sim, vox, mats), ref)
         assert same and err < 1e-4, (dims, pipeline, err)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="checks the gate alone, on host pointers")
+@pytest.mark.parametrize("dims,prec,status", [
+    # rows of 3^7, 5^5 and 2 3^7 points, and columns of 4 3^7, need more threads than the short
+    # radix plans have: past the gate with the plain executor's buffers (7: no device)
+    ((2187, 64, 24), capi.FP32, 7), ((3125, 64, 16), capi.FP32, 7), ((4374, 32, 24), capi.FP32, 7),
+    ((48, 8748, 8), capi.FP32, 7), ((16, 6561, 24), capi.FP32, 7), ((130, 130, 200), capi.FP32, 7),
+    # sides with short plans: refused (1)
+    ((2048, 64, 24), capi.FP32, 1), ((3072, 64, 16), capi.FP32, 1), ((48, 4096, 20), capi.FP32, 1),
+    ((81, 243, 150), capi.FP32, 1), ((125, 625, 40), capi.FP32, 1), ((144, 128, 160), capi.FP32, 1)])
+def test_requests_that_do_not_fit(dims, prec, status):
+    sim = capi.Sim(dims, 4, 2.0, [285.0, 286.0], (0, 5, 175), precision=prec, pipeline=capi.PIPE_MBASIS)
+    assert sim.resolved_pipeline() == capi.PIPE_MBASIS
+    buf = np.zeros(64)
+    p = ctypes.c_void_p(buf.ctypes.data)
+    assert capi.lib().cyr_simulate_device_noalloc(sim.ref, p, p, p, None) == status
