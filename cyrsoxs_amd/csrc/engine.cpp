@@ -138,16 +138,18 @@ struct Lanes {
 };
 
 // Queues the whole schedule: fork from `main`, each stream runs its members with
-// resident tables, join back into `main`.
+// resident tables, join back into `main`.  ran[i] (ran may be null): the smaller executor
+// that member i fell back to.
 cyr_status queue_schedule(const cyr_sim_desc *descs, const void *const *d_voxels, const double *const *mats,
-                          void *const *d_outs, const Schedule &s, Lanes &L, hipStream_t main) {
+                          void *const *d_outs, const Schedule &s, Lanes &L, hipStream_t main,
+                          int32_t *ran = nullptr) {
   CYR_HIP(hipEventRecord(L.fork, main));
   for (size_t l = 0; l < L.st.size(); l++) {
     CYR_HIP(hipStreamWaitEvent(L.st[l], L.fork, 0));
     for (uint32_t i : s.per_lane[l]) {
       const void *tab = reinterpret_cast<const unsigned char *>(s.tables.ptr) + s.table_off[i];
       CYR_TRY(run_simulation(&descs[i], s.geo[i], d_voxels[i], mats[i], d_outs[i], *L.wb[l], L.st[l], kRunResident,
-                             tab));
+                             tab, ran ? ran + i : nullptr));
     }
     CYR_HIP(hipEventRecord(L.ev[l], L.st[l]));
     CYR_HIP(hipStreamWaitEvent(main, L.ev[l], 0));
@@ -289,9 +291,21 @@ cyr_status cyr_batch_create(uint32_t count, const cyr_sim_desc *descs, const voi
   CYR_TRY(plan_schedule(count, p.descs.data(), p.matp.data(), (uint32_t)p.lanes.st.size(), p.cap, p.sched));
   CYR_TRY(tune_shapes(count, p.descs.data(), p.sched.geo, *p.lanes.wb[0], p.lanes.st[0]));
   // eager pass: sizes every buffer and creates every twiddle table, so the
-  // captured graph holds kernels and event edges only
-  CYR_TRY(queue_schedule(p.descs.data(), p.vox.data(), p.matp.data(), p.outs.data(), p.sched, p.lanes, p.cap));
-  CYR_HIP(hipStreamSynchronize(p.cap));
+  // captured graph holds kernels and event edges only.  A member whose buffers do not fit
+  // falls back to a smaller executor and frees those of its stream: the plan keeps that
+  // executor, and the pass is repeated until every member runs the one it has.
+  for (bool settled = false; !settled;) {
+    std::vector<int32_t> ran(count, -1);
+    CYR_TRY(queue_schedule(p.descs.data(), p.vox.data(), p.matp.data(), p.outs.data(), p.sched, p.lanes, p.cap,
+                           ran.data()));
+    CYR_HIP(hipStreamSynchronize(p.cap));
+    settled = true;
+    for (uint32_t i = 0; i < count; i++)
+      if (ran[i] >= 0) {
+        p.descs[i].pipeline = ran[i];
+        settled = false;
+      }
+  }
   CYR_HIP(hipStreamBeginCapture(p.cap, hipStreamCaptureModeRelaxed));
   const cyr_status qs = queue_schedule(p.descs.data(), p.vox.data(), p.matp.data(), p.outs.data(), p.sched, p.lanes,
                                        p.cap);

@@ -882,7 +882,7 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
 
 template <typename T>
 cyr_status run_impl(const cyr_sim_desc *d, const SimGeometry &g, const void *d_vox, const double *mats, T *d_out,
-                    WorkBuffers &wb, hipStream_t st, RunMode mode, const void *resident_tables) {
+                    WorkBuffers &wb, hipStream_t st, RunMode mode, const void *resident_tables, int32_t *ran) {
   Tables tb;
   const void *tables = resident_tables;
   if (mode == kRunResident) {
@@ -908,12 +908,13 @@ cyr_status run_impl(const cyr_sim_desc *d, const SimGeometry &g, const void *d_v
   if (s == CYR_E_NOMEM && !scratch_arena()) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     CYR_HIP(hipStreamIsCapturing(st, &cap));
-    if (cap == hipStreamCaptureStatusNone) {  // (capture follows an eager run, which sized the buffers)
+    if (cap == hipStreamCaptureStatusNone) {  // (captured members name the executor that fitted: ran)
       cyr_sim_desc q = *d;
       for (int p; s == CYR_E_NOMEM && (p = smaller_pipeline(&q, g)) >= 0;) {
         CYR_HIP(hipStreamSynchronize(st));
         for (auto &l : wb.lane) l.release();
         q.pipeline = p;
+        if (ran) *ran = p;
         s = execute(&q);
       }
     }
@@ -1085,10 +1086,11 @@ uint64_t work_bytes(const cyr_sim_desc *d, const SimGeometry &g) {
 }
 
 cyr_status run_simulation(const cyr_sim_desc *d, const SimGeometry &g, const void *d_vox, const double *mats,
-                          void *d_out, WorkBuffers &wb, hipStream_t st, RunMode mode, const void *resident_tables) {
+                          void *d_out, WorkBuffers &wb, hipStream_t st, RunMode mode, const void *resident_tables,
+                          int32_t *ran) {
   if (d->precision == CYR_FP64)
-    return run_impl<double>(d, g, d_vox, mats, reinterpret_cast<double *>(d_out), wb, st, mode, resident_tables);
-  return run_impl<float>(d, g, d_vox, mats, reinterpret_cast<float *>(d_out), wb, st, mode, resident_tables);
+    return run_impl<double>(d, g, d_vox, mats, reinterpret_cast<double *>(d_out), wb, st, mode, resident_tables, ran);
+  return run_impl<float>(d, g, d_vox, mats, reinterpret_cast<float *>(d_out), wb, st, mode, resident_tables, ran);
 }
 
 size_t table_bytes(const cyr_sim_desc *d, const SimGeometry &g) {

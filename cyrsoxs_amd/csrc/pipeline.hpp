@@ -62,10 +62,11 @@ uint64_t output_bytes(const cyr_sim_desc *d, const SimGeometry &g);
 // writes [nE][nK][Ny][Nx] of the compute precision to d_out.  Asynchronous on
 // `st` except for small table uploads; the caller synchronises.
 // kRunResident reads the constant tables at resident_tables (laid out as
-// fill_tables writes them); the other modes build and upload them.
+// fill_tables writes them); the other modes build and upload them.  Where the buffers of
+// the descriptor's executor do not fit and a smaller one runs, *ran (may be null) names it.
 cyr_status run_simulation(const cyr_sim_desc *d, const SimGeometry &g, const void *d_vox, const double *mats,
                           void *d_out, WorkBuffers &wb, hipStream_t st, RunMode mode = kRunSync,
-                          const void *resident_tables = nullptr);
+                          const void *resident_tables = nullptr, int32_t *ran = nullptr);
 
 // The simulation's constant tables (material constants, Hanning, E-basis
 // coefficients, rotation inverses): their size, and their contents on the host.

@@ -83,8 +83,8 @@ static cyr_status ensure_in_arena(ScratchArena &a, DeviceBuffer &b, size_t bytes
 // Test hook for the error path of a failed device allocation: with
 // CYR_TEST_FAIL_ALLOC=k in the environment, the device allocation after the next
 // k ones fails with CYR_E_NOMEM (and every later one, until the value changes)
-// without calling hipMalloc.
-static bool injected_alloc_failure() {
+// without calling hipMalloc; with CYR_TEST_FAIL_ALLOC=>n every one of more than n bytes.
+static bool injected_alloc_failure(size_t bytes) {
   static std::mutex mu;
   static std::string seen;
   static long left = -1;
@@ -97,8 +97,9 @@ static bool injected_alloc_failure() {
   }
   if (seen != v) {
     seen = v;
-    left = std::atol(v);
+    left = *v == '>' ? -1 : std::atol(v);
   }
+  if (*v == '>') return bytes > std::strtoull(v + 1, nullptr, 10);
   if (left < 0) return false;
   if (left == 0) return true;
   left--;
@@ -114,7 +115,7 @@ cyr_status ensure_buffer(DeviceBuffer &b, size_t bytes) {
     b.ptr = nullptr;
     b.bytes = 0;
   }
-  if (injected_alloc_failure()) return fail(CYR_E_NOMEM, "injected device allocation failure (CYR_TEST_FAIL_ALLOC)");
+  if (injected_alloc_failure(bytes)) return fail(CYR_E_NOMEM, "injected device allocation failure (CYR_TEST_FAIL_ALLOC)");
   void *p = nullptr;
   hipError_t e = hipMalloc(&p, bytes);
   if (e != hipSuccess) {
