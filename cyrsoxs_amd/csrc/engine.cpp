@@ -294,6 +294,8 @@ cyr_status cyr_batch_create(uint32_t count, const cyr_sim_desc *descs, const voi
   // captured graph holds kernels and event edges only.  A member whose buffers do not fit
   // falls back to a smaller executor and frees those of its stream: the plan keeps that
   // executor, and the pass is repeated until every member runs the one it has.
+  BandMap bands;
+  for (auto &w : p.lanes.wb) w->bands = &bands;
   for (bool settled = false; !settled;) {
     std::vector<int32_t> ran(count, -1);
     CYR_TRY(queue_schedule(p.descs.data(), p.vox.data(), p.matp.data(), p.outs.data(), p.sched, p.lanes, p.cap,
@@ -311,6 +313,7 @@ cyr_status cyr_batch_create(uint32_t count, const cyr_sim_desc *descs, const voi
                                        p.cap);
   hipGraph_t g = nullptr;
   const hipError_t ce = hipStreamEndCapture(p.cap, &g);
+  for (auto &w : p.lanes.wb) w->bands = nullptr;
   if (qs != CYR_OK) {
     if (g) (void)hipGraphDestroy(g);
     return qs;

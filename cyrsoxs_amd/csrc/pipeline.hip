@@ -583,21 +583,15 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
 // [e0, e0 + ne) for k, by (grid, k, |k| list): known after one eager run, so graph
 // capture can size its launches.
 std::mutex g_band_mu;
-// per band geometry: widest band, sum of the band widths, columns inside the row
-// spans, D4 (no finite plane value beyond sqrt(D4) / 2 pixels of the centre)
-struct BandWidths {
-  uint32_t J;
-  uint64_t wsum, ssum, d4;
-};
-std::map<std::vector<double>, BandWidths> g_band_widths;
+BandMap g_band_widths;
 
 // Band table of energies [e0, e0 + ne) for k vector k into `band`, its widest band
 // in *J and the sum of the widths in *wsum (read back once per distinct geometry,
-// which waits for the stream; a stream under graph capture needs them cached by
-// an earlier run).
+// which waits for the stream; a stream under graph capture needs them known from an
+// earlier run: `own`, if not null, keeps every geometry that its plan meets).
 cyr_status mbasis_band(const cyr_sim_desc *d, const SimGeometry &g, uint32_t k, uint32_t e0, uint32_t ne,
                        const double *d_kmag, int32_t *band, uint32_t *bmax, hipStream_t s, uint32_t *J,
-                       uint64_t *wsum, uint64_t *ssum, uint64_t *d4) {
+                       uint64_t *wsum, uint64_t *ssum, uint64_t *d4, BandMap *own) {
   const double kv[3] = {g.kvec[k].x, g.kvec[k].y, g.kvec[k].z};
   const EwaldGeom geo = make_ewald_geom(g.nx, g.ny, g.nz, d->phys_size, g.kmag[e0], kv, d->interpolation);
   const double kmax = *std::max_element(g.kmag.begin() + e0, g.kmag.begin() + e0 + ne);
@@ -605,17 +599,21 @@ cyr_status mbasis_band(const cyr_sim_desc *d, const SimGeometry &g, uint32_t k, 
                              kv[0], kv[1], kv[2]};
   key.insert(key.end(), g.kmag.begin() + e0, g.kmag.begin() + e0 + ne);
   bool known = false;
-  {
+  auto look = [&](const BandMap &m) {
+    const auto it = m.find(key);
+    if (it == m.end()) return;
+    *J = it->second.J;
+    *wsum = it->second.wsum;
+    *ssum = it->second.ssum;
+    *d4 = it->second.d4;
+    known = true;
+  };
+  if (own) look(*own);
+  if (!known) {
     std::lock_guard<std::mutex> lk(g_band_mu);
-    auto it = g_band_widths.find(key);
-    if (it != g_band_widths.end()) {
-      *J = it->second.J;
-      *wsum = it->second.wsum;
-      *ssum = it->second.ssum;
-      *d4 = it->second.d4;
-      known = true;
-    }
+    look(g_band_widths);
   }
+  if (known && own) own->emplace(key, BandWidths{*J, *wsum, *ssum, *d4});
   if (known) return launch_mbasis_bands(geo, d_kmag + e0, ne, kmax, band, bmax, false, s);
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   CYR_HIP(hipStreamIsCapturing(s, &cap));
@@ -627,6 +625,7 @@ cyr_status mbasis_band(const cyr_sim_desc *d, const SimGeometry &g, uint32_t k, 
   CYR_HIP(hipStreamSynchronize(s));
   const BandWidths bw{h[0], (uint64_t)h[1] | ((uint64_t)h[2] << 32), (uint64_t)h[3] | ((uint64_t)h[4] << 32),
                       (uint64_t)h[5] | ((uint64_t)h[6] << 32)};
+  if (own) own->emplace(key, bw);
   std::lock_guard<std::mutex> lk(g_band_mu);
   if (g_band_widths.size() >= 4096) g_band_widths.clear();  // bounded: entries are cheap to recompute
   g_band_widths[key] = bw;
@@ -701,16 +700,31 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
       uint32_t ne = tensor ? 1 : g.nE - e0, J = 0;
       uint64_t wsum = 0;  // sum over columns of the band widths
       uint64_t ssum = 0;  // columns inside the row spans (those some band reads)
-      uint64_t d4 = 0;    // (2 x the largest distance of a finite plane value from the centre)^2
-      for (;;) {
+      double rfin = 0;    // no plane value farther from the centre is finite
+      if (tensor) {
+        // one energy's bands are its one or two bins wide, and its disc bounds the columns:
+        // nothing to read back (ssum, wsum: of the disc, for the timing labels)
+        const double kv[3] = {g.kvec[k].x, g.kvec[k].y, g.kvec[k].z};
+        const EwaldGeom geo = make_ewald_geom(g.nx, g.ny, g.nz, d->phys_size, g.kmag[e0], kv, d->interpolation);
+        J = (uint32_t)ng;
+        rfin = ewald_radius(geo);
+        ssum = (uint64_t)std::min((double)P, M_PI * (geo.k / geo.dx) * (geo.k / geo.dy));
+        wsum = ssum * J;
         kt_begin(s);
-        CYR_TRY(mbasis_band(d, g, k, e0, ne, su.kmag, band, bmax, s, &J, &wsum, &ssum, &d4));
+        CYR_TRY(launch_mbasis_bands(geo, su.kmag + e0, 1, g.kmag[e0], band, bmax, false, s));
         kt_end("mbasis_bands", s, (double)P * 4);
+      }
+      while (!tensor) {
+        uint64_t d4 = 0;  // (2 rfin)^2
+        kt_begin(s);
+        CYR_TRY(mbasis_band(d, g, k, e0, ne, su.kmag, band, bmax, s, &J, &wsum, &ssum, &d4, wb.bands));
+        kt_end("mbasis_bands", s, (double)P * 4);
+        rfin = 0.5 * std::sqrt((double)d4);
         if (J <= cap || ne == 1) break;
         ne = (ne + 1) / 2;
       }
       // columns that some band reads: bin x is the shifted column Nx/2 - x
-      const uint32_t reach = (uint32_t)std::min(0.5 * std::sqrt((double)d4) + 2.0, 4294967294.0);
+      const uint32_t reach = (uint32_t)std::min(rfin + 2.0, 4294967294.0);
       if (J == 0) J = 1;  // no pixel sampled: the angles kernel writes NaN only
       CYR_TRY(ensure_buffer(lb.part, sizeof(cx<T>) * planes * nvol * J * P));
       cx<T> *own = reinterpret_cast<cx<T> *>(lb.part.ptr);
@@ -811,7 +825,7 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
       if (lab) {
         // the pixels the rotation may read: a box about the disc of finite values, its
         // columns from a cache line's first record on
-        const double reach = 0.5 * std::sqrt((double)d4) + kQuadMargin + 1.0;
+        const double reach = rfin + kQuadMargin + 1.0;
         auto box = [&](uint32_t n, uint32_t &lo, uint32_t &len) {
           const double a = std::max(0.0, n / 2.0 - reach), b = std::min((double)n, std::ceil(n / 2.0 + reach) + 1.0);
           lo = (uint32_t)a / 16 * 16;
@@ -841,8 +855,7 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
           CYR_TRY(launch_rotate_quad<T>(proj, inv, su.quad + (size_t)3 * k * g.nA, su.quad_t + (size_t)3 * k * g.nA,
                                         g.nA, g.nx, g.ny, d->rot_mask, AvgSink<T>(avg, out, ostride, P, det), n,
                                         su.tiles, g.quarter, su.otiles,
-                                        quad_turns<T>(g, k, gmin), 0.5 * std::sqrt((double)d4), pol,
-                                        sizeof(cx<T>) * V * pass_max, s));
+                                        quad_turns<T>(g, k, gmin), rfin, pol, sizeof(cx<T>) * V * pass_max, s));
           kt_end("rotate_quad", s, n * ((double)kQuadRecord * P * sizeof(T) + 8.0 * P));
           CYR_TRY(launch_detector_warp<T>(avg, out, ostride, n, g.nx, g.ny, det, d->rot_mask, s));
         }
@@ -869,7 +882,7 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
           kt_end("mbasis_angles", s, (double)planes * nvol * (double)wsum * cxb + n * (double)g.nA * P * sizeof(T));
           kt_begin(s);
           CYR_TRY(launch_rotate_all<T>(pr, inv, g.nA, g.nx, g.ny, d->rot_mask, AvgSink<T>(bavg, out, ostride, P, det), n, su.tiles,
-                                       0.5 * std::sqrt((double)d4), s));
+                                       rfin, s));
           kt_end("rotate_all", s, n * (double)(g.nA + 1) * P * sizeof(T));
           CYR_TRY(launch_detector_warp<T>(bavg, out, ostride, n, g.nx, g.ny, det, d->rot_mask, s));
         }

@@ -2,6 +2,9 @@
 // device-resident inputs.
 #pragma once
 
+#include <map>
+#include <vector>
+
 #include "common.hpp"
 #include "host_math.hpp"
 
@@ -15,6 +18,14 @@ struct LaneBuffers {
   void release();
   size_t bytes() const;
 };
+
+// Material basis, per band geometry (the key): widest band, sum of the band widths, columns
+// inside the row spans, D4 (no finite plane value beyond sqrt(D4) / 2 pixels of the centre).
+struct BandWidths {
+  uint32_t J;
+  uint64_t wsum, ssum, d4;
+};
+using BandMap = std::map<std::vector<double>, BandWidths>;
 
 struct WorkBuffers {
   LaneBuffers lane[2];
@@ -31,6 +42,9 @@ struct WorkBuffers {
   // cap on the E-basis energy lanes for work queued through this object (the
   // batch executor runs members concurrently instead)
   uint32_t max_lanes = 2;
+  // while a batch plan is made: the band widths its capture will ask for (the process's own
+  // table of them is bounded)
+  BandMap *bands = nullptr;
   cyr_status ensure_aux();
   // Asynchronous host -> device copy of n bytes through the pinned staging.
   cyr_status upload(void *dst, const void *src, size_t n, hipStream_t st);

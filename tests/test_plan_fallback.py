@@ -1,5 +1,6 @@
-"""Captured plans whose members' own executors do not fit the device: the plan runs the
-executor that the eager call falls back to."""
+"""Captured plans: members whose own executors do not fit the device (the plan runs the
+executor that the eager call falls back to), and members of more units than the process
+keeps band widths for."""
 import numpy as np
 import pytest
 
@@ -47,5 +48,33 @@ def test_plan_falls_back_as_the_eager_call(case, monkeypatch):
             torch.cuda.synchronize()
             for o, r in zip(outs, (small_ref, ref, ref)):
                 np.testing.assert_array_equal(o.cpu().numpy(), r.cpu().numpy())
+    finally:
+        plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pipeline,prec,nE,nK", [(capi.PIPE_EBASIS, capi.FP64, 4200, 1), (capi.PIPE_MBASIS, capi.FP32, 1, 4200)])
+def test_plan_of_many_units(pipeline, prec, nE, nK):
+    """More than 4096 (energy, k vector) units in one plan: its replays equal the eager call."""
+    print(f"plan of many units pipeline={pipeline}", flush=True)
+    dims, M = (10, 8, 6), 2
+    dt = torch.float64 if prec == capi.FP64 else torch.float32
+    energies = list(np.linspace(280.0, 300.0, nE))
+    tilt = np.linspace(0.0, 0.05, nK)
+    kv = np.stack([np.sin(tilt), np.zeros(nK), np.cos(tilt)], axis=1) if nK > 1 else None
+    vox = torch.from_numpy(random_euler(dims, M, 15)).to(dt).cuda()
+    mats = random_constants(nE, M, 16)
+    sim = capi.Sim(dims, M, 3.0, energies, (0, 90, 90), precision=prec, pipeline=pipeline, interpolation=1,
+                   **({"kvectors": kv, "case_type": 1} if nK > 1 else {}))
+    assert sim.resolved_pipeline() == pipeline
+    ref, out = (torch.empty((nE, nK, dims[1], dims[0]), dtype=dt, device="cuda") for _ in range(2))
+    capi.simulate_device(sim, vox, mats, ref)
+    plan = capi.BatchPlan([sim], [vox], [mats], [out], lanes=1)
+    try:
+        for rep in range(2):
+            out.fill_(0.0)
+            plan.launch()
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(out.cpu().numpy(), ref.cpu().numpy())
     finally:
         plan.close()
