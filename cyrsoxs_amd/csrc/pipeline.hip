@@ -445,6 +445,24 @@ double ewald_radius(const EwaldGeom &g) {
   return std::hypot(cx, cy) + g.k / std::min(g.dx, g.dy) + 2.0;
 }
 
+// The streams of `lanes` (1 or 2) units in flight: st, and the second one, which starts after
+// what st holds; and the wait of st for it.
+cyr_status fork_lanes(WorkBuffers &wb, uint32_t lanes, hipStream_t st, hipStream_t (&lane_st)[2]) {
+  lane_st[0] = lane_st[1] = st;
+  if (lanes < 2) return CYR_OK;
+  CYR_TRY(wb.ensure_aux());
+  lane_st[1] = wb.aux;
+  CYR_HIP(hipEventRecord(wb.ev_fork, st));
+  CYR_HIP(hipStreamWaitEvent(wb.aux, wb.ev_fork, 0));
+  return CYR_OK;
+}
+cyr_status join_lanes(WorkBuffers &wb, uint32_t lanes, hipStream_t st) {
+  if (lanes < 2) return CYR_OK;
+  CYR_HIP(hipEventRecord(wb.ev_join, wb.aux));
+  CYR_HIP(hipStreamWaitEvent(st, wb.ev_join, 0));
+  return CYR_OK;
+}
+
 // EBASIS: per (energy, k) unit the five tensor fields, their XY transforms, the
 // z DFT at the Ewald bins, then every angle as 2D work.  With two lanes, unit u
 // runs on stream u % 2 with its own work buffers and starts once unit u-1's
@@ -474,13 +492,8 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
     CYR_TRY(ensure_buffer(lb.part, sizeof(cx<T>) * P * ng * kEbFields * yz.nchunks));
     CYR_TRY(ensure_buffer(lb.dc, sizeof(double2) * kEbFields * g.nz));
   }
-  hipStream_t lane_st[2] = {st, st};
-  if (lanes > 1) {
-    CYR_TRY(wb.ensure_aux());
-    lane_st[1] = wb.aux;
-    CYR_HIP(hipEventRecord(wb.ev_fork, st));
-    CYR_HIP(hipStreamWaitEvent(wb.aux, wb.ev_fork, 0));
-  }
+  hipStream_t lane_st[2];
+  CYR_TRY(fork_lanes(wb, lanes, st, lane_st));
   const double cxb = su.cxb;
   const double part_bytes = cxb * P * ng * kEbFields * yz.nchunks;
   for (uint32_t u = 0; u < units; u++) {
@@ -572,11 +585,7 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
     }
     CYR_TRY(launch_detector_warp<T>(avg, out, 0, 1, g.nx, g.ny, det, d->rot_mask, s));
   }
-  if (lanes > 1) {
-    CYR_HIP(hipEventRecord(wb.ev_join, wb.aux));
-    CYR_HIP(hipStreamWaitEvent(st, wb.ev_join, 0));
-  }
-  return CYR_OK;
+  return join_lanes(wb, lanes, st);
 }
 
 // Widest Ewald band and the sum of the columns' band widths over energies
@@ -662,7 +671,7 @@ uint32_t mbasis_band_cap(const SimGeometry &g) {
 // fields of one energy at a time (E-basis on grids that don't run the fused Y/z kernel).
 template <typename T>
 cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_vox, T *d_out, WorkBuffers &wb,
-                     hipStream_t s, const Setup<T> &su, bool tensor) {
+                     hipStream_t st, const Setup<T> &su, bool tensor) {
   const uint64_t V = g.V, P = g.P;
   const bool hann = d->windowing == 1 && d->algorithm != 1;
   const bool three = g.nz > 1;
@@ -672,31 +681,43 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
   // laboratory frame: one quadratic form per pixel instead of every angle's projection
   const bool lab = d->reference_frame != 0;
   const uint32_t nb = lab && !tensor ? std::min(mbasis_energy_batch(g, sizeof(T)), g.nE) : 1;
-  LaneBuffers &lb = wb.lane[0];
-  CYR_TRY(ensure_buffer(lb.pol, sizeof(cx<T>) * V * pass_max));
-  CYR_TRY(ensure_buffer(lb.proj, sizeof(T) * P * (lab ? 4 * (uint64_t)nb : g.nA)));
-  CYR_TRY(ensure_buffer(lb.avg, sizeof(double) * P * nb));
-  CYR_TRY(ensure_buffer(lb.bins, sizeof(int32_t) * P + sizeof(uint32_t) * mbasis_bmax_words(g.nx, g.ny)));
+  // units of the tensor fields, like run_ebasis', may be in flight two at a time
+  const uint32_t lanes = tensor && g.nE * g.nK > 1 ? std::min(energy_lanes(), wb.max_lanes) : 1;
   // DC-neighbour sums: taken by the Y pass when it runs on a compile-time plan
   // (dc_slots partials per z slice), else by their own kernel (one per slice)
   const uint32_t dc_slots = fft_dc_slots<T>(g.nx, g.ny);
   const uint64_t dc_per = (uint64_t)g.nz * (dc_slots ? dc_slots : 1);
-  CYR_TRY(ensure_buffer(lb.dc, sizeof(double2) * nvol * (dc_per + 1)));
-  cx<T> *pol = reinterpret_cast<cx<T> *>(lb.pol.ptr);
-  int32_t *band = reinterpret_cast<int32_t *>(lb.bins.ptr);
-  uint32_t *bmax = reinterpret_cast<uint32_t *>(band + P);
-  const uint32_t *span = mbasis_span_table(bmax, g.nx, g.ny);
-  double2 *dcz = reinterpret_cast<double2 *>(lb.dc.ptr);
-  double2 *dcv = dcz + (uint64_t)nvol * dc_per;
-  T *proj = reinterpret_cast<T *>(lb.proj.ptr);
-  double *avg = reinterpret_cast<double *>(lb.avg.ptr);
+  for (uint32_t L = 0; L < lanes; L++) {
+    LaneBuffers &lb = wb.lane[L];
+    CYR_TRY(ensure_buffer(lb.pol, sizeof(cx<T>) * V * pass_max));
+    CYR_TRY(ensure_buffer(lb.proj, sizeof(T) * P * (lab ? 4 * (uint64_t)nb : g.nA)));
+    CYR_TRY(ensure_buffer(lb.avg, sizeof(double) * P * nb));
+    CYR_TRY(ensure_buffer(lb.bins, sizeof(int32_t) * P + sizeof(uint32_t) * mbasis_bmax_words(g.nx, g.ny)));
+    CYR_TRY(ensure_buffer(lb.dc, sizeof(double2) * nvol * (dc_per + 1)));
+    if (tensor) CYR_TRY(ensure_buffer(lb.part, sizeof(cx<T>) * nvol * ng * P));
+  }
+  hipStream_t lane_st[2];
+  CYR_TRY(fork_lanes(wb, lanes, st, lane_st));
   const double cxb = su.cxb;
   const uint32_t cap = mbasis_band_cap(g);
   const double vel = d->storage == CYR_STORE_NATIVE ? (double)sizeof(T) : 2.0;
 
+  uint32_t unit = 0;
   for (uint32_t k = 0; k < g.nK; k++) {
     const M3 Q = ebasis_frame(g, k);
-    for (uint32_t e0 = 0; e0 < g.nE;) {
+    for (uint32_t e0 = 0; e0 < g.nE; unit++) {
+      const uint32_t L = unit % lanes;
+      hipStream_t s = lane_st[L];
+      LaneBuffers &lb = wb.lane[L];
+      cx<T> *pol = reinterpret_cast<cx<T> *>(lb.pol.ptr);
+      int32_t *band = reinterpret_cast<int32_t *>(lb.bins.ptr);
+      uint32_t *bmax = reinterpret_cast<uint32_t *>(band + P);
+      const uint32_t *span = mbasis_span_table(bmax, g.nx, g.ny);
+      double2 *dcz = reinterpret_cast<double2 *>(lb.dc.ptr);
+      double2 *dcv = dcz + (uint64_t)nvol * dc_per;
+      T *proj = reinterpret_cast<T *>(lb.proj.ptr);
+      double *avg = reinterpret_cast<double *>(lb.avg.ptr);
+      if (lanes > 1 && unit > 0) CYR_HIP(hipStreamWaitEvent(s, wb.ev_polx[(unit - 1) % lanes], 0));
       uint32_t ne = tensor ? 1 : g.nE - e0, J = 0;
       uint64_t wsum = 0;  // sum over columns of the band widths
       uint64_t ssum = 0;  // columns inside the row spans (those some band reads)
@@ -756,6 +777,7 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
         const auto launch_x = tensor ? launch_xfields<T, kXTensor> : pair ? launch_xfields<T, kXPair> : launch_xfields<T, kXSingle>;
         CYR_TRY(launch_x(xa, d_vox, d->storage, d->morphology_type, hann, s));
         kt_end("xfields", s, (tensor ? g.M : pair ? 2.0 : 1.0) * 4.0 * vel * V + nv * (double)V * cxb);
+        if (lanes > 1) CYR_HIP(hipEventRecord(wb.ev_polx[L], s));
         FftDc fdc{dcz + (uint64_t)vb * dc_per, su.twz, span, reach};
         if (!dc_slots) {
           DcArgs<T> da{};
@@ -890,7 +912,7 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
       e0 += ne;
     }
   }
-  return CYR_OK;
+  return join_lanes(wb, lanes, st);
 }
 
 template <typename T>
@@ -925,6 +947,7 @@ cyr_status run_impl(const cyr_sim_desc *d, const SimGeometry &g, const void *d_v
       cyr_sim_desc q = *d;
       for (int p; s == CYR_E_NOMEM && (p = smaller_pipeline(&q, g)) >= 0;) {
         CYR_HIP(hipStreamSynchronize(st));
+        if (wb.aux) CYR_HIP(hipStreamSynchronize(wb.aux));
         for (auto &l : wb.lane) l.release();
         q.pipeline = p;
         if (ran) *ran = p;
@@ -935,6 +958,7 @@ cyr_status run_impl(const cyr_sim_desc *d, const SimGeometry &g, const void *d_v
   if (mode != kRunSync) return s;
   // drain the stream on errors too, so no queued launch outlives the call's buffers
   const hipError_t se = hipStreamSynchronize(st);
+  if (s != CYR_OK && wb.aux) (void)hipStreamSynchronize(wb.aux);
   kt_collect();
   if (s != CYR_OK) return s;
   if (se != hipSuccess) return hip_fail(se, "hipStreamSynchronize", __FILE__, __LINE__);
@@ -1072,8 +1096,9 @@ uint64_t work_bytes(const cyr_sim_desc *d, const SimGeometry &g) {
     // run_bands over the tensor fields of one energy: volumes, its one or two band
     // rows (a column's own bin and its interpolation partner), tables, DC sums, planes
     const uint64_t planes = d->reference_frame != 0 ? 4 : g.nA;
-    b += cs * g.V * kEbFields + cs * 2 * kEbFields * g.P + 4 * g.P + 4 * mbasis_bmax_words(g.nx, g.ny) +
-         16 * kEbFields * (mbasis_dc_per(d, g) + 1) + rs * g.P * planes + 8 * g.P;
+    const uint64_t lanes = (uint64_t)g.nE * g.nK > 1 ? energy_lanes() : 1;
+    b += lanes * (cs * g.V * kEbFields + cs * 2 * kEbFields * g.P + 4 * g.P + 4 * mbasis_bmax_words(g.nx, g.ny) +
+                  16 * kEbFields * (mbasis_dc_per(d, g) + 1) + rs * g.P * planes + 8 * g.P);
   } else if (pipe == CYR_PIPE_MBASIS) {
     // one pass of packed volumes, band values (own + mirror, at most the band cap),
     // band table, DC sums, per-angle projections, average
