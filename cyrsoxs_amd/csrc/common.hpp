@@ -104,6 +104,8 @@ template <typename T> __device__ inline double tw_cos(const cx<T> *tw, uint32_t 
   if constexpr (sizeof(T) == 4) return (double)tw[e].x + (double)tw[n + e].x;
   else return (double)tw[e].x;
 }
+// A value in another precision.
+template <typename C, typename T> __device__ inline cx<C> cx_as(cx<T> v) { return mk<C>((C)v.x, (C)v.y); }
 // v * w^e from a table of length n (tw: hi block; the residual block follows at tw + n).
 template <typename T> __device__ inline cx<T> cmul_tw(cx<T> v, const cx<T> *tw, uint32_t n, uint32_t e) {
   if constexpr (sizeof(T) == 4) return cmul_comp<T>(v, tw[e], tw[n + e]);

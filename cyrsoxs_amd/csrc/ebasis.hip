@@ -454,7 +454,8 @@ bool fused_supported(uint32_t nx, uint32_t ny, uint32_t nz, int precision) {
   LfShape s;
   uint32_t e;
   if (!ct_usable(nx, precision) && !lf_x_shape(nx, precision, P, s, e)) return false;
-  if (!ct_usable(ny, precision) && !(lf_plan(ny, precision, false, P) && lf_cols_shape(P, precision, 16, s))) return false;
+  const int py = lf_precision(ny, precision);
+  if (!ct_usable(ny, precision) && !(lf_plan(ny, py, false, P) && lf_cols_shape(P, py, 16, s))) return false;
   return nz == 1 || mbasis_zband_supported(nz, precision);
 }
 

@@ -252,21 +252,22 @@ struct AnyShape {
 };
 
 // Inputs: of one column, or of the block's rows (rows past the last read the last).
-template <typename T, bool CONTIG> struct AnyIn {
+template <typename T, typename C, bool CONTIG> struct AnyIn {
   const cx<T> *gp;
   uint64_t es;     // columns: element stride; rows: row stride
   uint32_t rows;   // rows of this block
-  __device__ inline cx<T> load(uint32_t p, uint32_t e, uint32_t r, uint32_t q) const {
-    if constexpr (CONTIG) return gp[(uint64_t)(p < rows ? p : rows - 1) * es + e + r * q];
-    else return stream_load<T>(gp + e * es + r * (q * es));
+  __device__ inline cx<C> load(uint32_t p, uint32_t e, uint32_t r, uint32_t q) const {
+    if constexpr (CONTIG) return cx_as<C, T>(gp[(uint64_t)(p < rows ? p : rows - 1) * es + e + r * q]);
+    else return cx_as<C, T>(stream_load<T>(gp + e * es + r * (q * es)));
   }
 };
 
-// TAB: the tables are in LDS (false: the longest pencils, read from memory).
-template <typename T, bool CONTIG, bool TAB>
-__global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<T> tb, AnyShape sh, PassArgs A) {
+// TAB: the tables are in LDS (false: the longest pencils, read from memory).  C: the
+// precision of the arithmetic (lf_precision).
+template <typename T, typename C, bool CONTIG, bool TAB>
+__global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<C> tb, AnyShape sh, PassArgs A) {
   extern __shared__ unsigned char smem_raw[];
-  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw);
+  cx<C> *lds = reinterpret_cast<cx<C> *>(smem_raw);
   uint32_t t = 0, p = 0, tile = blockIdx.x, vol = blockIdx.y;
   if constexpr (!CONTIG) {
     const uint32_t q = xcd_tile(blockIdx.x, gridDim.x);
@@ -285,14 +286,14 @@ __global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<T> tb, AnyShape sh,
   // (idle pencils read pencil 0 and write nothing)
   cx<T> *gp = reinterpret_cast<cx<T> *>(A.vol[vol]) + (uint64_t)o * A.outer_stride +
               (uint64_t)(active ? pencil : 0) * A.inner_stride;
-  LfLds<T> tab{tb.tw, tb.pos};
-  cx<T> *after = lds + (CONTIG ? A.pp * sh.pitch : tb.m << sh.lpp);
+  LfLds<C> tab{tb.tw, tb.tw + tb.m, tb.pos};
+  cx<C> *after = lds + (CONTIG ? A.pp * sh.pitch : tb.m << sh.lpp);
   const uint32_t *span = A.span;
   if constexpr (TAB) {
-    tab = lf_stage_tables<T>(tb, after);
+    tab = lf_stage_tables<C, true>(tb, after);
     if (!CONTIG && A.span) {
       uint32_t *ls = reinterpret_cast<uint32_t *>(reinterpret_cast<unsigned char *>(after) +
-                                                  lf_lds_tables<T>(tb.m, tb.nlast));
+                                                  lf_lds_tables<C, true>(tb.m, tb.nlast));
       for (uint32_t i = threadIdx.x; i < tb.n; i += blockDim.x) ls[i] = A.span[i];
       span = ls;
     }
@@ -327,14 +328,14 @@ __global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<T> tb, AnyShape sh,
     }
   }
   const uint32_t rows = CONTIG ? (A.inner_count - g * A.pp < A.pp ? A.inner_count - g * A.pp : A.pp) : 1;
-  AnyIn<T, CONTIG> in{gp, CONTIG ? A.inner_stride : A.elem_stride, rows};
+  AnyIn<T, C, CONTIG> in{gp, CONTIG ? A.inner_stride : A.elem_stride, rows};
   // the line's shifted x range (see fft_ct_kernel)
   const uint32_t n = A.inner_count, m = n / 2;
   const uint32_t x0 = g * A.pp, x1 = (x0 + A.pp < n ? x0 + A.pp : n) - 1;
   const bool lo_part = x0 <= m, hi_part = x1 > m;
   const uint32_t a0 = m - (x1 < m ? x1 : m), a1 = m - x0;
   const uint32_t b0 = n + m - x1, b1 = n + m - (x0 > m + 1 ? x0 : m + 1);
-  auto out = [&](uint32_t row, uint32_t k0, uint32_t r, uint32_t dk, cx<T> v) {
+  auto out = [&](uint32_t row, uint32_t k0, uint32_t r, uint32_t dk, cx<C> v) {
     const uint32_t k = k0 + r * dk;
     bool keep = CONTIG ? row < rows : active;
     if constexpr (!CONTIG) {
@@ -344,12 +345,12 @@ __global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<T> tb, AnyShape sh,
       }
     }
     if (keep) {
-      if constexpr (CONTIG) gp[row * in.es + k] = v;
-      else gp[k0 * in.es + r * (dk * in.es)] = v;
+      if constexpr (CONTIG) gp[row * in.es + k] = cx_as<T, C>(v);
+      else gp[k0 * in.es + r * (dk * in.es)] = cx_as<T, C>(v);
     }
   };
-  if constexpr (CONTIG) lf_run<false, false, T>(tb, tab, lds, LfRows{sh.pitch, sh.pad, A.pp}, in, out);
-  else lf_run<false, false, T>(tb, tab, lds, LfCols{sh.lpp, p, t, sh.tpp}, in, out);
+  if constexpr (CONTIG) lf_run<false, false, true, C>(tb, tab, lds, LfRows{sh.pitch, sh.pad, A.pp}, in, out);
+  else lf_run<false, false, true, C>(tb, tab, lds, LfCols{sh.lpp, p, t, sh.tpp}, in, out);
 }
 
 // Direct O(n^2) DFT of each pencil for lengths beyond the any-length tile (e.g. a
@@ -529,30 +530,33 @@ bool radix_sequence(uint32_t n, uint32_t cap, std::vector<uint32_t> &out, double
   return !out.empty();
 }
 
-// Forward FFT of a host vector whose length is a product of small primes.
-void host_fft(std::vector<std::complex<double>> &x) {
+// The tables are formed in extended precision and rounded once (their entries' errors
+// would add to those of the arithmetic).
+using xcomplex = std::complex<long double>;
+constexpr long double kPiL = 3.14159265358979323846264338327950288L;
+
+// exp(-2 pi i k / n)
+xcomplex root_of(uint64_t k, uint64_t n) {
+  const long double a = -2 * kPiL * (long double)(k % n) / (long double)n;
+  return {std::cos(a), std::sin(a)};
+}
+
+// Forward FFT of a host vector whose length is a product of small primes (roots: those of
+// the whole transform, `step` apart for this length).
+void host_fft(std::vector<xcomplex> &x, const std::vector<xcomplex> &roots, size_t step) {
   const size_t n = x.size();
   if (n == 1) return;
   size_t p = 2;
   while (n % p != 0) p++;
   const size_t m = n / p;
-  std::vector<std::vector<std::complex<double>>> sub(p, std::vector<std::complex<double>>(m));
+  std::vector<std::vector<xcomplex>> sub(p, std::vector<xcomplex>(m));
   for (size_t i = 0; i < n; i++) sub[i % p][i / p] = x[i];
-  for (auto &v : sub) host_fft(v);
+  for (auto &v : sub) host_fft(v, roots, step * p);
   for (size_t k = 0; k < n; k++) {
-    std::complex<double> acc = 0;
-    for (size_t r = 0; r < p; r++) {
-      const double a = -2.0 * M_PI * (double)((r * k) % n) / (double)n;
-      acc += sub[r][k % m] * std::complex<double>(std::cos(a), std::sin(a));
-    }
+    xcomplex acc = 0;
+    for (size_t r = 0; r < p; r++) acc += sub[r][k % m] * roots[(r * k) % n * step];
     x[k] = acc;
   }
-}
-
-// exp(-i pi k^2 / n), the argument reduced exactly
-std::complex<double> chirp_of(uint64_t k, uint32_t n) {
-  const double a = -M_PI * (double)((k * k) % (2ull * n)) / (double)n;
-  return {std::cos(a), std::sin(a)};
 }
 
 size_t al64(size_t x) { return (x + 63) & ~(size_t)63; }
@@ -560,7 +564,7 @@ size_t al64(size_t x) { return (x + 63) & ~(size_t)63; }
 template <typename T> struct LfOffsets {
   size_t tw, chirp, spec, pos, total;  // (the stages come first)
   explicit LfOffsets(const LfPlan &P) {
-    const size_t cs = sizeof(cx<T>);
+    const size_t cs = sizeof(cx<T>) * tw_blocks<T>();  // (FP32: and the residuals)
     tw = al64(sizeof(P.st));
     chirp = tw + al64(cs * P.m);
     spec = chirp + (P.blue ? al64(cs * P.n) : 0);
@@ -574,11 +578,14 @@ template <typename T> std::vector<unsigned char> lf_host(const LfPlan &P) {
   const LfOffsets<T> o(P);
   std::vector<unsigned char> h(o.total, 0);
   std::memcpy(h.data(), P.st, sizeof(P.st));
+  // entry i of a table of n, and its residual
+  auto put = [](cx<T> *t, uint32_t n, uint32_t i, const xcomplex &c) {
+    t[i] = mk<T>((T)c.real(), (T)c.imag());
+    if (tw_blocks<T>() == 2)
+      t[n + i] = mk<T>((T)(c.real() - (long double)t[i].x), (T)(c.imag() - (long double)t[i].y));
+  };
   cx<T> *tw = reinterpret_cast<cx<T> *>(h.data() + o.tw);
-  for (uint32_t k = 0; k < P.m; k++) {
-    const double a = 2.0 * M_PI * (double)k / (double)P.m;
-    tw[k] = mk<T>((T)std::cos(a), (T)-std::sin(a));
-  }
+  for (uint32_t k = 0; k < P.m; k++) put(tw, P.m, k, root_of(k, P.m));
   uint16_t *pos = reinterpret_cast<uint16_t *>(h.data() + o.pos);
   for (uint32_t k = 0; k < P.m; k++) {
     uint32_t x = k, at = 0;
@@ -590,16 +597,16 @@ template <typename T> std::vector<unsigned char> lf_host(const LfPlan &P) {
   }
   if (P.blue) {
     cx<T> *ch = reinterpret_cast<cx<T> *>(h.data() + o.chirp), *sp = reinterpret_cast<cx<T> *>(h.data() + o.spec);
-    std::vector<std::complex<double>> b(P.m, 0.0);
+    std::vector<xcomplex> b(P.m, 0.0L), roots(P.m);
+    for (uint32_t k = 0; k < P.m; k++) roots[k] = root_of(k, P.m);
     for (uint32_t k = 0; k < P.n; k++) {
-      const std::complex<double> c = chirp_of(k, P.n);
-      ch[k] = mk<T>((T)c.real(), (T)c.imag());
+      const xcomplex c = root_of((uint64_t)k * k, 2ull * P.n);  // exp(-i pi k^2 / n)
+      put(ch, P.n, k, c);
       b[k] = std::conj(c);
       if (k) b[P.m - k] = std::conj(c);
     }
-    host_fft(b);
-    for (uint32_t k = 0; k < P.m; k++)
-      sp[pos[k]] = mk<T>((T)(b[k].real() / P.m), (T)(b[k].imag() / P.m));
+    host_fft(b, roots, 1);
+    for (uint32_t k = 0; k < P.m; k++) put(sp, P.m, pos[k], b[k] / (long double)P.m);
   }
   return h;
 }
@@ -660,6 +667,12 @@ bool lf_plan(uint32_t n, int precision, bool narrow, LfPlan &P) {
   }
   P = it->second;
   return P.n != 0;
+}
+
+int lf_precision(uint32_t n, int precision) {
+  LfPlan P;
+  return precision == CYR_FP32 && n < kLfShortConvolution && lf_plan(n, CYR_FP32, false, P) && P.blue ? CYR_FP64
+                                                                                                      : precision;
 }
 
 template <typename T> cyr_status lf_tables(const LfPlan &P, LfTab<T> &t) {
@@ -733,9 +746,11 @@ uint32_t lf_threads(const LfPlan &P, uint32_t unit, uint32_t pencils) {
   return pick;
 }
 
-size_t lf_tables_lds(const LfPlan &P, int precision) {
+// (comp: with the FP32 residuals of compensated products)
+size_t lf_tables_lds(const LfPlan &P, int precision, bool comp) {
   const uint32_t nlast = P.st[P.nst - 1].nb;
-  return precision == CYR_FP64 ? lf_lds_tables<double>(P.m, nlast) : lf_lds_tables<float>(P.m, nlast);
+  if (precision == CYR_FP64) return lf_lds_tables<double, true>(P.m, nlast);
+  return comp ? lf_lds_tables<float, true>(P.m, nlast) : lf_lds_tables<float, false>(P.m, nlast);
 }
 
 // Column tiles: max_cols adjacent pencils where three blocks of them (with room for a
@@ -747,7 +762,7 @@ bool lf_cols_shape(const LfPlan &P, int precision, uint32_t max_cols, LfShape &s
   for (uint32_t lpp = 6; lpp-- > 0;) {
     if (1u << lpp > max_cols) continue;
     const uint32_t pp = 1u << lpp;
-    const size_t tile = cs * ((size_t)P.m << lpp), with = tile + lf_tables_lds(P, precision) + 4 * (size_t)P.n;
+    const size_t tile = cs * ((size_t)P.m << lpp), with = tile + lf_tables_lds(P, precision, true) + 4 * (size_t)P.n;
     if (lpp > 2 && with > cap / 3) continue;
     if (lpp > 0 && with > cap) continue;
     const bool tables = with <= cap;
@@ -766,9 +781,10 @@ bool lf_cols_shape(const LfPlan &P, int precision, uint32_t max_cols, LfShape &s
 }
 
 // Rows: 2048 points of transforms for 256 threads, or, with e elements of a row per
-// thread, as many rows as 256 threads hold.
+// thread, as many rows as 256 threads hold (plain twiddle products).
 bool lf_rows_shape(const LfPlan &P, int precision, uint32_t e, bool need_tables, LfShape &s) {
-  const size_t cs = precision == CYR_FP64 ? 16 : 8, cap = max_lds_bytes(), tab = lf_tables_lds(P, precision);
+  const size_t cs = precision == CYR_FP64 ? 16 : 8, cap = max_lds_bytes();
+  const size_t tab = lf_tables_lds(P, precision, e == 0);
   s = LfShape{};
   s.tpp = e ? (P.n + e - 1) / e : 0;
   if (s.tpp > kLfRowThreads) return false;
@@ -794,11 +810,9 @@ cyr_status launch_any(uint32_t n, bool contig, uint32_t nc, PassArgs &A, hipStre
   LfPlan P;
   LfShape s;
   *done = false;
-  if (!lf_plan(n, prec_of<T>(), false, P)) return CYR_OK;
-  if (!(contig ? lf_rows_shape(P, prec_of<T>(), 0, false, s) : lf_cols_shape(P, prec_of<T>(), 16, s)))
-    return CYR_OK;
-  LfTab<T> tb;
-  CYR_TRY(lf_tables<T>(P, tb));
+  const int prec = lf_precision(n, prec_of<T>());
+  if (!lf_plan(n, prec, false, P)) return CYR_OK;
+  if (!(contig ? lf_rows_shape(P, prec, 0, false, s) : lf_cols_shape(P, prec, 16, s))) return CYR_OK;
   A.pp = s.pp;
   column_groups(A);
   A.nvol = nc;
@@ -807,11 +821,20 @@ cyr_status launch_any(uint32_t n, bool contig, uint32_t nc, PassArgs &A, hipStre
     return fail(CYR_E_UNSUPPORTED, "FFT grid too large");
   const AnyShape sh{s.tpp, s.lpp, s.pitch, s.pad};
   const dim3 block(s.threads), grid = contig ? dim3((unsigned)tiles, nc) : dim3(xcd_grid(tiles * nc));
-#define CYR_ANY(C, TB) hipLaunchKernelGGL((fft_any_kernel<T, C, TB>), grid, block, s.lds, st, tb, sh, A)
-  if (contig && s.tables) CYR_ANY(true, true);
-  else if (contig) CYR_ANY(true, false);
-  else if (s.tables) CYR_ANY(false, true);
-  else CYR_ANY(false, false);
+#define CYR_ANY(C, CT, TB) hipLaunchKernelGGL((fft_any_kernel<T, C, CT, TB>), grid, block, s.lds, st, tb, sh, A)
+  if (prec != prec_of<T>()) {  // (short: the tables are in LDS)
+    LfTab<double> tb;
+    CYR_TRY(lf_tables<double>(P, tb));
+    if (contig) CYR_ANY(double, true, true);
+    else CYR_ANY(double, false, true);
+  } else {
+    LfTab<T> tb;
+    CYR_TRY(lf_tables<T>(P, tb));
+    if (contig && s.tables) CYR_ANY(T, true, true);
+    else if (contig) CYR_ANY(T, true, false);
+    else if (s.tables) CYR_ANY(T, false, true);
+    else CYR_ANY(T, false, false);
+  }
 #undef CYR_ANY
   CYR_LAUNCHED();
   *done = true;
@@ -833,7 +856,8 @@ template <typename T> bool fft_span_fits(uint32_t n) {
   if (!strided_ct<T>(n)) {
     LfPlan P;
     LfShape s;
-    return lf_plan(n, prec_of<T>(), false, P) && lf_cols_shape(P, prec_of<T>(), 16, s);
+    const int prec = lf_precision(n, prec_of<T>());
+    return lf_plan(n, prec, false, P) && lf_cols_shape(P, prec, 16, s);
   }
   const uint32_t pp = n <= 512 ? 16 : (n == 1024 ? 8 : 4), wg = pp * (n / ct_elements(n));
   const bool lo = tw_lo_in_lds<T>((size_t)pp * n, n, wg);
@@ -850,7 +874,8 @@ template <typename T> uint32_t fft_dc_slots(uint32_t nx, uint32_t ny) {
   }
   LfPlan P;
   LfShape s;
-  return lf_plan(ny, prec_of<T>(), false, P) && lf_cols_shape(P, prec_of<T>(), 16, s) ? 3 * (s.pp * s.tpp / 64) : 0;
+  const int prec = lf_precision(ny, prec_of<T>());
+  return lf_plan(ny, prec, false, P) && lf_cols_shape(P, prec, 16, s) ? 3 * (s.pp * s.tpp / 64) : 0;
 }
 
 template <typename T>

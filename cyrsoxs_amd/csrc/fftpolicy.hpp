@@ -157,6 +157,7 @@ template <typename T, int N, int E, bool CONTIG, int PP, int... R> struct CtFft 
   static constexpr int R0 = FirstOf<R...>::value, RL = LastOf<R...>::value;
   static constexpr int PE = CONTIG ? 1 : PP;
   static constexpr bool kCt = true;
+  using Comp = T;  // precision of the arithmetic
   struct Plan {};
   __device__ explicit CtFft(const Plan &) {}
   __device__ static constexpr bool holds(uint32_t, int) { return true; }
@@ -182,12 +183,14 @@ template <typename T, int N, int E, bool CONTIG, int PP, int... R> struct CtFft 
 };
 
 // Any length (lfft.hpp), rows: slot i of thread t is element t + i tpp (E tpp >= n;
-// the last slots may be empty).  Plain twiddle products.
-template <typename T, int E, bool NARROW> struct LfRowFft {
+// the last slots may be empty).  Plain twiddle products but in convolutions.  C: precision of
+// the arithmetic (lf_precision).
+template <typename T, int E, bool NARROW, typename C = T> struct LfRowFft {
   static constexpr int kE = E;
   static constexpr bool kCt = false, kNarrow = NARROW;
+  using Comp = C;
   struct Plan {
-    LfTab<T> tb;
+    LfTab<C> tb;
     uint32_t tpp;    // threads per row
     uint32_t pitch;  // LDS elements per row
     uint32_t pad;    // one slot of padding per 2^pad elements
@@ -197,24 +200,25 @@ template <typename T, int E, bool NARROW> struct LfRowFft {
   __device__ uint32_t in_pos(uint32_t t, int i) const { return t + (uint32_t)i * P.tpp; }
   __device__ bool holds(uint32_t t, int i) const { return t + (uint32_t)i * P.tpp < P.tb.n; }
   // (the tables lie behind the rows: stage() copies them, a barrier must follow)
-  __device__ void stage(cx<T> *lds, uint32_t pp) const { lf_stage_tables<T>(P.tb, lds + pp * P.pitch); }
+  __device__ void stage(cx<C> *lds, uint32_t pp) const { lf_stage_tables<C, false>(P.tb, lds + pp * P.pitch); }
   template <class OUT>
-  __device__ void transform(cx<T> (&v)[E], uint32_t t, uint32_t p, uint32_t pp, cx<T> *lds, OUT out) const {
-    const cx<T> *tw = lds + pp * P.pitch;
-    const LfLds<T> tab{tw, reinterpret_cast<const uint16_t *>(tw + P.tb.m)};
+  __device__ void transform(cx<T> (&v)[E], uint32_t t, uint32_t p, uint32_t pp, cx<C> *lds, OUT out) const {
+    const cx<C> *tw = lds + pp * P.pitch;
+    const LfLds<C> tab{tw, P.tb.tw + P.tb.m, reinterpret_cast<const uint16_t *>(tw + P.tb.m)};
     const LfRows ad{P.pitch, P.pad, pp};
 #pragma unroll
     for (int i = 0; i < E; i++)
       if (holds(t, i)) {
         const uint32_t e = in_pos(t, i);
-        lds[ad.at(p, e)] = P.tb.blue ? cmul<T>(v[i], P.tb.chirp[e]) : v[i];
+        const cx<C> x = cx_as<C, T>(v[i]);
+        lds[ad.at(p, e)] = P.tb.blue ? cmul_tw<C>(x, P.tb.chirp, P.tb.n, e) : x;
       }
     if (P.tb.blue)
-      for (uint32_t e = P.tb.n + t; e < P.tb.m; e += P.tpp) lds[ad.at(p, e)] = mk<T>(0, 0);
+      for (uint32_t e = P.tb.n + t; e < P.tb.m; e += P.tpp) lds[ad.at(p, e)] = mk<C>(0, 0);
     lds_sync();
-    LfNoInput<T> in;
-    auto emit = [&](uint32_t row, uint32_t k, uint32_t r, uint32_t dk, cx<T> x) { out(row, k + r * dk, x); };
-    lf_run<true, NARROW, T>(P.tb, tab, lds, ad, in, emit);
+    LfNoInput<C> in;
+    auto emit = [&](uint32_t row, uint32_t k, uint32_t r, uint32_t dk, cx<C> x) { out(row, k + r * dk, cx_as<T, C>(x)); };
+    lf_run<true, NARROW, false, C>(P.tb, tab, lds, ad, in, emit);
     lds_sync();  // the rows may be refilled
   }
 };

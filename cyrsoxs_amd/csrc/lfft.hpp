@@ -57,7 +57,8 @@ struct LfPlan {
 };
 
 // Device tables of one length: W_m^k (k < m); pos[k], the slot of output k (uint16);
-// Bluestein: chirp c_n (n < N) and the chirp's spectrum / m by slot.
+// Bluestein: chirp c_n (n < N) and the chirp's spectrum / m by slot.  In FP32 each of the
+// three is followed by its rounding residuals (cmul_tw).
 template <typename T> struct LfTab {
   uint32_t n, m, blue, nst;  // of the plan
   uint32_t nlast;            // butterflies of the last stage: pos[k] below it are used
@@ -68,6 +69,15 @@ template <typename T> struct LfTab {
   const cx<T> *spec;
   const uint16_t *pos;
 };
+
+// The precision of the arithmetic of a length: FP64 for FP32 pencils of fewer than 128 points
+// that need a convolution.  There the direct sum of compensated products is closer than an
+// FP32 convolution, whose intermediate values carry the pencil's mean through every slot:
+// values about an offset, errors 2.0 (23 points), 1.6 (47) and 1.2 (101) times the sum's;
+// from 128 on it is the sum that is further off (211: 0.84, 499: 0.61).  In FP64 the error
+// is the result's own rounding (101 x 94 x 21, 4 energies: 131 -> 158 us).
+constexpr uint32_t kLfShortConvolution = 128;
+int lf_precision(uint32_t n, int precision);
 
 // Plan of a length (false: longer than the tile limit).  lf_tables builds its
 // tables once per device (or in the caller's scratch arena).
@@ -117,6 +127,8 @@ template <> struct PrimeRoots<13> {
 };
 
 // X_j, X_(P-j) = a_0 + sum_k cos(2 pi j k / P) (a_k + a_(P-k)) -/+ i sum_k sin(...) (a_k - a_(P-k))
+// (FP32, 13: constants with their rounding residuals, without which 13 points were 1.18 times
+// as far off as the direct sum; 7 and 11 are no further than that either way)
 template <typename T, int P> __device__ inline void bfly_prime(cx<T> *a) {
   constexpr int H = (P - 1) / 2;
   cx<T> t[H], d[H];
@@ -136,7 +148,15 @@ template <typename T, int P> __device__ inline void bfly_prime(cx<T> *a) {
       constexpr int k = decltype(kc)::value;
       constexpr int e = (j * k) % P;
       constexpr T c = (T)PrimeRoots<P>::c[(e <= H ? e : P - e) - 1];
-      constexpr T s = (T)(e <= H ? PrimeRoots<P>::s[e - 1] : -PrimeRoots<P>::s[P - e - 1]);
+      constexpr double sd = e <= H ? PrimeRoots<P>::s[e - 1] : -PrimeRoots<P>::s[P - e - 1];
+      constexpr T s = (T)sd;
+      if constexpr (sizeof(T) == 4 && P == 13) {
+        constexpr T cl = (T)(PrimeRoots<P>::c[(e <= H ? e : P - e) - 1] - (double)c), sl = (T)(sd - (double)s);
+        m.x += cl * t[k - 1].x;
+        m.y += cl * t[k - 1].y;
+        n.x += sl * d[k - 1].x;
+        n.y += sl * d[k - 1].y;
+      }
       m.x += c * t[k - 1].x;
       m.y += c * t[k - 1].y;
       n.x += s * d[k - 1].x;
@@ -147,13 +167,19 @@ template <typename T, int P> __device__ inline void bfly_prime(cx<T> *a) {
   });
 }
 
+// v (c + i s) with both constants' rounding residuals (FP32), as the table's finest products
+template <typename T> __device__ inline cx<T> cmul_const(cx<T> v, double c, double s) {
+  const cx<T> hi = mk<T>((T)c, (T)s);
+  return cmul_comp<T>(v, hi, mk<T>((T)(c - (double)hi.x), (T)(s - (double)hi.y)));
+}
+
 template <typename T> __device__ inline void bfly6(cx<T> *a) {
-  const T h = (T)0.5, r = (T)0.86602540378443864676372317075293618347;
+  constexpr double r = 0.86602540378443864676372317075293618347;
   cx<T> e[3] = {a[0], a[2], a[4]}, o[3] = {a[1], a[3], a[5]};
   bfly3<T>(e);
   bfly3<T>(o);
-  o[1] = mk<T>(h * o[1].x + r * o[1].y, h * o[1].y - r * o[1].x);   // (1/2, -sqrt3/2)
-  o[2] = mk<T>(-h * o[2].x + r * o[2].y, -h * o[2].y - r * o[2].x); // (-1/2, -sqrt3/2)
+  o[1] = cmul_const<T>(o[1], 0.5, -r);
+  o[2] = cmul_const<T>(o[2], -0.5, -r);
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     a[k] = cadd<T>(e[k], o[k]);
@@ -163,9 +189,9 @@ template <typename T> __device__ inline void bfly6(cx<T> *a) {
 
 template <typename T> __device__ inline void bfly9(cx<T> *a) {
   // W_9^1, W_9^2, W_9^4
-  const cx<T> w1 = mk<T>((T)0.76604444311897803520239265055542, (T)-0.64278760968653932632264340990726);
-  const cx<T> w2 = mk<T>((T)0.17364817766693034885171662676931, (T)-0.98480775301220805936674302458952);
-  const cx<T> w4 = mk<T>((T)-0.93969262078590838405410927732473, (T)-0.34202014332566873304409961468226);
+  constexpr double c1 = 0.76604444311897803520239265055542, s1 = -0.64278760968653932632264340990726;
+  constexpr double c2 = 0.17364817766693034885171662676931, s2 = -0.98480775301220805936674302458952;
+  constexpr double c4 = -0.93969262078590838405410927732473, s4 = -0.34202014332566873304409961468226;
   cx<T> c[3][3];
 #pragma unroll
   for (int n = 0; n < 3; n++) {
@@ -174,10 +200,10 @@ template <typename T> __device__ inline void bfly9(cx<T> *a) {
     c[n][2] = a[n + 6];
     bfly3<T>(c[n]);
   }
-  c[1][1] = cmul<T>(c[1][1], w1);
-  c[1][2] = cmul<T>(c[1][2], w2);
-  c[2][1] = cmul<T>(c[2][1], w2);
-  c[2][2] = cmul<T>(c[2][2], w4);
+  c[1][1] = cmul_const<T>(c[1][1], c1, s1);
+  c[1][2] = cmul_const<T>(c[1][2], c2, s2);
+  c[2][1] = cmul_const<T>(c[2][1], c2, s2);
+  c[2][2] = cmul_const<T>(c[2][2], c4, s4);
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     cx<T> v[3] = {c[0][k], c[1][k], c[2][k]};
@@ -190,15 +216,15 @@ template <typename T> __device__ inline void bfly9(cx<T> *a) {
 
 template <typename T> __device__ inline void bfly10(cx<T> *a) {
   // W_10^k = (cos 36k, -sin 36k)
-  const T c1 = (T)0.80901699437494742410229341718282, s1 = (T)0.58778525229247312916870595463907;
-  const T c2 = (T)0.30901699437494742410229341718282, s2 = (T)0.95105651629515357211643933337938;
+  constexpr double c1 = 0.80901699437494742410229341718282, s1 = 0.58778525229247312916870595463907;
+  constexpr double c2 = 0.30901699437494742410229341718282, s2 = 0.95105651629515357211643933337938;
   cx<T> e[5] = {a[0], a[2], a[4], a[6], a[8]}, o[5] = {a[1], a[3], a[5], a[7], a[9]};
   bfly5<T>(e);
   bfly5<T>(o);
-  o[1] = cmul<T>(o[1], mk<T>(c1, -s1));
-  o[2] = cmul<T>(o[2], mk<T>(c2, -s2));
-  o[3] = cmul<T>(o[3], mk<T>(-c2, -s2));
-  o[4] = cmul<T>(o[4], mk<T>(-c1, -s1));
+  o[1] = cmul_const<T>(o[1], c1, -s1);
+  o[2] = cmul_const<T>(o[2], c2, -s2);
+  o[3] = cmul_const<T>(o[3], -c2, -s2);
+  o[4] = cmul_const<T>(o[4], -c1, -s1);
 #pragma unroll
   for (int k = 0; k < 5; k++) {
     a[k] = cadd<T>(e[k], o[k]);
@@ -258,19 +284,24 @@ inline uint32_t lf_row_pitch(uint32_t m, uint32_t pad) { return m + (m >> pad) +
 // pointer that could be either LDS or memory would make every twiddle load a flat
 // one).
 template <typename T> struct LfLds {
-  const cx<T> *tw;
+  const cx<T> *tw, *lo;  // (lo: FP32 residuals)
   const uint16_t *pos;
 };
+// Twiddle entries a block keeps: with COMP, FP32 residuals too.
+template <typename T, bool COMP> __host__ __device__ constexpr uint32_t lf_lds_twiddles(uint32_t m) {
+  return COMP ? tw_len<T>(m) : m;
+}
 // LDS bytes of the tables.
-template <typename T> __host__ __device__ constexpr size_t lf_lds_tables(uint32_t m, uint32_t nlast) {
-  return sizeof(cx<T>) * m + ((sizeof(uint16_t) * nlast + 15) & ~(size_t)15);
+template <typename T, bool COMP> __host__ __device__ constexpr size_t lf_lds_tables(uint32_t m, uint32_t nlast) {
+  return sizeof(cx<T>) * lf_lds_twiddles<T, COMP>(m) + ((sizeof(uint16_t) * nlast + 15) & ~(size_t)15);
 }
 // Copies them to `at` (a barrier must follow).
-template <typename T> __device__ inline LfLds<T> lf_stage_tables(const LfTab<T> &P, cx<T> *at) {
-  uint16_t *pos = reinterpret_cast<uint16_t *>(at + P.m);
-  for (uint32_t i = threadIdx.x; i < P.m; i += blockDim.x) at[i] = P.tw[i];
+template <typename T, bool COMP> __device__ inline LfLds<T> lf_stage_tables(const LfTab<T> &P, cx<T> *at) {
+  const uint32_t n = lf_lds_twiddles<T, COMP>(P.m);
+  uint16_t *pos = reinterpret_cast<uint16_t *>(at + n);
+  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) at[i] = P.tw[i];
   for (uint32_t i = threadIdx.x; i < P.nlast; i += blockDim.x) pos[i] = P.pos[i];
-  return LfLds<T>{at, pos};
+  return LfLds<T>{at, (COMP ? at : P.tw) + P.m, pos};
 }
 
 // ---- stages -------------------------------------------------------------------------
@@ -283,7 +314,12 @@ enum LfRole : uint32_t {
 };
 
 // Stage S of the block's pencils.
-template <typename T, int R, class AD, class IN, class OUT>
+// FP32: the finest twiddles (those of the first forward stage and of its inverse), the chirp
+// and its spectrum are compensated products, as the finest of the codelets' passes are.  The
+// twiddles' residuals lie in LDS beside them (200 x 240 x 50, 12 energies: 491 us with plain
+// products, 522 with residuals read from L2 ahead of the butterfly, 511 from LDS).  COMP
+// false: only in convolutions, from memory.
+template <typename T, int R, bool COMP, class AD, class IN, class OUT>
 __device__ inline void lf_stage(const LfTab<T> &P, const LfStage &S, uint32_t role, const LfLds<T> &tab, cx<T> *buf,
                                 const AD &ad, IN &in, OUT &out) {
   const uint32_t q = S.q, count = ad.count(S);
@@ -311,7 +347,7 @@ __device__ inline void lf_stage(const LfTab<T> &P, const LfStage &S, uint32_t ro
 #pragma unroll
         for (int r = 0; r < R; r++) {
           const uint32_t e = e0 + r * q;
-          const cx<T> c = cmul<T>(v[r], P.chirp[e < P.n ? e : 0]);
+          const cx<T> c = cmul_tw<T>(v[r], P.chirp, P.n, e < P.n ? e : 0);
           v[r] = e < P.n ? c : mk<T>(0, 0);
         }
       }
@@ -320,9 +356,21 @@ __device__ inline void lf_stage(const LfTab<T> &P, const LfStage &S, uint32_t ro
       for (int r = 0; r < R; r++) v[r] = buf[ad.at(p, a0, e0, r, q)];
     }
     const uint32_t w = j * S.ts;
-    if ((role & kLfInv) && !last) {
+    auto twiddle = [&] {
 #pragma unroll
       for (int r = 1; r < R; r++) v[r] = cmul<T>(v[r], tab.tw[r * w]);
+    };
+    const bool comp = sizeof(T) == 4 && S.ts == 1 && (COMP || P.blue);  // (uniform)
+    auto twiddle_comp = [&] {
+      if constexpr (sizeof(T) == 4) {
+        const cx<T> *lo = COMP ? tab.lo : P.tw + P.m;
+#pragma unroll
+        for (int r = 1; r < R; r++) v[r] = cmul_comp<T>(v[r], tab.tw[r * w], lo[r * w]);
+      }
+    };
+    if ((role & kLfInv) && !last) {
+      if (comp) twiddle_comp();
+      else twiddle();
     }
     bfly_any<T, R>(v);
     if constexpr (R <= 10) {
@@ -331,22 +379,22 @@ __device__ inline void lf_stage(const LfTab<T> &P, const LfStage &S, uint32_t ro
         // forward butterflies give the inverse transform (swapped back at the end)
 #pragma unroll
         for (int r = 0; r < R; r++) {
-          const cx<T> u = cmul<T>(v[r], P.spec[e0 + r]);
+          const cx<T> u = cmul_tw<T>(v[r], P.spec, P.m, e0 + r);
           v[r] = mk<T>(u.y, u.x);
         }
         bfly_any<T, R>(v);
       }
     }
     if (!(role & kLfInv) && !last) {
-#pragma unroll
-      for (int r = 1; r < R; r++) v[r] = cmul<T>(v[r], tab.tw[r * w]);
+      if (comp) twiddle_comp();
+      else twiddle();
     }
     if (role & kLfOut) {
       if (role & kLfInv) {
 #pragma unroll
         for (int r = 0; r < R; r++) {
           const uint32_t k = e0 + r * q;
-          if (k < P.n) out(p, k, 0, 0, cmul<T>(mk<T>(v[r].y, v[r].x), P.chirp[k]));
+          if (k < P.n) out(p, k, 0, 0, cmul_tw<T>(mk<T>(v[r].y, v[r].x), P.chirp, P.n, k));
         }
       } else {
 #pragma unroll
@@ -359,24 +407,24 @@ __device__ inline void lf_stage(const LfTab<T> &P, const LfStage &S, uint32_t ro
   }
 }
 
-template <bool NARROW, typename T, class AD, class IN, class OUT>
+template <bool NARROW, bool COMP, typename T, class AD, class IN, class OUT>
 __device__ inline void lf_stage_any(const LfTab<T> &P, uint32_t s, uint32_t role, const LfLds<T> &tab, cx<T> *buf,
                                     const AD &ad, IN &in, OUT &out) {
   const LfStage S = P.st[s];
   // (uniform over the grid; FP64 butterflies of 11 and 13 would spill: those lengths run
   // Bluestein)
   switch (S.radix) {
-    case 2: lf_stage<T, 2>(P, S, role, tab, buf, ad, in, out); break;
-    case 3: lf_stage<T, 3>(P, S, role, tab, buf, ad, in, out); break;
-    case 4: lf_stage<T, 4>(P, S, role, tab, buf, ad, in, out); break;
-    case 5: lf_stage<T, 5>(P, S, role, tab, buf, ad, in, out); break;
-    case 6: lf_stage<T, 6>(P, S, role, tab, buf, ad, in, out); break;
-    case 7: lf_stage<T, 7>(P, S, role, tab, buf, ad, in, out); break;
-    case 8: lf_stage<T, 8>(P, S, role, tab, buf, ad, in, out); break;
-    case 9: if constexpr (!NARROW) lf_stage<T, 9>(P, S, role, tab, buf, ad, in, out); break;
-    case 10: if constexpr (!NARROW) lf_stage<T, 10>(P, S, role, tab, buf, ad, in, out); break;
-    case 11: if constexpr (!NARROW && sizeof(T) == 4) lf_stage<T, 11>(P, S, role, tab, buf, ad, in, out); break;
-    default: if constexpr (!NARROW && sizeof(T) == 4) lf_stage<T, 13>(P, S, role, tab, buf, ad, in, out); break;
+    case 2: lf_stage<T, 2, COMP>(P, S, role, tab, buf, ad, in, out); break;
+    case 3: lf_stage<T, 3, COMP>(P, S, role, tab, buf, ad, in, out); break;
+    case 4: lf_stage<T, 4, COMP>(P, S, role, tab, buf, ad, in, out); break;
+    case 5: lf_stage<T, 5, COMP>(P, S, role, tab, buf, ad, in, out); break;
+    case 6: lf_stage<T, 6, COMP>(P, S, role, tab, buf, ad, in, out); break;
+    case 7: lf_stage<T, 7, COMP>(P, S, role, tab, buf, ad, in, out); break;
+    case 8: lf_stage<T, 8, COMP>(P, S, role, tab, buf, ad, in, out); break;
+    case 9: if constexpr (!NARROW) lf_stage<T, 9, COMP>(P, S, role, tab, buf, ad, in, out); break;
+    case 10: if constexpr (!NARROW) lf_stage<T, 10, COMP>(P, S, role, tab, buf, ad, in, out); break;
+    case 11: if constexpr (!NARROW && sizeof(T) == 4) lf_stage<T, 11, COMP>(P, S, role, tab, buf, ad, in, out); break;
+    default: if constexpr (!NARROW && sizeof(T) == 4) lf_stage<T, 13, COMP>(P, S, role, tab, buf, ad, in, out); break;
   }
 }
 
@@ -388,16 +436,16 @@ template <typename T> struct LfNoInput {
 // Transforms the block's pencils: in.load(p, e0, r, q) gives input e0 + r q < n of pencil
 // p, out(p, k0, r, dk, v) takes its output k0 + r dk (q and dk uniform: addresses step by
 // scalars).  FROM_LDS: the inputs are already stored in LDS, behind a barrier (Bluestein:
-// times the chirp, zeros from n on).  NARROW: a narrow plan.  Every thread of the block
+// times the chirp, zeros from n on).  NARROW: a narrow plan.  COMP: see lf_stage.  Every thread of the block
 // calls it; barriers separate the stages, none follows the last.
-template <bool FROM_LDS, bool NARROW, typename T, class AD, class IN, class OUT>
+template <bool FROM_LDS, bool NARROW, bool COMP, typename T, class AD, class IN, class OUT>
 __device__ inline void lf_run(const LfTab<T> &P, const LfLds<T> &tab, cx<T> *buf, const AD &ad, IN &in, OUT &out) {
   const uint32_t steps = P.blue ? 2 * P.nst - 1 : P.nst;
 #pragma unroll 1
   for (uint32_t i = 0; i < steps; i++) {
     uint32_t role = (!FROM_LDS && i == 0 ? kLfIn : 0) | (i + 1 == steps ? kLfOut : 0);
     if (P.blue) role |= i + 1 == P.nst ? kLfMid : i >= P.nst ? kLfInv : 0;
-    lf_stage_any<NARROW, T>(P, i < P.nst ? i : steps - 1 - i, role, tab, buf, ad, in, out);
+    lf_stage_any<NARROW, COMP, T>(P, i < P.nst ? i : steps - 1 - i, role, tab, buf, ad, in, out);
     if (i + 1 < steps) lds_sync();
   }
 }

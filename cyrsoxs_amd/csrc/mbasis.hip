@@ -368,12 +368,13 @@ hipError_t launch_zband_n(const BandArgs<T> &a, hipStream_t st, const cx<T> *tw)
 
 // The same for any length (lfft.hpp): the first stage loads the column's elements, the
 // last hands its outputs to the band test, so nothing but the band values leaves.
-// TAB: the tables are in LDS (false: the longest pencils, read from memory).
-template <typename T, bool TAB>
-__global__ void __launch_bounds__(1024) mbasis_zband_any_kernel(LfTab<T> tb, uint32_t tpp, uint32_t lpp,
+// TAB: the tables are in LDS (false: the longest pencils, read from memory).  C: the
+// precision of the arithmetic (lf_precision).
+template <typename T, typename C, bool TAB>
+__global__ void __launch_bounds__(1024) mbasis_zband_any_kernel(LfTab<C> tb, uint32_t tpp, uint32_t lpp,
                                                                 BandArgs<T> a) {
   extern __shared__ unsigned char smem_raw[];
-  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw);
+  cx<C> *lds = reinterpret_cast<cx<C> *>(smem_raw);
   const uint32_t PP = 1u << lpp, groups = (a.nx + PP - 1) >> lpp, per_vol = groups * a.ny;
   const uint32_t qb = xcd_chunk_tile(blockIdx.x, kZbandChunk);  // (as mbasis_zband_kernel)
   if (qb < a.count) {
@@ -403,9 +404,9 @@ __global__ void __launch_bounds__(1024) mbasis_zband_any_kernel(LfTab<T> tb, uin
   const uint32_t lom = bm & 0xffffu, wm = a.mir ? bm >> 16 : 0;
   cx<T> *own = a.own + (uint64_t)(a.vbase + v) * a.J * P + col;
   cx<T> *mir = a.mir + (uint64_t)(a.vbase + v) * a.J * P + cm;
-  LfLds<T> tab{tb.tw, tb.pos};
+  LfLds<C> tab{tb.tw, tb.tw + tb.m, tb.pos};
   if constexpr (TAB) {
-    tab = lf_stage_tables<T>(tb, lds + ((size_t)tb.m << lpp));
+    tab = lf_stage_tables<C, true>(tb, lds + ((size_t)tb.m << lpp));
     lds_sync();
   }
   const uint32_t N = a.nz;
@@ -414,34 +415,41 @@ __global__ void __launch_bounds__(1024) mbasis_zband_any_kernel(LfTab<T> tb, uin
     const cx<T> *base;
     uint64_t P;
     bool need;
-    __device__ cx<T> load(uint32_t, uint32_t e, uint32_t r, uint32_t q) const {
-      return need ? base[(uint64_t)e * P + r * (q * P)] : mk<T>(0, 0);
+    __device__ cx<C> load(uint32_t, uint32_t e, uint32_t r, uint32_t q) const {
+      return need ? cx_as<C, T>(base[(uint64_t)e * P + r * (q * P)]) : mk<C>(0, 0);
     }
   } in{base, P, need};
-  auto out = [&](uint32_t, uint32_t k0, uint32_t ks, uint32_t dk, cx<T> r) {
+  auto out = [&](uint32_t, uint32_t k0, uint32_t ks, uint32_t dk, cx<C> x) {
+    const cx<T> r = cx_as<T, C>(x);
     const uint32_t kz = k0 + ks * dk;
     const uint32_t j = unshift(kz, N) - lo;  // wraps above w when below the band
     if (j < w) own[(uint64_t)j * P] = r;
     const uint32_t jm = unshift(kz ? N - kz : 0, N) - lom;
     if (jm < wm) mir[(uint64_t)jm * P] = r;
   };
-  lf_run<false, false, T>(tb, tab, lds, LfCols{lpp, p, t, tpp}, in, out);
+  lf_run<false, false, true, C>(tb, tab, lds, LfCols{lpp, p, t, tpp}, in, out);
 }
 
 // Up to 32 columns.
 template <typename T> cyr_status launch_zband_any(const BandArgs<T> &a, hipStream_t st) {
-  const int prec = sizeof(T) == 8 ? CYR_FP64 : CYR_FP32;
+  const int native = sizeof(T) == 8 ? CYR_FP64 : CYR_FP32, prec = lf_precision(a.nz, native);
   LfPlan P;
   LfShape s;
   if (!lf_plan(a.nz, prec, false, P) || !lf_cols_shape(P, prec, 32, s))
     return fail(CYR_E_UNSUPPORTED, "Z band pass: length beyond the tile");
-  LfTab<T> tb;
-  CYR_TRY(lf_tables<T>(P, tb));
   const uint64_t tiles = (uint64_t)((a.nx + s.pp - 1) / s.pp) * a.ny * a.count;
   if (tiles > 0x7ffffff0ull) return fail(CYR_E_UNSUPPORTED, "Z band pass: grid too large");
   const dim3 grid(xcd_chunk_grid(tiles + a.count, kZbandChunk)), block(s.pp * s.tpp);
-  if (s.tables) hipLaunchKernelGGL((mbasis_zband_any_kernel<T, true>), grid, block, s.lds, st, tb, s.tpp, s.lpp, a);
-  else hipLaunchKernelGGL((mbasis_zband_any_kernel<T, false>), grid, block, s.lds, st, tb, s.tpp, s.lpp, a);
+  if (prec != native) {  // (short: the tables are in LDS)
+    LfTab<double> tb;
+    CYR_TRY(lf_tables<double>(P, tb));
+    hipLaunchKernelGGL((mbasis_zband_any_kernel<T, double, true>), grid, block, s.lds, st, tb, s.tpp, s.lpp, a);
+  } else {
+    LfTab<T> tb;
+    CYR_TRY(lf_tables<T>(P, tb));
+    if (s.tables) hipLaunchKernelGGL((mbasis_zband_any_kernel<T, T, true>), grid, block, s.lds, st, tb, s.tpp, s.lpp, a);
+    else hipLaunchKernelGGL((mbasis_zband_any_kernel<T, T, false>), grid, block, s.lds, st, tb, s.tpp, s.lpp, a);
+  }
   CYR_LAUNCHED();
   return CYR_OK;
 }
@@ -799,6 +807,7 @@ bool mbasis_zband_supported(uint32_t nz, int precision) {
   if (precision == CYR_FP64 ? zband_ct<double>(nz) : zband_ct<float>(nz)) return true;
   LfPlan P;
   LfShape s;
+  precision = lf_precision(nz, precision);
   return lf_plan(nz, precision, false, P) && lf_cols_shape(P, precision, 32, s);
 }
 

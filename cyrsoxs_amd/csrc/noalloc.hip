@@ -14,16 +14,22 @@
 
 #include "common.hpp"
 #include "fft.hpp"
+#include "lfft.hpp"
 #include "host_math.hpp"
 #include "pipeline.hpp"
 
 namespace cyr {
 namespace {
 
-// The array also holds the any-length transforms' tables (at most three lengths, of
-// 8 complex values and 2 bytes per point of a convolution up to 16384 points), so that
-// they take nothing from the documented size.
+// The array also holds the any-length transforms' tables, so that they take nothing from
+// the documented size: at most three lengths, each of 16 bytes (FP64 entries, or FP32 ones
+// with their residuals) for the twiddles and the spectrum of a convolution of m points and
+// for the chirp of fewer than m / 2 + 1, 2 bytes of digit reversal a point, and the stages.
 constexpr size_t kTableBytes = 3u * 1024u * 1024u;
+static_assert(3 * (16 * (size_t)(2 * kLfMaxConvolution + kLfMaxConvolution / 2 + 1) + 2 * kLfMaxConvolution + 1024) <=
+                      kTableBytes &&
+                  3 * (18 * (size_t)kLfMaxLength + 1024) <= kTableBytes,
+              "the tables of three lengths must fit");
 constexpr size_t kScratchBytes = CYR_NOALLOC_SCRATCH_BYTES + kTableBytes;
 static_assert(kScratchBytes % 256 == 0, "scratch size must keep 256-byte alignment");
 

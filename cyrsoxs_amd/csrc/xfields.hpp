@@ -168,7 +168,7 @@ __device__ inline void voxel_fields(const S *__restrict__ vox, const PolxArgs<T>
 // barriers and want all that fit without spilling.
 template <typename T, class F, int MODE> constexpr int x_min_waves() {
   if constexpr (F::kCt) return MODE == kXTensor && F::kE <= 8 ? 4 : 2;
-  else return sizeof(T) == 8 ? (F::kE <= 2 ? 3 : 2) : F::kNarrow && F::kE <= 4 ? 4 : 2;
+  else return sizeof(T) == 8 ? (F::kE <= 2 ? 3 : 2) : F::kNarrow && F::kE <= 4 && sizeof(typename F::Comp) == 4 ? 4 : 2;
 }
 
 // ---- fields + X FFT --------------------------------------------------------------
@@ -177,7 +177,7 @@ __global__ void __launch_bounds__(WG, (x_min_waves<T, F, MODE>()))
     xfields_kernel(typename F::Plan plan, PolxArgs<T> a, const S *__restrict__ vox, int morph, int hann) {
   constexpr int E = F::kE, NO = x_outputs<MODE>();
   extern __shared__ unsigned char smem_raw[];
-  cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw);
+  auto *lds = reinterpret_cast<cx<typename F::Comp> *>(smem_raw);
   const F fft(plan);
   const uint32_t tpp = a.tpp;
   const uint32_t t = threadIdx.x % tpp, p = threadIdx.x / tpp;
@@ -366,10 +366,12 @@ constexpr int ct_polx_wg(int N, int E) { return N / E <= 64 ? 64 : N / E; }
 // SIMD, where radices up to 13 took 182 (200 x 240 x 50, 3 materials: 109 -> 84 us per
 // volume; 101 x 94 x 21: 58 -> 37 us).  Lengths with factors 11 and 13 would be
 // Bluestein's in a narrow plan, so those keep the wide one in FP32 (156 x 156 x 64, 4
-// materials: 183 us per volume by Bluestein, 98 so).
+// materials: 183 us per volume by Bluestein, 98 so).  Short convolutions: narrow FP64 plans.
 constexpr uint64_t kXSplitThreads = 256 * 512;  // two waves per SIMD
 inline bool lf_x_shape(uint32_t n, int precision, LfPlan &P, LfShape &s, uint32_t &e) {
   e = precision == CYR_FP64 ? 2 : 4;
+  if (lf_precision(n, precision) != precision)
+    return lf_plan(n, CYR_FP64, true, P) && lf_rows_shape(P, CYR_FP64, e, true, s);
   const bool fits = lf_plan(n, precision, true, P);
   if (precision == CYR_FP32 && fits && P.blue) {
     LfPlan W;
@@ -399,10 +401,10 @@ template <typename T, int MODE> uint32_t x_split(uint64_t blocks, uint32_t threa
   return sizeof(T) == 4 && blocks * threads < kXSplitThreads ? (uint32_t)x_outputs<MODE>() : 1;
 }
 
-template <typename T, typename S, int E, bool NARROW, int MODE>
-hipError_t launch_xfields_lf(const LfTab<T> &tb, const LfShape &sh, hipStream_t st, const PolxArgs<T> &a,
+template <typename T, typename S, int E, bool NARROW, int MODE, typename C>
+hipError_t launch_xfields_lf(const LfTab<C> &tb, const LfShape &sh, hipStream_t st, const PolxArgs<T> &a,
                              const void *vox, int morph, int hann) {
-  using F = LfRowFft<T, E, NARROW>;
+  using F = LfRowFft<T, E, NARROW, C>;
   const typename F::Plan plan{tb, sh.tpp, sh.pitch, sh.pad};
   hipLaunchKernelGGL((xfields_kernel<T, S, F, kLfRowThreads, MODE>),
                      dim3(ceil_div(a.rows, sh.pp), x_split<T, MODE>(ceil_div(a.rows, sh.pp), sh.pp * sh.tpp)),
@@ -447,9 +449,11 @@ cyr_status launch_xfields(PolxArgs<T> a, const void *vox, int storage, int morph
   const int prec = sizeof(T) == 8 ? CYR_FP64 : CYR_FP32;
   const bool ct = ct_usable(a.nx, prec);
   LfTab<T> tb{};
+  LfTab<double> tb64{};
   LfShape sh;
   uint32_t e_lf = 0;
   bool narrow = true;
+  const bool conv64 = !ct && lf_precision(a.nx, prec) != prec;
   size_t lds = 0;
   if (ct) {
     // rows of <= 64 threads share one wave
@@ -465,7 +469,8 @@ cyr_status launch_xfields(PolxArgs<T> a, const void *vox, int storage, int morph
     if (!lf_x_shape(a.nx, prec, P, sh, e_lf))
       return fail(CYR_E_UNSUPPORTED, "fused X kernel: row does not fit its block");
     narrow = P.narrow;
-    CYR_TRY(lf_tables<T>(P, tb));
+    if (conv64) CYR_TRY(lf_tables<double>(P, tb64));
+    else CYR_TRY(lf_tables<T>(P, tb));
     a.tpp = sh.tpp;
     a.pp = sh.pp;
   }
@@ -476,7 +481,9 @@ cyr_status launch_xfields(PolxArgs<T> a, const void *vox, int storage, int morph
   auto go = [&](auto tag) {
     using S = decltype(tag);
     if (ct) e = launch_xfields_ct_n<T, S, MODE>(a.nx, grid, lds, st, a, vox, morph, hann ? 1 : 0, &found);
-    else if (!narrow) {
+    else if (conv64) {
+      if constexpr (sizeof(T) == 4) e = launch_xfields_lf<T, S, E0, true, MODE>(tb64, sh, st, a, vox, morph, hann ? 1 : 0);
+    } else if (!narrow) {
       if constexpr (sizeof(T) == 4) e = launch_xfields_lf<T, S, E0, false, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
     } else if (e_lf == E0) e = launch_xfields_lf<T, S, E0, true, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
     else if (e_lf == 2 * E0) e = launch_xfields_lf<T, S, 2 * E0, true, MODE>(tb, sh, st, a, vox, morph, hann ? 1 : 0);
