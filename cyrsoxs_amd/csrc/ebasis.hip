@@ -220,7 +220,7 @@ __global__ void __launch_bounds__(256) ebasis_dc_kernel(DcArgs<T> a) {
 // of the block calls it (barriers inside).
 template <typename T, int NG>
 __device__ inline bool eb_fields(const AnglesArgs<T> &a, uint64_t t, uint32_t &X, uint32_t &Y,
-                                 cx<T> (&F)[NG][kEbFields], double (&md)[NG][6], T &w1) {
+                                 cx<T> (&F)[NG][kEbFields], double (&md)[NG][6], double &w1) {
   const EwaldGeom &g = a.g;
   const uint64_t P2 = (uint64_t)g.nx * g.ny;
   // the block holding the pixel of FFT bin (0, 0) (X = Nx/2, Y = Ny/2) first sums
@@ -286,30 +286,33 @@ __device__ inline bool eb_fields(const AnglesArgs<T> &a, uint64_t t, uint32_t &X
   }
 #pragma unroll
   for (int q = 0; q < NG; q++) scatter_matrix(g, X, Y, three ? z0 + q : 0, md[q]);
-  w1 = (T)f;
+  w1 = f;
   return true;
 }
 
 // ---- laboratory frame: the quadratic form ------------------------------------------
-// One record per pixel (12 B) in place of every angle's projection written here and
-// gathered again by the rotation (4 B per pixel and angle each way): one energy of
-// 256^2 x 64 with 36 angles, 47 + 33 us for the two kernels.
+// One record per pixel (24 B) in place of every angle's projection written here and
+// gathered again by the rotation (4 B per pixel and angle each way).  The forms and what is
+// sampled from them are FP64 in FP32 runs too: an angle's intensity is a sum of squares, so
+// its own projection has a few roundings of itself, while the form's three terms cancel
+// where it is small; and the angles' sums then carry no roundings of weights and taps.
+// One energy of 256^2 x 64 with 36 angles: the two kernels 47 + 33 us by angle, 14 + 26 us so.
 template <typename T, int NG>
 __global__ void __launch_bounds__(256) ebasis_quad_kernel(AnglesArgs<T> a) {
   const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t X, Y;
   cx<T> F[NG][kEbFields];
   double md[NG][6];
-  T w1;
+  double w1;
   const bool fine = eb_fields<T, NG>(a, t, X, Y, F, md, w1);
   if (t >= (uint64_t)a.g.nx * a.g.ny) return;
   if (!fine) {
     Y = (uint32_t)(t / a.g.nx);
     X = (uint32_t)(t - (uint64_t)Y * a.g.nx);
   }
-  T *o = a.quad + (uint64_t)quad_index(X, Y, a.g.nx, a.g.ny) * kQuadRecord;
-  if (!fine) o[0] = o[1] = o[2] = qnan<T>();
-  else quad_form_write<T, NG>(a.Q, F, md, w1, o);
+  double *o = a.quad + (uint64_t)quad_index(X, Y, a.g.nx, a.g.ny) * kQuadRecord;
+  if (!fine) o[0] = o[1] = o[2] = qnan<double>();
+  else quad_form_write<double, T, NG>(a.Q, F, md, w1, o);
 }
 
 // ---- material frame: every angle's intensity ----------------------------------------
@@ -320,7 +323,7 @@ __global__ void __launch_bounds__(256) ebasis_angles_kernel(AnglesArgs<T> a) {
   uint32_t X, Y;
   cx<T> F[NG][kEbFields];
   double md[NG][6];
-  T w1;
+  double w1;
   const bool fine = eb_fields<T, NG>(a, t, X, Y, F, md, w1);
   if (t >= P2) return;
   if (!fine) {
@@ -347,7 +350,7 @@ __global__ void __launch_bounds__(256) ebasis_angles_kernel(AnglesArgs<T> a) {
       I[q] = scatter_intensity<T>(md[q], pv);
     }
     T out;
-    if constexpr (NG == 2) out = (1 - w1) * I[0] + w1 * I[1];
+    if constexpr (NG == 2) out = (1 - (T)w1) * I[0] + (T)w1 * I[1];
     else out = I[0];
     a.proj[(uint64_t)an * P2 + t] = out;
   }
@@ -529,7 +532,7 @@ template <typename T> cyr_status launch_ebasis_dc(const DcArgs<T> &a, hipStream_
 template <typename T> cyr_status launch_ebasis_angles(const AnglesArgs<T> &a, int ng, hipStream_t st) {
   const uint64_t P = (uint64_t)a.g.nx * a.g.ny;
   const dim3 grid(ceil_div(P, 256)), block(256);
-  if (a.quad) {
+  if (a.quad) {  // (laboratory frame)
     if (ng == 2) hipLaunchKernelGGL((ebasis_quad_kernel<T, 2>), grid, block, 0, st, a);
     else hipLaunchKernelGGL((ebasis_quad_kernel<T, 1>), grid, block, 0, st, a);
   } else if (ng == 2) {

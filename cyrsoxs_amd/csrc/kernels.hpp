@@ -143,8 +143,8 @@ template <typename T> struct AnglesArgs {
   const T *amat;                   // [nA][kEbAmat]
   uint32_t nA;
   T *proj;                         // [nA][Ny][Nx] (material frame), or
-  T *quad;                         // [P][3] in quad_index order (laboratory frame)
-  Mat3<T> Q;                       // frame e1, e2, k^ (quadratic form)
+  double *quad;                    // [P][3] in quad_index order (laboratory frame)
+  Mat3<double> Q;                  // frame e1, e2, k^ (quadratic form)
 };
 template <typename T> cyr_status launch_ebasis_angles(const AnglesArgs<T> &a, int ng, hipStream_t st);
 
@@ -197,12 +197,14 @@ template <typename T> struct MbAnglesArgs {
   uint32_t nA;
   T *proj;                         // [ne][nA][Ny][Nx] (per-angle projections), or
   T *quad;                         // [ne][P][3] in quad_index order: laboratory frame, the intensity's quadratic form
+  double *quad64;                  // the same in FP64 (M = 0)
   Mat3<T> Q;                       // frame e1, e2, k^ (quadratic form)
+  Mat3<double> Q64;
   const double *kmag;              // |k| of the ne energies (mats holds ne x M)
   uint32_t ne;
   uint32_t bx, by, bw, bh;         // quadratic forms: of the pixels [bx, bx + bw) x [by, by + bh)
 };
-// ne energies in one launch: with quad one quadratic form per pixel (laboratory frame),
+// ne energies in one launch: with quad or quad64 one quadratic form per pixel (laboratory frame),
 // else every angle's projection.
 template <typename T> cyr_status launch_mbasis_angles(const MbAnglesArgs<T> &a, int ng, hipStream_t st);
 
@@ -281,7 +283,8 @@ void rotation_orbit_tile_order(uint32_t n, uint32_t *out);
 uint32_t rotation_quarter_turns(uint32_t nx, uint32_t ny, uint32_t nA, uint32_t quarter);
 // Laboratory frame: the same for ne energies from their per-pixel quadratic forms
 // quad[ne][P][3] (quad_index order; I(theta) = c^2 q0 + s^2 q1 + 2 c s q2) with
-// coef[a] = (c^2, s^2, 2 c s) (FP64; coef_t: the same in the compute precision)
+// coef[a] = (c^2, s^2, 2 c s) (FP64; coef_t: the same in the forms' precision T, in which
+// they are sampled and combined; O: the output's)
 // into avg (ne patterns); each angle's taps serve several energies.  quarter (angle
 // steps per 90 degrees, 0 = none) with otiles (orbit tile order) lets each tap
 // cell serve the angles a quarter turn apart.  scratch: room for the sums over an angle's
@@ -298,9 +301,9 @@ struct QuadTurns {
   bool turn = false;   // and those of a + 1 quarter turn are (q1, q0, -q2) of a's
   double rin = 0;      // pixels from the centre within which plane values are finite (a hint)
 };
-template <typename T>
+template <typename T, typename O>
 cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double *coef, const T *coef_t, uint32_t nA,
-                              uint32_t nx, uint32_t ny, int rot_mask, const AvgSink<T> &avg, uint32_t ne,
+                              uint32_t nx, uint32_t ny, int rot_mask, const AvgSink<O> &avg, uint32_t ne,
                               const uint32_t *tiles,
                               uint32_t quarter, const uint32_t *otiles, QuadTurns turns, double rfin, void *scratch,
                               size_t scratch_bytes, hipStream_t st);

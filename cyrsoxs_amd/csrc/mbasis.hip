@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "fft.hpp"
 #include "fftpolicy.hpp"
@@ -485,7 +486,7 @@ __device__ inline void add_basis(int r, const MatConst<T> &mc, const cx<T> &x, c
 // matrices md[q] and the linear weight w1 of bin z0 + 1.
 template <typename T, int NG>
 __device__ inline int mb_fields(const MbAnglesArgs<T> &a, uint32_t X, uint32_t Y, cx<T> (&F)[NG][kEbFields],
-                                double (&md)[NG][6], T &w1) {
+                                double (&md)[NG][6], double &w1) {
   const EwaldGeom &g = a.g;
   const uint64_t P2 = (uint64_t)g.nx * g.ny;
   uint32_t z0 = 0;
@@ -502,7 +503,7 @@ __device__ inline int mb_fields(const MbAnglesArgs<T> &a, uint32_t X, uint32_t Y
   for (int q = 0; q < NG; q++) dc[q] = ix == 0 && iy == 0 && (three ? unshift(z0 + q, g.nz) == 0 : true);
   const uint64_t slab = (uint64_t)a.J * P2;
   const cx<T> *own = a.own + (uint64_t)j0 * P2 + col, *mir = a.mir + (uint64_t)j0 * P2 + col;
-  w1 = (T)f;
+  w1 = f;
   if (a.M == 0) {  // five complex tensor fields, no packing
 #pragma unroll
     for (int q = 0; q < NG; q++)
@@ -585,7 +586,7 @@ __global__ void __launch_bounds__(256) mbasis_angles_kernel(MbAnglesArgs<T> a) {
   const uint32_t Y = (uint32_t)(t / a.g.nx), X = (uint32_t)(t - (uint64_t)Y * a.g.nx);
   cx<T> F[NG][kEbFields];
   double md[NG][6];
-  T w1;
+  double w1;
   if (!mb_fields<T, NG>(a, X, Y, F, md, w1)) {
     for (uint32_t an = 0; an < a.nA; an++) a.proj[(uint64_t)an * P2 + t] = mb_qnan<T>();
     return;
@@ -610,30 +611,31 @@ __global__ void __launch_bounds__(256) mbasis_angles_kernel(MbAnglesArgs<T> a) {
       I[q] = scatter_intensity<T>(md[q], pv);
     }
     T out;
-    if constexpr (NG == 2) out = (1 - w1) * I[0] + w1 * I[1];
+    if constexpr (NG == 2) out = (1 - (T)w1) * I[0] + (T)w1 * I[1];
     else out = I[0];
     a.proj[(uint64_t)an * P2 + t] = out;
   }
 }
 
-// One (pixel, energy): a holds the energy's |k| and constants.
-template <typename T, int NG>
-__device__ inline void quad_pixel_energy(const MbAnglesArgs<T> &a, uint32_t X, uint32_t Y, T *o) {
+// One (pixel, energy): a holds the energy's |k| and constants.  R: the form's precision.
+template <typename T, typename R, int NG>
+__device__ inline void quad_pixel_energy(const MbAnglesArgs<T> &a, uint32_t X, uint32_t Y, R *o) {
   cx<T> F[NG][kEbFields];
   double md[NG][6];
-  T w1;
+  double w1;
   if (!mb_fields<T, NG>(a, X, Y, F, md, w1)) {
-    o[0] = o[1] = o[2] = mb_qnan<T>();
+    o[0] = o[1] = o[2] = mb_qnan<R>();
     return;
   }
-  quad_form_write<T, NG>(a.Q, F, md, w1, o);
+  if constexpr (sizeof(R) == sizeof(T)) quad_form_write<T, T, NG>(a.Q, F, md, (T)w1, o);
+  else quad_form_write<R, T, NG>(a.Q64, F, md, w1, o);
 }
 
 // Only the pixels of a box about the Ewald disc: the rotation samples nothing beyond it
 // (2048^2 film at 1 nm, 50 energies: 267 -> 155 us per 10 energies; 512^2 in FP64: 30 -> 21 us).
 constexpr uint32_t kQuadChunk = 16;  // pixel blocks per XCD chunk of the quadratic-form grids
-template <typename T, int NG>
-__global__ void __launch_bounds__(256) mbasis_quad_kernel(MbAnglesArgs<T> a) {
+template <typename T, typename R, int NG>
+__global__ void __launch_bounds__(256) mbasis_quad_kernel(MbAnglesArgs<T> a, R *quad) {
   const uint64_t P2 = (uint64_t)a.g.nx * a.g.ny;
   // 1D grid in XCD order over (pixel block, energy), energy fastest: the ne
   // energies of a pixel block read the same band columns and run on one XCD
@@ -647,7 +649,7 @@ __global__ void __launch_bounds__(256) mbasis_quad_kernel(MbAnglesArgs<T> a) {
   a.g.k = a.kmag[e];
   a.mats += (uint64_t)e * a.M;
   const uint32_t r = (uint32_t)(t / a.bw), X = a.bx + (uint32_t)(t - (uint64_t)r * a.bw), Y = a.by + r;
-  quad_pixel_energy<T, NG>(a, X, Y, a.quad + ((uint64_t)e * P2 + quad_index(X, Y, a.g.nx, a.g.ny)) * kQuadRecord);
+  quad_pixel_energy<T, R, NG>(a, X, Y, quad + ((uint64_t)e * P2 + quad_index(X, Y, a.g.nx, a.g.ny)) * kQuadRecord);
 }
 
 // Two energies (2 ep, 2 ep + 1) of one pixel per thread.  Neighbouring energies'
@@ -684,8 +686,8 @@ __global__ void __launch_bounds__(256) mbasis_quad2_kernel(MbAnglesArgs<T> a) {
   const bool three = !a.g.enable2d;
   const uint32_t gap = z0[0] > z0[1] ? z0[0] - z0[1] : z0[1] - z0[0];
   if (!kind0 || !kind1 || (ix == 0 && iy == 0) || (three && gap > 1)) {
-    quad_pixel_energy<T, NG>(ak[0], X, Y, o0);
-    if (two) quad_pixel_energy<T, NG>(ak[1], X, Y, o1);
+    quad_pixel_energy<T, T, NG>(ak[0], X, Y, o0);
+    if (two) quad_pixel_energy<T, T, NG>(ak[1], X, Y, o1);
     return;
   }
   const uint64_t col = (uint64_t)iy * a.g.nx + ix;
@@ -762,7 +764,7 @@ __global__ void __launch_bounds__(256) mbasis_quad2_kernel(MbAnglesArgs<T> a) {
       F[k][q][3].y += iso[k][q].y;
       scatter_matrix(ak[k].g, X, Y, three ? z0[k] + q : 0, md[q]);
     }
-    quad_form_write<T, NG>(a.Q, F[k], md, (T)f[k], k ? o1 : o0);
+    quad_form_write<T, T, NG>(a.Q, F[k], md, (T)f[k], k ? o1 : o0);
   }
 }
 
@@ -839,10 +841,10 @@ template <typename T> cyr_status launch_mbasis_angles(const MbAnglesArgs<T> &a, 
   const uint64_t P = (uint64_t)a.g.nx * a.g.ny;
   if (!a.kmag || a.ne == 0 || a.ne > 65535) return fail(CYR_E_INVALID, "material basis: energy table missing");
   const dim3 grid(ceil_div(P, 256), a.ne), block(256);
-  if (a.quad) {
+  if (a.quad || a.quad64) {
     // FP32: energies in pairs (one thread per pixel and pair); FP64 (whose pair
     // kernel would hold 256 registers) and single energies: one at a time
-    const bool paired = a.ne >= 2 && sizeof(T) == 4;
+    const bool paired = a.quad && a.ne >= 2 && sizeof(T) == 4;
     const uint32_t per = paired ? (a.ne + 1) / 2 : a.ne;
     if (!a.bw || !a.bh || (uint64_t)a.bx + a.bw > a.g.nx || (uint64_t)a.by + a.bh > a.g.ny)
       return fail(CYR_E_INVALID, "quadratic form: box outside the plane");
@@ -859,8 +861,13 @@ template <typename T> cyr_status launch_mbasis_angles(const MbAnglesArgs<T> &a, 
       }
     }
     if (!launched) {
-      if (ng == 2) hipLaunchKernelGGL((mbasis_quad_kernel<T, 2>), g2, block, 0, st, a);
-      else hipLaunchKernelGGL((mbasis_quad_kernel<T, 1>), g2, block, 0, st, a);
+      auto one = [&](auto *quad) {
+        using R = std::remove_pointer_t<decltype(quad)>;
+        if (ng == 2) hipLaunchKernelGGL((mbasis_quad_kernel<T, R, 2>), g2, block, 0, st, a, quad);
+        else hipLaunchKernelGGL((mbasis_quad_kernel<T, R, 1>), g2, block, 0, st, a, quad);
+      };
+      if (a.quad64) one(a.quad64);
+      else one(a.quad);
     }
   } else {
     if (ng == 2) hipLaunchKernelGGL((mbasis_angles_kernel<T, 2>), grid, block, 0, st, a);

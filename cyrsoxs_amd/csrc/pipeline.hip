@@ -18,6 +18,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "fft.hpp"
@@ -463,6 +464,17 @@ cyr_status join_lanes(WorkBuffers &wb, uint32_t lanes, hipStream_t st) {
   return CYR_OK;
 }
 
+// E-basis, laboratory frame: FP64 quadratic forms instead of every angle's projection,
+// where they take no more memory (so what fitted fits).
+bool ebasis_forms(const cyr_sim_desc *d, const SimGeometry &g) {
+  return d->reference_frame != 0 &&
+         kQuadRecord * sizeof(double) <= (uint64_t)g.nA * (d->precision == CYR_FP64 ? 8 : 4);
+}
+// Bytes per pixel of either.
+uint64_t ebasis_plane_bytes(const cyr_sim_desc *d, const SimGeometry &g) {
+  return ebasis_forms(d, g) ? kQuadRecord * sizeof(double) : (uint64_t)g.nA * (d->precision == CYR_FP64 ? 8 : 4);
+}
+
 // EBASIS: per (energy, k) unit the five tensor fields, their XY transforms, the
 // z DFT at the Ewald bins, then every angle as 2D work.  With two lanes, unit u
 // runs on stream u % 2 with its own work buffers and starts once unit u-1's
@@ -476,8 +488,7 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
   const int ng = (g.nz > 1 && d->interpolation == 1) ? 2 : 1;
   const uint32_t units = g.nE * g.nK;
   const uint32_t lanes = units > 1 ? std::min(energy_lanes(), wb.max_lanes) : 1;
-  // laboratory frame: one quadratic form per pixel instead of every angle's projection
-  const bool lab = d->reference_frame != 0;
+  const bool forms = ebasis_forms(d, g);
   YzArgs<T> yz{};
   yz.nx = g.nx;
   yz.ny = g.ny;
@@ -486,7 +497,7 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
   for (uint32_t L = 0; L < lanes; L++) {
     LaneBuffers &lb = wb.lane[L];
     CYR_TRY(ensure_buffer(lb.pol, sizeof(cx<T>) * V * kEbFields));
-    CYR_TRY(ensure_buffer(lb.proj, sizeof(T) * P * (lab ? kQuadRecord : g.nA)));
+    CYR_TRY(ensure_buffer(lb.proj, P * ebasis_plane_bytes(d, g)));
     CYR_TRY(ensure_buffer(lb.avg, sizeof(double) * P));
     CYR_TRY(ensure_buffer(lb.bins, sizeof(int32_t) * P));
     CYR_TRY(ensure_buffer(lb.part, sizeof(cx<T>) * P * ng * kEbFields * yz.nchunks));
@@ -504,7 +515,6 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
     int32_t *kzt = reinterpret_cast<int32_t *>(lb.bins.ptr);
     cx<T> *part = reinterpret_cast<cx<T> *>(lb.part.ptr);
     double2 *dcz = reinterpret_cast<double2 *>(lb.dc.ptr);
-    T *proj = reinterpret_cast<T *>(lb.proj.ptr);
     double *avg = reinterpret_cast<double *>(lb.avg.ptr);
     if (lanes > 1 && u > 0) CYR_HIP(hipStreamWaitEvent(s, wb.ev_polx[(u - 1) % lanes], 0));
     const double kv[3] = {g.kvec[k].x, g.kvec[k].y, g.kvec[k].z};
@@ -563,18 +573,20 @@ cyr_status run_ebasis(const cyr_sim_desc *d, const SimGeometry &g, const void *d
     const double rfin = ewald_radius(geo);
     const double *det = &g.det_inv[(size_t)k * 6];
     const AvgSink<T> sink(avg, out, 0, P, det);
-    if (lab) {
-      aa.quad = proj;
-      aa.Q = m3<T>(Q);
+    if (forms) {
+      aa.quad = reinterpret_cast<double *>(lb.proj.ptr);
+      aa.Q = m3<double>(Q);
       kt_begin(s);
       CYR_TRY(launch_ebasis_angles<T>(aa, ng, s));
-      kt_end("ebasis_quad", s, part_bytes + (double)kQuadRecord * P * sizeof(T));
+      kt_end("ebasis_quad", s, part_bytes + 8.0 * kQuadRecord * P);
+      const double *coef = su.quad + (size_t)3 * k * g.nA;
       kt_begin(s);
-      CYR_TRY(launch_rotate_quad<T>(proj, inv, su.quad + (size_t)3 * k * g.nA, su.quad_t + (size_t)3 * k * g.nA, g.nA,
-                                    g.nx, g.ny, d->rot_mask, sink, 1, su.tiles, g.quarter, su.otiles,
-                                    quad_turns<T>(g, k, geo), rfin, pol, sizeof(cx<T>) * V * kEbFields, s));
-      kt_end("rotate_quad", s, (double)kQuadRecord * P * sizeof(T) + 8.0 * P);
+      CYR_TRY((launch_rotate_quad<double, T>(aa.quad, inv, coef, coef, g.nA, g.nx, g.ny, d->rot_mask, sink, 1, su.tiles,
+                                             g.quarter, su.otiles, quad_turns<double>(g, k, geo), rfin, pol,
+                                             sizeof(cx<T>) * V * kEbFields, s)));
+      kt_end("rotate_quad", s, 8.0 * kQuadRecord * P + 8.0 * P);
     } else {
+      T *proj = reinterpret_cast<T *>(lb.proj.ptr);
       aa.proj = proj;
       kt_begin(s);
       CYR_TRY(launch_ebasis_angles<T>(aa, ng, s));
@@ -679,8 +691,8 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
   const uint32_t nvol = tensor ? kEbFields : mbasis_volumes(g.M), pass_max = nvol < 7 ? nvol : 7;
   const uint64_t planes = tensor ? 1 : 2;  // band values: own, and those of the mirrored bins
   // laboratory frame: one quadratic form per pixel instead of every angle's projection
-  const bool lab = d->reference_frame != 0;
-  const uint32_t nb = lab && !tensor ? std::min(mbasis_energy_batch(g, sizeof(T)), g.nE) : 1;
+  const bool forms = tensor ? ebasis_forms(d, g) : d->reference_frame != 0;
+  const uint32_t nb = forms && !tensor ? std::min(mbasis_energy_batch(g, sizeof(T)), g.nE) : 1;
   // units of the tensor fields, like run_ebasis', may be in flight two at a time
   const uint32_t lanes = tensor && g.nE * g.nK > 1 ? std::min(energy_lanes(), wb.max_lanes) : 1;
   // DC-neighbour sums: taken by the Y pass when it runs on a compile-time plan
@@ -690,7 +702,7 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
   for (uint32_t L = 0; L < lanes; L++) {
     LaneBuffers &lb = wb.lane[L];
     CYR_TRY(ensure_buffer(lb.pol, sizeof(cx<T>) * V * pass_max));
-    CYR_TRY(ensure_buffer(lb.proj, sizeof(T) * P * (lab ? 4 * (uint64_t)nb : g.nA)));
+    CYR_TRY(ensure_buffer(lb.proj, tensor ? P * ebasis_plane_bytes(d, g) : sizeof(T) * P * (forms ? 4 * (uint64_t)nb : g.nA)));
     CYR_TRY(ensure_buffer(lb.avg, sizeof(double) * P * nb));
     CYR_TRY(ensure_buffer(lb.bins, sizeof(int32_t) * P + sizeof(uint32_t) * mbasis_bmax_words(g.nx, g.ny)));
     CYR_TRY(ensure_buffer(lb.dc, sizeof(double2) * nvol * (dc_per + 1)));
@@ -844,7 +856,8 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
       aa.amat = su.amat + (size_t)kEbAmat * k * g.nA;
       aa.nA = g.nA;
       aa.Q = m3<T>(Q);
-      if (lab) {
+      aa.Q64 = m3<double>(Q);
+      if (forms) {
         // the pixels the rotation may read: a box about the disc of finite values, its
         // columns from a cache line's first record on
         const double reach = rfin + kQuadMargin + 1.0;
@@ -863,22 +876,28 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
           aa.kmag = su.kmag + b0;
           aa.ne = n;
           aa.mats = su.mats + (size_t)b0 * g.M;
-          aa.quad = proj;
+          if (tensor) aa.quad64 = reinterpret_cast<double *>(proj);
+          else aa.quad = proj;
+          const double rec = kQuadRecord * (tensor ? 8.0 : sizeof(T));
           kt_begin(s);
           CYR_TRY(launch_mbasis_angles<T>(aa, ng, s));
           // unique inputs: the group's band values (own + mirror, each column's band
           // width, shared by its energies) and the band table; outputs: n
           // quadratic-form planes
           const double bp = (double)aa.bw * aa.bh;
-          kt_end("mbasis_quad", s, (double)planes * nvol * (double)wsum * cxb + 4.0 * bp + n * (double)kQuadRecord * bp * sizeof(T));
+          kt_end("mbasis_quad", s, (double)planes * nvol * (double)wsum * cxb + 4.0 * bp + n * rec * bp);
           EwaldGeom gmin = aa.g;  // (the batch's smallest disc)
           for (uint32_t i = 1; i < n; i++) gmin.k = std::min(gmin.k, g.kmag[b0 + i]);
+          auto rotate = [&](auto *quad, const auto *coef_t) {
+            using R = std::remove_pointer_t<decltype(quad)>;
+            return launch_rotate_quad<R, T>(quad, inv, su.quad + (size_t)3 * k * g.nA, coef_t + (size_t)3 * k * g.nA,
+                                            g.nA, g.nx, g.ny, d->rot_mask, AvgSink<T>(avg, out, ostride, P, det), n,
+                                            su.tiles, g.quarter, su.otiles, quad_turns<R>(g, k, gmin), rfin, pol,
+                                            sizeof(cx<T>) * V * pass_max, s);
+          };
           kt_begin(s);
-          CYR_TRY(launch_rotate_quad<T>(proj, inv, su.quad + (size_t)3 * k * g.nA, su.quad_t + (size_t)3 * k * g.nA,
-                                        g.nA, g.nx, g.ny, d->rot_mask, AvgSink<T>(avg, out, ostride, P, det), n,
-                                        su.tiles, g.quarter, su.otiles,
-                                        quad_turns<T>(g, k, gmin), rfin, pol, sizeof(cx<T>) * V * pass_max, s));
-          kt_end("rotate_quad", s, n * ((double)kQuadRecord * P * sizeof(T) + 8.0 * P));
+          CYR_TRY(tensor ? rotate(aa.quad64, su.quad) : rotate(aa.quad, su.quad_t));
+          kt_end("rotate_quad", s, n * (rec * P + 8.0 * P));
           CYR_TRY(launch_detector_warp<T>(avg, out, ostride, n, g.nx, g.ny, det, d->rot_mask, s));
         }
       } else {
@@ -1095,10 +1114,9 @@ uint64_t work_bytes(const cyr_sim_desc *d, const SimGeometry &g) {
   if (pipe == CYR_PIPE_EBASIS && !ebasis_yz_supported(g.nx, g.ny, g.nz, d->precision)) {
     // run_bands over the tensor fields of one energy: volumes, its one or two band
     // rows (a column's own bin and its interpolation partner), tables, DC sums, planes
-    const uint64_t planes = d->reference_frame != 0 ? 4 : g.nA;
     const uint64_t lanes = (uint64_t)g.nE * g.nK > 1 ? energy_lanes() : 1;
     b += lanes * (cs * g.V * kEbFields + cs * 2 * kEbFields * g.P + 4 * g.P + 4 * mbasis_bmax_words(g.nx, g.ny) +
-                  16 * kEbFields * (mbasis_dc_per(d, g) + 1) + rs * g.P * planes + 8 * g.P);
+                  16 * kEbFields * (mbasis_dc_per(d, g) + 1) + g.P * ebasis_plane_bytes(d, g) + 8 * g.P);
   } else if (pipe == CYR_PIPE_MBASIS) {
     // one pass of packed volumes, band values (own + mirror, at most the band cap),
     // band table, DC sums, per-angle projections, average
@@ -1113,7 +1131,7 @@ uint64_t work_bytes(const cyr_sim_desc *d, const SimGeometry &g) {
     const uint64_t nch = ebasis_max_chunks(g.nx, g.ny, g.nz, d->precision);
     const uint64_t lanes = (uint64_t)g.nE * g.nK > 1 ? energy_lanes() : 1;
     b += lanes * (cs * g.V * kEbFields + 4 * g.P + cs * g.P * 2 * kEbFields * nch + 16 * kEbFields * g.nz +
-                  rs * g.P * (d->reference_frame != 0 ? kQuadRecord : g.nA) + 8 * g.P);
+                  g.P * ebasis_plane_bytes(d, g) + 8 * g.P);
   } else {
     b += cs * g.V * 3 + rs * g.P + 8 * g.P * 2 + 4 * g.P;
     if (d->algorithm == 1) b += cs * g.V * 6;

@@ -10,15 +10,17 @@ namespace cyr {
 
 // With E(theta) = c e1 + s e2 the polarization is p = c u + s v, u = Q (F0, F1, F2),
 // v = Q (F1, F3, F4), so I(theta) = c^2 |M u|^2 + s^2 |M v|^2 + 2 c s Re<M u, M v>.
-// quad[pixel] = (|Mu|^2, |Mv|^2, Re<Mu, Mv>), interpolated between the bins.
-template <typename T, int NG>
-__device__ inline void quad_form_write(const Mat3<T> &Q, const cx<T> (&F)[NG][kEbFields], const double (&md)[NG][6],
+// quad[pixel] = (|Mu|^2, |Mv|^2, Re<Mu, Mv>), interpolated between the bins.  T: the forms'
+// precision (fields S).
+template <typename T, typename S, int NG>
+__device__ inline void quad_form_write(const Mat3<T> &Q, const cx<S> (&F)[NG][kEbFields], const double (&md)[NG][6],
                                        T w1, T *o) {
   T qa[NG], qb[NG], qm[NG];
 #pragma unroll
   for (int q = 0; q < NG; q++) {
     cx<T> u[3], v[3], mu[3], mv[3];
-    const cx<T> ue[3] = {F[q][0], F[q][1], F[q][2]}, ve[3] = {F[q][1], F[q][3], F[q][4]};
+    const cx<T> ue[3] = {cx_as<T, S>(F[q][0]), cx_as<T, S>(F[q][1]), cx_as<T, S>(F[q][2])};
+    const cx<T> ve[3] = {ue[1], cx_as<T, S>(F[q][3]), cx_as<T, S>(F[q][4])};
 #pragma unroll
     for (int i = 0; i < 3; i++) {
       u[i] = mk<T>(Q.m[3 * i] * ue[0].x + Q.m[3 * i + 1] * ue[1].x + Q.m[3 * i + 2] * ue[2].x,

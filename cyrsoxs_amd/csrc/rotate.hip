@@ -243,8 +243,8 @@ __device__ inline void quad_add(const QPoint &p, const Rec<T> (&tp)[NE][4], cons
   quad_combine<T, NE>(p.inside, sm, c, rot_mask, acc, cnt);
 }
 
-template <typename T, int NE>
-__device__ inline void quad_store(const AvgSink<T> &avg, uint64_t t, uint32_t e0, uint32_t ne, uint32_t nA,
+template <typename O, int NE>
+__device__ inline void quad_store(const AvgSink<O> &avg, uint64_t t, uint32_t e0, uint32_t ne, uint32_t nA,
                                   int rot_mask, const double (&acc)[NE], const uint32_t (&cnt)[NE]) {
 #pragma unroll
   for (int e = 0; e < NE; e++) {
@@ -269,10 +269,10 @@ __device__ inline void quad_pixel(const T *const (&qp)[NE], const double *__rest
 }
 
 // grid y: groups of NE energies (ne in total)
-template <typename T, int NE>
+template <typename T, typename O, int NE>
 __global__ void __launch_bounds__(256) rotate_quad_kernel(const T *__restrict__ quad, const double *__restrict__ inv_tab,
                                                           const double *__restrict__ coef, uint32_t nA, uint32_t nx,
-                                                          uint32_t ny, int rot_mask, AvgSink<T> avg,
+                                                          uint32_t ny, int rot_mask, AvgSink<O> avg,
                                                           uint32_t ne, const uint32_t *__restrict__ tiles,
                                                           uint32_t ntiles) {
   const uint64_t P = (uint64_t)nx * ny;
@@ -285,7 +285,7 @@ __global__ void __launch_bounds__(256) rotate_quad_kernel(const T *__restrict__ 
   double acc[NE] = {};
   uint32_t cnt[NE] = {};
   quad_pixel<T, NE>(qp, inv_tab, coef, nA, nx, ny, X, Y, rot_mask, acc, cnt);
-  quad_store<T, NE>(avg, (uint64_t)Y * nx + X, e0, ne, nA, rot_mask, acc, cnt);
+  quad_store<O, NE>(avg, (uint64_t)Y * nx + X, e0, ne, nA, rot_mask, acc, cnt);
 }
 
 // The same for planes too small to fill the chip: S waves of a block take S runs of the
@@ -294,12 +294,12 @@ __global__ void __launch_bounds__(256) rotate_quad_kernel(const T *__restrict__ 
 // there are 4 S times as many waves as one tile per block and four energies give:
 // 256^2, one energy, 36 angles: 70 us (quarter-turn orbits, 64 blocks) -> 20 us; 64^2,
 // 3 energies, 6 angles: 32 -> 6.5 us.
-template <typename T, int S>
+template <typename T, typename O, int S>
 __global__ void __launch_bounds__(64 * S) rotate_quad_split_kernel(const T *__restrict__ quad,
                                                                    const double *__restrict__ inv_tab,
                                                                    const double *__restrict__ coef, uint32_t nA,
                                                                    uint32_t nx, uint32_t ny, int rot_mask,
-                                                                   AvgSink<T> avg,
+                                                                   AvgSink<O> avg,
                                                                    const uint32_t *__restrict__ tiles,
                                                                    uint32_t ntiles) {
   __shared__ double sum[S][64];
@@ -328,14 +328,14 @@ __global__ void __launch_bounds__(64 * S) rotate_quad_split_kernel(const T *__re
     acc[0] += sum[i][l];
     cnt[0] += num[i][l];
   }
-  quad_store<T, 1>(avg, (uint64_t)Y * nx + X, e, e + 1, nA, rot_mask, acc, cnt);
+  quad_store<O, 1>(avg, (uint64_t)Y * nx + X, e, e + 1, nA, rot_mask, acc, cnt);
 }
 
 // Tiles of the general order beyond every finite plane value: the averages
 // rotate_quad_kernel would form there (NaN, or 0 with the rotation mask), as in
 // orbit_fill_kernel.  Same tile and pixel layout as tile_pixel.
-template <typename T, int NE>
-__global__ void __launch_bounds__(256) quad_fill_kernel(AvgSink<T> avg, uint32_t nx, uint32_t ny,
+template <typename O, int NE>
+__global__ void __launch_bounds__(256) quad_fill_kernel(AvgSink<O> avg, uint32_t nx, uint32_t ny,
                                                         uint32_t ne, int rot_mask, const uint32_t *__restrict__ tiles,
                                                         uint32_t first) {
   const uint64_t P = (uint64_t)nx * ny;
@@ -405,10 +405,10 @@ constexpr int kRawBufferFlags = 0x00020000;
 // Row 0 (n pixels), column 0 below it (n - 1) and the centre, which are in no orbit: pixel
 // j of them by every angle, a quarter of the angles a wave.  Pixels farther than rcut from
 // the centre sample nothing finite.
-template <typename T, int NE, bool RM, int R>
+template <typename T, typename O, int NE, bool RM, int R>
 __device__ inline void orbit_tail(const T *const (&qp)[NE], const double *__restrict__ inv_tab,
                                   const double *__restrict__ coef, uint32_t nA, uint32_t n, double rcut, uint32_t j,
-                                  uint32_t w, uint32_t l, uint32_t e0, uint32_t ne, AvgSink<T> avg,
+                                  uint32_t w, uint32_t l, uint32_t e0, uint32_t ne, AvgSink<O> avg,
                                   double (&sum)[4][4][NE][64], uint32_t (&num)[R][R][NE][64]) {
   const uint32_t h = n / 2;
   const bool in = j < 2 * n;
@@ -437,7 +437,7 @@ __device__ inline void orbit_tail(const T *const (&qp)[NE], const double *__rest
       acc[e] += sum[i][0][e][l];
       if constexpr (RM) cnt[e] += num[i][0][e][l];
     }
-  quad_store<T, NE>(avg, (uint64_t)Y * n + X, e0, ne, nA, RM, acc, cnt);
+  quad_store<O, NE>(avg, (uint64_t)Y * n + X, e0, ne, nA, RM, acc, cnt);
 }
 
 // A block holds one 8 x 8 quadrant of a tile of orbits; its wave i samples the points of
@@ -446,11 +446,11 @@ __device__ inline void orbit_tail(const T *const (&qp)[NE], const double *__rest
 // 512^2 FP64 film, 10 energies x 72 angles: 128 us for one energy -> 111 us for all ten;
 // 2048^2 film, 10 energies x 180 angles: 1.19 ms, as before).  The waves' sums meet in LDS,
 // added in orbit order.
-template <typename T, int NE, int Q, bool RM>
+template <typename T, typename O, int NE, int Q, bool RM>
 __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__ quad, const double *__restrict__ inv_tab,
                                                            const double *__restrict__ coef,
                                                            const T *__restrict__ coef_t, uint32_t nA, uint32_t A4,
-                                                           uint32_t n, AvgSink<T> avg, uint32_t ne,
+                                                           uint32_t n, AvgSink<O> avg, uint32_t ne,
                                                            const uint32_t *__restrict__ otiles, uint32_t n_otiles,
                                                            double rcut, int share) {
   __shared__ double sum[4][4][NE][64];
@@ -464,7 +464,7 @@ __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__
 #pragma unroll
   for (int e = 0; e < NE; e++) qp[e] = quad + (uint64_t)(e0 + e < ne ? e0 + e : e0) * P * kQuadRecord;
   if (qb >= 4 * n_otiles) {
-    orbit_tail<T, NE, RM>(qp, inv_tab, coef, nA, n, rcut, (qb - 4 * n_otiles) * 64 + l, i, l, e0, ne, avg, sum, num);
+    orbit_tail<T, O, NE, RM>(qp, inv_tab, coef, nA, n, rcut, (qb - 4 * n_otiles) * 64 + l, i, l, e0, ne, avg, sum, num);
     return;
   }
   const uint32_t tt = otiles[qb >> 2];
@@ -614,7 +614,7 @@ __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__
       if constexpr (RM) c[e] += num[j][q][e][l];
     }
   }
-  quad_store<T, NE>(avg, (uint64_t)PYi * n + PXi, e0, ne, nA, RM, a, c);
+  quad_store<O, NE>(avg, (uint64_t)PYi * n + PXi, e0, ne, nA, RM, a, c);
 }
 
 // Full turns (Q = 4): the sum over an angle's four quarter turns first, then the angles.
@@ -669,12 +669,12 @@ __global__ void __launch_bounds__(256) quad_sym_kernel(const T *__restrict__ qua
 // angles each.  Points near a cell edge or the image border, and samples of records that
 // the exact path decides, are replayed pair by pair from the planes themselves, as in
 // rotate_orbit_kernel (the same margins), wave i taking those of orbit pixel i.
-template <typename T, int NE, bool RM>
+template <typename T, typename O, int NE, bool RM>
 __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 5 : 4) rotate_sym_kernel(const T *__restrict__ quad, const T *__restrict__ sym,
                                                          const double *__restrict__ inv_tab,
                                                          const double *__restrict__ coef, const T *__restrict__ coef_t,
                                                          uint32_t nA, uint32_t A4, uint32_t n,
-                                                         AvgSink<T> avg, uint32_t ne,
+                                                         AvgSink<O> avg, uint32_t ne,
                                                          const uint32_t *__restrict__ otiles, uint32_t n_otiles,
                                                          double rcut) {
   __shared__ double sum[4][4][NE][64];
@@ -690,7 +690,7 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 5 : 4) rotate_sym_kernel
   for (int e = 0; e < NE; e++) qp[e] = quad + (uint64_t)(e0 + e < ne ? e0 + e : e0) * P * kQuadRecord;
   if (qb >= 4 * n_otiles) {
     if constexpr (!RM)  // (with the mask rotate_orbit_kernel runs too, and takes them)
-      orbit_tail<T, NE, RM>(qp, inv_tab, coef, nA, n, rcut, (qb - 4 * n_otiles) * 64 + l, i, l, e0, ne, avg, sum, num);
+      orbit_tail<T, O, NE, RM>(qp, inv_tab, coef, nA, n, rcut, (qb - 4 * n_otiles) * 64 + l, i, l, e0, ne, avg, sum, num);
     return;
   }
   const uint32_t tt = otiles[qb >> 2];
@@ -807,15 +807,15 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 5 : 4) rotate_sym_kernel
       ex[e] += sum[w][i][e][l];
       if constexpr (RM) exn[e] += num[w][i][e][l];
     }
-  quad_store<T, NE>(avg, (uint64_t)py(i) * n + px(i), e0, ne, nA, RM, ex, exn);
+  quad_store<O, NE>(avg, (uint64_t)py(i) * n + px(i), e0, ne, nA, RM, ex, exn);
 }
 
 // Orbit tiles beyond every finite plane value (their pixels' taps, within 1.5
 // pixels of points as far from the centre as the pixel, are all NaN): the
 // averages rotate_orbit_kernel would form there, NaN, or 0 with the rotation
 // mask (no valid sample).  Same tile and pixel layout as rotate_orbit_kernel.
-template <typename T, int NE, bool RM>
-__global__ void __launch_bounds__(256) orbit_fill_kernel(AvgSink<T> avg, uint32_t n, uint32_t ne,
+template <typename O, int NE, bool RM>
+__global__ void __launch_bounds__(256) orbit_fill_kernel(AvgSink<O> avg, uint32_t n, uint32_t ne,
                                                          const uint32_t *__restrict__ otiles, uint32_t first) {
   const uint64_t P = (uint64_t)n * n;
   const uint32_t h = n / 2;
@@ -968,30 +968,30 @@ cyr_status launch_rotate_all(const T *proj, const double *inv_tab, uint32_t nA, 
   return CYR_OK;
 }
 
-template <typename T, int NE, bool RM>
+template <typename T, typename O, int NE, bool RM>
 hipError_t launch_orbit_rm(uint32_t Q, dim3 grid, hipStream_t st, const T *quad, const double *inv_tab,
-                           const double *coef, const T *coef_t, uint32_t nA, uint32_t A4, uint32_t n, const AvgSink<T> &avg,
+                           const double *coef, const T *coef_t, uint32_t nA, uint32_t A4, uint32_t n, const AvgSink<O> &avg,
                            uint32_t ne, const uint32_t *otiles, uint32_t n_otiles, double rcut, int share) {
   switch (Q) {
     case 2:
-      hipLaunchKernelGGL((rotate_orbit_kernel<T, NE, 2, RM>), grid, dim3(256), 0, st, quad, inv_tab, coef, coef_t, nA,
+      hipLaunchKernelGGL((rotate_orbit_kernel<T, O, NE, 2, RM>), grid, dim3(256), 0, st, quad, inv_tab, coef, coef_t, nA,
                          A4, n, avg, ne, otiles, n_otiles, rcut, share);
       break;
     case 3:
-      hipLaunchKernelGGL((rotate_orbit_kernel<T, NE, 3, RM>), grid, dim3(256), 0, st, quad, inv_tab, coef, coef_t, nA,
+      hipLaunchKernelGGL((rotate_orbit_kernel<T, O, NE, 3, RM>), grid, dim3(256), 0, st, quad, inv_tab, coef, coef_t, nA,
                          A4, n, avg, ne, otiles, n_otiles, rcut, share);
       break;
     default:
-      hipLaunchKernelGGL((rotate_orbit_kernel<T, NE, 4, RM>), grid, dim3(256), 0, st, quad, inv_tab, coef, coef_t, nA,
+      hipLaunchKernelGGL((rotate_orbit_kernel<T, O, NE, 4, RM>), grid, dim3(256), 0, st, quad, inv_tab, coef, coef_t, nA,
                          A4, n, avg, ne, otiles, n_otiles, rcut, share);
       break;
   }
   return hipGetLastError();
 }
 
-template <typename T>
+template <typename T, typename O>
 cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double *coef, const T *coef_t, uint32_t nA,
-                              uint32_t nx, uint32_t ny, int rot_mask, const AvgSink<T> &avg, uint32_t ne,
+                              uint32_t nx, uint32_t ny, int rot_mask, const AvgSink<O> &avg, uint32_t ne,
                               const uint32_t *tiles,
                               uint32_t quarter, const uint32_t *otiles, QuadTurns turns, double rfin, void *scratch,
                               size_t scratch_bytes, hipStream_t st) {
@@ -1008,14 +1008,14 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
   if ((uint64_t)n_act * 4 * ne < kSplitWaves) {
     const dim3 grid(xcd_grid(4ull * n_act), 1, ne);
     if ((uint64_t)n_act * 16 * ne < kSplitWaves && nA >= 8)
-      hipLaunchKernelGGL((rotate_quad_split_kernel<T, 16>), grid, dim3(1024), 0, st, quad, inv_tab, coef, nA, nx, ny,
+      hipLaunchKernelGGL((rotate_quad_split_kernel<T, O, 16>), grid, dim3(1024), 0, st, quad, inv_tab, coef, nA, nx, ny,
                          rot_mask, avg, tiles, n_act);
     else
-      hipLaunchKernelGGL((rotate_quad_split_kernel<T, 4>), grid, dim3(256), 0, st, quad, inv_tab, coef, nA, nx, ny,
+      hipLaunchKernelGGL((rotate_quad_split_kernel<T, O, 4>), grid, dim3(256), 0, st, quad, inv_tab, coef, nA, nx, ny,
                          rot_mask, avg, tiles, n_act);
     CYR_LAUNCHED();
     if (n_act < ntiles) {
-      hipLaunchKernelGGL((quad_fill_kernel<T, 1>), dim3(ntiles - n_act, 1, ne), dim3(256), 0, st, avg, nx, ny, ne,
+      hipLaunchKernelGGL((quad_fill_kernel<O, 1>), dim3(ntiles - n_act, 1, ne), dim3(256), 0, st, avg, nx, ny, ne,
                          rot_mask, tiles, n_act);
       CYR_LAUNCHED();
     }
@@ -1053,13 +1053,13 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
       for (uint32_t b0 = 0; b0 < ne;) {
         const uint32_t nb = (uint32_t)std::min<uint64_t>(fit, ne - b0);
         const T *qb = quad + (uint64_t)b0 * nx * nx * kQuadRecord;
-        const AvgSink<T> ab = avg.from(b0);
+        const AvgSink<O> ab = avg.from(b0);
         const dim3 gs(tx * tx, nb);
         const dim3 gr(xcd_grid(rot_mask ? 4ull * o_sym : blocks), 1, ceil_div(nb, 2));
         auto run = [&](auto rm) {
           constexpr bool RM = decltype(rm)::value;
           hipLaunchKernelGGL((quad_sym_kernel<T, RM>), gs, dim3(256), 0, st, qb, sym, nx, tx, rskip);
-          hipLaunchKernelGGL((rotate_sym_kernel<T, 2, RM>), gr, dim3(256), 0, st, qb, sym, inv_tab, coef, coef_t, nA,
+          hipLaunchKernelGGL((rotate_sym_kernel<T, O, 2, RM>), gr, dim3(256), 0, st, qb, sym, inv_tab, coef, coef_t, nA,
                              quarter, nx, ab, nb, otiles, o_sym, rcut);
         };
         if (rot_mask) run(std::true_type{});
@@ -1072,16 +1072,16 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
     if (!o_sym || rot_mask) {
       const uint32_t o_n = o_act - o_sym;
       const dim3 grid(xcd_grid(4ull * o_n + ceil_div(2ull * nx, 64)), 1, ceil_div(ne, 2));
-      e = rot_mask ? launch_orbit_rm<T, 2, true>(Q, grid, st, quad, inv_tab, coef, coef_t, nA, quarter, nx, avg, ne,
+      e = rot_mask ? launch_orbit_rm<T, O, 2, true>(Q, grid, st, quad, inv_tab, coef, coef_t, nA, quarter, nx, avg, ne,
                                                   otiles + o_sym, o_n, rcut, turns.share ? 1 : 0)
-                   : launch_orbit_rm<T, 2, false>(Q, grid, st, quad, inv_tab, coef, coef_t, nA, quarter, nx, avg, ne,
+                   : launch_orbit_rm<T, O, 2, false>(Q, grid, st, quad, inv_tab, coef, coef_t, nA, quarter, nx, avg, ne,
                                                    otiles, o_n, rcut, turns.share ? 1 : 0);
       if (e != hipSuccess) return hip_fail(e, "rotate_orbit_kernel", __FILE__, __LINE__);
     }
     if (o_act < n_otiles) {
       const dim3 gf(n_otiles - o_act, 1, ceil_div(ne, 2));
-      if (rot_mask) hipLaunchKernelGGL((orbit_fill_kernel<T, 2, true>), gf, dim3(256), 0, st, avg, nx, ne, otiles, o_act);
-      else hipLaunchKernelGGL((orbit_fill_kernel<T, 2, false>), gf, dim3(256), 0, st, avg, nx, ne, otiles, o_act);
+      if (rot_mask) hipLaunchKernelGGL((orbit_fill_kernel<O, 2, true>), gf, dim3(256), 0, st, avg, nx, ne, otiles, o_act);
+      else hipLaunchKernelGGL((orbit_fill_kernel<O, 2, false>), gf, dim3(256), 0, st, avg, nx, ne, otiles, o_act);
       e = hipGetLastError();
       if (e != hipSuccess) return hip_fail(e, "orbit_fill_kernel", __FILE__, __LINE__);
     }
@@ -1092,18 +1092,18 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
   // set in cache (measured 19% faster there, equal at 512^2).
   const bool one = (uint64_t)nx * ny * kQuadRecord * sizeof(T) > (16ull << 20);
   if (one)
-    hipLaunchKernelGGL((rotate_quad_kernel<T, 1>), dim3(xcd_grid(n_act), 1, ne), dim3(256), 0, st, quad, inv_tab,
+    hipLaunchKernelGGL((rotate_quad_kernel<T, O, 1>), dim3(xcd_grid(n_act), 1, ne), dim3(256), 0, st, quad, inv_tab,
                        coef, nA, nx, ny, rot_mask, avg, ne, tiles, n_act);
   else
-    hipLaunchKernelGGL((rotate_quad_kernel<T, 4>), dim3(xcd_grid(n_act), 1, ceil_div(ne, 4)), dim3(256), 0, st, quad,
+    hipLaunchKernelGGL((rotate_quad_kernel<T, O, 4>), dim3(xcd_grid(n_act), 1, ceil_div(ne, 4)), dim3(256), 0, st, quad,
                        inv_tab, coef, nA, nx, ny, rot_mask, avg, ne, tiles, n_act);
   CYR_LAUNCHED();
   if (n_act < ntiles) {
     if (one)
-      hipLaunchKernelGGL((quad_fill_kernel<T, 1>), dim3(ntiles - n_act, 1, ne), dim3(256), 0, st, avg, nx, ny, ne, rot_mask,
+      hipLaunchKernelGGL((quad_fill_kernel<O, 1>), dim3(ntiles - n_act, 1, ne), dim3(256), 0, st, avg, nx, ny, ne, rot_mask,
                          tiles, n_act);
     else
-      hipLaunchKernelGGL((quad_fill_kernel<T, 4>), dim3(ntiles - n_act, 1, ceil_div(ne, 4)), dim3(256), 0, st, avg, nx, ny,
+      hipLaunchKernelGGL((quad_fill_kernel<O, 4>), dim3(ntiles - n_act, 1, ceil_div(ne, 4)), dim3(256), 0, st, avg, nx, ny,
                          ne, rot_mask, tiles, n_act);
     CYR_LAUNCHED();
   }
@@ -1134,15 +1134,21 @@ cyr_status launch_warp(const T *src, T *dst, uint32_t nx, uint32_t ny, const dou
                                                   const AvgSink<T> &, hipStream_t);                                \
   template cyr_status launch_rotate_all<T>(const T *, const double *, uint32_t, uint32_t, uint32_t, int,           \
                                            const AvgSink<T> &, uint32_t, const uint32_t *, double, hipStream_t);   \
-  template cyr_status launch_rotate_quad<T>(const T *, const double *, const double *, const T *, uint32_t,        \
-                                            uint32_t, uint32_t, int, const AvgSink<T> &, uint32_t,                 \
-                                            const uint32_t *, uint32_t, const uint32_t *, QuadTurns, double,       \
-                                            void *, size_t, hipStream_t);                                          \
   template cyr_status launch_detector_warp<T>(const double *, T *, uint64_t, uint32_t, uint32_t, uint32_t,         \
                                               const double *, int, hipStream_t);                                   \
   template cyr_status launch_warp<T>(const T *, T *, uint32_t, uint32_t, const double *, hipStream_t);
 CYR_INST(float)
 CYR_INST(double)
+#undef CYR_INST
+
+#define CYR_INST(T, O)                                                                                            \
+  template cyr_status launch_rotate_quad<T, O>(const T *, const double *, const double *, const T *, uint32_t,    \
+                                               uint32_t, uint32_t, int, const AvgSink<O> &, uint32_t,             \
+                                               const uint32_t *, uint32_t, const uint32_t *, QuadTurns, double,   \
+                                               void *, size_t, hipStream_t);
+CYR_INST(float, float)
+CYR_INST(double, float)
+CYR_INST(double, double)
 #undef CYR_INST
 
 }  // namespace cyr
