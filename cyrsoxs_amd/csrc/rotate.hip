@@ -625,11 +625,14 @@ __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__
 // and as S(s y) = P S(y), pixel s x takes the same sample with P, s^2 x and s^3 x the
 // values of x and s x: one gather per orbit and angle a < A4, a quarter of those
 // rotate_orbit_kernel makes, from the quadrant u, v in [0, n/2 - 1] about the centre alone
-// (every y turns into it; P where by an odd number of quarter turns).  Bound by its
-// gathers through L1 and its FP64 points: 2048^2 film, 10 energies x 180 angles 1.19 ms by
-// orbits -> 0.40 ms and 24 us for S (a wave replaying all four pixels of its
-// own deferred angles, not one pixel of all: 0.46 ms; 1 or 4 energies a pass, not 2: 0.51,
-// 0.46 ms).
+// (every y turns into it; P where by an odd number of quarter turns).  S is summed in FP64
+// and kept in the forms' precision, rounded once; its samples, their weights and the angles'
+// values are FP64, so in FP32 a pair carries fewer roundings than by orbits (against 64 bits,
+// 512^2 films, 72 angles with the mask: 2.17e-7 where orbits leave 2.20e-7 and FP32 sums and
+// samples 2.19e-7).  Bound by its gathers through L1 and its FP64 points: 2048^2 film, 10
+// energies x 180 angles 1.19 ms by orbits -> 0.48 ms with S (FP32 sums and samples: 0.45 ms;
+// S kept in FP64, 2.17e-7 too: 0.84 ms; a wave replaying all four pixels of its own deferred
+// angles, not one pixel of all, or 1 or 4 energies a pass, not 2: 4 to 11 % slower).
 
 // The quadrant's S of ne planes.  Where a value is not finite the record says what the
 // samples that read it come to: q0 and q1 NaN, no pair there has a value (with the mask:
@@ -645,24 +648,24 @@ __global__ void __launch_bounds__(256) quad_sym_kernel(const T *__restrict__ qua
   T *o = sym + ((uint64_t)blockIdx.y * h * h + quad_index(u, v, h, h)) * kQuadRecord;
   const uint32_t idx[4] = {quad_index(h + u, h + v, n, n), quad_index(h - v, h + u, n, n),
                            quad_index(h - u, h - v, n, n), quad_index(h + v, h - u, n, n)};
-  T r[4][3];
+  double r[4][3];
 #pragma unroll
   for (int i = 0; i < 4; i++)
 #pragma unroll
-    for (int c = 0; c < 3; c++) r[i][c] = q[(uint64_t)idx[i] * kQuadRecord + c];
-  const T nan = (T)__longlong_as_double(0x7ff8000000000000ll);
-  T s0 = (r[0][0] + r[2][0]) + (r[1][1] + r[3][1]), s1 = (r[0][1] + r[2][1]) + (r[1][0] + r[3][0]);
-  const T s2 = (r[0][2] + r[2][2]) - (r[1][2] + r[3][2]);
-  if (!(isfinite(s0) && isfinite(s1) && isfinite(s2))) {
+    for (int c = 0; c < 3; c++) r[i][c] = (double)q[(uint64_t)idx[i] * kQuadRecord + c];
+  const double nan = __longlong_as_double(0x7ff8000000000000ll);
+  double s0 = (r[0][0] + r[2][0]) + (r[1][1] + r[3][1]), s1 = (r[0][1] + r[2][1]) + (r[1][0] + r[3][0]);
+  const double s2 = (r[0][2] + r[2][2]) - (r[1][2] + r[3][2]);
+  if (!(isfinite((T)s0) && isfinite((T)s1) && isfinite((T)s2))) {
     uint32_t bad = 0;
 #pragma unroll
     for (int i = 0; i < 4; i++) bad += isnan(r[i][0]) || isnan(r[i][1]) || isnan(r[i][2]) ? 1 : 0;
     s0 = nan;
-    s1 = bad >= (RM ? 4u : 1u) ? nan : (T)0;
+    s1 = bad >= (RM ? 4u : 1u) ? nan : 0.0;
   }
-  o[0] = s0;
-  o[1] = s1;
-  o[2] = s2;
+  o[0] = (T)s0;
+  o[1] = (T)s1;
+  o[2] = (T)s2;
 }
 
 // A block holds one 8 x 8 quadrant of a tile of orbits; its waves take a quarter of the
@@ -672,7 +675,7 @@ __global__ void __launch_bounds__(256) quad_sym_kernel(const T *__restrict__ qua
 template <typename T, typename O, int NE, bool RM>
 __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 5 : 4) rotate_sym_kernel(const T *__restrict__ quad, const T *__restrict__ sym,
                                                          const double *__restrict__ inv_tab,
-                                                         const double *__restrict__ coef, const T *__restrict__ coef_t,
+                                                         const double *__restrict__ coef,
                                                          uint32_t nA, uint32_t A4, uint32_t n,
                                                          AvgSink<O> avg, uint32_t ne,
                                                          const uint32_t *__restrict__ otiles, uint32_t n_otiles,
@@ -733,7 +736,7 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 5 : 4) rotate_sym_kernel
       const uint32_t x0 = inside ? (uint32_t)fx0 : 0u, y0 = inside ? (uint32_t)fy0 : 0u;
       const uint32_t o00 = quad_index(x0, y0, h, h) * rb, o10 = quad_index(x0 + 1, y0, h, h) * rb;
       const uint32_t o01 = quad_index(x0, y0 + 1, h, h) * rb, o11 = quad_index(x0 + 1, y0 + 1, h, h) * rb;
-      typename Tap3<T>::v t[NE][4];
+      Rec<T> t[NE][4];
 #pragma unroll
       for (int e = 0; e < NE; e++) {
         t[e][0] = tap_load<T>(rs[e], o00);
@@ -741,28 +744,28 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 5 : 4) rotate_sym_kernel
         t[e][2] = tap_load<T>(rs[e], o01);
         t[e][3] = tap_load<T>(rs[e], o11);
       }
-      const T fxT = (T)fx, fyT = (T)fy, gx = (T)1 - fxT, gy = (T)1 - fyT;
-      const T w00 = gx * gy, w10 = fxT * gy, w01 = gx * fyT, w11 = fxT * fyT;
-      T sm[NE][3];
+      const double gx = 1 - fx, gy = 1 - fy;
+      const double w00 = gx * gy, w10 = fx * gy, w01 = gx * fy, w11 = fx * fy;
+      double sm[NE][3];
       bool exact = !safe;
 #pragma unroll
       for (int e = 0; e < NE; e++) {
-        sm[e][0] = w00 * t[e][0].x + w10 * t[e][1].x + w01 * t[e][2].x + w11 * t[e][3].x;
-        sm[e][1] = w00 * t[e][0].y + w10 * t[e][1].y + w01 * t[e][2].y + w11 * t[e][3].y;
-        sm[e][2] = w00 * t[e][0].z + w10 * t[e][1].z + w01 * t[e][2].z + w11 * t[e][3].z;
+        sm[e][0] = w00 * (double)t[e][0].x + w10 * (double)t[e][1].x + w01 * (double)t[e][2].x + w11 * (double)t[e][3].x;
+        sm[e][1] = w00 * (double)t[e][0].y + w10 * (double)t[e][1].y + w01 * (double)t[e][2].y + w11 * (double)t[e][3].y;
+        sm[e][2] = w00 * (double)t[e][0].z + w10 * (double)t[e][1].z + w01 * (double)t[e][2].z + w11 * (double)t[e][3].z;
         exact = exact || (inside && isnan(sm[e][0]) && !isnan(sm[e][1]));
       }
       if (exact) {
         defer |= 1ull << (a - a0);
         continue;
       }
-      const T *c = coef_t + 3 * (uint64_t)a;
-      const T c0 = odd ? c[1] : c[0], c1 = odd ? c[0] : c[1], c2 = odd ? -c[2] : c[2];
+      const double *c = coef + 3 * (uint64_t)a;
+      const double c0 = odd ? c[1] : c[0], c1 = odd ? c[0] : c[1], c2 = odd ? -c[2] : c[2];
       if constexpr (!RM) dead = dead || !inside;
 #pragma unroll
       for (int e = 0; e < NE; e++) {
-        const double v0 = (double)(c0 * sm[e][0] + c1 * sm[e][1] + c2 * sm[e][2]);
-        const double v1 = (double)(c1 * sm[e][0] + c0 * sm[e][1] - c2 * sm[e][2]);
+        const double v0 = c0 * sm[e][0] + c1 * sm[e][1] + c2 * sm[e][2];
+        const double v1 = c1 * sm[e][0] + c0 * sm[e][1] - c2 * sm[e][2];
         if constexpr (RM) {
           const bool ok = inside && !isnan(sm[e][1]);
           acc[0][e] += ok ? v0 : 0.0;
@@ -1050,8 +1053,9 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
       T *sym = reinterpret_cast<T *>(scratch);
       const double rskip = rfin >= 0 ? rfin + kQuadMargin : 4.0 * nx;
       const uint32_t tx = ceil_div(rfin >= 0 ? std::min(h, (uint32_t)rskip + 1) : h, 16);
+      const uint32_t passes = ceil_div(ne, fit), per = ceil_div(ne, passes);  // (alike)
       for (uint32_t b0 = 0; b0 < ne;) {
-        const uint32_t nb = (uint32_t)std::min<uint64_t>(fit, ne - b0);
+        const uint32_t nb = std::min(per, ne - b0);
         const T *qb = quad + (uint64_t)b0 * nx * nx * kQuadRecord;
         const AvgSink<O> ab = avg.from(b0);
         const dim3 gs(tx * tx, nb);
@@ -1059,7 +1063,7 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
         auto run = [&](auto rm) {
           constexpr bool RM = decltype(rm)::value;
           hipLaunchKernelGGL((quad_sym_kernel<T, RM>), gs, dim3(256), 0, st, qb, sym, nx, tx, rskip);
-          hipLaunchKernelGGL((rotate_sym_kernel<T, O, 2, RM>), gr, dim3(256), 0, st, qb, sym, inv_tab, coef, coef_t, nA,
+          hipLaunchKernelGGL((rotate_sym_kernel<T, O, 2, RM>), gr, dim3(256), 0, st, qb, sym, inv_tab, coef, nA,
                              quarter, nx, ab, nb, otiles, o_sym, rcut);
         };
         if (rot_mask) run(std::true_type{});

@@ -33,3 +33,26 @@ def test_cancelling_forms(dims):
     assert sim.num_angles == 11 and sim.resolved_pipeline() == capi.PIPE_EBASIS
     err, same = pattern_rel_l2(capi.simulate(sim, vox, mats), ref)
     assert same and err < 1e-4, (dims, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rot_mask", [0, 1])
+@pytest.mark.parametrize("n", [64, 256])
+def test_whole_turns_of_large_values(n, rot_mask):
+    """Whole turns of FP32 forms whose sum over the quarter turns exceeds FP32's largest value
+    (3.4e38) while each is below it (four Bragg peaks of 2e38, 90 degrees apart): FP32 against
+    FP64, 1e-4 as above."""
+    print(f"large values {n} mask={rot_mask}", flush=True)
+    dims, V = (n, n, 1), n * n
+    a = 2 * np.pi * 8 * np.arange(n) / n
+    vox = np.zeros((1, V, 4))
+    vox[0, :, 3] = (2 + np.cos(a)[:, None] + np.cos(a)[None, :]).reshape(V)
+    mats = np.array([[[1 - 2e-3, 1e-3, 1 - 1e-3, 5e-4]]])
+    kw = dict(interpolation=1, morphology_type=1, rot_mask=rot_mask, pipeline=capi.PIPE_MBASIS)
+    one = capi.simulate(capi.Sim(dims, 1, 1.0, [285.0], (0, 1, 0), precision=capi.FP64, **kw), vox, mats)
+    vox *= np.sqrt(2e38 / np.nanmax(one))
+    args = (dims, 1, 1.0, [285.0], (0.0, 2.0, 358.0))
+    ref = capi.simulate(capi.Sim(*args, precision=capi.FP64, **kw), vox, mats)
+    got = capi.simulate(capi.Sim(*args, **kw), vox, mats).astype(np.float64)
+    err, same = pattern_rel_l2(got / 1e38, ref / 1e38)
+    assert same and err < 1e-4, (n, rot_mask, err)
