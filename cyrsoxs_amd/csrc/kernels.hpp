@@ -197,7 +197,7 @@ template <typename T> struct MbAnglesArgs {
   uint32_t nA;
   T *proj;                         // [ne][nA][Ny][Nx] (per-angle projections), or
   T *quad;                         // [ne][P][3] in quad_index order: laboratory frame, the intensity's quadratic form
-  double *quad64;                  // the same in FP64 (M = 0)
+  double *quad64;                  // the same, formed and kept in FP64
   Mat3<T> Q;                       // frame e1, e2, k^ (quadratic form)
   Mat3<double> Q64;
   const double *kmag;              // |k| of the ne energies (mats holds ne x M)

@@ -483,9 +483,10 @@ __device__ inline void add_basis(int r, const MatConst<T> &mc, const cx<T> &x, c
 
 // ---- per energy: the tensor fields at a pixel's Ewald bins ----------------------
 // Returns 0 for a NaN pixel; else fills F[q] (bin z0 + q), the scattering
-// matrices md[q] and the linear weight w1 of bin z0 + 1.
-template <typename T, int NG>
-__device__ inline int mb_fields(const MbAnglesArgs<T> &a, uint32_t X, uint32_t Y, cx<T> (&F)[NG][kEbFields],
+// matrices md[q] and the linear weight w1 of bin z0 + 1.  C: the precision in which the
+// packed values are separated and combined.
+template <typename T, int NG, typename C = T>
+__device__ inline int mb_fields(const MbAnglesArgs<T> &a, uint32_t X, uint32_t Y, cx<C> (&F)[NG][kEbFields],
                                 double (&md)[NG][6], double &w1) {
   const EwaldGeom &g = a.g;
   const uint64_t P2 = (uint64_t)g.nx * g.ny;
@@ -510,55 +511,58 @@ __device__ inline int mb_fields(const MbAnglesArgs<T> &a, uint32_t X, uint32_t Y
 #pragma unroll
       for (int c = 0; c < kEbFields; c++) {
         const double2 d = a.dcv[c];
-        F[q][c] = dc[q] ? mk<T>((T)d.x, (T)d.y) : own[(uint64_t)c * slab + (uint64_t)q * P2];
+        F[q][c] = dc[q] ? mk<C>((C)d.x, (C)d.y) : cx_as<C, T>(own[(uint64_t)c * slab + (uint64_t)q * P2]);
       }
 #pragma unroll
     for (int q = 0; q < NG; q++) scatter_matrix(g, X, Y, three ? z0 + q : 0, md[q]);
     return kind;
   }
-  auto fetch = [&](uint32_t v, int q, cx<T> &z, cx<T> &zm) {
+  auto fetch = [&](uint32_t v, int q, cx<C> &z, cx<C> &zm) {
     if (dc[q]) {
       const double2 d = a.dcv[v];
-      z = zm = mk<T>((T)d.x, (T)d.y);
+      z = zm = mk<C>((C)d.x, (C)d.y);
     } else {
-      z = own[(uint64_t)v * slab + (uint64_t)q * P2];
-      zm = mir[(uint64_t)v * slab + (uint64_t)q * P2];
+      z = cx_as<C, T>(own[(uint64_t)v * slab + (uint64_t)q * P2]);
+      zm = cx_as<C, T>(mir[(uint64_t)v * slab + (uint64_t)q * P2]);
     }
   };
-  cx<T> iso[NG];
+  cx<C> iso[NG];
+  auto as_c = [](const MatConst<T> &m) {
+    return MatConst<C>{(C)m.ar, (C)m.ai, (C)m.br, (C)m.bi, (C)m.cr, (C)m.ci, (C)m.dr, (C)m.di};
+  };
 #pragma unroll
   for (int q = 0; q < NG; q++) {
-    iso[q] = mk<T>(0, 0);
+    iso[q] = mk<C>(0, 0);
 #pragma unroll
-    for (int c = 0; c < kEbFields; c++) F[q][c] = mk<T>(0, 0);
+    for (int c = 0; c < kEbFields; c++) F[q][c] = mk<C>(0, 0);
   }
   const uint32_t pairs = a.M / 2;
   for (uint32_t p = 0; p < pairs; p++) {
-    const MatConst<T> ma = a.mats[2 * p], mb = a.mats[2 * p + 1];
+    const MatConst<C> ma = as_c(a.mats[2 * p]), mb = as_c(a.mats[2 * p + 1]);
 #pragma unroll
     for (int r = 0; r < 7; r++) {
 #pragma unroll
       for (int q = 0; q < NG; q++) {
-        cx<T> z, zm, xa, xb;
+        cx<C> z, zm, xa, xb;
         fetch(7 * p + r, q, z, zm);
-        unpack<T>(z, zm, xa, xb);
-        add_basis<T>(r, ma, xa, iso[q], F[q]);
-        add_basis<T>(r, mb, xb, iso[q], F[q]);
+        unpack<C>(z, zm, xa, xb);
+        add_basis<C>(r, ma, xa, iso[q], F[q]);
+        add_basis<C>(r, mb, xb, iso[q], F[q]);
       }
     }
   }
   if (a.M & 1) {  // last material alone: (alpha, beta), (q00, q11), (q01, q02), (q12, -)
-    const MatConst<T> mc = a.mats[a.M - 1];
+    const MatConst<C> mc = as_c(a.mats[a.M - 1]);
     const uint32_t vb = 7 * pairs;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
 #pragma unroll
       for (int q = 0; q < NG; q++) {
-        cx<T> z, zm, xa, xb;
+        cx<C> z, zm, xa, xb;
         fetch(vb + r, q, z, zm);
-        unpack<T>(z, zm, xa, xb);
-        add_basis<T>(2 * r, mc, xa, iso[q], F[q]);
-        if (r < 3) add_basis<T>(2 * r + 1, mc, xb, iso[q], F[q]);
+        unpack<C>(z, zm, xa, xb);
+        add_basis<C>(2 * r, mc, xa, iso[q], F[q]);
+        if (r < 3) add_basis<C>(2 * r + 1, mc, xb, iso[q], F[q]);
       }
     }
   }
@@ -620,15 +624,15 @@ __global__ void __launch_bounds__(256) mbasis_angles_kernel(MbAnglesArgs<T> a) {
 // One (pixel, energy): a holds the energy's |k| and constants.  R: the form's precision.
 template <typename T, typename R, int NG>
 __device__ inline void quad_pixel_energy(const MbAnglesArgs<T> &a, uint32_t X, uint32_t Y, R *o) {
-  cx<T> F[NG][kEbFields];
+  cx<R> F[NG][kEbFields];
   double md[NG][6];
   double w1;
-  if (!mb_fields<T, NG>(a, X, Y, F, md, w1)) {
+  if (!mb_fields<T, NG, R>(a, X, Y, F, md, w1)) {
     o[0] = o[1] = o[2] = mb_qnan<R>();
     return;
   }
   if constexpr (sizeof(R) == sizeof(T)) quad_form_write<T, T, NG>(a.Q, F, md, (T)w1, o);
-  else quad_form_write<R, T, NG>(a.Q64, F, md, w1, o);
+  else quad_form_write<R, R, NG>(a.Q64, F, md, w1, o);
 }
 
 // Only the pixels of a box about the Ewald disc: the rotation samples nothing beyond it

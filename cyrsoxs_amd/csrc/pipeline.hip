@@ -675,6 +675,24 @@ uint32_t mbasis_band_cap(const SimGeometry &g) {
   return cap > floor_cap ? cap : floor_cap;
 }
 
+// Laboratory frame of the material basis in FP32: the forms are combined from the band
+// values, kept and sampled in FP64 where there are few of them, so that AUTO, which takes
+// this executor on small grids for time, gives up no precision to the others (against 64
+// bits, rms over eight seeds, FP32 / FP64 / per-angle FFTs: 250^2 film, 26 angles 1.05 /
+// 0.93 / 0.91e-7; 40 x 44 x 12 vector 1.45 / 1.10 / 0.93e-7; 100 x 100 x 20, one angle 1.90 /
+// 1.32 / 1.73e-7).  64^3, 3 energies: 85 us either way; it costs about 0.16 ns a form, and
+// more forms stay FP32: 200 x 240 x 50, 12 energies: 511 against 602 us, where plain is
+// further off (1.8 against 1.2e-7); 2048^2 film, 50 energies: 4.0 against 8.0 ms, where the
+// E-basis is no closer (1.9 against 1.6e-7).  The records take the place of the averages
+// that the detector warp would read: only where it is the identity.
+constexpr uint64_t kForms64 = 1ull << 18;  // pixels x energies
+bool mbasis_forms64(const cyr_sim_desc *d, const SimGeometry &g) {
+  if (d->precision == CYR_FP64 || d->reference_frame == 0 || g.P * g.nE > kForms64) return false;
+  for (uint32_t k = 0; k < g.nK; k++)
+    if (!identity_warp(&g.det_inv[(size_t)k * 6])) return false;
+  return true;
+}
+
 // MBASIS: per (k, energy group) the seven real basis fields of every material
 // (packed two per complex volume), their 3D FFTs, and their values in the band
 // of Ewald bins the group samples (plus the mirrored bins); then per energy the
@@ -692,6 +710,7 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
   const uint64_t planes = tensor ? 1 : 2;  // band values: own, and those of the mirrored bins
   // laboratory frame: one quadratic form per pixel instead of every angle's projection
   const bool forms = tensor ? ebasis_forms(d, g) : d->reference_frame != 0;
+  const bool forms64 = tensor || mbasis_forms64(d, g);  // (of the forms: in FP64)
   const uint32_t nb = forms && !tensor ? std::min(mbasis_energy_batch(g, sizeof(T)), g.nE) : 1;
   // units of the tensor fields, like run_ebasis', may be in flight two at a time
   const uint32_t lanes = tensor && g.nE * g.nK > 1 ? std::min(energy_lanes(), wb.max_lanes) : 1;
@@ -702,8 +721,12 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
   for (uint32_t L = 0; L < lanes; L++) {
     LaneBuffers &lb = wb.lane[L];
     CYR_TRY(ensure_buffer(lb.pol, sizeof(cx<T>) * V * pass_max));
-    CYR_TRY(ensure_buffer(lb.proj, tensor ? P * ebasis_plane_bytes(d, g) : sizeof(T) * P * (forms ? 4 * (uint64_t)nb : g.nA)));
-    CYR_TRY(ensure_buffer(lb.avg, sizeof(double) * P * nb));
+    if (forms64 && !tensor) {
+      CYR_TRY(ensure_buffer(lb.proj, sizeof(double) * kQuadRecord * P * nb));
+    } else {
+      CYR_TRY(ensure_buffer(lb.proj, tensor ? P * ebasis_plane_bytes(d, g) : sizeof(T) * P * (forms ? 4 * (uint64_t)nb : g.nA)));
+      CYR_TRY(ensure_buffer(lb.avg, sizeof(double) * P * nb));
+    }
     CYR_TRY(ensure_buffer(lb.bins, sizeof(int32_t) * P + sizeof(uint32_t) * mbasis_bmax_words(g.nx, g.ny)));
     CYR_TRY(ensure_buffer(lb.dc, sizeof(double2) * nvol * (dc_per + 1)));
     if (tensor) CYR_TRY(ensure_buffer(lb.part, sizeof(cx<T>) * nvol * ng * P));
@@ -876,9 +899,9 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
           aa.kmag = su.kmag + b0;
           aa.ne = n;
           aa.mats = su.mats + (size_t)b0 * g.M;
-          if (tensor) aa.quad64 = reinterpret_cast<double *>(proj);
+          if (forms64) aa.quad64 = reinterpret_cast<double *>(proj);
           else aa.quad = proj;
-          const double rec = kQuadRecord * (tensor ? 8.0 : sizeof(T));
+          const double rec = kQuadRecord * (forms64 ? 8.0 : sizeof(T));
           kt_begin(s);
           CYR_TRY(launch_mbasis_angles<T>(aa, ng, s));
           // unique inputs: the group's band values (own + mirror, each column's band
@@ -896,7 +919,7 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
                                             sizeof(cx<T>) * V * pass_max, s);
           };
           kt_begin(s);
-          CYR_TRY(tensor ? rotate(aa.quad64, su.quad) : rotate(aa.quad, su.quad_t));
+          CYR_TRY(forms64 ? rotate(aa.quad64, su.quad) : rotate(aa.quad, su.quad_t));
           kt_end("rotate_quad", s, n * (rec * P + 8.0 * P));
           CYR_TRY(launch_detector_warp<T>(avg, out, ostride, n, g.nx, g.ny, det, d->rot_mask, s));
         }

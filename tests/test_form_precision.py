@@ -10,11 +10,11 @@ less.  Bar as in every FP32 parity test, 1e-4 of the FP64 oracle.
 import numpy as np
 import pytest
 
-from cyrsoxs_amd import capi
+from cyrsoxs_amd import capi, synthetic
 from oracle import oracle as O
 from tests.helpers import pattern_rel_l2
 
-pytest.importorskip("torch")
+torch = pytest.importorskip("torch")
 
 
 @pytest.mark.gpu
@@ -56,3 +56,38 @@ def test_whole_turns_of_large_values(n, rot_mask):
     got = capi.simulate(capi.Sim(*args, **kw), vox, mats).astype(np.float64)
     err, same = pattern_rel_l2(got / 1e38, ref / 1e38)
     assert same and err < 1e-4, (n, rot_mask, err)
+
+
+def _smooth(shape, seed):
+    f = torch.randn(shape, generator=torch.Generator().manual_seed(seed), dtype=torch.float64)
+    return synthetic.gaussian_filter_periodic(f, 3.0).reshape(-1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims,angles", [((40, 44, 12), (0.0, 10.0, 170.0)), ((100, 100, 20), (0.0, 1.0, 0.0))])
+def test_few_forms_of_the_material_basis(dims, angles):
+    """Small grids in FP32: the material basis, which AUTO takes for time, leaves no more than
+    the per-angle executor.  Both errors (against FP64) are sums of a few roundings at the
+    brightest pixels, about 25 % apart from seed to seed when averaged over eight, so their
+    ratio stays below 1 + sqrt(2) x 0.25 = 1.35 (FP32 combinations and forms: 1.6)."""
+    M, energies, err = 3, [281.0, 284.0, 286.0, 289.0], {}
+    for seed in range(8):
+        nx, ny, nz = dims
+        logits = torch.stack([_smooth((nz, ny, nx), 100 * seed + m) for m in range(M)])
+        logits = (logits - logits.mean(1, keepdim=True)) / logits.std(1, keepdim=True)
+        phi = torch.softmax(logits, 0).numpy()
+        rng = np.random.default_rng(seed)
+        d = rng.normal(size=(M, phi.shape[1], 3))
+        d /= np.linalg.norm(d, axis=-1, keepdims=True)
+        s = rng.uniform(0, 1, size=phi.shape)
+        vox = np.concatenate([d * np.sqrt(phi * s)[..., None], (phi * (1 - s))[..., None]], -1).astype(np.float32)
+        mats = synthetic.lorentzian_constants(energies, M, seed=seed)
+        kw = dict(interpolation=1, morphology_type=1)
+        run = lambda prec, pipe: capi.simulate(capi.Sim(dims, M, 2.0, energies, angles, precision=prec, pipeline=pipe, **kw),
+                                               vox, mats)
+        ref = run(capi.FP64, capi.PIPE_PLAIN)
+        for pipe in (capi.PIPE_PLAIN, capi.PIPE_MBASIS):
+            err.setdefault(pipe, []).append(pattern_rel_l2(run(capi.FP32, pipe), ref)[0])
+    rms = {p: float(np.sqrt(np.mean(np.square(e)))) for p, e in err.items()}
+    print(rms)
+    assert rms[capi.PIPE_MBASIS] < 1.35 * rms[capi.PIPE_PLAIN], rms
