@@ -329,8 +329,23 @@ cyr_status run_plain(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
   uint32_t nb = 1;
   if (!full && wb.max_lanes > 1 && !scratch_arena())
     nb = (uint32_t)std::min<uint64_t>({(64ull << 20) / angle_bytes + 1, (uint64_t)kPolAngles, (uint64_t)g.nA});
-  if (nb > 1 && ensure_buffer(lb.pol, angle_bytes * nb) != CYR_OK) nb = 1;
-  CYR_TRY(ensure_buffer(lb.pol, angle_bytes * nb));
+  auto buffers = [&](uint32_t n) -> cyr_status {
+    CYR_TRY(ensure_buffer(lb.pol, angle_bytes * n));
+    if (alg1) CYR_TRY(ensure_buffer(wb.nt, sizeof(cx<T>) * V * 6));
+    if (full) CYR_TRY(ensure_buffer(wb.scatter, sizeof(T) * V));
+    CYR_TRY(ensure_buffer(lb.proj, sizeof(T) * P * n));
+    CYR_TRY(ensure_buffer(wb.acc, sizeof(double) * P));
+    CYR_TRY(ensure_buffer(wb.count, sizeof(uint32_t) * P));
+    return ensure_buffer(lb.avg, sizeof(double) * P);
+  };
+  cyr_status bs = buffers(nb);
+  if (bs == CYR_E_NOMEM && nb > 1) {  // what fits one angle at a time must fit
+    CYR_HIP(hipStreamSynchronize(st));
+    lb.release();
+    nb = 1;
+    bs = buffers(nb);
+  }
+  CYR_TRY(bs);
   cx<T> *pol = reinterpret_cast<cx<T> *>(lb.pol.ptr);
   cx<T> *vols[3 * kPolAngles];
   void *vptr[3 * kPolAngles];
@@ -338,12 +353,6 @@ cyr_status run_plain(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
     vols[c] = pol + (uint64_t)c * V;
     vptr[c] = vols[c];
   }
-  if (alg1) CYR_TRY(ensure_buffer(wb.nt, sizeof(cx<T>) * V * 6));
-  if (full) CYR_TRY(ensure_buffer(wb.scatter, sizeof(T) * V));
-  CYR_TRY(ensure_buffer(lb.proj, sizeof(T) * P * nb));
-  CYR_TRY(ensure_buffer(wb.acc, sizeof(double) * P));
-  CYR_TRY(ensure_buffer(wb.count, sizeof(uint32_t) * P));
-  CYR_TRY(ensure_buffer(lb.avg, sizeof(double) * P));
   T *proj = reinterpret_cast<T *>(lb.proj.ptr);
   double *acc = reinterpret_cast<double *>(wb.acc.ptr);
   uint32_t *count = reinterpret_cast<uint32_t *>(wb.count.ptr);

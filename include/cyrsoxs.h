@@ -274,7 +274,9 @@ uint32_t cyr_num_angles(double start, double increment, double end);
  * PLAIN; where its buffers exceed a limit, a smaller one may run instead of an
  * error); -1 for an invalid descriptor.  No counterpart in the reference. */
 int32_t cyr_resolved_pipeline(const cyr_sim_desc *desc);
-/* Device bytes a simulation holds while it runs (morphology + work volumes). */
+/* Device bytes a simulation holds while it runs (morphology + work volumes).  The plain
+ * executor of cyr_simulate and cyr_simulate_device takes up to 64 MB more for small grids,
+ * where that fits. */
 uint64_t cyr_footprint_bytes(const cyr_sim_desc *desc);
 /* Frees the library's per-device caches (work buffers, twiddle tables, batch
  * streams, upload staging).  It waits for calls that are using them and returns
