@@ -367,7 +367,7 @@ constexpr int ct_polx_wg(int N, int E) { return N / E <= 64 ? 64 : N / E; }
 // volume; 101 x 94 x 21: 58 -> 37 us).  Lengths with factors 11 and 13 would be
 // Bluestein's in a narrow plan, so those keep the wide one in FP32 (156 x 156 x 64, 4
 // materials: 183 us per volume by Bluestein, 98 so).  Short convolutions: narrow FP64 plans.
-constexpr uint64_t kXSplitThreads = 256 * 512;  // two waves per SIMD
+constexpr uint64_t kXSplitThreads = 256 * 384;  // one and a half waves per SIMD
 inline bool lf_x_shape(uint32_t n, int precision, LfPlan &P, LfShape &s, uint32_t &e) {
   e = precision == CYR_FP64 ? 2 : 4;
   if (lf_precision(n, precision) != precision)
@@ -393,12 +393,15 @@ inline bool ct_usable(uint32_t n, int precision) {
 
 // Blocks over which the any-length outputs are split (each evaluates the voxels again,
 // from L2): all of them when the rows alone leave the chip short of waves, so that the
-// chain of transforms that a block runs one after another is one transform long
-// (101 x 94 x 21, a pair: 120 -> 58 us).  Not for the compile-time plans, whose
-// transforms are short (64^3: 13.7 against 15.2 us), nor for FP64, whose sines cost
-// more than the chain (64^3: 40 against 79 us).
+// chain of transforms that a block runs one after another is one transform long.  A pair of
+// materials, split / not (us), by threads of the rows alone: FP32 32 x 32 x 16 (4k) 8.4 /
+// 21.2, 101 x 94 x 21 (51k) 44.8 / 75.2, 147 x 147 x 16 (87k) 29.7 / 38.7, 200 x 240 x 8
+// (96k) 29.9 / 34.7, 96 x 96 x 48 (111k) 37.1 / 34.7, 1000 x 500 (125k) 47 / 42; FP64, whose
+// sines weigh more, 250 x 250 (31k) 22.5 / 36.3, 50 x 60 x 20 (30k) 20.9 / 29.2, 300 x 271
+// (41k) 27.6 / 38.6, 500 x 500 (125k) 56 / 42, 200 x 240 x 8 (192k) 87 / 61.  Not for the
+// compile-time plans, whose transforms are short (64^3: 13.7 against 15.2 us).
 template <typename T, int MODE> uint32_t x_split(uint64_t blocks, uint32_t threads) {
-  return sizeof(T) == 4 && blocks * threads < kXSplitThreads ? (uint32_t)x_outputs<MODE>() : 1;
+  return blocks * threads < kXSplitThreads ? (uint32_t)x_outputs<MODE>() : 1;
 }
 
 template <typename T, typename S, int E, bool NARROW, int MODE, typename C>
