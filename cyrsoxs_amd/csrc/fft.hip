@@ -293,7 +293,7 @@ __global__ void __launch_bounds__(1024) fft_any_kernel(LfTab<C> tb, AnyShape sh,
     tab = lf_stage_tables<C, true>(tb, after);
     if (!CONTIG && A.span) {
       uint32_t *ls = reinterpret_cast<uint32_t *>(reinterpret_cast<unsigned char *>(after) +
-                                                  lf_lds_tables<C, true>(tb.m, tb.nlast));
+                                                  lf_lds_tables<C>(tb.m, tb.nlast, !tb.blue));
       for (uint32_t i = threadIdx.x; i < tb.n; i += blockDim.x) ls[i] = A.span[i];
       span = ls;
     }
@@ -564,9 +564,9 @@ size_t al64(size_t x) { return (x + 63) & ~(size_t)63; }
 template <typename T> struct LfOffsets {
   size_t tw, chirp, spec, pos, total;  // (the stages come first)
   explicit LfOffsets(const LfPlan &P) {
-    const size_t cs = sizeof(cx<T>) * tw_blocks<T>();  // (FP32: and the residuals)
+    const size_t cs = sizeof(cx<T>);
     tw = al64(sizeof(P.st));
-    chirp = tw + al64(cs * P.m);
+    chirp = tw + al64(cs * tw_len<T>(P.m));
     spec = chirp + (P.blue ? al64(cs * P.n) : 0);
     pos = spec + (P.blue ? al64(cs * P.m) : 0);
     total = pos + al64(sizeof(uint16_t) * P.m);
@@ -578,14 +578,13 @@ template <typename T> std::vector<unsigned char> lf_host(const LfPlan &P) {
   const LfOffsets<T> o(P);
   std::vector<unsigned char> h(o.total, 0);
   std::memcpy(h.data(), P.st, sizeof(P.st));
-  // entry i of a table of n, and its residual
-  auto put = [](cx<T> *t, uint32_t n, uint32_t i, const xcomplex &c) {
-    t[i] = mk<T>((T)c.real(), (T)c.imag());
-    if (tw_blocks<T>() == 2)
-      t[n + i] = mk<T>((T)(c.real() - (long double)t[i].x), (T)(c.imag() - (long double)t[i].y));
-  };
+  auto round = [](const xcomplex &c) { return mk<T>((T)c.real(), (T)c.imag()); };
   cx<T> *tw = reinterpret_cast<cx<T> *>(h.data() + o.tw);
-  for (uint32_t k = 0; k < P.m; k++) put(tw, P.m, k, root_of(k, P.m));
+  for (uint32_t k = 0; k < P.m; k++) {
+    const xcomplex c = root_of(k, P.m);
+    tw[k] = round(c);
+    if (tw_blocks<T>() == 2) tw[P.m + k] = round(c - xcomplex(tw[k].x, tw[k].y));
+  }
   uint16_t *pos = reinterpret_cast<uint16_t *>(h.data() + o.pos);
   for (uint32_t k = 0; k < P.m; k++) {
     uint32_t x = k, at = 0;
@@ -601,12 +600,12 @@ template <typename T> std::vector<unsigned char> lf_host(const LfPlan &P) {
     for (uint32_t k = 0; k < P.m; k++) roots[k] = root_of(k, P.m);
     for (uint32_t k = 0; k < P.n; k++) {
       const xcomplex c = root_of((uint64_t)k * k, 2ull * P.n);  // exp(-i pi k^2 / n)
-      put(ch, P.n, k, c);
+      ch[k] = round(c);
       b[k] = std::conj(c);
       if (k) b[P.m - k] = std::conj(c);
     }
     host_fft(b, roots, 1);
-    for (uint32_t k = 0; k < P.m; k++) put(sp, P.m, pos[k], b[k] / (long double)P.m);
+    for (uint32_t k = 0; k < P.m; k++) sp[pos[k]] = round(b[k] / (long double)P.m);
   }
   return h;
 }
@@ -749,8 +748,8 @@ uint32_t lf_threads(const LfPlan &P, uint32_t unit, uint32_t pencils) {
 // (comp: with the FP32 residuals of compensated products)
 size_t lf_tables_lds(const LfPlan &P, int precision, bool comp) {
   const uint32_t nlast = P.st[P.nst - 1].nb;
-  if (precision == CYR_FP64) return lf_lds_tables<double, true>(P.m, nlast);
-  return comp ? lf_lds_tables<float, true>(P.m, nlast) : lf_lds_tables<float, false>(P.m, nlast);
+  comp = comp && !P.blue;
+  return precision == CYR_FP64 ? lf_lds_tables<double>(P.m, nlast, comp) : lf_lds_tables<float>(P.m, nlast, comp);
 }
 
 // Column tiles: max_cols adjacent pencils where three blocks of them (with room for a

@@ -183,8 +183,8 @@ template <typename T, int N, int E, bool CONTIG, int PP, int... R> struct CtFft 
 };
 
 // Any length (lfft.hpp), rows: slot i of thread t is element t + i tpp (E tpp >= n;
-// the last slots may be empty).  Plain twiddle products but in convolutions.  C: precision of
-// the arithmetic (lf_precision).
+// the last slots may be empty).  Plain twiddle products.  C: precision of the arithmetic
+// (lf_precision).
 template <typename T, int E, bool NARROW, typename C = T> struct LfRowFft {
   static constexpr int kE = E;
   static constexpr bool kCt = false, kNarrow = NARROW;
@@ -204,14 +204,14 @@ template <typename T, int E, bool NARROW, typename C = T> struct LfRowFft {
   template <class OUT>
   __device__ void transform(cx<T> (&v)[E], uint32_t t, uint32_t p, uint32_t pp, cx<C> *lds, OUT out) const {
     const cx<C> *tw = lds + pp * P.pitch;
-    const LfLds<C> tab{tw, P.tb.tw + P.tb.m, reinterpret_cast<const uint16_t *>(tw + P.tb.m)};
+    const LfLds<C> tab{tw, nullptr, reinterpret_cast<const uint16_t *>(tw + P.tb.m)};
     const LfRows ad{P.pitch, P.pad, pp};
 #pragma unroll
     for (int i = 0; i < E; i++)
       if (holds(t, i)) {
         const uint32_t e = in_pos(t, i);
         const cx<C> x = cx_as<C, T>(v[i]);
-        lds[ad.at(p, e)] = P.tb.blue ? cmul_tw<C>(x, P.tb.chirp, P.tb.n, e) : x;
+        lds[ad.at(p, e)] = P.tb.blue ? cmul<C>(x, P.tb.chirp[e]) : x;
       }
     if (P.tb.blue)
       for (uint32_t e = P.tb.n + t; e < P.tb.m; e += P.tpp) lds[ad.at(p, e)] = mk<C>(0, 0);

@@ -57,8 +57,8 @@ struct LfPlan {
 };
 
 // Device tables of one length: W_m^k (k < m); pos[k], the slot of output k (uint16);
-// Bluestein: chirp c_n (n < N) and the chirp's spectrum / m by slot.  In FP32 each of the
-// three is followed by its rounding residuals (cmul_tw).
+// Bluestein: chirp c_n (n < N) and the chirp's spectrum / m by slot.  In FP32 the twiddles
+// are followed by their rounding residuals.
 template <typename T> struct LfTab {
   uint32_t n, m, blue, nst;  // of the plan
   uint32_t nlast;            // butterflies of the last stage: pos[k] below it are used
@@ -70,13 +70,14 @@ template <typename T> struct LfTab {
   const uint16_t *pos;
 };
 
-// The precision of the arithmetic of a length: FP64 for FP32 pencils of fewer than 128 points
-// that need a convolution.  There the direct sum of compensated products is closer than an
-// FP32 convolution, whose intermediate values carry the pencil's mean through every slot:
-// values about an offset, errors 2.0 (23 points), 1.6 (47) and 1.2 (101) times the sum's;
-// from 128 on it is the sum that is further off (211: 0.84, 499: 0.61).  In FP64 the error
-// is the result's own rounding (101 x 94 x 21, 4 energies: 131 -> 158 us).
-constexpr uint32_t kLfShortConvolution = 128;
+// The precision of the arithmetic of a length: FP64 for FP32 pencils of fewer than 208 points
+// that need a convolution.  There the direct sum of compensated products is as close as an
+// FP32 convolution or closer, whose intermediate values carry the pencil's mean through every
+// slot: values about an offset, errors 2.0 (23 points), 1.6 (47), 1.2 (101) and 1.06 (202)
+// times the sum's; from 211 on (0.86) it is the sum that is further off (499: 0.63), with
+// compensated products in the convolution hardly more (0.82, 0.61).  In FP64 the error is
+// the result's own rounding (101 x 94 x 21, 4 energies: 131 -> 153 us).
+constexpr uint32_t kLfShortConvolution = 208;
 int lf_precision(uint32_t n, int precision);
 
 // Plan of a length (false: longer than the tile limit).  lf_tables builds its
@@ -287,21 +288,21 @@ template <typename T> struct LfLds {
   const cx<T> *tw, *lo;  // (lo: FP32 residuals)
   const uint16_t *pos;
 };
-// Twiddle entries a block keeps: with COMP, FP32 residuals too.
-template <typename T, bool COMP> __host__ __device__ constexpr uint32_t lf_lds_twiddles(uint32_t m) {
-  return COMP ? tw_len<T>(m) : m;
+// Twiddle entries a block keeps: with comp (not in convolutions), FP32 residuals too.
+template <typename T> __host__ __device__ constexpr uint32_t lf_lds_twiddles(uint32_t m, bool comp) {
+  return comp ? (uint32_t)tw_len<T>(m) : m;
 }
 // LDS bytes of the tables.
-template <typename T, bool COMP> __host__ __device__ constexpr size_t lf_lds_tables(uint32_t m, uint32_t nlast) {
-  return sizeof(cx<T>) * lf_lds_twiddles<T, COMP>(m) + ((sizeof(uint16_t) * nlast + 15) & ~(size_t)15);
+template <typename T> __host__ __device__ constexpr size_t lf_lds_tables(uint32_t m, uint32_t nlast, bool comp) {
+  return sizeof(cx<T>) * lf_lds_twiddles<T>(m, comp) + ((sizeof(uint16_t) * nlast + 15) & ~(size_t)15);
 }
 // Copies them to `at` (a barrier must follow).
 template <typename T, bool COMP> __device__ inline LfLds<T> lf_stage_tables(const LfTab<T> &P, cx<T> *at) {
-  const uint32_t n = lf_lds_twiddles<T, COMP>(P.m);
+  const uint32_t n = lf_lds_twiddles<T>(P.m, COMP && !P.blue);
   uint16_t *pos = reinterpret_cast<uint16_t *>(at + n);
   for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) at[i] = P.tw[i];
   for (uint32_t i = threadIdx.x; i < P.nlast; i += blockDim.x) pos[i] = P.pos[i];
-  return LfLds<T>{at, (COMP ? at : P.tw) + P.m, pos};
+  return LfLds<T>{at, at + P.m, pos};
 }
 
 // ---- stages -------------------------------------------------------------------------
@@ -314,11 +315,10 @@ enum LfRole : uint32_t {
 };
 
 // Stage S of the block's pencils.
-// FP32: the finest twiddles (those of the first forward stage and of its inverse), the chirp
-// and its spectrum are compensated products, as the finest of the codelets' passes are.  The
-// twiddles' residuals lie in LDS beside them (200 x 240 x 50, 12 energies: 491 us with plain
-// products, 522 with residuals read from L2 ahead of the butterfly, 511 from LDS).  COMP
-// false: only in convolutions, from memory.
+// COMP, FP32: the finest twiddles, those of the first stage, are compensated products, as the
+// finest of the codelets' passes are (not in convolutions).  Their residuals lie in LDS
+// beside them (200 x 240 x 50, 12 energies: 491 us with plain products, 522 with residuals
+// read from L2 ahead of the butterfly, 511 from LDS).
 template <typename T, int R, bool COMP, class AD, class IN, class OUT>
 __device__ inline void lf_stage(const LfTab<T> &P, const LfStage &S, uint32_t role, const LfLds<T> &tab, cx<T> *buf,
                                 const AD &ad, IN &in, OUT &out) {
@@ -347,7 +347,7 @@ __device__ inline void lf_stage(const LfTab<T> &P, const LfStage &S, uint32_t ro
 #pragma unroll
         for (int r = 0; r < R; r++) {
           const uint32_t e = e0 + r * q;
-          const cx<T> c = cmul_tw<T>(v[r], P.chirp, P.n, e < P.n ? e : 0);
+          const cx<T> c = cmul<T>(v[r], P.chirp[e < P.n ? e : 0]);
           v[r] = e < P.n ? c : mk<T>(0, 0);
         }
       }
@@ -357,21 +357,17 @@ __device__ inline void lf_stage(const LfTab<T> &P, const LfStage &S, uint32_t ro
     }
     const uint32_t w = j * S.ts;
     auto twiddle = [&] {
+      if constexpr (COMP && sizeof(T) == 4) {
+        if (S.ts == 1 && !P.blue) {  // (uniform)
+#pragma unroll
+          for (int r = 1; r < R; r++) v[r] = cmul_comp<T>(v[r], tab.tw[r * w], tab.lo[r * w]);
+          return;
+        }
+      }
 #pragma unroll
       for (int r = 1; r < R; r++) v[r] = cmul<T>(v[r], tab.tw[r * w]);
     };
-    const bool comp = sizeof(T) == 4 && S.ts == 1 && (COMP || P.blue);  // (uniform)
-    auto twiddle_comp = [&] {
-      if constexpr (sizeof(T) == 4) {
-        const cx<T> *lo = COMP ? tab.lo : P.tw + P.m;
-#pragma unroll
-        for (int r = 1; r < R; r++) v[r] = cmul_comp<T>(v[r], tab.tw[r * w], lo[r * w]);
-      }
-    };
-    if ((role & kLfInv) && !last) {
-      if (comp) twiddle_comp();
-      else twiddle();
-    }
+    if ((role & kLfInv) && !last) twiddle();
     bfly_any<T, R>(v);
     if constexpr (R <= 10) {
       if (role & kLfMid) {
@@ -379,22 +375,19 @@ __device__ inline void lf_stage(const LfTab<T> &P, const LfStage &S, uint32_t ro
         // forward butterflies give the inverse transform (swapped back at the end)
 #pragma unroll
         for (int r = 0; r < R; r++) {
-          const cx<T> u = cmul_tw<T>(v[r], P.spec, P.m, e0 + r);
+          const cx<T> u = cmul<T>(v[r], P.spec[e0 + r]);
           v[r] = mk<T>(u.y, u.x);
         }
         bfly_any<T, R>(v);
       }
     }
-    if (!(role & kLfInv) && !last) {
-      if (comp) twiddle_comp();
-      else twiddle();
-    }
+    if (!(role & kLfInv) && !last) twiddle();
     if (role & kLfOut) {
       if (role & kLfInv) {
 #pragma unroll
         for (int r = 0; r < R; r++) {
           const uint32_t k = e0 + r * q;
-          if (k < P.n) out(p, k, 0, 0, cmul_tw<T>(mk<T>(v[r].y, v[r].x), P.chirp, P.n, k));
+          if (k < P.n) out(p, k, 0, 0, cmul<T>(mk<T>(v[r].y, v[r].x), P.chirp[k]));
         }
       } else {
 #pragma unroll

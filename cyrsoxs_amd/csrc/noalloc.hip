@@ -22,8 +22,8 @@ namespace cyr {
 namespace {
 
 // The array also holds the any-length transforms' tables, so that they take nothing from
-// the documented size: at most three lengths, each of 16 bytes (FP64 entries, or FP32 ones
-// with their residuals) for the twiddles and the spectrum of a convolution of m points and
+// the documented size: at most three lengths, each of 16 bytes (FP64 entries, or FP32
+// twiddles with their residuals) for the twiddles and the spectrum of a convolution of m points and
 // for the chirp of fewer than m / 2 + 1, 2 bytes of digit reversal a point, and the stages.
 constexpr size_t kTableBytes = 3u * 1024u * 1024u;
 static_assert(3 * (16 * (size_t)(2 * kLfMaxConvolution + kLfMaxConvolution / 2 + 1) + 2 * kLfMaxConvolution + 1024) <=

@@ -1,6 +1,6 @@
 """Rounding errors of single-axis transforms without a codelet, against extended precision.
 
-FP32, sides below 128 that need a convolution: the arithmetic is FP64, so an output's error
+FP32, sides below 208 that need a convolution: the arithmetic is FP64, so an output's error
 is its own rounding, at most 2^-24 = 6e-8 of it, also where the pencil has a large mean.
 FP64: up to eleven steps (2 x 4 stages, three products), each about 0.8 x 2^-53 rms, times
 sqrt(m / n) <= 1.75 for a convolution's longer pencil: sqrt(11) x 0.8 x 1.1e-16 x 1.75 = 5.1e-16,
@@ -31,7 +31,7 @@ def _rel(a, b):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("axis", [0, 1])
-@pytest.mark.parametrize("n", [17, 23, 31, 34, 47, 61, 94, 101, 127])
+@pytest.mark.parametrize("n", [17, 23, 31, 34, 47, 61, 94, 101, 127, 155, 202])
 def test_short_fp32_convolutions(n, axis):
     rng = np.random.default_rng(n)
     x = 1 + 0.1 * rng.normal(size=(n, 600)) + 0.1j * rng.normal(size=(n, 600))
