@@ -723,8 +723,8 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
   const uint32_t nb = forms && !tensor ? std::min(mbasis_energy_batch(g, sizeof(T)), g.nE) : 1;
   // units of the tensor fields, like run_ebasis', may be in flight two at a time
   const uint32_t lanes = tensor && g.nE * g.nK > 1 ? std::min(energy_lanes(), wb.max_lanes) : 1;
-  // DC-neighbour sums: taken by the Y pass when it runs on a compile-time plan
-  // (dc_slots partials per z slice), else by their own kernel (one per slice)
+  // DC-neighbour sums: taken by the Y pass (dc_slots partials per z slice), or, on planes of
+  // two columns, by their own kernel (one per slice)
   const uint32_t dc_slots = fft_dc_slots<T>(g.nx, g.ny);
   const uint64_t dc_per = (uint64_t)g.nz * (dc_slots ? dc_slots : 1);
   for (uint32_t L = 0; L < lanes; L++) {

@@ -630,9 +630,9 @@ __global__ void __launch_bounds__(256) rotate_orbit_kernel(const T *__restrict__
 // values are FP64, so in FP32 a pair carries fewer roundings than by orbits (against 64 bits,
 // 512^2 films, 72 angles with the mask: 2.17e-7 where orbits leave 2.20e-7 and FP32 sums and
 // samples 2.19e-7).  Bound by its gathers through L1 and its FP64 points: 2048^2 film, 10
-// energies x 180 angles 1.19 ms by orbits -> 0.48 ms with S (FP32 sums and samples: 0.45 ms;
-// S kept in FP64, 2.17e-7 too: 0.84 ms; a wave replaying all four pixels of its own deferred
-// angles, not one pixel of all, or 1 or 4 energies a pass, not 2: 4 to 11 % slower).
+// energies x 180 angles 1.19 ms by orbits -> 0.43 ms and 25 us for S (FP32 sums and samples:
+// 0.40 ms; S kept in FP64, 2.17e-7 too: 0.78 ms; a wave replaying all four pixels of its own
+// deferred angles, not one pixel of all, or 1 or 4 energies a pass, not 2: 4 to 11 % slower).
 
 // The quadrant's S of ne planes.  Where a value is not finite the record says what the
 // samples that read it come to: q0 and q1 NaN, no pair there has a value (with the mask:
@@ -1063,8 +1063,12 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
         auto run = [&](auto rm) {
           constexpr bool RM = decltype(rm)::value;
           hipLaunchKernelGGL((quad_sym_kernel<T, RM>), gs, dim3(256), 0, st, qb, sym, nx, tx, rskip);
-          hipLaunchKernelGGL((rotate_sym_kernel<T, O, 2, RM>), gr, dim3(256), 0, st, qb, sym, inv_tab, coef, nA,
-                             quarter, nx, ab, nb, otiles, o_sym, rcut);
+          if (nb == 1)  // (one plane, not gathered twice)
+            hipLaunchKernelGGL((rotate_sym_kernel<T, O, 1, RM>), gr, dim3(256), 0, st, qb, sym, inv_tab, coef, nA,
+                               quarter, nx, ab, nb, otiles, o_sym, rcut);
+          else
+            hipLaunchKernelGGL((rotate_sym_kernel<T, O, 2, RM>), gr, dim3(256), 0, st, qb, sym, inv_tab, coef, nA,
+                               quarter, nx, ab, nb, otiles, o_sym, rcut);
         };
         if (rot_mask) run(std::true_type{});
         else run(std::false_type{});
@@ -1076,10 +1080,15 @@ cyr_status launch_rotate_quad(const T *quad, const double *inv_tab, const double
     if (!o_sym || rot_mask) {
       const uint32_t o_n = o_act - o_sym;
       const dim3 grid(xcd_grid(4ull * o_n + ceil_div(2ull * nx, 64)), 1, ceil_div(ne, 2));
-      e = rot_mask ? launch_orbit_rm<T, O, 2, true>(Q, grid, st, quad, inv_tab, coef, coef_t, nA, quarter, nx, avg, ne,
-                                                  otiles + o_sym, o_n, rcut, turns.share ? 1 : 0)
-                   : launch_orbit_rm<T, O, 2, false>(Q, grid, st, quad, inv_tab, coef, coef_t, nA, quarter, nx, avg, ne,
-                                                   otiles, o_n, rcut, turns.share ? 1 : 0);
+      auto run = [&](auto energies, auto rm) {
+        return launch_orbit_rm<T, O, decltype(energies)::value, decltype(rm)::value>(
+            Q, grid, st, quad, inv_tab, coef, coef_t, nA, quarter, nx, avg, ne, rot_mask ? otiles + o_sym : otiles, o_n,
+            rcut, turns.share ? 1 : 0);
+      };
+      using One = std::integral_constant<int, 1>;
+      using Two = std::integral_constant<int, 2>;
+      e = rot_mask ? (ne == 1 ? run(One{}, std::true_type{}) : run(Two{}, std::true_type{}))
+                   : (ne == 1 ? run(One{}, std::false_type{}) : run(Two{}, std::false_type{}));
       if (e != hipSuccess) return hip_fail(e, "rotate_orbit_kernel", __FILE__, __LINE__);
     }
     if (o_act < n_otiles) {
