@@ -31,7 +31,7 @@
 //   ebasis_quad_kernel   laboratory frame: sums the chunks, applies the DC replacement
 //                        and writes the pixel's quadratic form (quadform.hpp), which
 //                        the rotation evaluates at every angle
-//   ebasis_angles_kernel material frame: for every angle p~ = A(theta) F (A = frame x
+//   ebasis_angles_kernel material frame and short angle lists: for every angle p~ = A(theta) F (A = frame x
 //                        E coefficients, 3 x 5, FP64-built) and the Ewald intensity
 // Grids whose Ny has no compile-time codelet, and most in FP64 (ebasis_yz_supported), take
 // the band passes of mbasis.hip over the five tensor fields instead of ebasis_yz_kernel.
@@ -315,7 +315,7 @@ __global__ void __launch_bounds__(256) ebasis_quad_kernel(AnglesArgs<T> a) {
   else quad_form_write<double, T, NG>(a.Q, F, md, w1, o);
 }
 
-// ---- material frame: every angle's intensity ----------------------------------------
+// ---- material frame, short angle lists: every angle's intensity ----------------------------------------
 template <typename T, int NG>
 __global__ void __launch_bounds__(256) ebasis_angles_kernel(AnglesArgs<T> a) {
   const uint64_t P2 = (uint64_t)a.g.nx * a.g.ny;

@@ -13,7 +13,7 @@
 // at slot pos[kk], the digit reversal, so nothing is reordered.
 //
 // Lengths with a prime factor above 13 (FP64: above 7) run Bluestein's algorithm in
-// the same tile: with c_n = exp(-i pi n^2 / N), X_k = c_k sum_n (x_n c_n) conj(c_(k-n)),
+// the same tile (short ones in FP64 arithmetic, lf_precision): with c_n = exp(-i pi n^2 / N), X_k = c_k sum_n (x_n c_n) conj(c_(k-n)),
 // a circular convolution of length M >= 2N - 1 (M = 2^a 3^b 5^c 7^d).  The forward
 // transform leaves digit-reversed order, the spectrum of the chirp is stored in
 // that order, and the stages run backwards (decimation in time, digit-reversed in,

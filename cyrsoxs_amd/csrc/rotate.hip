@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(256) rotate_all_kernel(const T *__restrict__ p
 // q = (q0, q1, q2): I(theta) = c^2 q0 + s^2 q1 + 2 c s q2.  Bilinear sampling is
 // linear, so the three components are sampled (same taps, weights and validity
 // as bilinear_sample; a tap of zero weight contributes nothing, NaN included)
-// and combined once per angle, in the storage precision (FP64 runs: FP64).  Each
+// and combined once per angle, in the forms' precision.  Each
 // angle's back-mapped point, taps and weights serve NE energies.
 
 // Back-mapped point of one (pixel, angle): validity, top-left tap, fractions.
@@ -189,7 +189,7 @@ template <typename T, int NE>
 __device__ inline void quad_sums(const QPoint &p, const Rec<T> (&tp)[NE][4], T (&sm)[NE][3]) {
   const double gx = 1 - p.fx, gy = 1 - p.fy;
   const double wd[4] = {gx * gy, p.fx * gy, gx * p.fy, p.fx * p.fy};
-  // taps are interpolated in the storage precision (the weights rounded once per
+  // taps are interpolated in the forms' precision (the weights rounded once per
   // angle); which taps count (weight exactly 0 or not) is decided on the FP64
   // weights, and the sum over angles stays FP64
   T w[4];
@@ -368,7 +368,7 @@ __global__ void __launch_bounds__(256) quad_fill_kernel(AvgSink<O> avg, uint32_t
 // its tap cell, validity and nonzero weights, so they reuse its bilinear sums
 // (only the weights' last bits can differ from a pair's own).  Such points take
 // the lean path: no zero-weight tests, taps through 32-bit buffer offsets (the
-// plane is below 2 GiB), the intensity in the compute precision, and one value
+// plane is below 2 GiB), the intensity in the forms' precision, and one value
 // for the pairs q and q + 2 when their coefficients are equal (`share`).  The
 // rest (a point on or near a pixel edge: angles at exact multiples of 90 degrees,
 // or special angles such as 60 degrees on the axes) is recorded per angle in a
