@@ -459,7 +459,8 @@ bool fused_supported(uint32_t nx, uint32_t ny, uint32_t nz, int precision) {
   if (!ct_usable(nx, precision) && !lf_x_shape(nx, precision, P, s, e)) return false;
   const int py = lf_precision(ny, precision);
   if (!ct_usable(ny, precision) && !(lf_plan(ny, py, false, P) && lf_cols_shape(P, py, 16, s))) return false;
-  return nz == 1 || mbasis_zband_supported(nz, precision);
+  // (Nz beyond the band pass: the volumes' Z pass by the direct sum, which needs a pencil in LDS)
+  return (size_t)nz * (precision == CYR_FP64 ? 16 : 8) <= device_max_lds();
 }
 
 uint32_t ebasis_max_chunks(uint32_t nx, uint32_t ny, uint32_t nz, int precision) {

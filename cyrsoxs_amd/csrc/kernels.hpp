@@ -69,8 +69,8 @@ cyr_status launch_igor_shift(cx<T> *vol, uint32_t nx, uint32_t ny, uint32_t nz, 
 // p~ = A F.
 constexpr int kEbFields = 5;
 constexpr int kEbAmat = 3 * kEbFields;
-// True when every side has a transform whose tile fits the fused kernels (other
-// grids run the plain executor).
+// True when the X and Y sides have transforms whose tiles fit the fused kernels and a
+// Z pencil fits in LDS (other grids run the plain executor).
 bool fused_supported(uint32_t nx, uint32_t ny, uint32_t nz, int precision);
 // True when the fused Y / z-bin kernel takes the grid (a compile-time plan for Ny).
 bool ebasis_yz_supported(uint32_t nx, uint32_t ny, uint32_t nz, int precision);
@@ -182,7 +182,8 @@ template <typename T> struct BandArgs {
 };
 template <typename T> cyr_status launch_mbasis_extract(const BandArgs<T> &a, hipStream_t st);
 // Z FFT of the Y-transformed volumes writing only the band values (vol[] is read,
-// not overwritten), 3D; launch_mbasis_extract copies them in 2D.
+// not overwritten), 3D; launch_mbasis_extract copies them in 2D, and behind a Z pass
+// over the volumes for the Nz that the band pass has no tile for.
 bool mbasis_zband_supported(uint32_t nz, int precision);
 template <typename T> cyr_status launch_mbasis_zband(const BandArgs<T> &a, hipStream_t st);
 template <typename T> struct MbAnglesArgs {

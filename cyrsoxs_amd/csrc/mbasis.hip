@@ -14,10 +14,10 @@
 //
 // Launches per (k, energy group): mbasis_bands_kernel (+ a reduction the first time),
 // then per material pass xfields_kernel (pair/single mode) -> Y FFT pass with the
-// DC neighbour sums -> mbasis_zband_kernel (Z FFT writing only band values; in 2D
-// mbasis_extract_kernel), which also forms the DC values; then per batch of energies
-// mbasis_quad_kernel (material frame: mbasis_angles_kernel) and the shared rotation /
-// detector kernels.
+// DC neighbour sums -> mbasis_zband_kernel (Z FFT writing only band values; in 2D, and
+// behind a Z pass where Nz has no tile, mbasis_extract_kernel), which also forms the DC
+// values; then per batch of energies mbasis_quad_kernel (material frame:
+// mbasis_angles_kernel) and the shared rotation / detector kernels.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -251,26 +251,29 @@ template <typename T> __device__ inline void dc_value(const BandArgs<T> &a, uint
   }
 }
 
-// ---- band values of the transformed packed planes (2D) ---------------------------
-// own[v][0][col] = Z_v(col),  mir[v][0][col] = Z_v(-col) for sampled columns.
-// Grid: (columns + 1 block, volume).
+// ---- band values of the transformed packed volumes --------------------------------
+// own[v][j][col] = Z_v(col, kz(Zlo + j)),  mir[v][j][col] = Z_v(-col, -kz(Zlo + j)) for
+// j < width(col): 2D (kz = 0), and 3D where the transformed pencils are written back.
+// Grid: (columns + 1 block, j, volume).
 template <typename T>
 __global__ void __launch_bounds__(256) mbasis_extract_kernel(BandArgs<T> a) {
   const uint64_t P = (uint64_t)a.nx * a.ny;
   const uint64_t col = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t v = blockIdx.y;
+  const uint32_t j = blockIdx.y, v = blockIdx.z;
   if (blockIdx.x == gridDim.x - 1) {  // one block past the columns
     __shared__ double2 part[4];
-    dc_value<T>(a, v, part);
+    if (j == 0) dc_value<T>(a, v, part);
     return;
   }
-  if (col >= P || a.band[col] == 0) return;
+  const uint32_t b = col < P ? (uint32_t)a.band[col] : 0;
+  if (j >= (b >> 16)) return;
+  const uint32_t kz = a.nz > 1 ? unshift((b & 0xffffu) + j, a.nz) : 0, mz = kz ? a.nz - kz : 0;
   const uint32_t iy = (uint32_t)(col / a.nx), ix = (uint32_t)(col - (uint64_t)iy * a.nx);
   const uint32_t mx = ix ? a.nx - ix : 0, my = iy ? a.ny - iy : 0;
   const cx<T> *Z = a.vol[v];
-  const uint64_t o = (uint64_t)(a.vbase + v) * a.J * P + col;
-  a.own[o] = Z[col];
-  if (a.mir) a.mir[o] = Z[(uint64_t)my * a.nx + mx];
+  const uint64_t o = ((uint64_t)(a.vbase + v) * a.J + j) * P + col;
+  a.own[o] = Z[(uint64_t)kz * P + col];
+  if (a.mir) a.mir[o] = Z[(uint64_t)mz * P + (uint64_t)my * a.nx + mx];
 }
 
 // ---- Z FFT fused with the band extraction --------------------------------------
@@ -795,9 +798,9 @@ uint32_t *mbasis_span_table(uint32_t *bmax, uint32_t, uint32_t ny) { return bmax
 
 template <typename T> cyr_status launch_mbasis_extract(const BandArgs<T> &a, hipStream_t st) {
   if (a.count == 0) return CYR_OK;
-  if (a.count > (uint32_t)kXMaxOut || a.J == 0 || a.nz != 1) return fail(CYR_E_INVALID, "band extraction: bad shape");
+  if (a.count > (uint32_t)kXMaxOut || a.J == 0 || a.J > 65535) return fail(CYR_E_INVALID, "band extraction: bad shape");
   const uint64_t P = (uint64_t)a.nx * a.ny;
-  hipLaunchKernelGGL((mbasis_extract_kernel<T>), dim3(ceil_div(P, 256) + 1, a.count), dim3(256), 0, st, a);
+  hipLaunchKernelGGL((mbasis_extract_kernel<T>), dim3(ceil_div(P, 256) + 1, a.J, a.count), dim3(256), 0, st, a);
   CYR_LAUNCHED();
   return CYR_OK;
 }

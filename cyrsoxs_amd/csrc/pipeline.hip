@@ -860,8 +860,14 @@ cyr_status run_bands(const cyr_sim_desc *d, const SimGeometry &g, const void *d_
         ba.dcv = dcv;
         ba.dc_per = dc_per;
         ba.dc_cnt = three ? 6.0 : 4.0;
+        const bool zband = three && mbasis_zband_supported(g.nz, d->precision);
+        if (three && !zband) {
+          kt_begin(s);
+          CYR_TRY(fft_axis<T>(vptr, nv, g.nx, g.ny, g.nz, 2, s));
+          kt_end("fft_z", s, 2.0 * nv * (double)V * cxb);
+        }
         kt_begin(s);
-        if (three) {
+        if (zband) {
           // reads the volumes' columns inside the row spans; writes each column's band
           // values and those of its mirror column (own + mir)
           CYR_TRY(launch_mbasis_zband<T>(ba, s));
